@@ -87,55 +87,58 @@ __global__ __launch_bounds__(256) void k_classify(const u64* __restrict__ coord,
 // 8-texel depth rows share 128-byte lines, are then read through one L2.
 // ---------------------------------------------------------------------------------------
 
-// kList (several z-tiles): the wave's columns are col_list[c0 .. c0+7], the z-tile's columns with
-// leaf nodes in column order, *n_list of them; ncol (at most the leaf node count) bounds the grid.
+// kList: the wave's columns are col_list[c0 .. c0+7], *n_list of them in all (with several z-tiles,
+// the z-tile's columns with leaf nodes in column order; or those that k_leaf_lanes left), and the
+// workgroups stride over the list; ncol (at most the leaf node count) bounds it.
 // Otherwise the wave's columns are c0 .. c0+7 of all ncol.
-template <bool kList>
+template <bool kList, u32 kCols>
 __global__ __launch_bounds__(64 * kLeafWaves) void k_leaf_waves(LeafColumns lc, u32 ncol, u32 nleaf,
                                                                 const float* __restrict__ depth, u32 N, u32 T,
                                                                 const float2* __restrict__ lv3,
                                                                 u32* __restrict__ mask_out, u64* __restrict__ leafm,
-                                                                u32* __restrict__ runhead,
+                                                                u32* __restrict__ runhead, u64* __restrict__ hash_out,
                                                                 u32 unit_chunk,
                                                                 u64* __restrict__ tab, u32 tab_slots,
                                                                 const u32* __restrict__ col_list,
                                                                 const u32* __restrict__ n_list) {
     // Per lane: f_t and the breadth-first index of node `lane` of each of the wave's columns (a lane
     // only ever reads back its own entries, so the arrays need no barrier).
-    __shared__ int s_f[kLeafWaves][kLeafCols][64];
-    __shared__ u32 s_b[kLeafWaves][kLeafCols][64];
+    __shared__ int s_f[kLeafWaves][kCols][64];
+    __shared__ u32 s_b[kLeafWaves][kCols][64];
     // A chunk's changed-node flags (leaf_column): byte j + 1 for node q0 + j, byte 65 a sink.
     __shared__ uint8_t s_chg[kLeafWaves][128];
     // The wave index is uniform across the wave; saying so keeps the column bases in scalar registers.
     const u32 lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // Workgroups are dealt to the XCDs in turn; XCD x takes the contiguous units [x*unit_chunk, ...).
     // A column list fills only its first units, so there consecutive units go to different XCDs.
-    const u32 unit = kList ? blockIdx.x : (blockIdx.x % kXcds) * unit_chunk + blockIdx.x / kXcds;
-    const u32 c0 = (unit * kLeafWaves + wave) * kLeafCols;
+    u32 unit = kList ? blockIdx.x : (blockIdx.x % kXcds) * unit_chunk + blockIdx.x / kXcds;
+    const u32 nvalid = kList ? min(*n_list, ncol) : ncol;  // columns of this launch
+    do {
+    const u32 c0 = (unit * kLeafWaves + wave) * kCols;
+    if (kList && c0 >= nvalid) break;
     // Every load below is unconditional (addresses clamped into range, values masked afterwards), so
     // the compiler counts them exactly and waits only for what each step uses.
-    const u32 nvalid = kList ? min(*n_list, ncol) : ncol;  // columns of this launch
     const u32 clast = kList ? (nvalid ? nvalid - 1 : 0u) : ncol - 1;
-    // lane k < kLeafCols: column c0 + k of the launch (list entries past nvalid are never read)
-    const u32 my_slot = min(c0 + (lane & (kLeafCols - 1)), clast);
+    // lane k < kCols: column c0 + k of the launch (list entries past nvalid are never read)
+    const u32 my_slot = min(c0 + (lane & (kCols - 1)), clast);
     const u32 my_col = kList ? (nvalid ? col_list[my_slot] : 0u) : my_slot;
     uint4 ci = lc.info[my_col];
-    if (lane >= kLeafCols || c0 + lane >= nvalid) ci = make_uint4(0u, 0u, 0u, 0u);
+    if (lane >= kCols || c0 + lane >= nvalid) ci = make_uint4(0u, 0u, 0u, 0u);
     // Addresses are a wave-uniform base (the column's block, its run of indices) plus a per-lane
     // offset computed once, so every load takes its address from scalar registers and one vector
     // offset, with no per-column vector arithmetic.
     // Byte offset of texel (lane & 7, lane >> 3) of a column's block: below 2^32 (N <= 2^21), so a
     // load takes it as its 32-bit vector offset from the block's scalar base.
     const u32 loff = 4u * ((lane >> 3) * N + (lane & 7));
-    float d[kLeafCols];
+    float d[kCols];
     // Without a list, a wave's columns are c0 .. c0+7 of one row of level-3 texels when the row
     // holds a multiple of 8 columns: their blocks are 32 bytes apart, one base and immediate offsets.
-    const bool row_run = !kList && lc.w3 >= kLeafCols && c0 + kLeafCols <= ncol;
+    const bool row_run = !kList && lc.w3 >= kCols && c0 + kCols <= ncol;
     if (row_run) {
         const u32 x3 = c0 & (lc.w3 - 1), y3 = c0 >> lc.w3_shift;
         const char* blk = reinterpret_cast<const char*>(depth + ((size_t)(8 * y3) * N + 8 * x3)) + loff;
 #pragma unroll
-        for (u32 k = 0; k < kLeafCols; ++k) {
+        for (u32 k = 0; k < kCols; ++k) {
             const float* p = reinterpret_cast<const float*>(blk + 32 * k);
             if (T > 1) {
                 d[k] = 0.0f;
@@ -149,7 +152,7 @@ __global__ __launch_bounds__(64 * kLeafWaves) void k_leaf_waves(LeafColumns lc, 
         // values are never used.  With one z-tile every column has nodes, and the check would only
         // cost issue slots.
 #pragma unroll
-        for (u32 k = 0; k < kLeafCols; ++k) {
+        for (u32 k = 0; k < kCols; ++k) {
             const u32 c = kList ? __builtin_amdgcn_readlane(my_col, k) : min(c0 + k, clast);
             const u32 x3 = c & (lc.w3 - 1), y3 = c >> lc.w3_shift;
             const float* blk = depth + ((size_t)(8 * y3) * N + 8 * x3);
@@ -158,7 +161,7 @@ __global__ __launch_bounds__(64 * kLeafWaves) void k_leaf_waves(LeafColumns lc, 
         }
     } else {
 #pragma unroll
-        for (u32 k = 0; k < kLeafCols; ++k) {
+        for (u32 k = 0; k < kCols; ++k) {
             const u32 c = kList ? __builtin_amdgcn_readlane(my_col, k) : min(c0 + k, clast);
             const u32 x3 = c & (lc.w3 - 1), y3 = c >> lc.w3_shift;
             const float* blk = depth + ((size_t)(8 * y3) * N + 8 * x3);
@@ -166,23 +169,23 @@ __global__ __launch_bounds__(64 * kLeafWaves) void k_leaf_waves(LeafColumns lc, 
             d[k] = __builtin_nontemporal_load(reinterpret_cast<const float*>(reinterpret_cast<const char*>(blk) + loff));
         }
     }
-    u32 b[kLeafCols];
+    u32 b[kCols];
 #pragma unroll
-    for (u32 k = 0; k < kLeafCols; ++k) {
+    for (u32 k = 0; k < kCols; ++k) {
         const u32 cnt = __builtin_amdgcn_readlane(ci.x, k), st = __builtin_amdgcn_readlane(ci.y, k);
         const u32* run = lc.bfs + (cnt ? st : 0u);  // st + lane < nleaf for lane < cnt: the counts sum to it
         b[k] = run[(lane < cnt) ? lane : 0u];
     }
     const float HT = (float)(N * T);
     // The columns' minimum and maximum f from their level-3 pyramid texels (the 8x8 blocks' depth
-    // minimum and maximum): lane k < kLeafCols holds column k's, lane k + kLeafCols its maximum.
+    // minimum and maximum): lane k < kCols holds column k's, lane k + kCols its maximum.
     // A block holding a NaN takes them from its texels instead (the pyramid keeps a NaN only as a
     // first operand, so its extremes do not tell).
     const float2 ext = lv3[my_col];
-    const int fext = leaf_f(((lane & kLeafCols) ? ext.y : ext.x) * HT);
+    const int fext = leaf_f(((lane & kCols) ? ext.y : ext.x) * HT);
     u32 nan_cols = 0;
 #pragma unroll
-    for (u32 k = 0; k < kLeafCols; ++k) {
+    for (u32 k = 0; k < kCols; ++k) {
         const float D = d[k] * HT;
         if (__ballot(!(D == D))) nan_cols |= 1u << k;
         s_f[wave][k][lane] = leaf_f(D);
@@ -196,17 +199,81 @@ __global__ __launch_bounds__(64 * kLeafWaves) void k_leaf_waves(LeafColumns lc, 
         const u32 base = __builtin_amdgcn_readlane(ci.y, k);
         const int zs = (int)__builtin_amdgcn_readlane(ci.z, k);
         const int f = s_f[wave][k][lane];
-        int fmin = __builtin_amdgcn_readlane(fext, k), fmax = __builtin_amdgcn_readlane(fext, k + kLeafCols);
+        int fmin = __builtin_amdgcn_readlane(fext, k), fmax = __builtin_amdgcn_readlane(fext, k + kCols);
         if ((nan_cols >> k) & 1u) {
             fmin = __ockl_wfred_min_i32(f);
             fmax = __ockl_wfred_max_i32(f);
         }
         // (with one wave per workgroup its flags sit at a constant LDS address)
         leaf_column(f, fmin, fmax, zs, cnt, s_b[wave][k][lane], lc.bfs + base, 0u, nleaf,
-                    kLeafWaves == 1 ? s_chg[0] : s_chg[wave], lane, mask_out, leafm, runhead);
+                    kLeafWaves == 1 ? s_chg[0] : s_chg[wave], lane, mask_out, leafm, runhead, hash_out);
     }
+    unit += gridDim.x;
+    } while (kList);
     // The leaf level's merge table is cleared here, after all the work (stores issued earlier
     // would be waited for with the loads): this kernel leaves HBM bandwidth to spare.
+    clear_table(tab, tab_slots);
+}
+
+// The same with one column per lane (leaf_lane), for launches with enough columns to fill the chip
+// that way: a workgroup takes 16 x 16 columns, each of its waves 8 x 8 (whose nodes lie close together
+// in breadth-first order), or 256 columns of the list.
+template <bool kList>
+struct MapCols {
+    LeafColumns lc;
+    const float* depth;
+    u32 N;
+    float HT;
+    const u32* list;
+    u32 nlist, first, tx, ty;
+    __device__ void operator()(u32 slot, LeafCol& c) const {
+        u32 x, y;
+        uint4 ci = make_uint4(0u, 0u, 0u, 0u);
+        if (kList) {
+            const bool in = first + slot < nlist;
+            const u32 col = in ? list[first + slot] : 0u;
+            x = col & (lc.w3 - 1);
+            y = col >> lc.w3_shift;
+            if (in) ci = lc.info[col];
+        } else {
+            x = 16 * tx + 8 * ((slot >> 6) & 1u) + (slot & 7u);
+            y = 16 * ty + 8 * (slot >> 7) + ((slot >> 3) & 7u);
+            ci = lc.info[(y << lc.w3_shift) + x];
+        }
+        c.col = (y << lc.w3_shift) + x;
+        c.blk = depth + ((size_t)(8 * y) * N + 8 * x);
+        c.pitch = N;
+        c.HT = HT;
+        c.cnt = ci.x;
+        c.start = ci.y;
+        c.zs = (int)ci.z;
+        c.gtag = 0;
+    }
+};
+
+// Even bits of v, packed.
+__device__ inline u32 even_bits(u32 v) {
+    v &= 0x55555555u;
+    v = (v | (v >> 1)) & 0x33333333u;
+    v = (v | (v >> 2)) & 0x0F0F0F0Fu;
+    v = (v | (v >> 4)) & 0x00FF00FFu;
+    return (v | (v >> 8)) & 0xFFFFu;
+}
+
+template <bool kList>
+__global__ __launch_bounds__(kLaneThreads) void k_leaf_lanes(LeafColumns lc, u32 ncol, const float* __restrict__ depth, u32 N,
+                                                             u32 T, LeafOut o, u32 unit_chunk, u64* __restrict__ tab,
+                                                             u32 tab_slots, const u32* __restrict__ col_list,
+                                                             const u32* __restrict__ n_list) {
+    // Tiles of a map in Morton order, a contiguous range of them per XCD; a list's in turn.
+    const u32 unit = kList ? blockIdx.x : (blockIdx.x % kXcds) * unit_chunk + blockIdx.x / kXcds;
+    MapCols<kList> cols{lc, depth, N, (float)(N * T), col_list, 0u, unit * kLaneThreads, even_bits(unit), even_bits(unit >> 1)};
+    if (kList) cols.nlist = min(*n_list, ncol);
+    if (unit * kLaneThreads < (kList ? cols.nlist : ncol)) {
+        LeafCol c;
+        cols(threadIdx.x, c);
+        leaf_lanes(c, o);
+    }
     clear_table(tab, tab_slots);
 }
 
@@ -227,7 +294,8 @@ __global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 
 }
 
 __global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
-                                                                    const u32* __restrict__ runhead, u32 n,
+                                                                    const u32* __restrict__ runhead,
+                                                                    const u64* __restrict__ hash, u32 n,
                                                                     u64* __restrict__ tab, u32 S, u32* __restrict__ tslot,
                                                                     u32* __restrict__ full, u64* __restrict__ zero,
                                                                     u32 nzero, u32 hbits) {
@@ -248,21 +316,27 @@ __global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* _
         const u32 i = i0 + k * kLeafInsertThreads;
         rh[k] = (i < n) ? runhead[i] : kNoRep;
     }
-    // The key hash of each run's first node (the run's smallest index), from its mask and
-    // leafmasks (its row at its own index): computed here, lane-parallel, rather than wave-uniform
-    // in the leaf kernel.
-    u32 hm[kLeafPer];
-#pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        hm[k] = (rh[k] == i) ? mask[i] : 0u;
-    }
+    // The key hash of each run's first node (the run's smallest index): from the leaf kernel where
+    // a lane walked its column, else from its mask and leafmasks (its row at its own index).
     u64 h[kLeafPer];
 #pragma unroll
     for (u32 k = 0; k < kLeafPer; ++k) {
         const u32 i = i0 + k * kLeafInsertThreads;
-        h[k] = (rh[k] == i) ? weaken_hash(leaf_key_hash(hm[k], leafm + (size_t)i * 8), hbits) : 0ull;
-        if (h[k] == 0ull && rh[k] == i) h[k] = 1ull;
+        h[k] = (hash && rh[k] == i) ? hash[i] : 0ull;
+    }
+    u32 hm[kLeafPer];
+#pragma unroll
+    for (u32 k = 0; k < kLeafPer; ++k) {
+        const u32 i = i0 + k * kLeafInsertThreads;
+        hm[k] = (rh[k] == i && h[k] == 0ull) ? mask[i] : 0u;
+    }
+#pragma unroll
+    for (u32 k = 0; k < kLeafPer; ++k) {
+        const u32 i = i0 + k * kLeafInsertThreads;
+        if (rh[k] != i) continue;
+        if (h[k] == 0ull) h[k] = leaf_key_hash(hm[k], leafm + (size_t)i * 8);
+        h[k] = weaken_hash(h[k], hbits);
+        if (h[k] == 0ull) h[k] = 1ull;
     }
     __syncthreads();
     u32 ls[kLeafPer];
@@ -935,6 +1009,10 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         lv[L].off = A.take<u32>(c);
     }
     u64* leafm = leaf ? A.take<u64>(c2 * 8) : nullptr;
+    // The run heads' key hashes, from the leaf kernel to the leaf insert, in the place of the leaf
+    // level's unique list and offsets (two arrays side by side), which the ranks scan writes later.
+    const bool lane_leaf = leaf && (col_list ? std::min<u64>(ncol, cnt[2]) : ncol) >= kLaneLeafMin;
+    u64* leaf_hash = lane_leaf ? reinterpret_cast<u64*>(lv[2].uniq) : nullptr;
     u32* runhead = leaf ? A.take<u32>(c2) : nullptr;
     u32* colbfs = leaf ? A.take<u32>(c2) : nullptr;
     u32* clist = col_list ? A.take<u32>(ncol) : nullptr;
@@ -1008,13 +1086,29 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
             const u32 unit_chunk = ceil_div<u32>(units, kXcds);
             const u32 slots = use_table ? leaf_table_slots(c, small_leaf) : 0u;
             // The leaf level is the first merged: its table is cleared by this kernel.
-            if (col_list)
-                CPVS_LAUNCH("leaf_waves", k_leaf_waves<true>, dim3(unit_chunk * kXcds), dim3(64 * kLeafWaves), 0, s, lc,
-                            bound, c, p->depth, N, T, p->lv[3], lv[2].mask, leafm, runhead, unit_chunk, tab,
+            if (lane_leaf) {
+                // (the list of slow columns lies where the representatives are written later)
+                const LeafOut lo{colbfs, lv[2].mask, leafm, runhead, leaf_hash, rep, meta + kMetaSlow, c};
+                const u32 tiles = ceil_div<u32>(bound, kLaneThreads);
+                const u32 chunk = ceil_div<u32>(tiles, kXcds);
+                if (col_list)
+                    CPVS_LAUNCH("leaf_lanes", k_leaf_lanes<true>, dim3(tiles), dim3(kLaneThreads), 0, s, lc, bound, p->depth,
+                                N, T, lo, chunk, tab, slots, clist, nclist);
+                else
+                    CPVS_LAUNCH("leaf_lanes", k_leaf_lanes<false>, dim3(chunk * kXcds), dim3(kLaneThreads), 0, s, lc, bound,
+                                p->depth, N, T, lo, chunk, tab, slots, nullptr, nullptr);
+                const u32 sbound = std::min(bound, c);
+                CPVS_LAUNCH("leaf_waves", (k_leaf_waves<true, kSlowCols>),
+                            dim3(std::min(ceil_div<u32>(sbound, kLeafWaves * kSlowCols), kSlowWaves / kLeafWaves)),
+                            dim3(64 * kLeafWaves), 0, s, lc, sbound, c, p->depth, N, T, p->lv[3], lv[2].mask, leafm, runhead,
+                            leaf_hash, 0u, tab, 0u, rep, meta + kMetaSlow);
+            } else if (col_list)
+                CPVS_LAUNCH("leaf_waves", (k_leaf_waves<true, kLeafCols>), dim3(unit_chunk * kXcds), dim3(64 * kLeafWaves), 0, s, lc,
+                            bound, c, p->depth, N, T, p->lv[3], lv[2].mask, leafm, runhead, nullptr, unit_chunk, tab,
                             slots, clist, nclist);
             else
-                CPVS_LAUNCH("leaf_waves", k_leaf_waves<false>, dim3(unit_chunk * kXcds), dim3(64 * kLeafWaves), 0, s, lc,
-                            bound, c, p->depth, N, T, p->lv[3], lv[2].mask, leafm, runhead, unit_chunk, tab,
+                CPVS_LAUNCH("leaf_waves", (k_leaf_waves<false, kLeafCols>), dim3(unit_chunk * kXcds), dim3(64 * kLeafWaves), 0, s, lc,
+                            bound, c, p->depth, N, T, p->lv[3], lv[2].mask, leafm, runhead, nullptr, unit_chunk, tab,
                             slots, nullptr, nullptr);
             break;
         }
@@ -1069,7 +1163,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
             if (L == deepest && !is_leaf) CPVS_LAUNCH("table_clear", k_table_clear, grid1d(Sl), dim3(256), 0, s, tab, Sl);
             if (is_leaf) {
                 CPVS_LAUNCH("insert_leaf", k_insert_leaf, dim3(ceil_div<u32>(c, kLeafWindow)), dim3(kLeafInsertThreads), 0, s,
-                            lv[2].mask, leafm, runhead, c, tab, Sl, tslot, meta + kMetaFull, rpart, nzero,
+                            lv[2].mask, leafm, runhead, leaf_hash, c, tab, Sl, tslot, meta + kMetaFull, rpart, nzero,
                             ctx->leaf_hash_bits.load());
                 CPVS_LAUNCH("resolve", k_resolve<LeafEq>, grid1d(c, kNodeThreads), dim3(kNodeThreads), 0, s, tslot, tab, runhead, c,
                             LeafEq{lv[2].mask, leafm, nullptr, c}, rep, meta + kMetaColl, lv[2].mask, 1u, rpart, rrounds);

@@ -257,7 +257,8 @@ __device__ inline u32 write_lane(u32 old, u32 v, u32 l) {
 // breadth-first index of node lane (the first 64 nodes), bfs_run[q] that of node q.  Writes each
 // node's run head (the breadth-first index of its run's first node), and for every run head its
 // mask (with gtag, a forest's DAG index, in the upper half) and the leafmasks of its partial slices
-// in the row at its own index (8 slots per node).  fl: the wave's 128 bytes of LDS flags.
+// in the row at its own index (8 slots per node); hash_out (may be null) gets 0 for each head.
+// fl: the wave's 128 bytes of LDS flags.
 //
 // Node q differs from node q-1 iff some texel's h = f + 8 - 8*zs has h - 8q in [0, 14]: q =
 // floor(h/8), or floor(h/8) - 1 when h mod 8 != 7.  Each lane flags its (at most two) nodes in LDS,
@@ -266,7 +267,7 @@ __device__ inline u32 write_lane(u32 old, u32 v, u32 l) {
 // between them; the fences keep the compiler from moving them across one another.
 __device__ inline void leaf_column(int f, int fmin, int fmax, int zs, u32 cnt, u32 first_bfs, const u32* bfs_run,
                                    u32 gtag, u32 nleaf, uint8_t* fl, u32 lane, u32* __restrict__ mask_out,
-                                   u64* __restrict__ leafm, u32* __restrict__ runhead) {
+                                   u64* __restrict__ leafm, u32* __restrict__ runhead, u64* __restrict__ hash_out) {
     const int h = f + 8 - 8 * zs;
     const int qa = h >> 3;  // floor(h / 8)
     const bool below = (h & 7) != 7;
@@ -326,7 +327,10 @@ __device__ inline void leaf_column(int f, int fmin, int fmax, int zs, u32 cnt, u
         // nleaf bounds every index (only exceeded if the column map were inconsistent).
         if (lane < qn && bfs < nleaf) {
             runhead[bfs] = my_head_bfs;
-            if ((chg >> lane) & 1ull) mask_out[bfs] = my_mask;
+            if ((chg >> lane) & 1ull) {
+                mask_out[bfs] = my_mask;
+                if (hash_out) hash_out[bfs] = 0ull;  // the leaf insert computes it from the row
+            }
         }
     };
     // The first chunk's indices are staged; a longer column (box walls) loads the rest here.
@@ -335,8 +339,149 @@ __device__ inline void leaf_column(int f, int fmin, int fmax, int zs, u32 cnt, u
 }
 
 constexpr u32 kXcds = 8;
-constexpr u32 kLeafCols = 8;
+constexpr u32 kLeafCols = 1;
 constexpr u32 kLeafWaves = 1;
+
+// ---------------------------------------------------------------------------------------
+// Leaf columns, one column per lane.  A smooth surface crosses an 8x8 block in a few slices, all
+// of them in one to three nodes; such a column's 64 texels stay in one lane's registers, and each
+// partial slice's leafmask is 64 compares and carries (two instructions per texel for 64 columns
+// at once, where the wave-per-column walk issues a ballot, its placement and the scalar work of a
+// run head for one).  A column with more than kLaneSlices partial slices or kLaneNodes nodes (box
+// walls, steep surfaces) or with a texel that is not finite goes to a list that the wave-per-column
+// kernel walks in a launch of its own: shared out inside the workgroup, a box's edge kept four waves
+// busy long after the other workgroups were done.
+// ---------------------------------------------------------------------------------------
+constexpr u32 kLaneThreads = 256;  // columns per workgroup
+constexpr int kLaneSlices = 16;
+constexpr u32 kLaneNodes = 4;
+
+// One level-3 column: its index and 8x8 depth block, its leaf nodes' count, first column slot and
+// first z, and its DAG's tag.
+struct LeafCol {
+    u32 col;
+    const float* blk;
+    u32 pitch;
+    float HT;
+    u32 cnt, start;
+    int zs;
+    u32 gtag;
+};
+struct LeafOut {
+    const u32* bfs;  // column slot -> breadth-first index
+    u32* mask;
+    u64* leafm;
+    u32* runhead;
+    u64* hash;  // key hash of every run head whose column a lane walked, 0 for the others'
+    u32* slow;  // the columns left to the wave-per-column kernel, *n_slow of them
+    u32* n_slow;
+    u32 nleaf;
+};
+
+// m with the bits of one texel's compare shifted in: 2 m + (zf <= d), two instructions.
+__device__ inline u32 shift_in_le(u32 m, float zf, float d) {
+    asm("v_cmp_le_f32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(zf), "v"(d) : "vcc");
+    return m;
+}
+
+// Walks one column per lane; returns false when the column must be walked by a wave.
+__device__ inline bool leaf_lane(const LeafCol& c, const LeafOut& o) {
+    if (c.cnt == 0) return true;
+    if (c.cnt > kLaneNodes) return false;
+    float D[64];
+#pragma unroll
+    for (u32 r = 0; r < 8; ++r) {
+        const float4* row = reinterpret_cast<const float4*>(c.blk + (size_t)r * c.pitch);
+        const float4 a = row[0], b = row[1];
+        D[8 * r + 0] = a.x, D[8 * r + 1] = a.y, D[8 * r + 2] = a.z, D[8 * r + 3] = a.w;
+        D[8 * r + 4] = b.x, D[8 * r + 5] = b.y, D[8 * r + 6] = b.z, D[8 * r + 7] = b.w;
+    }
+    u32 b[kLaneNodes];
+#pragma unroll
+    for (u32 q = 0; q < kLaneNodes; ++q) b[q] = o.bfs[c.start + min(q, c.cnt - 1)];
+    float lo = D[0], hi = D[0], sum = D[0];
+#pragma unroll
+    for (u32 t = 1; t < 64; ++t) {
+        lo = fminf(lo, D[t]);
+        hi = fmaxf(hi, D[t]);
+        sum += D[t];
+    }
+    // Slices below zlo are lit at every texel, slices from zhi on at none (scaling by HT keeps the
+    // order, and leaf_f is non-decreasing).
+    const int zlo = leaf_f(lo * c.HT) + 1, zhi = leaf_f(hi * c.HT) + 1;
+    const bool finite = sum - sum == 0.0f;  // no NaN or infinity (one that only the sum makes is set aside too)
+    if (!finite || zhi - zlo > kLaneSlices) return false;
+#pragma unroll
+    for (u32 t = 0; t < 64; ++t) D[t] *= c.HT;
+    const int z0 = 8 * c.zs, z1 = z0 + 8 * (int)c.cnt;  // the column's slices
+    auto node_mask = [&](int zb) {
+        const u32 cmin = (u32)min(max(zlo - zb, 0), 8), cmax = (u32)min(max(zhi - zb, 0), 8);
+        const u32 below_min = (1u << (2 * cmin)) - 1u, below_max = (1u << (2 * cmax)) - 1u;
+        return (0x5555u & below_min) | (0xAAAAu & below_max & ~below_min) | c.gtag;
+    };
+    // A node heads a run unless it is all lit or all shadow as the node below it.
+    u32 head = 0, prev = 0;
+#pragma unroll
+    for (u32 q = 0; q < kLaneNodes; ++q) {
+        if (q >= c.cnt) break;
+        const u32 m = node_mask(z0 + 8 * (int)q);
+        const bool part = (m & 0xAAAAu) != 0;
+        const bool is_head = q == 0 || part || m != prev;
+        prev = m;
+        if (is_head) head = b[q];
+        if (b[q] < o.nleaf) {  // (only exceeded if the column map were inconsistent)
+            o.runhead[b[q]] = head;
+            if (is_head) {
+                o.mask[b[q]] = m;
+                if (!part) {
+                    const u64 h = LeafHash(m).value();
+                    o.hash[b[q]] = h ? h : 1ull;
+                }
+            }
+        }
+    }
+    // The partial slices, in order: leafmask, its place in its node's row, the node's key hash.
+    const int ze = min(zhi, z1);
+    u32 bq = 0, k = 0;
+    LeafHash hs(0);
+    for (int z = max(zlo, z0); z < ze; ++z) {
+        const float zf = (float)z + 0.5f;
+        u32 mlo = 0, mhi = 0;
+#pragma unroll
+        for (int t = 31; t >= 0; --t) mlo = shift_in_le(mlo, zf, D[t]);
+#pragma unroll
+        for (int t = 63; t >= 32; --t) mhi = shift_in_le(mhi, zf, D[t]);
+        const u32 q = (u32)(z - z0) >> 3;
+        if (k == 0) {
+            bq = q == 0 ? b[0] : q == 1 ? b[1] : q == 2 ? b[2] : b[3];
+            hs = LeafHash(node_mask(z0 + 8 * (int)q));
+        }
+        const u64 m = ((u64)mhi << 32) | mlo;
+        if (bq < o.nleaf) o.leafm[(size_t)bq * 8 + k] = m;
+        hs.add(m);
+        ++k;
+        if ((z & 7) == 7 || z + 1 == ze) {
+            const u64 h = hs.value();
+            if (bq < o.nleaf) o.hash[bq] = h ? h : 1ull;
+            k = 0;
+        }
+    }
+    return true;
+}
+
+// The lanes' columns, those set aside appended to the list (one atomic per wave).
+__device__ inline void leaf_lanes(const LeafCol& c, const LeafOut& o) {
+    const bool slow = !leaf_lane(c, o);
+    const u64 m = __ballot(slow);
+    if (!m) return;
+    const u32 lane = threadIdx.x & 63;
+    u32 at = 0;
+    if (lane == (u32)__builtin_ctzll(m)) at = atomicAdd(o.n_slow, (u32)__popcll(m));
+    at = __builtin_amdgcn_readlane(at, __builtin_ctzll(m));
+    // (a listed column has a node, so the list holds at most nleaf)
+    const u32 k = at + (u32)__popcll(m & ((1ull << lane) - 1ull));
+    if (slow && k < o.nleaf) o.slow[k] = c.col;
+}
 
 // Children ranks of inner node i (slots j >= k are 0).  All eight loads are issued before any is
 // used, so a node costs one memory round trip, not one per child.
@@ -346,18 +491,25 @@ __device__ inline void load_child_ranks(const u32* cstart, const u32* child_rank
     for (u32 j = 0; j < 8; ++j) r[j] = (j < k) ? child_rank[s + j] : 0u;
 }
 
+// Key hash of an inner node: a sum of (mask, child ranks) times fixed odd 64-bit constants, whose
+// collisions need an exact zero of the differences' sum mod 2^64, then a mixer that is a bijection.
+// Two 32-bit multiplies per child instead of a chain of two 64-bit ones: in the one-workgroup
+// merge of the small levels, four waves per SIMD hash four nodes per thread and level, and the
+// chained form's multiplies alone were most of its time.
 __device__ inline u64 inner_key_hash(const u32* mask, const u32* cstart, const u32* child_rank, u32 i) {
+    constexpr u64 kMul[9] = {0x9E3779B97F4A7C15ull, 0xC2B2AE3D27D4EB4Full, 0x165667B19E3779F9ull, 0xD6E8FEB86659FD93ull,
+                             0xA0761D6478BD642Full, 0xE7037ED1A0B428DBull, 0x8EBC6AF09C88C6E3ull, 0x589965CC75374CC3ull,
+                             0x1D8E4E27C47D124Full};
     const u32 m = mask[i];
     const u32 k = num_children(m);
-    u64 h = hash_step(kHashSeed, m);
+    u64 h = kHashSeed + m * kMul[8];
     if (k) {
         u32 r[8];
         load_child_ranks(cstart, child_rank, i, k, r);
 #pragma unroll
-        for (u32 j = 0; j < 8; ++j)
-            if (j < k) h = hash_step(h, r[j]);
+        for (u32 j = 0; j < 8; ++j) h += r[j] * kMul[j];  // (slots past the children are 0)
     }
-    return h;
+    return mix64(h);
 }
 
 // A merge hash cut to its low `bits` bits, in both the tag and the slot position, so that distinct
@@ -681,7 +833,8 @@ enum : int {
     kMetaRoot = 4 * kMaxLevels + 2,      // root mask
     kMetaSortColl = 4 * kMaxLevels + 3,  // 32-bit key collisions resolved by a scan (sort merge)
     kMetaFull = 4 * kMaxLevels + 4,      // table inserts that found no free slot (table merge)
-    kMetaWords = 4 * kMaxLevels + 5,
+    kMetaSlow = 4 * kMaxLevels + 5,      // leaf columns left to the wave-per-column kernel
+    kMetaWords = 4 * kMaxLevels + 6,
 };
 
 
@@ -730,6 +883,11 @@ __device__ inline void write_leaf_node(u32 r, const u32* __restrict__ uniq, cons
 }
 
 
+// Launches over this many columns walk them one per lane (a map's are then at least 16 x 16).
+constexpr u64 kLaneLeafMin = 1u << 15;
+constexpr u32 kSlowCols = 1;
+constexpr u32 kSlowWaves = 8192;  // waves that stride over the columns left to them: the chip's 32 per CU
+
 inline u32 table_slots(u32 n) {
     u32 S = 1024;
     while (S < n + n / 2 + 1) S <<= 1;
@@ -743,7 +901,8 @@ inline u32 leaf_table_slots(u32 c, bool small) { return table_slots((small && c 
 // Non-template kernels defined in build.hip.
 __global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 S);
 __global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
-                                                                    const u32* __restrict__ runhead, u32 n,
+                                                                    const u32* __restrict__ runhead,
+                                                                    const u64* __restrict__ hash, u32 n,
                                                                     u64* __restrict__ tab, u32 S, u32* __restrict__ tslot,
                                                                     u32* __restrict__ full, u64* __restrict__ zero,
                                                                     u32 nzero, u32 hbits);

@@ -232,7 +232,7 @@ template <u32 kCols, u32 kWaves>
 __global__ __launch_bounds__(64 * kWaves) void k_forest_leaf(const uint4* __restrict__ colinfo, const u32* __restrict__ colbfs,
                                                              const FItem* __restrict__ items, u32 nleaf,
                                                              u32* __restrict__ mask_out, u64* __restrict__ leafm,
-                                                             u32* __restrict__ runhead,
+                                                             u32* __restrict__ runhead, u64* __restrict__ hash_out,
                                                              u64* __restrict__ tab, u32 tab_slots,
                                                              const u32* __restrict__ col_list, const u32* __restrict__ n_list,
                                                              u32 list_cap) {
@@ -240,8 +240,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_forest_leaf(const uint4* __rest
     __shared__ u32 s_b[kWaves][kCols][64];
     __shared__ uint8_t s_chg[kWaves][128];  // each wave's changed-node flags (leaf_column)
     const u32 lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const u32 c0 = (blockIdx.x * kWaves + wave) * kCols;
     const u32 nvalid = min(*n_list, list_cap);
+    for (u32 c0 = (blockIdx.x * kWaves + wave) * kCols; c0 < nvalid; c0 += gridDim.x * kWaves * kCols) {
     const u32 clast = nvalid ? nvalid - 1 : 0u;
     const u32 my_col = nvalid ? col_list[min(c0 + (lane & (kCols - 1)), clast)] : 0u;
     uint4 ci = colinfo[my_col];
@@ -300,7 +300,34 @@ __global__ __launch_bounds__(64 * kWaves) void k_forest_leaf(const uint4* __rest
             fmax = __ockl_wfred_max_i32(f);
         }
         leaf_column(f, fmin, fmax, zs, cnt, s_b[wave][k][lane], colbfs + base, gtag, nleaf,
-                    kWaves == 1 ? s_chg[0] : s_chg[wave], lane, mask_out, leafm, runhead);
+                    kWaves == 1 ? s_chg[0] : s_chg[wave], lane, mask_out, leafm, runhead, hash_out);
+    }
+    }
+    clear_table(tab, tab_slots);
+}
+
+// The same with one column per lane (leaf_lane) over the list.
+__global__ __launch_bounds__(kLaneThreads) void k_forest_lanes(const uint4* __restrict__ colinfo, const FItem* __restrict__ items,
+                                                               LeafOut o, u64* __restrict__ tab, u32 tab_slots,
+                                                               const u32* __restrict__ col_list,
+                                                               const u32* __restrict__ n_list, u32 list_cap) {
+    const u32 n = min(*n_list, list_cap), k = blockIdx.x * kLaneThreads + threadIdx.x;
+    if (blockIdx.x * kLaneThreads < n) {
+        LeafCol c{};
+        if (k < n) {
+            c.col = col_list[k];
+            const uint4 ci = colinfo[c.col];
+            const FItem& it = items[ci.w];
+            const u32 local = c.col - it.col_base, x3 = local & (it.w3 - 1), y3 = local >> it.w3_shift;
+            c.blk = it.depth + ((size_t)(8 * y3) * it.N + 8 * x3);
+            c.pitch = it.N;
+            c.HT = (float)(it.N * it.T);
+            c.cnt = ci.x;
+            c.start = ci.y;
+            c.zs = (int)ci.z;
+            c.gtag = ci.w << 16;
+        }
+        leaf_lanes(c, o);
     }
     clear_table(tab, tab_slots);
 }
@@ -418,24 +445,34 @@ constexpr int kRetrySort = -1010;
 constexpr int kRetryFull = -1011;
 constexpr int kRetryExact = -1012;  // the counts exceed the emitted nodes (a map with NaN depths)
 
-// Launches the leaf kernel in the shape the options name.
+// Launches the leaf kernels: one column per lane and a wave for each column left over, or, below
+// kLaneLeafMin columns, waves only, in the shape the options name.  n_slow and slow: the columns
+// left over (room for lo.nleaf).
 void launch_leaf(const ForestOpts& o, u32 units_cols, hipStream_t s, const uint4* colinfo, const u32* colbfs,
-                 const FItem* items, u32 nleaf, u32* mask, u64* leafm, u32* runhead, u64* tab,
-                 u32 slots, const u32* clist, const u32* nclist, u32 cap) {
+                 const FItem* items, u32 nleaf, u32* mask, u64* leafm, u32* runhead, u64* hash, u32* slow, u32* n_slow,
+                 u64* tab, u32 slots, const u32* clist, const u32* nclist, u32 cap) {
+    if (hash) {
+        const LeafOut lo{colbfs, mask, leafm, runhead, hash, slow, n_slow, nleaf};
+        CPVS_LAUNCH("forest_lanes", k_forest_lanes, dim3(ceil_div<u32>(units_cols, kLaneThreads)), dim3(kLaneThreads), 0, s,
+                    colinfo, items, lo, tab, slots, clist, nclist, cap);
+        CPVS_LAUNCH("forest_leaf", (k_forest_leaf<kSlowCols, 1>), dim3(std::min(ceil_div<u32>(units_cols, kSlowCols), kSlowWaves)),
+                    dim3(64), 0, s, colinfo, colbfs, items, nleaf, mask, leafm, runhead, hash, tab, 0u, slow, n_slow, cap);
+        return;
+    }
     const u32 per = o.leaf_cols * o.leaf_waves;
     const dim3 grid((units_cols + per - 1) / per);
     if (o.leaf_cols == 4 && o.leaf_waves == 1)
         CPVS_LAUNCH("forest_leaf", (k_forest_leaf<4, 1>), grid, dim3(64), 0, s, colinfo, colbfs, items, nleaf, mask, leafm,
-                    runhead, tab, slots, clist, nclist, cap);
+                    runhead, nullptr, tab, slots, clist, nclist, cap);
     else if (o.leaf_cols == 4)
         CPVS_LAUNCH("forest_leaf", (k_forest_leaf<4, 2>), grid, dim3(128), 0, s, colinfo, colbfs, items, nleaf, mask, leafm,
-                    runhead, tab, slots, clist, nclist, cap);
+                    runhead, nullptr, tab, slots, clist, nclist, cap);
     else if (o.leaf_waves == 1)
         CPVS_LAUNCH("forest_leaf", (k_forest_leaf<8, 1>), grid, dim3(64), 0, s, colinfo, colbfs, items, nleaf, mask, leafm,
-                    runhead, tab, slots, clist, nclist, cap);
+                    runhead, nullptr, tab, slots, clist, nclist, cap);
     else
         CPVS_LAUNCH("forest_leaf", (k_forest_leaf<8, 2>), grid, dim3(128), 0, s, colinfo, colbfs, items, nleaf, mask, leafm,
-                    runhead, tab, slots, clist, nclist, cap);
+                    runhead, nullptr, tab, slots, clist, nclist, cap);
 }
 
 // Pinned staging of one forest build.
@@ -636,6 +673,9 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         lv.uniq[L] = A.take<u32>(c);
         lv.off[L] = A.take<u32>(c);
     }
+    // The run heads' key hashes, from the leaf kernel to the leaf insert, in the place of the leaf
+    // level's unique list and offsets (two arrays side by side), which the ranks scan writes later.
+    u64* leaf_hash = (C[2] && std::min<u64>(ncol, C[2]) >= kLaneLeafMin) ? reinterpret_cast<u64*>(lv.uniq[2]) : nullptr;
     u64* leafm = A.take<u64>(c2 * 8);
     u32* runhead = A.take<u32>(c2);
     u32* colbfs = A.take<u32>(c2);
@@ -692,8 +732,8 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         const u32 slots2 = use_table ? leaf_table_slots((u32)C[2], small_leaf) : 0u;
         if (C[2]) {
             const u32 bound = (u32)std::min<u64>(ncol, C[2]);
-            launch_leaf(o, bound, s, colinfo, colbfs, items, (u32)C[2], lv.mask[2], leafm, runhead, tab, slots2,
-                        clist, nclist, bound);
+            launch_leaf(o, bound, s, colinfo, colbfs, items, (u32)C[2], lv.mask[2], leafm, runhead, leaf_hash, rep,
+                        meta + kMetaSlow, tab, slots2, clist, nclist, bound);
         }
         // Bottom-up merge over every level with nodes (roots included: a root is alone in its DAG).
         int prev = -1;  // the level merged before (its ranks are the next level's child ranks)
@@ -714,7 +754,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
                 if (!is_leaf && prev < 0) CPVS_LAUNCH("table_clear", k_table_clear, grid_of(Sl, 256), dim3(256), 0, s, tab, Sl);
                 if (is_leaf) {
                     CPVS_LAUNCH("insert_leaf", k_insert_leaf, dim3(ceil_div<u32>(c, kLeafWindow)), dim3(kLeafInsertThreads), 0, s,
-                                lv.mask[2], leafm, runhead, c, tab, Sl, tslot, meta + kMetaFull, rpart, nzero,
+                                lv.mask[2], leafm, runhead, leaf_hash, c, tab, Sl, tslot, meta + kMetaFull, rpart, nzero,
                                 ctx->leaf_hash_bits.load());
                     CPVS_LAUNCH("resolve", k_resolve<LeafEq>, grid_of(c, kNodeThreads), dim3(kNodeThreads), 0, s, tslot, tab,
                                 runhead, c, LeafEq{lv.mask[2], leafm, nullptr, c}, rep, meta + kMetaColl, lv.mask[2], 1u,
