@@ -29,7 +29,7 @@
 #include <cstdio>
 #include <cstring>
 
-#include "build_parts.hpp"
+#include "merge.hpp"
 
 namespace cpvs {
 
@@ -277,274 +277,11 @@ __global__ __launch_bounds__(kLaneThreads) void k_leaf_lanes(LeafColumns lc, u32
     clear_table(tab, tab_slots);
 }
 
-// ---------------------------------------------------------------------------------------
-// 3. Merge.
-// ---------------------------------------------------------------------------------------
-// --- (a) hash table --------------------------------------------------------------------------
-
-// One 64-bit word per slot: the key hash's high 32 bits (its tag) above the smallest node index
-// with that hash, so a probe touches one cache line and a new key costs one atomic.  ~0 marks an
-// empty slot (node indices stay below 2^32 - 1).  Two keys whose tags are equal and whose probe
-// chains meet share a slot; the full-key compare in k_resolve then sends the build down the
-// sorting path, as for equal 64-bit hashes.
-
-__global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 S) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < S) tab[i] = kEmptySlot;
-}
-
-__global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
-                                                                    const u32* __restrict__ runhead,
-                                                                    const u64* __restrict__ hash, u32 n,
-                                                                    u64* __restrict__ tab, u32 S, u32* __restrict__ tslot,
-                                                                    u32* __restrict__ full, u64* __restrict__ zero,
-                                                                    u32 nzero, u32 hbits) {
-    __shared__ u64 gh[kLeafSlots];
-    __shared__ u32 gi[kLeafSlots];  // smallest node index of the slot's hash, then its global slot
-    __shared__ unsigned short glist[kLeafWindow];  // LDS slots in use
-    __shared__ u32 gcount;
-    clear_partials(zero, nzero);
-    for (u32 j = threadIdx.x; j < kLeafSlots; j += blockDim.x) {
-        gh[j] = 0ull;  // 0 marks an empty LDS slot
-        gi[j] = kNoRep;
-    }
-    if (threadIdx.x == 0) gcount = 0;
-    const u32 i0 = blockIdx.x * kLeafWindow + threadIdx.x;
-    u32 rh[kLeafPer];
-#pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        rh[k] = (i < n) ? runhead[i] : kNoRep;
-    }
-    // The key hash of each run's first node (the run's smallest index): from the leaf kernel where
-    // a lane walked its column, else from its mask and leafmasks (its row at its own index).
-    u64 h[kLeafPer];
-#pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        h[k] = (hash && rh[k] == i) ? hash[i] : 0ull;
-    }
-    u32 hm[kLeafPer];
-#pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        hm[k] = (rh[k] == i && h[k] == 0ull) ? mask[i] : 0u;
-    }
-#pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        if (rh[k] != i) continue;
-        if (h[k] == 0ull) h[k] = leaf_key_hash(hm[k], leafm + (size_t)i * 8);
-        h[k] = weaken_hash(h[k], hbits);
-        if (h[k] == 0ull) h[k] = 1ull;
-    }
-    __syncthreads();
-    u32 ls[kLeafPer];
-#pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        ls[k] = 0;
-        if (rh[k] != i) continue;
-        u32 sl = (u32)(h[k] ^ (h[k] >> 29)) & (kLeafSlots - 1);
-        for (;;) {
-            const u64 cur = atomicCAS(reinterpret_cast<unsigned long long*>(gh + sl), 0ull, (unsigned long long)h[k]);
-            if (cur == 0ull) {
-                glist[atomicAdd(&gcount, 1u)] = (unsigned short)sl;
-                break;
-            }
-            if (cur == h[k]) break;
-            sl = (sl + 1) & (kLeafSlots - 1);
-        }
-        atomicMin(gi + sl, i);
-        ls[k] = sl;
-    }
-    __syncthreads();
-    const u32 m = gcount;  // at most kLeafWindow
-    for (u32 j = threadIdx.x; j < m; j += blockDim.x) {
-        const u32 sl = glist[j];
-        gi[sl] = table_insert(tab, S, gh[sl], gi[sl], full);
-    }
-    __syncthreads();
-#pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        if (rh[k] == i) tslot[i] = gi[ls[k]];
-    }
-}
-
-__global__ __launch_bounds__(kInsertBlock) void k_insert_inner(const u32* __restrict__ mask, const u32* __restrict__ cstart,
-                                                               const u32* __restrict__ child_rank, u32 n, u64* __restrict__ tab,
-                                                               u32 S, u32* __restrict__ tslot, u32* __restrict__ full,
-                                                               u64* __restrict__ zero, u32 nzero, u32 hbits) {
-    clear_partials(zero, nzero);
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool act = i < n;
-    const u64 h = act ? weaken_hash(inner_key_hash(mask, cstart, child_rank, i), hbits) : 0ull;
-    const u32 slot = table_insert_group(tab, S, h, i, act, full);
-    if (act) tslot[i] = slot;
-}
-
-// --- (b) radix sort ----------------------------------------------------------------------------
-
-__global__ __launch_bounds__(256) void k_sortkeys_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
-                                                       const u32* __restrict__ runhead,
-                                                       u32 n, u32* __restrict__ skey, u32* __restrict__ sval) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    u32 h = runhead[i];  // the key is the run's first node's
-    h = (h < n) ? h : i;
-    skey[i] = fold32(leaf_key_hash(mask[h], leafm + (size_t)h * 8));
-    sval[i] = i;
-}
-
-__global__ __launch_bounds__(256) void k_sortkeys_inner(const u32* __restrict__ mask, const u32* __restrict__ cstart,
-                                                        const u32* __restrict__ child_rank, u32 n, u32* __restrict__ skey,
-                                                        u32* __restrict__ sval) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    skey[i] = fold32(inner_key_hash(mask, cstart, child_rank, i));
-    sval[i] = i;
-}
-
-// --- ranks -------------------------------------------------------------------------------------
-
-// Copies take their first occurrence's rank.  The merge table of the next level (tab_slots > 0)
-// is cleared here too: this level's last table read (k_resolve) ran before.
-__global__ __launch_bounds__(kNodeThreads) void k_rank_copies(const u32* __restrict__ rep, const u32* __restrict__ runhead, u32 count,
-                                                     u32* __restrict__ rank, u64* __restrict__ tab, u32 tab_slots) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) {
-        u32 r = rep[i];
-        const u32 h = runhead ? runhead[i] : i;  // loaded with rep[i]: most leaf nodes need it
-        if (r == kNoRep) r = (h < count) ? rep[h] : kNoRep;
-        if (r != i && r < count) rank[i] = rank[r];
-    }
-    clear_table(tab, tab_slots);
-}
-
-__global__ void k_root_init(u32* rank, u32* uniq, u32* n_uniq) {
-    rank[0] = 0;
-    uniq[0] = 0;
-    *n_uniq = 1;
-}
-
 // First launch after the scratch is laid out when no level is small: the root's coordinate, and
 // the meta words zeroed (k_small_topdown does both otherwise).
 __global__ void k_start(u64* root_coord, u64 root, u32* meta, u32 meta_words) {
     *root_coord = root;
     for (u32 i = 0; i < meta_words; ++i) meta[i] = 0u;
-}
-
-// ---------------------------------------------------------------------------------------
-// 4. Compress.
-// ---------------------------------------------------------------------------------------
-// B[R] = 0, B[L-1] = B[L] + S[L]; total = B[bottom] + S[bottom] (levels absent have S = 0).  One
-// thread; every S is loaded before any base is stored (stored one by one behind each load, the
-// loads would wait for one another).
-__device__ inline void level_bases(u32* meta, int R, int bottom) {
-    u32 S[kMaxLevels];
-#pragma unroll
-    for (int L = 0; L < kMaxLevels; ++L) S[L] = meta[kMetaS + L];
-    unsigned long long acc = 0;
-#pragma unroll
-    for (int L = kMaxLevels - 1; L >= 0; --L) {
-        if (L <= R && L >= bottom) {
-            meta[kMetaB + L] = (u32)acc;
-            acc += S[L];
-        }
-    }
-    meta[kMetaW] = (acc > 0xFFFFFFFFull) ? 0xFFFFFFFFu : (u32)acc;
-}
-
-// The build's readback: the metadata block copied to pinned host memory by the whole workgroup,
-// one word per thread (after a barrier, so that thread 0's bases are in).
-__device__ inline void meta_to_host(const u32* meta, u32* host_meta) {
-    __syncthreads();
-    for (u32 i = threadIdx.x; i < kMetaWords; i += blockDim.x) host_meta[i] = meta[i];
-    __threadfence_system();
-}
-
-__global__ __launch_bounds__(128) void k_level_bases(u32* __restrict__ meta, int R, int bottom,
-                                                     const u32* __restrict__ root_mask, u32* __restrict__ host_meta) {
-    if (threadIdx.x == 0) {
-        meta[kMetaRoot] = *root_mask;
-        level_bases(meta, R, bottom);
-    }
-    meta_to_host(meta, host_meta);
-}
-
-// Every level's words in one launch: once the offsets and bases are known the levels' words are
-// independent, and a launch per level costs a launch each.  Level k takes the blocks
-// [first[k], first[k+1]), one unique node per thread.
-struct WriteLevel {
-    const u32* uniq;
-    const u32* mask;
-    const u32* cstart;
-    const u32* off;
-    const u32* child_rank;  // null at the deepest level
-    const u32* child_off;
-    u32 child_n;            // nodes of the child level
-    u32 U, base, child_base, leaf;
-    int L;                  // the octree level (k_write_levels_dev reads U and the bases of meta)
-};
-struct WriteArgs {
-    int nlev;
-    u32 first[kMaxLevels + 1];
-    WriteLevel lv[kMaxLevels];
-    const u64* leafm;
-    u32 nleaf;  // nodes of the leaf level (at least 1)
-};
-
-__global__ __launch_bounds__(kNodeThreads) void k_write_levels(WriteArgs a, u32* __restrict__ out) {
-    int k = 0;
-    while (k + 1 < a.nlev && blockIdx.x >= a.first[k + 1]) ++k;
-    const WriteLevel& l = a.lv[k];
-    const u32 r = (blockIdx.x - a.first[k]) * blockDim.x + threadIdx.x;
-    if (r >= l.U) return;
-    if (l.leaf)
-        write_leaf_node(r, l.uniq, l.mask, a.leafm, a.nleaf, l.off, l.base, out);
-    else
-        write_inner_node(r, l.uniq, l.mask, l.cstart, l.off, l.base, l.child_rank, l.child_off, l.child_base, l.child_n,
-                         out);
-}
-
-// The same with the unique counts and level bases read from the metadata block, so that it runs
-// right behind the merge with no host readback between: a grid-stride loop over the levels'
-// blocks (their number is known on the device only), the words into a staging area of the
-// pre-merge word bound.
-__global__ __launch_bounds__(kNodeThreads) void k_write_levels_dev(WriteArgs a, const u32* __restrict__ meta,
-                                                                  u32* __restrict__ out, u64 cap) {
-    __shared__ u32 s_first[kMaxLevels + 1], s_U[kMaxLevels], s_base[kMaxLevels], s_cbase[kMaxLevels];
-    if (threadIdx.x == 0) {
-        u32 acc = 0;
-        for (int k = 0; k < a.nlev; ++k) {
-            const int L = a.lv[k].L;
-            s_U[k] = meta[kMetaU + L];
-            s_base[k] = meta[kMetaB + L];
-            s_cbase[k] = a.lv[k].child_rank ? meta[kMetaB + L - 1] : 0u;
-            s_first[k] = acc;
-            acc += (s_U[k] + kNodeThreads - 1) / kNodeThreads;
-        }
-        s_first[a.nlev] = acc;
-    }
-    __syncthreads();
-    const u32 nb = s_first[a.nlev];
-    for (u32 vb = blockIdx.x; vb < nb; vb += gridDim.x) {
-        int k = 0;
-        while (k + 1 < a.nlev && vb >= s_first[k + 1]) ++k;
-        const WriteLevel& l = a.lv[k];
-        const u32 r = (vb - s_first[k]) * blockDim.x + threadIdx.x;
-        if (r >= s_U[k]) continue;
-        // Offsets lie below the word count, itself below the staging's pre-merge bound; a node
-        // that would not fit (only if the build were inconsistent, which the host then reports)
-        // is not written.
-        if ((u64)s_base[k] + l.off[r] + 17 > cap) continue;
-        if (l.leaf)
-            write_leaf_node(r, l.uniq, l.mask, a.leafm, a.nleaf, l.off, s_base[k], out);
-        else
-            write_inner_node(r, l.uniq, l.mask, l.cstart, l.off, s_base[k], l.child_rank, l.child_off, s_cbase[k],
-                             l.child_n, out);
-    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -557,18 +294,21 @@ struct Level {
     u64* coord = nullptr;
     u32* mask = nullptr;
     u32* cstart = nullptr;
-    u32* rank = nullptr;
+    u32* id = nullptr;
     u32* uniq = nullptr;
     u32* off = nullptr;
+    u64* first = nullptr;
+    u64* tab = nullptr;
+    u32 slots = 0;
 };
 
 // ---------------------------------------------------------------------------------------
 // Small levels in one workgroup.  The upper octree levels hold few nodes (at 8192^2 the levels
 // above 6 hold a few thousand together), yet each costs about ten launches of the per-level
 // path at several microseconds apiece.  A level of at most kSmallMax nodes is handled by one
-// 1024-thread workgroup instead, all such levels in one launch per phase: top-down
-// classification and child emission, bottom-up merge (hash table in LDS), and compress
-// (size scans, level bases, words).  Results are those of the per-level path.
+// 1024-thread workgroup instead, all such levels in one launch per phase: top-down classification
+// and child emission, and bottom-up inserts (hash tables in LDS).  Results are those of the
+// per-level path.
 // ---------------------------------------------------------------------------------------
 // Measured at 8192^2: a limit of 4096 nodes beats 2048 (1.29 against 1.31 ms per build) and 8192
 // (1.34 ms: one workgroup then spends more on the 7.9 K-node level than its per-level launches do).
@@ -576,6 +316,11 @@ constexpr u32 kSmallMax = 4096;
 constexpr int kSmallThreads = 1024;
 constexpr u32 kSmallPer = kSmallMax / kSmallThreads;  // nodes per thread
 constexpr u32 kSmallSlots = 2 * kSmallMax;             // LDS table of 8-byte slots: 64 KB
+inline u32 small_slots(u32 c) {
+    u32 S = 64;
+    while (S < 2 * c) S <<= 1;
+    return S;
+}
 
 struct SmallArgs {
     int R, Ls, deepest;  // the small levels are [Ls, R]; deepest = lowest level with nodes
@@ -583,13 +328,13 @@ struct SmallArgs {
     u64* coord[kMaxLevels];
     u32* mask[kMaxLevels];
     u32* cstart[kMaxLevels];
-    u32* rank[kMaxLevels];
-    u32* uniq[kMaxLevels];
-    u32* off[kMaxLevels];
+    u32* id[kMaxLevels];
+    u64* tab[kMaxLevels];
+    u32 slots[kMaxLevels];
+    u32 n_below;       // nodes of the level below Ls
+    const u32* heads;  // run heads when that level is the leaf level, else null
     const float2* lv[kMaxLevels];
     u32* meta;
-    u32* host_meta;  // pinned host copy of meta, written when the compress step is done
-    u32 sizes_in_merge;  // every larger level has its word offsets: k_small_merge finishes compress
 };
 
 // Exclusive sum over the workgroup, one value per thread; *total = the sum.
@@ -678,168 +423,60 @@ __device__ inline u32 lds_insert(u64* tab, u32 S, u64 h, u32 i) {
     }
 }
 
-// Merge of the small levels Ls .. R-1 (the root is never merged), then the root's rank.  A node
-// takes the smallest index with its slot's tag; if that node's key differs (a collision of tags
-// or of 64-bit hashes), it looks for its first occurrence by comparing keys with every lower index.
-// The small levels' ranks are also kept in LDS (two buffers: a level and its children), where the
-// next level's keys, key compares and the rank copies read them.  A level's masks and child starts
-// are loaded while the level below is merged, and staged in LDS for the keys and compares.
-__global__ __launch_bounds__(kSmallThreads) void k_small_merge(SmallArgs a) {
+// Inserts of the small levels Ls .. R-1 (the root is never merged), each into a table in LDS that is
+// then copied to the level's own.  The identities are also kept in LDS (two buffers: a level and its
+// children), where the next level's keys read them, and a level's masks and child starts are loaded
+// while the level below is inserted.
+__global__ __launch_bounds__(kSmallThreads) void k_small_insert(SmallArgs a) {
     __shared__ u64 tab[kSmallSlots];
-    __shared__ u32 s_wave[kSmallThreads / kWave];
-    __shared__ u32 s_rank[2][kSmallMax];
-    __shared__ u32 s_mask[kSmallMax];
-    __shared__ u32 s_cstart[kSmallMax];
-    u32 pm[kSmallPer], pc[kSmallPer];  // masks and child starts of the next level's nodes
-    auto prefetch = [&](int L) {
-        const u32 c = a.count[L], E = small_per_thread(c), i0 = threadIdx.x * E;
+    __shared__ u32 s_id[2][kSmallMax];
+    u32 pm[kSmallPer], pc[kSmallPer];  // masks and child starts of the level's nodes
+    auto load = [&](int L) {
+        const u32 c = a.count[L];
 #pragma unroll
         for (u32 e = 0; e < kSmallPer; ++e) {
-            const u32 i = i0 + e;
-            pm[e] = 0;
-            pc[e] = 0;
-            if (e < E && i < c) {
-                pm[e] = a.mask[L][i];
-                pc[e] = a.cstart[L][i];
-            }
+            const u32 i = e * kSmallThreads + threadIdx.x;
+            pm[e] = (i < c) ? a.mask[L][i] : 0u;
+            pc[e] = (i < c) ? a.cstart[L][i] : 0u;
         }
     };
-    if (a.Ls < a.R) prefetch(a.Ls);
+    if (a.Ls < a.R) load(a.Ls);
     for (int L = a.Ls; L < a.R; ++L) {
-        const u32 c = a.count[L];  // at most kSmallMax
-        u32 S = 64;
-        while (S < 2 * c) S <<= 1;
+        const u32 c = a.count[L], S = a.slots[L];
         for (u32 j = threadIdx.x; j < S; j += kSmallThreads) tab[j] = kEmptySlot;
-        {
-            const u32 E = small_per_thread(c), i0 = threadIdx.x * E;
+        u64 h[kSmallPer];
 #pragma unroll
-            for (u32 e = 0; e < kSmallPer; ++e) {
-                const u32 i = i0 + e;
-                if (e < E && i < c) {
-                    s_mask[i] = pm[e];
-                    s_cstart[i] = pc[e];
+        for (u32 e = 0; e < kSmallPer; ++e) {
+            const u32 i = e * kSmallThreads + threadIdx.x;
+            h[e] = 0;
+            if (i >= c) continue;
+            const u32 k = (L > a.deepest) ? num_children(pm[e]) : 0u;
+            u32 r[8] = {};
+            if (k) {
+                // The first small level's children are in memory.
+                if (L == a.Ls) {
+                    load_child_ids(ChildIds{a.id[L - 1], a.heads, a.n_below}, pc[e], k, r);
+                } else {
+#pragma unroll
+                    for (u32 j = 0; j < 8; ++j) r[j] = (j < k) ? s_id[(L - 1) & 1][min(pc[e] + j, kSmallMax - 1)] : 0u;
                 }
             }
+            h[e] = inner_key_hash(pm[e], r);
         }
-        __syncthreads();
-        if (L + 1 < a.R) prefetch(L + 1);
-        // The first small level's children were ranked by the multi-workgroup path, in memory.
-        const u32* child_rank = (L > a.deepest) ? ((L > a.Ls) ? s_rank[(L - 1) & 1] : a.rank[L - 1]) : nullptr;
-        u32* rank_l = s_rank[L & 1];
-        const u32 E = small_per_thread(c), i0 = threadIdx.x * E;
-        u32 slot[kSmallPer];
+        if (L + 1 < a.R) load(L + 1);
+        __syncthreads();  // the table is clear
 #pragma unroll
         for (u32 e = 0; e < kSmallPer; ++e) {
-            const u32 i = i0 + e;
-            slot[e] = 0;
-            if (e < E && i < c) slot[e] = lds_insert(tab, S, inner_key_hash(s_mask, s_cstart, child_rank, i), i);
+            const u32 i = e * kSmallThreads + threadIdx.x;
+            if (i >= c) continue;
+            const u32 slot = lds_insert(tab, S, h[e], i);
+            s_id[L & 1][i] = slot;
+            a.id[L][i] = slot;
         }
-        __syncthreads();
-        const InnerEq eq{s_mask, s_cstart, child_rank};
-        // One scan of (first occurrences << 16 | their words) gives ranks and word offsets (a level
-        // of at most kSmallMax nodes of at most 9 words keeps the low half below 2^16).
-        u32 rep[kSmallPer], sz[kSmallPer], packed = 0;
-#pragma unroll
-        for (u32 e = 0; e < kSmallPer; ++e) {
-            const u32 i = i0 + e;
-            rep[e] = i;
-            sz[e] = 0;
-            if (e < E && i < c) {
-                u32 r = (u32)tab[slot[e]];
-                if (r != i && !eq(i, r)) {
-                    r = i;
-                    for (u32 j = 0; j < i; ++j)
-                        if (eq(i, j)) {
-                            r = j;
-                            break;
-                        }
-                }
-                rep[e] = r;
-                if (r == i) {
-                    sz[e] = 1u + num_children(s_mask[i]);
-                    packed += (1u << 16) + sz[e];
-                }
-            }
-        }
-        u32 total;
-        const u32 ex = small_scan(packed, s_wave, &total);
-        u32 rk = ex >> 16, of = ex & 0xFFFFu;
-#pragma unroll
-        for (u32 e = 0; e < kSmallPer; ++e) {
-            const u32 i = i0 + e;
-            if (e < E && i < c && rep[e] == i) {
-                a.rank[L][i] = rk;
-                rank_l[i] = rk;
-                a.uniq[L][rk] = i;
-                if (a.sizes_in_merge) a.off[L][rk] = of;
-                ++rk;
-                of += sz[e];
-            }
-        }
-        if (threadIdx.x == 0) {
-            a.meta[kMetaU + L] = total >> 16;
-            if (a.sizes_in_merge) a.meta[kMetaS + L] = total & 0xFFFFu;
-        }
-        __syncthreads();  // first occurrences ranked
-#pragma unroll
-        for (u32 e = 0; e < kSmallPer; ++e) {
-            const u32 i = i0 + e;
-            if (e < E && i < c && rep[e] != i) {
-                const u32 r = rank_l[rep[e]];
-                a.rank[L][i] = r;
-                rank_l[i] = r;
-            }
-        }
-        __syncthreads();  // the next level reads these ranks
+        __syncthreads();  // every insert is in; the next level reads these identities
+        for (u32 j = threadIdx.x; j < S; j += kSmallThreads) a.tab[L][j] = tab[j];
+        // (each thread clears for the next level the slots that it has just copied)
     }
-    if (threadIdx.x == 0) {
-        a.rank[a.R][0] = 0;
-        a.uniq[a.R][0] = 0;
-        a.meta[kMetaU + a.R] = 1;
-        if (a.sizes_in_merge) {
-            // What k_small_compress does otherwise: the root's size, the level bases, the readback.
-            const u32 root = a.mask[a.R][0];
-            a.off[a.R][0] = 0;
-            a.meta[kMetaS + a.R] = 1u + num_children(root);
-            a.meta[kMetaRoot] = root;
-            level_bases(a.meta, a.R, a.deepest);
-        }
-    }
-    if (a.sizes_in_merge) meta_to_host(a.meta, a.host_meta);  // uniform: every thread reaches the barrier
-}
-
-// Size scans of the small levels (1 + k words per unique node), then the level bases of all
-// levels (the per-level scans of the larger levels ran before).
-__global__ __launch_bounds__(kSmallThreads) void k_small_compress(SmallArgs a) {
-    __shared__ u32 s_wave[kSmallThreads / kWave];
-    for (int L = a.R; L >= a.Ls; --L) {
-        const u32 U = a.meta[kMetaU + L];
-        const u32 E = small_per_thread(U), i0 = threadIdx.x * E;
-        u32 sz[kSmallPer], sum = 0;
-#pragma unroll
-        for (u32 e = 0; e < kSmallPer; ++e) {
-            const u32 r = i0 + e;
-            sz[e] = (e < E && r < U) ? 1u + num_children(a.mask[L][a.uniq[L][r]]) : 0u;
-            sum += sz[e];
-        }
-        u32 total;
-        u32 ex = small_scan(sum, s_wave, &total);
-#pragma unroll
-        for (u32 e = 0; e < kSmallPer; ++e) {
-            const u32 r = i0 + e;
-            if (e < E && r < U) {
-                a.off[L][r] = ex;
-                ex += sz[e];
-            }
-        }
-        if (threadIdx.x == 0) a.meta[kMetaS + L] = total;
-    }
-    __syncthreads();  // every level's size (thread 0 wrote them) before the bases
-    if (threadIdx.x == 0) {
-        a.meta[kMetaRoot] = a.mask[a.R][0];
-        level_bases(a.meta, a.R, a.deepest);
-    }
-    meta_to_host(a.meta, a.host_meta);
 }
 
 // The DAG's word buffer: from the admission's allocator when it has one (a server keeps its budget
@@ -850,6 +487,32 @@ void* alloc_words(cpvs_ctx* ctx, const Admit* admit, u64 words) {
 }
 
 inline dim3 grid1d(u32 n, u32 block = 256) { return dim3(ceil_div<u32>(n ? n : 1, block)); }
+
+// The small levels [Ls, R] of a build with these node counts (R + 1: none).
+int small_levels(const u64* cnt, int deepest, int R, bool use_table, bool leaf) {
+    int Ls = R + 1;
+    if (use_table && leaf)
+        for (int L = R; L >= std::max(deepest, 3) && cnt[L] <= kSmallMax; --L) Ls = L;
+    return Ls;
+}
+int deepest_level(const u64* cnt, int bottom, int R) {
+    int d = R;  // lowest level with nodes (the counts are exact)
+    while (d > bottom && cnt[d - 1] > 0) --d;
+    return d;
+}
+// Slots of level L's table (0: the root and absent levels have none).  With the sort merge one entry
+// per node.
+u32 level_slots(const u64* cnt, int L, int R, int Ls, bool use_table, bool leaf, bool small_leaf) {
+    if (L >= R || !cnt[L]) return 0;
+    if (!use_table) return (u32)cnt[L];
+    if (L >= Ls) return small_slots((u32)cnt[L]);
+    return (leaf && L == 2) ? leaf_table_slots((u32)cnt[L], small_leaf) : table_slots((u32)cnt[L]);
+}
+u64 bound_words_of(const u64* cnt, int bottom, int R, bool leaf) {
+    u64 w = 0;
+    for (int L = bottom; L <= R; ++L) w += cnt[L] + ((L > bottom) ? cnt[L - 1] : 0) + ((leaf && L == 2) ? 16 * cnt[L] : 0);
+    return w;
+}
 
 constexpr int kRetryWithSort = -1000;
 constexpr int kRetryFullTable = -1001;
@@ -957,31 +620,18 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     // --- scratch sizing ----------------------------------------------------------------------
     u32 cmax = 1;
     for (int L = bottom; L < R; ++L) cmax = cnt[L] > cmax ? (u32)cnt[L] : cmax;
-    const u32 S = table_slots(cmax);
     const u32 scan_n = (leaf && ncol > cmax) ? ncol : cmax;
-    size_t need = meta_bytes + col_bytes;
-    for (int L = bottom; L <= R; ++L) {
-        const size_t c = cnt[L] ? cnt[L] : 1;
-        need += arena_bytes(c, 8) + 5 * arena_bytes(c, 4);
-    }
     const size_t c2 = leaf ? (cnt[2] ? cnt[2] : 1) : 1;
-    if (leaf) need += arena_bytes(c2 * 8, 8) + 2 * arena_bytes(c2, 4);  // leafmask rows, run heads, column map
-    need += 2 * arena_bytes(cmax, 4);
     const bool col_list = leaf && T > 1;  // compact the z-tile's columns with leaf nodes
-    if (col_list) need += arena_bytes(ncol, 4) + arena_bytes(1, 4);
-    if (use_table) need += arena_bytes(S, 8);
-    else need += 4 * arena_bytes(cmax, 4) + arena_bytes(sort_scratch_words(cmax), 4);
-    need += arena_bytes(scan_scratch_words(scan_n), 4);
-    need += 1 << 20;
+    const int deepest = deepest_level(cnt, bottom, R);
+    const int Ls = small_levels(cnt, deepest, R, use_table, leaf);
     // Pre-merge words bound the DAG: mask and child pointers per node, two words per partial slice
     // at the leaves.  The words are written into a staging area of that size right behind the
     // merge (no host readback before the write), then copied to an exact allocation; a caller's
-    // output buffer (into) is written directly after the readback instead.
-    u64 bound_words = 0;
-    for (int L = bottom; L <= R; ++L)
-        bound_words += cnt[L] + ((L > bottom) ? cnt[L - 1] : 0) + ((leaf && L == 2) ? 16 * cnt[L] : 0);
+    // output buffer (into) is written directly.
+    const u64 bound_words = bound_words_of(cnt, bottom, R, leaf);
     const bool staged = !into;
-    if (staged) need += arena_bytes(bound_words + 17, 4);  // 17 words of slack for the bound check
+    const size_t need = build_scratch_bytes(cnt, R, leaf, ncol, col_list, use_table, small_leaf, staged);
     if (admit) {
         rc = admit->fn(admit->user, A, need, 4 * bound_words);
         if (rc) return rc;
@@ -998,38 +648,54 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     // meta is zeroed by the first kernel below (k_small_topdown or k_start).
 
     Level lv[kMaxLevels];
+    u32 ntiles = 0;
+    size_t tab_slots = 0, clear_slots = 0;  // of all levels; of those whose tables a launch must clear
     for (int L = bottom; L <= R; ++L) {
         const size_t c = cnt[L] ? cnt[L] : 1;
+        const bool is_leaf = leaf && L == 2;
         lv[L].count = (u32)cnt[L];
-        lv[L].coord = A.take<u64>(c);
+        lv[L].coord = is_leaf ? nullptr : A.take<u64>(c);
         lv[L].mask = A.take<u32>(c);
-        lv[L].cstart = A.take<u32>(c);
-        lv[L].rank = A.take<u32>(c);
+        lv[L].cstart = is_leaf ? nullptr : A.take<u32>(c);
+        lv[L].id = A.take<u32>(c);
         lv[L].uniq = A.take<u32>(c);
         lv[L].off = A.take<u32>(c);
+        lv[L].first = A.take<u64>(first_words((u32)c));
+        lv[L].slots = level_slots(cnt, L, R, Ls, use_table, leaf, small_leaf);
+        tab_slots += lv[L].slots;
+        if (L < Ls) clear_slots += lv[L].slots;
+        ntiles += ceil_div<u32>((u32)cnt[L], kTileNodes);
     }
+    u64* tab = A.take<u64>(tab_slots);
+    {
+        u64* t0 = tab;  // deepest level first: the tables to clear are one run
+        for (int L = bottom; L <= R; ++L) {
+            lv[L].tab = t0;
+            t0 += lv[L].slots;
+        }
+    }
+    u32* tile_sums = A.take<u32>(ntiles);
+    u64* tile_pre = A.take<u64>(ntiles);
     u64* leafm = leaf ? A.take<u64>(c2 * 8) : nullptr;
     // The run heads' key hashes, from the leaf kernel to the leaf insert, in the place of the leaf
-    // level's unique list and offsets (two arrays side by side), which the ranks scan writes later.
+    // level's unique list and offsets (two arrays side by side), which k_offsets writes later.
     const bool lane_leaf = leaf && (col_list ? std::min<u64>(ncol, cnt[2]) : ncol) >= kLaneLeafMin;
     u64* leaf_hash = lane_leaf ? reinterpret_cast<u64*>(lv[2].uniq) : nullptr;
     u32* runhead = leaf ? A.take<u32>(c2) : nullptr;
     u32* colbfs = leaf ? A.take<u32>(c2) : nullptr;
     u32* clist = col_list ? A.take<u32>(ncol) : nullptr;
     u32* nclist = col_list ? A.take<u32>(1) : nullptr;
-    u32* rep = A.take<u32>(cmax);
-    u32* tslot = A.take<u32>(cmax);  // table slot of each node, or segment starts when sorting
-    u32* seg = tslot;
-    u64* tab = use_table ? A.take<u64>(S) : nullptr;
-    u32 *skey = nullptr, *sval = nullptr, *ktmp = nullptr, *vtmp = nullptr, *sort_scratch = nullptr;
+    SortScratch srt{};
     if (!use_table) {
-        skey = A.take<u32>(cmax);
-        sval = A.take<u32>(cmax);
-        ktmp = A.take<u32>(cmax);
-        vtmp = A.take<u32>(cmax);
-        sort_scratch = A.take<u32>(sort_scratch_words(cmax));
+        srt.skey = A.take<u32>(cmax);
+        srt.sval = A.take<u32>(cmax);
+        srt.ktmp = A.take<u32>(cmax);
+        srt.vtmp = A.take<u32>(cmax);
+        srt.seg = A.take<u32>(cmax);
+        srt.sort_scratch = A.take<u32>(sort_scratch_words(cmax));
     }
     u32* scan_scratch = A.take<u32>(scan_scratch_words(scan_n));
+    srt.scan_scratch = scan_scratch;
     u32* staging = staged ? A.take<u32>(bound_words + 17) : nullptr;
     if (A.used > A.cap) {
         set_error("build: scratch layout exceeds its reservation (%zu > %zu)", A.used, A.cap);
@@ -1050,26 +716,22 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
 
     // --- 1/2. BFS classification -------------------------------------------------------------
     const u64 root = pack_xyz(0, 0, 2 * t);  // create(): root offset (0,0,2*zTileIndex)
-    int deepest = R;  // lowest level with nodes (the counts are exact)
-    while (deepest > bottom && cnt[deepest - 1] > 0) --deepest;
     // Small levels [Ls, R] go through the one-workgroup kernels (with the hash-table merge).
-    int Ls = R + 1;
-    if (use_table && leaf)
-        for (int L = R; L >= std::max(deepest, 3) && cnt[L] <= kSmallMax; --L) Ls = L;
     SmallArgs sa{};
     sa.R = R;
     sa.Ls = Ls;
     sa.deepest = deepest;
     sa.meta = meta;
-    sa.host_meta = reinterpret_cast<u32*>(pinned);
+    sa.n_below = (Ls - 1 >= bottom && Ls - 1 < R) ? std::max<u32>(lv[Ls - 1].count, 1u) : 1u;
+    sa.heads = (leaf && Ls == 3) ? runhead : nullptr;
     for (int L = bottom; L <= R; ++L) {
         sa.count[L] = lv[L].count;
         sa.coord[L] = lv[L].coord;
         sa.mask[L] = lv[L].mask;
         sa.cstart[L] = lv[L].cstart;
-        sa.rank[L] = lv[L].rank;
-        sa.uniq[L] = lv[L].uniq;
-        sa.off[L] = lv[L].off;
+        sa.id[L] = lv[L].id;
+        sa.tab[L] = lv[L].tab;
+        sa.slots[L] = lv[L].slots;
         sa.lv[L] = p->lv[L];
     }
     const int top_big = std::min(R, Ls - 1);  // highest level of the per-level path
@@ -1084,11 +746,10 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
             const u32 bound = col_list ? std::min(ncol, c) : ncol;
             const u32 units = ceil_div<u32>(bound, kLeafWaves * kLeafCols);
             const u32 unit_chunk = ceil_div<u32>(units, kXcds);
-            const u32 slots = use_table ? leaf_table_slots(c, small_leaf) : 0u;
-            // The leaf level is the first merged: its table is cleared by this kernel.
+            const u32 slots = use_table ? (u32)clear_slots : 0u;  // the merge's tables are cleared here
             if (lane_leaf) {
-                // (the list of slow columns lies where the representatives are written later)
-                const LeafOut lo{colbfs, lv[2].mask, leafm, runhead, leaf_hash, rep, meta + kMetaSlow, c};
+                // (the list of slow columns lies where the identities are written later)
+                const LeafOut lo{colbfs, lv[2].mask, leafm, runhead, leaf_hash, lv[2].id, meta + kMetaSlow, c};
                 const u32 tiles = ceil_div<u32>(bound, kLaneThreads);
                 const u32 chunk = ceil_div<u32>(tiles, kXcds);
                 if (col_list)
@@ -1101,7 +762,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
                 CPVS_LAUNCH("leaf_waves", (k_leaf_waves<true, kSlowCols>),
                             dim3(std::min(ceil_div<u32>(sbound, kLeafWaves * kSlowCols), kSlowWaves / kLeafWaves)),
                             dim3(64 * kLeafWaves), 0, s, lc, sbound, c, p->depth, N, T, p->lv[3], lv[2].mask, leafm, runhead,
-                            leaf_hash, 0u, tab, 0u, rep, meta + kMetaSlow);
+                            leaf_hash, 0u, tab, 0u, lv[2].id, meta + kMetaSlow);
             } else if (col_list)
                 CPVS_LAUNCH("leaf_waves", (k_leaf_waves<true, kLeafCols>), dim3(unit_chunk * kXcds), dim3(64 * kLeafWaves), 0, s, lc,
                             bound, c, p->depth, N, T, p->lv[3], lv[2].mask, leafm, runhead, nullptr, unit_chunk, tab,
@@ -1133,121 +794,36 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     }
     CPVS_HIP_CHECK(hipGetLastError());
 
-    // Levels merged below (not the root, not the small levels) whose word count surely fits 32
-    // bits get ranks and offsets from one 64-bit scan.
-    auto fused_sizes = [&](int L) {
-        const u64 per_node = (leaf && L == 2) ? 17ull : 9ull;
-        return L >= deepest && L < std::min(R, Ls) && (u64)lv[L].count * per_node < 0xFFFFFFFFull;
-    };
-    // With every larger level's offsets known from its ranks scan, the small-level merge also
-    // computes the small levels' offsets and all level bases (no separate compress launch).
-    sa.sizes_in_merge = 1u;
-    for (int L = deepest; L < std::min(R, Ls); ++L)
-        if (!fused_sizes(L)) sa.sizes_in_merge = 0u;
-
     // --- 3. merge, bottom-up (the root is never merged) --------------------------------------
+    MArgs ma{};
+    ma.leafm = leafm;
+    ma.heads = runhead;
+    ma.nleaf = (u32)c2;
+    u32 tile = 0;
+    for (int L = deepest; L <= R; ++L) {
+        const Level& v = lv[L];
+        ma.tile0[ma.nlev] = tile;
+        tile += ceil_div<u32>(v.count, kTileNodes);
+        ma.lv[ma.nlev++] = MLevel{v.mask, v.cstart, v.id, v.tab, v.first, v.uniq, v.off, v.count, v.slots, L,
+                                  (leaf && L == 2) ? 1u : 0u, L == R ? 1u : 0u};
+    }
+    ma.tile0[ma.nlev] = tile;
+    // Without a leaf level its kernel did not clear the tables.
+    if (use_table && clear_slots && !(leaf && deepest == 2))
+        CPVS_LAUNCH("table_clear", k_table_clear, grid1d((u32)clear_slots), dim3(256), 0, s, tab, (u32)clear_slots);
     for (int L = deepest; L < std::min(R, Ls); ++L) {
-        const u32 c = lv[L].count;
-        const bool is_leaf = leaf && L == 2;
-        const u32* child_rank = (L > deepest) ? lv[L - 1].rank : nullptr;
-        const u32* rh = is_leaf ? runhead : nullptr;
-        // Levels ranked by the 64-bit scan take its tile partials from k_resolve (table merge): no
-        // reduce pass.  Tiles of more than one round are summed with atomics into partials that the
-        // insert kernel clears.
-        u64* rpart = (use_table && fused_sizes(L)) ? reinterpret_cast<u64*>(scan_scratch) : nullptr;
-        const u32 rrounds = scan_rounds(c);
-        const u32 nzero = (rpart && rrounds > 1) ? ceil_div<u32>(c, rrounds * kScanThreads) : 0u;
-        if (use_table) {
-            const u32 Sl = is_leaf ? leaf_table_slots(c, small_leaf) : table_slots(c);
-            // Cleared by the leaf kernel (leaf level) or the previous level's k_rank_copies.
-            if (L == deepest && !is_leaf) CPVS_LAUNCH("table_clear", k_table_clear, grid1d(Sl), dim3(256), 0, s, tab, Sl);
-            if (is_leaf) {
-                CPVS_LAUNCH("insert_leaf", k_insert_leaf, dim3(ceil_div<u32>(c, kLeafWindow)), dim3(kLeafInsertThreads), 0, s,
-                            lv[2].mask, leafm, runhead, leaf_hash, c, tab, Sl, tslot, meta + kMetaFull, rpart, nzero,
-                            ctx->leaf_hash_bits.load());
-                CPVS_LAUNCH("resolve", k_resolve<LeafEq>, grid1d(c, kNodeThreads), dim3(kNodeThreads), 0, s, tslot, tab, runhead, c,
-                            LeafEq{lv[2].mask, leafm, nullptr, c}, rep, meta + kMetaColl, lv[2].mask, 1u, rpart, rrounds);
-            } else {
-                CPVS_LAUNCH("insert_inner", k_insert_inner, grid1d(c, kInsertBlock), dim3(kInsertBlock), 0, s, lv[L].mask,
-                            lv[L].cstart, child_rank, c,
-                            tab, Sl, tslot, meta + kMetaFull, rpart, nzero, ctx->inner_hash_bits.load());
-                CPVS_LAUNCH("resolve", k_resolve<InnerEq>, grid1d(c, kNodeThreads), dim3(kNodeThreads), 0, s, tslot, tab, nullptr, c,
-                            InnerEq{lv[L].mask, lv[L].cstart, child_rank}, rep, meta + kMetaColl, lv[L].mask, 0u, rpart, rrounds);
-            }
-        } else {
-            if (is_leaf)
-                CPVS_LAUNCH("sortkeys", k_sortkeys_leaf, grid1d(c), dim3(256), 0, s, lv[2].mask, leafm, runhead, c, skey,
-                            sval);
-            else
-                CPVS_LAUNCH("sortkeys", k_sortkeys_inner, grid1d(c), dim3(256), 0, s, lv[L].mask, lv[L].cstart, child_rank, c,
-                            skey, sval);
-            radix_sort_pairs(skey, sval, ktmp, vtmp, c, 32, sort_scratch, s);
-            device_scan(SegHeadIn{skey}, SegStartOut{seg}, c, OpMax{}, nullptr, scan_scratch, s);
-            if (is_leaf)
-                CPVS_LAUNCH("representative", k_representative<LeafEq>, grid1d(c), dim3(256), 0, s, sval, seg, c,
-                            LeafEq{lv[2].mask, leafm, runhead, c}, rep, meta + kMetaSortColl);
-            else
-                CPVS_LAUNCH("representative", k_representative<InnerEq>, grid1d(c), dim3(256), 0, s, sval, seg, c,
-                            InnerEq{lv[L].mask, lv[L].cstart, child_rank}, rep, meta + kMetaSortColl);
-            rh = nullptr;  // every node got its representative directly
-        }
-        if (fused_sizes(L) && rpart)  // tile partials came from k_resolve
-            device_scan_from_partials(FirstSizeIn{rep, lv[L].mask, is_leaf ? 1u : 0u},
-                                      FirstSizeOut{lv[L].rank, lv[L].uniq, lv[L].off, meta + kMetaU + L, meta + kMetaS + L, c},
-                                      c, OpSum64{}, nullptr, rpart, s);
-        else if (fused_sizes(L))
-            device_scan(FirstSizeIn{rep, lv[L].mask, is_leaf ? 1u : 0u},
-                        FirstSizeOut{lv[L].rank, lv[L].uniq, lv[L].off, meta + kMetaU + L, meta + kMetaS + L, c}, c, OpSum64{},
-                        nullptr, scan_scratch, s);
+        if (use_table)
+            merge_insert(ma, L - deepest, leaf_hash, meta,
+                         (leaf && L == 2) ? ctx->leaf_hash_bits.load() : ctx->inner_hash_bits.load(), s);
         else
-            device_scan(FirstFlagIn{rep}, FirstRankOut{lv[L].rank, lv[L].uniq}, c, OpSum{}, meta + kMetaU + L, scan_scratch, s);
-        const u32 S_next = (use_table && L + 1 < std::min(R, Ls)) ? table_slots(lv[L + 1].count) : 0u;
-        CPVS_LAUNCH("rank_copies", k_rank_copies, grid1d(c, kNodeThreads), dim3(kNodeThreads), 0, s, rep, rh, c, lv[L].rank, tab, S_next);
+            merge_sort_level(ma, L - deepest, srt, meta, s);
     }
-    if (Ls <= R)
-        CPVS_LAUNCH("small_merge", k_small_merge, dim3(1), dim3(kSmallThreads), 0, s, sa);
-    else
-        CPVS_LAUNCH("root_init", k_root_init, dim3(1), dim3(1), 0, s, lv[R].rank, lv[R].uniq, meta + kMetaU + R);
+    if (Ls < R) CPVS_LAUNCH("small_insert", k_small_insert, dim3(1), dim3(kSmallThreads), 0, s, sa);
+    // --- 4. first occurrences, offsets, bases, words; one readback -------------------------
+    merge_finish(ma, !use_table, tile_sums, tile_pre, meta, R, reinterpret_cast<u32*>(pinned), s);
+    merge_write(ma, meta, staged ? staging : into->words, staged ? bound_words : into->cap, s);
     CPVS_HIP_CHECK(hipGetLastError());
-
-    // --- 4. compress: sizes, bases, one readback, write -------------------------------------
-    for (int L = top_big; L >= deepest; --L) {
-        if (fused_sizes(L)) continue;  // offsets came with the ranks
-        const u32 c = lv[L].count;
-        const u32 is_leaf = (leaf && L == 2) ? 1u : 0u;
-        device_scan(UniqueSizeIn{lv[L].uniq, lv[L].mask, meta + kMetaU + L, is_leaf},
-                    UniqueOffOut{lv[L].off, meta + kMetaU + L, meta + kMetaS + L, c}, c, OpSum64{}, nullptr, scan_scratch, s);
-    }
-    if (Ls <= R) {
-        if (!sa.sizes_in_merge) CPVS_LAUNCH("small_compress", k_small_compress, dim3(1), dim3(kSmallThreads), 0, s, sa);
-    } else {
-        CPVS_LAUNCH("level_bases", k_level_bases, dim3(1), dim3(128), 0, s, meta, R, deepest, lv[R].mask,
-                    reinterpret_cast<u32*>(pinned));
-    }
-    // The word writer's per-level arrays (the counts and bases come from meta or the readback).
-    WriteArgs wa{};
-    u32 wmax = 0;  // blocks of the largest possible write (every node unique)
-    for (int L = R; L >= deepest; --L) {
-        WriteLevel& w = wa.lv[wa.nlev++];
-        const bool kids = L > deepest;
-        w.uniq = lv[L].uniq;
-        w.mask = lv[L].mask;
-        w.cstart = lv[L].cstart;
-        w.off = lv[L].off;
-        w.child_rank = kids ? lv[L - 1].rank : nullptr;
-        w.child_off = kids ? lv[L - 1].off : nullptr;
-        w.child_n = kids ? std::max<u32>(lv[L - 1].count, 1u) : 1u;
-        w.leaf = (leaf && L == 2) ? 1u : 0u;
-        w.L = L;
-        wmax += ceil_div<u32>(lv[L].count ? lv[L].count : 1, kNodeThreads);
-    }
-    wa.leafm = leafm;
-    wa.nleaf = (u32)c2;
-    if (staged)
-        CPVS_LAUNCH("write_levels", k_write_levels_dev, dim3(std::min<u32>(wmax, 2048)), dim3(kNodeThreads), 0, s, wa, meta,
-                    staging, bound_words + 17);
-    CPVS_HIP_CHECK(hipGetLastError());
-    CPVS_HIP_CHECK(hipStreamSynchronize(s));  // the bases kernel copied meta into pinned
+    CPVS_HIP_CHECK(hipStreamSynchronize(s));  // k_totals copied meta into pinned
     u32 hm[kMetaWords];
     std::memcpy(hm, pinned, sizeof(hm));
 
@@ -1277,39 +853,24 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
                   (unsigned long long)into->cap);
         return CPVS_EINVAL;
     }
-    u32* d_words = into ? into->words : static_cast<u32*>(alloc_words(ctx, admit, total ? total : 1));
-    if (!d_words) {
-        set_error("build: hipMalloc of %llu DAG words failed", (unsigned long long)total);
-        return CPVS_ENOMEM;
-    }
-    if (staged) {
-        if (total) CPVS_LAUNCH("copy_words", k_copy_words, dim3(std::min<u64>(ceil_div<u64>(total, 1024), 4096)),
-                               dim3(256), 0, s, staging, d_words, total);
-    } else {
-        u32 wblocks = 0;
-        for (int k = 0; k < wa.nlev; ++k) {
-            WriteLevel& w = wa.lv[k];
-            w.U = hm[kMetaU + w.L];
-            w.base = hm[kMetaB + w.L];
-            w.child_base = w.child_rank ? hm[kMetaB + w.L - 1] : 0u;
-            wa.first[k] = wblocks;
-            wblocks += ceil_div<u32>(w.U, kNodeThreads);
-        }
-        wa.first[wa.nlev] = wblocks;
-        if (wblocks) CPVS_LAUNCH("write_levels", k_write_levels, dim3(wblocks), dim3(kNodeThreads), 0, s, wa, d_words);
-    }
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) {
-        if (!into) ctx->buffers.give(d_words);
-        return hip_fail(e, "build write", __FILE__, __LINE__);
-    }
     if (into) {
         into->nwords = total;
         into->root_mask = hm[kMetaRoot];
         return CPVS_OK;
     }
-
+    u32* d_words = static_cast<u32*>(alloc_words(ctx, admit, total ? total : 1));
+    if (!d_words) {
+        set_error("build: hipMalloc of %llu DAG words failed", (unsigned long long)total);
+        return CPVS_ENOMEM;
+    }
+    if (total) CPVS_LAUNCH("copy_words", k_copy_words, dim3(std::min<u64>(ceil_div<u64>(total, 1024), 4096)), dim3(256), 0, s,
+                           staging, d_words, total);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) {
+        ctx->buffers.give(d_words);
+        return hip_fail(e, "build write", __FILE__, __LINE__);
+    }
     cpvs_dag* d = new cpvs_dag();
     d->ctx = ctx;
     d->n = n;
@@ -1331,6 +892,33 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
 }
 
 }  // namespace
+
+// What build_once lays out: cnt the nodes per level (bottom .. R), ncol the leaf columns.
+size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_list, bool use_table, bool small_leaf,
+                           bool staged) {
+    const int bottom = leaf ? 2 : 0;
+    const int Ls = small_levels(cnt, deepest_level(cnt, bottom, R), R, use_table, leaf);
+    size_t need = arena_bytes(kMetaWords, sizeof(u32)) + (leaf ? arena_bytes(ncol, sizeof(uint4)) : 0);
+    u32 cmax = 1, ntiles = 0;
+    size_t slots = 0;
+    for (int L = bottom; L <= R; ++L) {
+        const size_t c = cnt[L] ? cnt[L] : 1;
+        if (L < R) cmax = cnt[L] > cmax ? (u32)cnt[L] : cmax;
+        const bool is_leaf = leaf && L == 2;
+        need += (is_leaf ? 0 : arena_bytes(c, 8) + arena_bytes(c, 4)) + 4 * arena_bytes(c, 4) +
+                arena_bytes(first_words((u32)c), 8);
+        slots += level_slots(cnt, L, R, Ls, use_table, leaf, small_leaf);
+        ntiles += ceil_div<u32>((u32)cnt[L], kTileNodes);
+    }
+    need += arena_bytes(slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(ntiles, 8);
+    const size_t c2 = leaf ? (cnt[2] ? cnt[2] : 1) : 1;
+    if (leaf) need += arena_bytes(c2 * 8, 8) + 2 * arena_bytes(c2, 4);  // leafmask rows, run heads, column map
+    if (col_list) need += arena_bytes(ncol, 4) + arena_bytes(1, 4);
+    if (!use_table) need += 5 * arena_bytes(cmax, 4) + arena_bytes(sort_scratch_words(cmax), 4);
+    need += arena_bytes(scan_scratch_words((leaf && ncol > cmax) ? ncol : cmax), 4);
+    if (staged) need += arena_bytes(bound_words_of(cnt, bottom, R, leaf) + 17, 4);
+    return need + (1 << 20);
+}
 
 // A build that finds its merge table too small runs again with a full-size table, one with a key
 // collision again with the sort merge, and one whose counts exceed the emitted nodes again with

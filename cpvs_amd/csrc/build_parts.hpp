@@ -483,32 +483,50 @@ __device__ inline void leaf_lanes(const LeafCol& c, const LeafOut& o) {
     if (slow && k < o.nleaf) o.slow[k] = c.col;
 }
 
-// Children ranks of inner node i (slots j >= k are 0).  All eight loads are issued before any is
-// used, so a node costs one memory round trip, not one per child.
-__device__ inline void load_child_ranks(const u32* cstart, const u32* child_rank, u32 i, u32 k, u32 r[8]) {
-    const u32 s = k ? cstart[i] : 0u;
+// The identity of each node of a level for its parents' keys: equal for equal subtrees, different
+// otherwise (up to hash collisions, which k_resolve finds): the node's merge-table slot, or its first
+// occurrence's index with the sort merge.  With heads set the level is the leaf level and only runs'
+// first nodes (heads[c] == c) have theirs yet: a child takes its run's, and it is stored for the
+// child as well (each node has one parent).
+struct ChildIds {
+    u32* id;
+    const u32* heads;
+    u32 n;  // nodes of the level: bounds every index (first children past a level's emitted nodes)
+};
+
+// Identities of k children from node s on (entries j >= k are 0).  All loads of a stage are issued
+// before any is used, so a node costs one memory round trip per stage, not one per child.
+__device__ inline void load_child_ids(const ChildIds& c, u32 s, u32 k, u32 r[8]) {
+    u32 at[8];
 #pragma unroll
-    for (u32 j = 0; j < 8; ++j) r[j] = (j < k) ? child_rank[s + j] : 0u;
+    for (u32 j = 0; j < 8; ++j) at[j] = min(s + j, c.n - 1);
+    if (!c.heads) {
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j) r[j] = (j < k) ? c.id[at[j]] : 0u;
+        return;
+    }
+    u32 h[8];
+#pragma unroll
+    for (u32 j = 0; j < 8; ++j) h[j] = (j < k) ? c.heads[at[j]] : 0u;
+#pragma unroll
+    for (u32 j = 0; j < 8; ++j) r[j] = (j < k) ? c.id[min(h[j], c.n - 1)] : 0u;
+#pragma unroll
+    for (u32 j = 0; j < 8; ++j)
+        if (j < k && h[j] != at[j]) c.id[at[j]] = r[j];
 }
 
-// Key hash of an inner node: a sum of (mask, child ranks) times fixed odd 64-bit constants, whose
-// collisions need an exact zero of the differences' sum mod 2^64, then a mixer that is a bijection.
-// Two 32-bit multiplies per child instead of a chain of two 64-bit ones: in the one-workgroup
-// merge of the small levels, four waves per SIMD hash four nodes per thread and level, and the
-// chained form's multiplies alone were most of its time.
-__device__ inline u64 inner_key_hash(const u32* mask, const u32* cstart, const u32* child_rank, u32 i) {
+// Key hash of an inner node with mask m, k children and their identities r: a sum of (mask,
+// identities) times fixed odd 64-bit constants, whose collisions need an exact zero of the
+// differences' sum mod 2^64, then a mixer that is a bijection.  Two 32-bit multiplies per child
+// instead of a chain of two 64-bit ones: in the one-workgroup merge of the small levels, four waves
+// per SIMD hash four nodes per thread and level, and a chain's multiplies alone were much of its time.
+__device__ inline u64 inner_key_hash(u32 m, const u32 (&r)[8]) {
     constexpr u64 kMul[9] = {0x9E3779B97F4A7C15ull, 0xC2B2AE3D27D4EB4Full, 0x165667B19E3779F9ull, 0xD6E8FEB86659FD93ull,
                              0xA0761D6478BD642Full, 0xE7037ED1A0B428DBull, 0x8EBC6AF09C88C6E3ull, 0x589965CC75374CC3ull,
                              0x1D8E4E27C47D124Full};
-    const u32 m = mask[i];
-    const u32 k = num_children(m);
     u64 h = kHashSeed + m * kMul[8];
-    if (k) {
-        u32 r[8];
-        load_child_ranks(cstart, child_rank, i, k, r);
 #pragma unroll
-        for (u32 j = 0; j < 8; ++j) h += r[j] * kMul[j];  // (slots past the children are 0)
-    }
+    for (u32 j = 0; j < 8; ++j) h += r[j] * kMul[j];  // (entries past the children are 0)
     return mix64(h);
 }
 
@@ -550,19 +568,20 @@ struct LeafEq {
 struct InnerEq {
     const u32* mask;
     const u32* cstart;
-    const u32* child_rank;
+    const u32* child_id;  // null at the deepest level
+    u32 child_n;
     __device__ bool operator()(u32 a, u32 b) const {
-        // Masks and first-child indices are loaded together (one round trip before the ranks).
+        // Masks and first-child indices are loaded together (one round trip before the identities).
         const u32 m = mask[a], mb = mask[b];
         const u32 ca = cstart[a], cb = cstart[b];
         if (m != mb) return false;
-        const u32 k = num_children(m);
+        const u32 k = child_id ? num_children(m) : 0u;
         if (!k) return true;
         u32 ra[8], rb[8];
 #pragma unroll
         for (u32 j = 0; j < 8; ++j) {
-            ra[j] = (j < k) ? child_rank[ca + j] : 0u;
-            rb[j] = (j < k) ? child_rank[cb + j] : 0u;
+            ra[j] = (j < k) ? child_id[min(ca + j, child_n - 1)] : 0u;
+            rb[j] = (j < k) ? child_id[min(cb + j, child_n - 1)] : 0u;
         }
         bool eq = true;
 #pragma unroll
@@ -570,7 +589,6 @@ struct InnerEq {
         return eq;
     }
 };
-
 
 // Open addressing, linear probing.  Large groups of equal keys hit one slot, so the slot is read
 // first, and only an empty slot or a larger index costs an atomic.  A slot only ever goes from
@@ -582,9 +600,9 @@ struct InnerEq {
 // 104 µs against a plain load.
 // A probe gives up after kMaxProbes occupied slots (a table too small for its keys: the leaf
 // level's table is sized for a quarter of its nodes), counts that in *full and returns a slot in
-// range; the host then builds again with a larger table.  Node i's representative is then still a
-// node r with rep[r] = r (k_resolve reads whatever the returned slot holds and checks the keys),
-// so every index the rest of the build derives stays in range.
+// range; the host then builds again with a larger table (k_resolve reads whatever the returned slot
+// holds, bounds it and checks the keys, so every index that the rest of the build derives stays in
+// range).
 constexpr u32 kMaxProbes = 256;
 __device__ inline u32 table_insert(u64* tab, u32 S, u64 h, u32 i, u32* full) {
     const u32 tag = (u32)(h >> 32);
@@ -644,13 +662,6 @@ __device__ inline u32 table_insert_group(u64* tab, u32 S, u64 h, u32 i, bool act
     return active ? gs[ls] : 0u;
 }
 
-// zero[0 .. nzero): the ranks scan's tile partials that k_resolve adds into next (cleared here, in a
-// launch that runs anyway).
-__device__ inline void clear_partials(u64* zero, u32 nzero) {
-    const u32 stride = gridDim.x * blockDim.x;
-    for (u32 j = blockIdx.x * blockDim.x + threadIdx.x; j < nzero; j += stride) zero[j] = 0ull;
-}
-
 // The leaf level: only a run's first node is inserted (1.3 M of 6.7 M nodes at 8192^2), so each
 // thread takes kLeafPer nodes and a workgroup merges a window of kLeafWindow nodes in LDS.  The
 // window's distinct hashes are listed as they are found, and the list is spread over the threads
@@ -662,48 +673,8 @@ constexpr u32 kLeafSlots = 2 * kLeafWindow;  // LDS table at most half full, so 
 static_assert(kLeafSlots <= 65536, "LDS slot numbers are listed as 16-bit values");
 
 
-// Threads per workgroup of the one-thread-per-node merge and write kernels (at 8192^2, 128 and 256
-// tie; 512 and 1024 make resolve and the writes slower by 5-10 µs).
+// Threads per workgroup of the write kernels (at 8192^2, 128 and 256 tie; 512 and 1024 are slower).
 constexpr u32 kNodeThreads = 256;
-
-// With partials set, each workgroup also reduces the ranks scan's input over its nodes (FirstSizeIn:
-// 1 << 32 | the node's words, for a first occurrence) into the partial of the scan tile it lies in
-// (tiles of `rounds` workgroups: a store for one, an atomic add into a partial the insert kernel
-// cleared otherwise), so the scan that follows needs no reduce pass.
-static_assert(kNodeThreads == kScanThreads, "resolve workgroups are the ranks scan's rounds");
-template <class Eq>
-__global__ __launch_bounds__(kNodeThreads) void k_resolve(const u32* __restrict__ tslot, const u64* __restrict__ tab,
-                                                 const u32* __restrict__ runhead, u32 n, Eq eq, u32* __restrict__ rep,
-                                                 u32* __restrict__ collisions, const u32* __restrict__ mask, u32 leaf,
-                                                 u64* __restrict__ partials, u32 rounds) {
-    __shared__ u64 s_wave[kNodeThreads / kWave];
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    u64 v = 0;
-    if (i < n) {
-        if (runhead && runhead[i] != i) {
-            rep[i] = kNoRep;  // resolved through its run's first node
-        } else {
-            u32 r = (u32)tab[tslot[i]];  // the smallest index with this node's tag
-            if (r >= n) r = i;
-            if (r != i && !eq(i, r)) {
-                atomicAdd(collisions, 1u);  // two keys share a 64-bit hash: the build is redone by sorting
-                r = i;
-            }
-            rep[i] = r;
-            if (partials && r == i) v = (1ull << 32) | (u64)(1u + (num_children(mask[i]) << leaf));
-        }
-    }
-    if (partials) {  // uniform across the launch
-        v = block_reduce(v, s_wave, OpSum64{});
-        if (threadIdx.x == 0) {
-            if (rounds == 1)
-                partials[blockIdx.x] = v;
-            else if (v)
-                atomicAdd(reinterpret_cast<unsigned long long*>(partials + blockIdx.x / rounds), (unsigned long long)v);
-        }
-    }
-}
-
 
 // Segment start of each sorted position: max-scan of (key differs from predecessor ? p : 0).
 struct SegHeadIn {
@@ -741,87 +712,6 @@ __global__ __launch_bounds__(256) void k_representative(const u32* __restrict__ 
 }
 
 
-struct FirstFlagIn {
-    const u32* rep;
-    __device__ u32 operator()(u32 i) const { return rep[i] == i ? 1u : 0u; }
-};
-struct FirstRankOut {
-    u32* rank;
-    u32* uniq;
-    __device__ void operator()(u32 i, u32 ex, u32 first) const {
-        if (first) {
-            rank[i] = ex;
-            uniq[ex] = i;
-        }
-    }
-};
-
-// Ranks and word offsets in one scan: first occurrences in index order are the uniques in rank
-// order, so a scan of (first ? 1 : 0, first ? node size : 0) -- packed as a u64 whose halves
-// cannot carry (size sums stay below 2^32) -- gives each first occurrence its rank and its offset.
-struct FirstSizeIn {
-    const u32* rep;
-    const u32* mask;
-    u32 leaf;  // 1 at the leafmask level (two words per partial child)
-    __device__ u64 operator()(u32 i) const {
-        const u32 r = rep[i], m = mask[i];  // both loads issued together (a select, not a branch)
-        const u64 v = (1ull << 32) | (u64)(1u + (num_children(m) << leaf));
-        return (r == i) ? v : 0ull;
-    }
-};
-struct FirstSizeOut {
-    u32* rank;
-    u32* uniq;
-    u32* off;
-    u32* n_uniq;  // device: the level's unique count
-    u32* words;   // device: the level's word count
-    u32 n;
-    __device__ void operator()(u32 i, u64 ex, u64 v) const {
-        if (v) {
-            const u32 r = (u32)(ex >> 32);
-            rank[i] = r;
-            uniq[r] = i;
-            off[r] = (u32)ex;
-        }
-        if (i == n - 1) {
-            const u64 t = ex + v;
-            *n_uniq = (u32)(t >> 32);
-            *words = (u32)t;
-        }
-    }
-};
-
-
-// Sizes of the unique nodes of a level whose word count may pass 2^32 (the levels not ranked by
-// the fused 64-bit scan hold at least 2^32 / 17 nodes).  The sums run in 64 bits; an offset or a
-// level total at or above 2^32 is stored saturated, so the host sees the overflow and rejects the
-// DAG before anything is written.
-struct UniqueSizeIn {
-    const u32* uniq;
-    const u32* mask;
-    const u32* n_uniq;  // device count of uniques of the level
-    u32 leaf;           // 1 at the leafmask level (two words per partial child)
-    __device__ u64 operator()(u32 r) const {
-        if (r >= *n_uniq) return 0ull;
-        return 1ull + (u64)(num_children(mask[uniq[r]]) << leaf);
-    }
-};
-
-__device__ inline u32 saturate32(u64 v) { return v > 0xFFFFFFFFull ? 0xFFFFFFFFu : (u32)v; }
-
-// Offsets of the unique nodes only (the scan runs over the level's node count, which the host
-// knows, while the unique count is on the device), and the level's word count.
-struct UniqueOffOut {
-    u32* off;
-    const u32* n_uniq;
-    u32* words;  // device: the level's word count (saturated)
-    u32 n;
-    __device__ void operator()(u32 r, u64 ex, u64 v) const {
-        if (r < *n_uniq) off[r] = saturate32(ex);
-        if (r == n - 1) *words = saturate32(ex + v);
-    }
-};
-
 // Device metadata block (u32 words).
 enum : int {
     kMetaU = 0,                          // uniques per level
@@ -838,51 +728,6 @@ enum : int {
 };
 
 
-// Unique node r of an inner level: [mask, absolute offsets of its partial children].
-// child_n (the child level's nodes) bounds the child ranks read as indices: ranks past a level's
-// emitted children were never written (the host then rejects the build's words).
-__device__ inline void write_inner_node(u32 r, const u32* __restrict__ uniq, const u32* __restrict__ mask,
-                                        const u32* __restrict__ cstart, const u32* __restrict__ off, u32 base,
-                                        const u32* __restrict__ child_rank, const u32* __restrict__ child_off, u32 child_base,
-                                        u32 child_n, u32* __restrict__ out) {
-    const u32 i = uniq[r];
-    const u32 o = base + off[r];
-    const u32 m = mask[i];
-    out[o] = m;
-    const u32 k = num_children(m);
-    if (!k) return;
-    u32 cr[8];
-    load_child_ranks(cstart, child_rank, i, k, cr);
-    u32 co[8];
-#pragma unroll
-    for (u32 j = 0; j < 8; ++j) co[j] = (j < k) ? child_off[min(cr[j], child_n - 1)] : 0u;
-#pragma unroll
-    for (u32 j = 0; j < 8; ++j)
-        if (j < k) out[o + 1 + j] = child_base + co[j];
-}
-
-// Unique leaf node r: [mask, (lo, hi) of each partial slice's leafmask].
-__device__ inline void write_leaf_node(u32 r, const u32* __restrict__ uniq, const u32* __restrict__ mask,
-                                       const u64* __restrict__ leafm, u32 nleaf, const u32* __restrict__ off, u32 base,
-                                       u32* __restrict__ out) {
-    const u32 i = min(uniq[r], nleaf - 1);  // a first occurrence, which heads its run: its own row
-    const u32 o = base + off[r];
-    const u32 m = mask[i];
-    out[o] = m;
-    const u32 k = num_children(m);
-    const u64* p = leafm + (size_t)i * 8;
-    u64 v[8];
-#pragma unroll
-    for (u32 j = 0; j < 8; ++j) v[j] = (j < k) ? p[j] : 0ull;
-#pragma unroll
-    for (u32 j = 0; j < 8; ++j)
-        if (j < k) {
-            out[o + 1 + 2 * j] = (u32)v[j];
-            out[o + 2 + 2 * j] = (u32)(v[j] >> 32);
-        }
-}
-
-
 // Launches over this many columns walk them one per lane (a map's are then at least 16 x 16).
 constexpr u64 kLaneLeafMin = 1u << 15;
 constexpr u32 kSlowCols = 1;
@@ -897,26 +742,5 @@ inline u32 table_slots(u32 n) {
 // node (measured: 256^2 and 512^2 maps fill 85-96% of a quarter-size table, 1024^2 40%, 8192^2 4%).
 constexpr u32 kSmallLeafTableMin = 1u << 20;
 inline u32 leaf_table_slots(u32 c, bool small) { return table_slots((small && c >= kSmallLeafTableMin) ? c / 4 : c); }
-
-// Non-template kernels defined in build.hip.
-__global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 S);
-__global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
-                                                                    const u32* __restrict__ runhead,
-                                                                    const u64* __restrict__ hash, u32 n,
-                                                                    u64* __restrict__ tab, u32 S, u32* __restrict__ tslot,
-                                                                    u32* __restrict__ full, u64* __restrict__ zero,
-                                                                    u32 nzero, u32 hbits);
-__global__ __launch_bounds__(kInsertBlock) void k_insert_inner(const u32* __restrict__ mask, const u32* __restrict__ cstart,
-                                                               const u32* __restrict__ child_rank, u32 n, u64* __restrict__ tab,
-                                                               u32 S, u32* __restrict__ tslot, u32* __restrict__ full,
-                                                               u64* __restrict__ zero, u32 nzero, u32 hbits);
-__global__ __launch_bounds__(256) void k_sortkeys_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
-                                                       const u32* __restrict__ runhead,
-                                                       u32 n, u32* __restrict__ skey, u32* __restrict__ sval);
-__global__ __launch_bounds__(256) void k_sortkeys_inner(const u32* __restrict__ mask, const u32* __restrict__ cstart,
-                                                        const u32* __restrict__ child_rank, u32 n, u32* __restrict__ skey,
-                                                        u32* __restrict__ sval);
-__global__ __launch_bounds__(kNodeThreads) void k_rank_copies(const u32* __restrict__ rep, const u32* __restrict__ runhead, u32 count,
-                                                     u32* __restrict__ rank, u64* __restrict__ tab, u32 tab_slots);
 
 }  // namespace cpvs

@@ -513,30 +513,17 @@ int cpvs_estimate_build(cpvs_ctx* ctx, const cpvs_pyramid* p, uint32_t t, uint32
     u64 cnt[kMaxLevels] = {};
     sum_node_counts(lay, pinned_partials(ctx->pinned), cnt);
     cnt[R] = 1;
-    u64 cmax = 1, per_level = 0, words = 0;
-    for (int L = bottom; L <= R; ++L) {
-        const u64 c = cnt[L] ? cnt[L] : 1;
-        cmax = c > cmax ? c : cmax;
-        per_level += arena_bytes(c, 8) + 5 * arena_bytes(c, 4);
-        // Pre-merge words: mask + one pointer per child (two words per partial slice at leaves).
+    u64 words = 0;
+    // Pre-merge words: mask + one pointer per child (two words per partial slice at leaves).
+    for (int L = bottom; L <= R; ++L)
         words += cnt[L] + ((L > bottom) ? cnt[L - 1] : 0) + ((bottom == 2 && L == 2) ? 16 * cnt[L] : 0);
-    }
-    const u64 c2 = (bottom == 2) ? (cnt[2] ? cnt[2] : 1) : 0;
-    const u64 ncol = (bottom == 2) ? (u64)(p->N >> 3) * (p->N >> 3) : 0;
-    const u64 leaf = (bottom == 2) ? arena_bytes(c2 * 8, 8) + 2 * arena_bytes(c2, 4) +
-                                         arena_bytes(ncol, 16)
-                                   : 0;
-    u64 slots = 1024;
-    while (slots < cmax + cmax / 2 + 1) slots <<= 1;
-    const u64 merge = (ctx->merge_mode == CPVS_MERGE_TABLE)
-                          ? arena_bytes(slots, 8)
-                          : 4 * arena_bytes(cmax, 4) + arena_bytes(sort_scratch_words((u32)cmax), 4);
-    const u64 temps = 2 * arena_bytes(cmax, 4) + merge + arena_bytes(scan_scratch_words((u32)(cmax > ncol ? cmax : ncol)), 4) +
-                      (1 << 20);
+    const u32 ncol = leafm ? (p->N >> 3) * (p->N >> 3) : 0u;
     if (nodes)
         for (int L = 0; L < n; ++L) nodes[L] = cnt[L];
-    // The words are staged at their pre-merge bound before the exact allocation.
-    if (scratch_bytes) *scratch_bytes = per_level + leaf + temps + arena_bytes(words + 17, 4);
+    // (with a full-size leaf table, which a build may fall back to)
+    if (scratch_bytes)
+        *scratch_bytes = build_scratch_bytes(cnt, R, leafm, ncol, leafm && T > 1, ctx->merge_mode == CPVS_MERGE_TABLE, false,
+                                             true);
     if (max_dag_bytes) *max_dag_bytes = 4 * words;
     return CPVS_OK;
     GUARD_END

@@ -22,7 +22,7 @@
 #include <cstring>
 #include <vector>
 
-#include "build_parts.hpp"
+#include "merge.hpp"
 
 namespace cpvs {
 
@@ -122,7 +122,10 @@ struct FLevels {
     u64* coord[kMaxLevels];
     u32* mask[kMaxLevels];
     u32* cstart[kMaxLevels];
-    u32* rank[kMaxLevels];
+    u32* id[kMaxLevels];
+    u64* tab[kMaxLevels];  // (k_offsets) rank << 32 | word offset of a first occurrence, at its identity
+    u32 slots[kMaxLevels];
+    u32 count[kMaxLevels];
     u32* uniq[kMaxLevels];
     u32* off[kMaxLevels];
 };
@@ -358,14 +361,16 @@ __global__ void k_forest_bases(const FItem* __restrict__ items, u32 M, FLevels l
             const u32 s = seg[k];
             u32 S = 0, U = 0, o0 = 0;
             if (s != kNone) {
-                // Ranks bounded by the level's unique nodes: a rank past the level's emitted children
-                // was never written (the host then rejects the forest's words).
-                const u32 Ul = meta[kMetaU + L], rmax = Ul ? Ul - 1 : 0u;
-                const u32 r0 = min(lv.rank[L][s], rmax);
-                o0 = lv.off[L][r0];
+                // A segment's first node is a first occurrence (keys hold the DAG's index): its rank and
+                // offset.  The identity is bounded: past a level's emitted children it was never
+                // written (the host then rejects the forest's words).
+                const u32 Ul = meta[kMetaU + L];
+                auto at = [&](u32 node) { return lv.tab[L][min(lv.id[L][node], lv.slots[L] - 1)]; };
+                const u64 v0 = at(s);
+                o0 = (u32)v0;
                 const u32 e = nxt[k];
-                const u32 r1 = (e != kNone) ? min(lv.rank[L][e], rmax) : Ul;
-                const u32 o1 = (e != kNone) ? lv.off[L][r1] : meta[kMetaS + L];
+                const u64 v1 = (e != kNone) ? at(e) : (((u64)Ul << 32) | meta[kMetaS + L]);
+                const u32 r0 = (u32)(v0 >> 32), r1 = (u32)(v1 >> 32), o1 = (u32)v1;
                 S = o1 - o0;
                 U = r1 - r0;
             }
@@ -423,12 +428,12 @@ __global__ __launch_bounds__(kNodeThreads) void k_forest_write(FWriteArgs a, FLe
             }
         return;
     }
-    u32 cr[8];
-    load_child_ranks(lv.cstart[L], lv.rank[L - 1], i, kc, cr);
-    const u32 cb = B[gk - 1], co0 = base_off[gk - 1];
-    u32 co[8];
+    const u32 cb = B[gk - 1], co0 = base_off[gk - 1], s = lv.cstart[L][i];
+    u32 id[8], co[8];
 #pragma unroll
-    for (u32 j = 0; j < 8; ++j) co[j] = (j < kc) ? lv.off[L - 1][cr[j]] : 0u;
+    for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? lv.id[L - 1][min(s + j, lv.count[L - 1] - 1)] : 0u;
+#pragma unroll
+    for (u32 j = 0; j < 8; ++j) co[j] = (j < kc) ? (u32)lv.tab[L - 1][min(id[j], lv.slots[L - 1] - 1)] : 0u;
 #pragma unroll
     for (u32 j = 0; j < 8; ++j)
         if (j < kc) out[o + 1 + j] = cb + (co[j] - co0);
@@ -638,21 +643,29 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         for (int L = Rmax + 1; L < kMaxLevels; ++L) st.seg[(size_t)f * kKL + L] = st.nxt[(size_t)f * kKL + L] = kNone;
 
     // --- scratch ----------------------------------------------------------------------------------
-    u32 cmax = 1;
-    for (int L = Lmin; L <= Rmax; ++L) cmax = std::max<u32>(cmax, (u32)C[L]);
-    const u32 S = table_slots(cmax);
+    u32 cmax = 1, ntiles = 0, slots[kMaxLevels] = {};
+    size_t tab_slots = 0;
+    for (int L = Lmin; L <= Rmax; ++L) {
+        const u32 c = (u32)C[L];
+        cmax = std::max<u32>(cmax, c);
+        if (!c) continue;
+        slots[L] = !use_table ? c : (L == 2) ? leaf_table_slots(c, small_leaf) : table_slots(c);
+        tab_slots += slots[L];
+        ntiles += ceil_div<u32>(c, kTileNodes);
+    }
+    if (tab_slots > 0xFFFFFFFFull) return kForestTooLarge;
     const u32 scan_n = (u32)std::max<u64>(ncol, cmax);
     const size_t c2 = C[2] ? C[2] : 1;
     size_t need = head;
     for (int L = Lmin; L <= Rmax; ++L) {
         const size_t c = C[L] ? C[L] : 1;
-        need += (L > 2 ? arena_bytes(c, 8) + arena_bytes(c, 4) : 0) + 4 * arena_bytes(c, 4);  // no coords, starts at leaves
+        need += (L > 2 ? arena_bytes(c, 8) + arena_bytes(c, 4) : 0) + 4 * arena_bytes(c, 4) +  // no coords, starts at leaves
+                arena_bytes(first_words((u32)c), 8);
     }
+    need += arena_bytes(tab_slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(ntiles, 8);
     need += arena_bytes(c2 * 8, 8) + 2 * arena_bytes(c2, 4);  // leafmask rows, run heads, column map
     need += arena_bytes(ncol, 4) + arena_bytes(1, 4);
-    need += 2 * arena_bytes(cmax, 4);
-    if (use_table) need += arena_bytes(S, 8);
-    else need += 4 * arena_bytes(cmax, 4) + arena_bytes(sort_scratch_words(cmax), 4);
+    if (!use_table) need += 5 * arena_bytes(cmax, 4) + arena_bytes(sort_scratch_words(cmax), 4);
     need += arena_bytes(scan_scratch_words(scan_n), 4);
     need += 1 << 20;
     bool moved = false;
@@ -664,36 +677,48 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         if (rc) return rc;
     }
     FLevels lv{};
+    u64* first[kMaxLevels] = {};
     for (int L = Lmin; L <= Rmax; ++L) {
         const size_t c = C[L] ? C[L] : 1;
         lv.coord[L] = (L > 2) ? A.take<u64>(c) : nullptr;
         lv.mask[L] = A.take<u32>(c);
         lv.cstart[L] = (L > 2) ? A.take<u32>(c) : nullptr;
-        lv.rank[L] = A.take<u32>(c);
+        lv.id[L] = A.take<u32>(c);
         lv.uniq[L] = A.take<u32>(c);
         lv.off[L] = A.take<u32>(c);
+        first[L] = A.take<u64>(first_words((u32)c));
+        lv.slots[L] = slots[L];
+        lv.count[L] = (u32)c;
     }
+    u64* tab = A.take<u64>(tab_slots);
+    {
+        u64* t0 = tab;
+        for (int L = Lmin; L <= Rmax; ++L) {
+            lv.tab[L] = t0;
+            t0 += slots[L];
+        }
+    }
+    u32* tile_sums = A.take<u32>(ntiles);
+    u64* tile_pre = A.take<u64>(ntiles);
     // The run heads' key hashes, from the leaf kernel to the leaf insert, in the place of the leaf
-    // level's unique list and offsets (two arrays side by side), which the ranks scan writes later.
+    // level's unique list and offsets (two arrays side by side), which k_offsets writes later.
     u64* leaf_hash = (C[2] && std::min<u64>(ncol, C[2]) >= kLaneLeafMin) ? reinterpret_cast<u64*>(lv.uniq[2]) : nullptr;
     u64* leafm = A.take<u64>(c2 * 8);
     u32* runhead = A.take<u32>(c2);
     u32* colbfs = A.take<u32>(c2);
     u32* clist = A.take<u32>(ncol ? ncol : 1);
     u32* nclist = A.take<u32>(1);
-    u32* rep = A.take<u32>(cmax);
-    u32* tslot = A.take<u32>(cmax);
-    u32* segs = tslot;
-    u64* tab = use_table ? A.take<u64>(S) : nullptr;
-    u32 *skey = nullptr, *sval = nullptr, *ktmp = nullptr, *vtmp = nullptr, *sort_scratch = nullptr;
+    SortScratch srt{};
     if (!use_table) {
-        skey = A.take<u32>(cmax);
-        sval = A.take<u32>(cmax);
-        ktmp = A.take<u32>(cmax);
-        vtmp = A.take<u32>(cmax);
-        sort_scratch = A.take<u32>(sort_scratch_words(cmax));
+        srt.skey = A.take<u32>(cmax);
+        srt.sval = A.take<u32>(cmax);
+        srt.ktmp = A.take<u32>(cmax);
+        srt.vtmp = A.take<u32>(cmax);
+        srt.seg = A.take<u32>(cmax);
+        srt.sort_scratch = A.take<u32>(sort_scratch_words(cmax));
     }
     u32* scan_scratch = A.take<u32>(scan_scratch_words(scan_n));
+    srt.scan_scratch = scan_scratch;
     if (A.used > A.cap) {
         set_error("forest: scratch layout exceeds its reservation (%zu > %zu)", A.used, A.cap);
         return CPVS_EINTERNAL;
@@ -729,73 +754,36 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
                 device_scan(ChildCountIn{lv.mask[L]}, emit, c, OpSum{}, meta + kMetaC + L, scan_scratch, s);
             }
         }
-        const u32 slots2 = use_table ? leaf_table_slots((u32)C[2], small_leaf) : 0u;
-        if (C[2]) {
+        if (C[2]) {  // (its kernel clears every level's table)
             const u32 bound = (u32)std::min<u64>(ncol, C[2]);
-            launch_leaf(o, bound, s, colinfo, colbfs, items, (u32)C[2], lv.mask[2], leafm, runhead, leaf_hash, rep,
-                        meta + kMetaSlow, tab, slots2, clist, nclist, bound);
+            launch_leaf(o, bound, s, colinfo, colbfs, items, (u32)C[2], lv.mask[2], leafm, runhead, leaf_hash, lv.id[2],
+                        meta + kMetaSlow, tab, use_table ? (u32)tab_slots : 0u, clist, nclist, bound);
+        } else if (use_table) {
+            CPVS_LAUNCH("table_clear", k_table_clear, grid_of(tab_slots, 256), dim3(256), 0, s, tab, (u32)tab_slots);
         }
         // Bottom-up merge over every level with nodes (roots included: a root is alone in its DAG).
-        int prev = -1;  // the level merged before (its ranks are the next level's child ranks)
+        MArgs ma{};
+        ma.leafm = leafm;
+        ma.heads = runhead;
+        ma.nleaf = (u32)c2;
+        u32 tile = 0;
         for (int L = Lmin; L <= Rmax; ++L) {
             const u32 c = (u32)C[L];
-            if (!c) {
-                prev = -1;
-                continue;
-            }
-            const bool is_leaf = (L == 2);
-            const u32* child_rank = (L > 2 && C[L - 1]) ? lv.rank[L - 1] : nullptr;
-            const u32* rh = is_leaf ? runhead : nullptr;
-            u64* rpart = use_table ? reinterpret_cast<u64*>(scan_scratch) : nullptr;
-            const u32 rrounds = scan_rounds(c);
-            const u32 nzero = (rpart && rrounds > 1) ? ceil_div<u32>(c, rrounds * kScanThreads) : 0u;
-            if (use_table) {
-                const u32 Sl = is_leaf ? slots2 : table_slots(c);
-                if (!is_leaf && prev < 0) CPVS_LAUNCH("table_clear", k_table_clear, grid_of(Sl, 256), dim3(256), 0, s, tab, Sl);
-                if (is_leaf) {
-                    CPVS_LAUNCH("insert_leaf", k_insert_leaf, dim3(ceil_div<u32>(c, kLeafWindow)), dim3(kLeafInsertThreads), 0, s,
-                                lv.mask[2], leafm, runhead, leaf_hash, c, tab, Sl, tslot, meta + kMetaFull, rpart, nzero,
-                                ctx->leaf_hash_bits.load());
-                    CPVS_LAUNCH("resolve", k_resolve<LeafEq>, grid_of(c, kNodeThreads), dim3(kNodeThreads), 0, s, tslot, tab,
-                                runhead, c, LeafEq{lv.mask[2], leafm, nullptr, c}, rep, meta + kMetaColl, lv.mask[2], 1u,
-                                rpart, rrounds);
-                } else {
-                    CPVS_LAUNCH("insert_inner", k_insert_inner, grid_of(c, kInsertBlock), dim3(kInsertBlock), 0, s, lv.mask[L],
-                                lv.cstart[L], child_rank, c, tab, Sl, tslot, meta + kMetaFull, rpart, nzero,
-                                ctx->inner_hash_bits.load());
-                    CPVS_LAUNCH("resolve", k_resolve<InnerEq>, grid_of(c, kNodeThreads), dim3(kNodeThreads), 0, s, tslot, tab,
-                                nullptr, c, InnerEq{lv.mask[L], lv.cstart[L], child_rank}, rep, meta + kMetaColl, lv.mask[L],
-                                0u, rpart, rrounds);
-                }
-                device_scan_from_partials(FirstSizeIn{rep, lv.mask[L], is_leaf ? 1u : 0u},
-                                          FirstSizeOut{lv.rank[L], lv.uniq[L], lv.off[L], meta + kMetaU + L, meta + kMetaS + L,
-                                                       c},
-                                          c, OpSum64{}, nullptr, rpart, s);
-            } else {
-                if (is_leaf)
-                    CPVS_LAUNCH("sortkeys", k_sortkeys_leaf, grid_of(c, 256), dim3(256), 0, s, lv.mask[2], leafm, runhead, c,
-                                skey, sval);
-                else
-                    CPVS_LAUNCH("sortkeys", k_sortkeys_inner, grid_of(c, 256), dim3(256), 0, s, lv.mask[L], lv.cstart[L],
-                                child_rank, c, skey, sval);
-                radix_sort_pairs(skey, sval, ktmp, vtmp, c, 32, sort_scratch, s);
-                device_scan(SegHeadIn{skey}, SegStartOut{segs}, c, OpMax{}, nullptr, scan_scratch, s);
-                if (is_leaf)
-                    CPVS_LAUNCH("representative", k_representative<LeafEq>, grid_of(c, 256), dim3(256), 0, s, sval, segs, c,
-                                LeafEq{lv.mask[2], leafm, runhead, c}, rep, meta + kMetaSortColl);
-                else
-                    CPVS_LAUNCH("representative", k_representative<InnerEq>, grid_of(c, 256), dim3(256), 0, s, sval, segs, c,
-                                InnerEq{lv.mask[L], lv.cstart[L], child_rank}, rep, meta + kMetaSortColl);
-                rh = nullptr;
-                device_scan(FirstSizeIn{rep, lv.mask[L], is_leaf ? 1u : 0u},
-                            FirstSizeOut{lv.rank[L], lv.uniq[L], lv.off[L], meta + kMetaU + L, meta + kMetaS + L, c}, c,
-                            OpSum64{}, nullptr, scan_scratch, s);
-            }
-            const u32 S_next = (use_table && L + 1 <= Rmax && C[L + 1]) ? table_slots((u32)C[L + 1]) : 0u;
-            CPVS_LAUNCH("rank_copies", k_rank_copies, grid_of(c, kNodeThreads), dim3(kNodeThreads), 0, s, rep, rh, c,
-                        lv.rank[L], tab, S_next);
-            prev = L;
+            if (!c) continue;
+            ma.tile0[ma.nlev] = tile;
+            tile += ceil_div<u32>(c, kTileNodes);
+            ma.lv[ma.nlev++] = MLevel{lv.mask[L], lv.cstart[L], lv.id[L], lv.tab[L], first[L], lv.uniq[L], lv.off[L],
+                                      c, lv.slots[L], L, L == 2 ? 1u : 0u, 0u};
         }
+        ma.tile0[ma.nlev] = tile;
+        for (int k = 0; k < ma.nlev; ++k) {
+            if (use_table)
+                merge_insert(ma, k, leaf_hash, meta,
+                             ma.lv[k].leaf ? ctx->leaf_hash_bits.load() : ctx->inner_hash_bits.load(), s);
+            else
+                merge_sort_level(ma, k, srt, meta, s);
+        }
+        merge_finish(ma, !use_table, tile_sums, tile_pre, meta, -1, nullptr, s);
         FBasesOut ho;
         ho.meta_host = st.back;
         ho.total = st.back + kMetaWords;

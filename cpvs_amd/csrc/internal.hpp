@@ -255,6 +255,11 @@ struct DagOut {
 int build_dag(cpvs_ctx* ctx, Arena& A, u64* pinned, int merge_mode, const cpvs_pyramid* p, u32 t, u32 T, hipStream_t s,
               cpvs_dag** out, const Admit* admit = nullptr, DagOut* into = nullptr);
 
+// The scratch bytes that build_dag needs for a map with cnt[L] nodes at level L (root level R) and
+// ncol leaf columns (see build.hip).
+size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_list, bool use_table, bool small_leaf,
+                           bool staged);
+
 // noalloc.hip: finds this device's fixed scratch (once per device); called by cpvs_ctx_create.
 int noalloc_setup(int device);
 

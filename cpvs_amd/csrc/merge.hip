@@ -1,0 +1,475 @@
+// merge.hip -- equal subtrees merged level by level, and the DAG's words.
+//
+// Bottom-up, each level takes one launch: the key of every node -- its mask and the partial
+// leafmasks, or its mask and its children's identities -- goes into the level's hash table, and the
+// slot it ends in is the node's own identity for its parents' keys.  Slots never move, so equal keys
+// have equal identities before anything is known of their order; what needs a finished table is
+// left to three launches over all levels at once:
+//   k_resolve   per node the smallest index in its slot, the full-key compare against it, and a bit
+//               for each first occurrence; the first occurrences and words of each 1024-node tile;
+//   k_totals    a scan of the tiles, the levels' totals and bases;
+//   k_offsets   rank and word offset of every first occurrence, in index order, which is the order
+//               that mergeLevel's linear search gives (src/CompressedShadowUtil.h:154-182).
+// Ranks as identities took four launches a level (insert, resolve, scan, rank copies), and the copies
+// alone read and wrote every node of the leaf level.
+//
+// Keys that a table cannot tell apart are found by the compares, and the build is done again with
+// the sort merge, whose identities are first occurrences' indices.
+#include "merge.hpp"
+
+namespace cpvs {
+
+// --- the table merge -------------------------------------------------------------------------
+
+// One 64-bit word per slot: the key hash's high 32 bits (its tag) above the smallest node index
+// with that hash, so a probe touches one cache line and a new key costs one atomic.  ~0 marks an
+// empty slot (node indices stay below 2^32 - 1).  Two keys whose tags are equal and whose probe
+// chains meet share a slot; the full-key compare in k_resolve then sends the build down the
+// sorting path, as for equal 64-bit hashes.
+
+__global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 S) {
+    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < S) tab[i] = kEmptySlot;
+}
+
+__global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
+                                                                    const u32* __restrict__ runhead,
+                                                                    const u64* __restrict__ hash, u32 n,
+                                                                    u64* __restrict__ tab, u32 S, u32* __restrict__ tslot,
+                                                                    u32* __restrict__ full, u32 hbits) {
+    __shared__ u64 gh[kLeafSlots];
+    __shared__ u32 gi[kLeafSlots];  // smallest node index of the slot's hash, then its global slot
+    __shared__ unsigned short glist[kLeafWindow];  // LDS slots in use
+    __shared__ u32 gcount;
+    for (u32 j = threadIdx.x; j < kLeafSlots; j += blockDim.x) {
+        gh[j] = 0ull;  // 0 marks an empty LDS slot
+        gi[j] = kNoRep;
+    }
+    if (threadIdx.x == 0) gcount = 0;
+    const u32 i0 = blockIdx.x * kLeafWindow + threadIdx.x;
+    u32 rh[kLeafPer];
+#pragma unroll
+    for (u32 k = 0; k < kLeafPer; ++k) {
+        const u32 i = i0 + k * kLeafInsertThreads;
+        rh[k] = (i < n) ? runhead[i] : kNoRep;
+    }
+    // The key hash of each run's first node (the run's smallest index): from the leaf kernel where
+    // a lane walked its column, else from its mask and leafmasks (its row at its own index).
+    u64 h[kLeafPer];
+#pragma unroll
+    for (u32 k = 0; k < kLeafPer; ++k) {
+        const u32 i = i0 + k * kLeafInsertThreads;
+        h[k] = (hash && rh[k] == i) ? hash[i] : 0ull;
+    }
+    u32 hm[kLeafPer];
+#pragma unroll
+    for (u32 k = 0; k < kLeafPer; ++k) {
+        const u32 i = i0 + k * kLeafInsertThreads;
+        hm[k] = (rh[k] == i && h[k] == 0ull) ? mask[i] : 0u;
+    }
+#pragma unroll
+    for (u32 k = 0; k < kLeafPer; ++k) {
+        const u32 i = i0 + k * kLeafInsertThreads;
+        if (rh[k] != i) continue;
+        if (h[k] == 0ull) h[k] = leaf_key_hash(hm[k], leafm + (size_t)i * 8);
+        h[k] = weaken_hash(h[k], hbits);
+        if (h[k] == 0ull) h[k] = 1ull;
+    }
+    __syncthreads();
+    u32 ls[kLeafPer];
+#pragma unroll
+    for (u32 k = 0; k < kLeafPer; ++k) {
+        const u32 i = i0 + k * kLeafInsertThreads;
+        ls[k] = 0;
+        if (rh[k] != i) continue;
+        u32 sl = (u32)(h[k] ^ (h[k] >> 29)) & (kLeafSlots - 1);
+        for (;;) {
+            const u64 cur = atomicCAS(reinterpret_cast<unsigned long long*>(gh + sl), 0ull, (unsigned long long)h[k]);
+            if (cur == 0ull) {
+                glist[atomicAdd(&gcount, 1u)] = (unsigned short)sl;
+                break;
+            }
+            if (cur == h[k]) break;
+            sl = (sl + 1) & (kLeafSlots - 1);
+        }
+        atomicMin(gi + sl, i);
+        ls[k] = sl;
+    }
+    __syncthreads();
+    const u32 m = gcount;  // at most kLeafWindow
+    for (u32 j = threadIdx.x; j < m; j += blockDim.x) {
+        const u32 sl = glist[j];
+        gi[sl] = table_insert(tab, S, gh[sl], gi[sl], full);
+    }
+    __syncthreads();
+#pragma unroll
+    for (u32 k = 0; k < kLeafPer; ++k) {
+        const u32 i = i0 + k * kLeafInsertThreads;
+        if (rh[k] == i) tslot[i] = gi[ls[k]];
+    }
+}
+
+__global__ __launch_bounds__(kInsertBlock) void k_insert_inner(const u32* __restrict__ mask, const u32* __restrict__ cstart,
+                                                               ChildIds ch, u32 n, u64* __restrict__ tab, u32 S,
+                                                               u32* __restrict__ id, u32* __restrict__ full, u32 hbits) {
+    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool act = i < n;
+    u64 h = 0;
+    if (act) {
+        const u32 m = mask[i], s = cstart[i];
+        const u32 k = ch.id ? num_children(m) : 0u;
+        u32 r[8] = {};
+        if (k) load_child_ids(ch, s, k, r);
+        h = weaken_hash(inner_key_hash(m, r), hbits);
+    }
+    const u32 slot = table_insert_group(tab, S, h, i, act, full);
+    if (act) id[i] = slot;
+}
+
+// --- the sort merge --------------------------------------------------------------------------
+
+__global__ __launch_bounds__(256) void k_sortkeys_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
+                                                       const u32* __restrict__ runhead,
+                                                       u32 n, u32* __restrict__ skey, u32* __restrict__ sval) {
+    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    u32 h = runhead[i];  // the key is the run's first node's
+    h = (h < n) ? h : i;
+    skey[i] = fold32(leaf_key_hash(mask[h], leafm + (size_t)h * 8));
+    sval[i] = i;
+}
+
+__global__ __launch_bounds__(256) void k_sortkeys_inner(const u32* __restrict__ mask, const u32* __restrict__ cstart,
+                                                        ChildIds ch, u32 n, u32* __restrict__ skey, u32* __restrict__ sval) {
+    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const u32 m = mask[i], s = cstart[i];
+    const u32 k = ch.id ? num_children(m) : 0u;
+    u32 r[8] = {};
+    if (k) load_child_ids(ch, s, k, r);
+    skey[i] = fold32(inner_key_hash(m, r));
+    sval[i] = i;
+}
+
+// --- first occurrences -----------------------------------------------------------------------
+
+__device__ inline int level_of_tile(const MArgs& a, u32 tile) {
+    int k = 0;
+    while (k + 1 < a.nlev && tile >= a.tile0[k + 1]) ++k;
+    return k;
+}
+
+__device__ inline u32 node_words(u32 m, u32 leaf) { return 1u + (num_children(m) << leaf); }
+
+template <bool kSorted>
+__global__ __launch_bounds__(kTileThreads) void k_resolve(MArgs a, u32* __restrict__ tile_sums, u32* __restrict__ collisions) {
+    __shared__ u32 s_wave[kTileThreads / kWave];
+    const int k = level_of_tile(a, blockIdx.x);
+    const MLevel& l = a.lv[k];
+    const u32 n = l.n, base = (blockIdx.x - a.tile0[k]) * kTileNodes + threadIdx.x;
+    // The loads of the tile's rounds are issued together, stage by stage.
+    u32 r[kTileRounds];
+    bool act[kTileRounds];
+#pragma unroll
+    for (int j = 0; j < kTileRounds; ++j) {
+        const u32 i = base + j * kTileThreads;
+        act[j] = i < n;
+        if (l.leaf && act[j]) act[j] = a.heads[i] == i;  // a first occurrence heads its run
+    }
+#pragma unroll
+    for (int j = 0; j < kTileRounds; ++j) r[j] = (act[j] && !l.lone) ? l.id[base + j * kTileThreads] : 0u;
+    if (!kSorted) {
+#pragma unroll
+        for (int j = 0; j < kTileRounds; ++j) r[j] = (act[j] && !l.lone) ? (u32)l.tab[min(r[j], l.slots - 1)] : 0u;
+    }
+    u32 acc = 0;  // first occurrences << 16 | their words (at most 1024 and 17408)
+#pragma unroll
+    for (int j = 0; j < kTileRounds; ++j) {
+        const u32 i = base + j * kTileThreads;
+        bool first = false;
+        if (act[j]) {
+            if (l.lone || r[j] >= n) r[j] = i;
+            first = r[j] == i;
+            const int kc = a.child(k);
+            if (!kSorted && l.lone && kc >= 0 && a.lv[kc].leaf) {
+                // A root over leaves (a 16 x 16 map) had no insert to store its children's identities.
+                u32 unused[8];
+                load_child_ids(ChildIds{a.lv[kc].id, a.heads, a.lv[kc].n}, l.cstart[i], num_children(l.mask[i]), unused);
+            }
+            if (!kSorted && !first) {
+                const bool same = l.leaf ? LeafEq{l.mask, a.leafm, nullptr, n}(i, r[j])
+                                         : InnerEq{l.mask, l.cstart, kc >= 0 ? a.lv[kc].id : nullptr, kc >= 0 ? a.lv[kc].n : 1u}(i, r[j]);
+                if (!same) {
+                    atomicAdd(collisions, 1u);  // two keys share a slot: the build is redone by sorting
+                    first = true;
+                }
+            }
+            if (first) acc += (1u << 16) | node_words(l.mask[i], l.leaf);
+        }
+        const u64 bits = __ballot(first);
+        if ((threadIdx.x & (kWave - 1)) == 0 && i < n) l.first[i / 64] = bits;
+    }
+    acc = block_reduce(acc, s_wave, OpSum{});
+    if (threadIdx.x == 0) tile_sums[blockIdx.x] = acc;
+}
+
+// B[R] = 0, B[L-1] = B[L] + S[L]; total = B[bottom] + S[bottom] (levels absent have S = 0).
+__device__ inline void level_bases(u32* meta, int R) {
+    u32 S[kMaxLevels];
+#pragma unroll
+    for (int L = 0; L < kMaxLevels; ++L) S[L] = meta[kMetaS + L];
+    unsigned long long acc = 0;
+#pragma unroll
+    for (int L = kMaxLevels - 1; L >= 0; --L) {
+        if (L <= R) {
+            meta[kMetaB + L] = (u32)acc;
+            acc += S[L];
+        }
+    }
+    meta[kMetaW] = (acc > 0xFFFFFFFFull) ? 0xFFFFFFFFu : (u32)acc;
+}
+
+__device__ inline u32 saturate32(u64 v) { return v > 0xFFFFFFFFull ? 0xFFFFFFFFu : (u32)v; }
+
+// One workgroup: a scan over all tiles, each thread a contiguous run of them.  A tile's prefix is
+// relative to its level's first tile; word sums run in 64 bits, and a prefix or a level total at
+// or above 2^32 is stored saturated, so that the host rejects the DAG.
+constexpr u32 kTotalsThreads = 1024;
+__global__ __launch_bounds__(kTotalsThreads) void k_totals(MArgs a, const u32* __restrict__ tile_sums,
+                                                           u64* __restrict__ tile_pre, u32* __restrict__ meta, int R,
+                                                           u32* __restrict__ host_meta) {
+    __shared__ u32 s_c[kTotalsThreads / kWave];
+    __shared__ u64 s_w[kTotalsThreads / kWave];
+    __shared__ u32 lev_c[kMaxLevels + 1];  // first occurrences and words before each level
+    __shared__ u64 lev_w[kMaxLevels + 1];
+    const u32 nt = a.tile0[a.nlev];
+    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    const u32 E = ceil_div<u32>(nt, kTotalsThreads);
+    const u32 b = min(threadIdx.x * E, nt), e = min(b + E, nt);
+    u32 c = 0;
+    u64 w = 0;
+#pragma unroll 4
+    for (u32 i = b; i < e; ++i) {
+        const u32 v = tile_sums[i];
+        c += v >> 16;
+        w += v & 0xFFFFu;
+    }
+    const u32 ci = wave_inclusive_scan(c, OpSum{});
+    const u64 wi = wave_inclusive_scan(w, OpSum64{});
+    if (lane == kWave - 1) {
+        s_c[wid] = ci;
+        s_w[wid] = wi;
+    }
+    __syncthreads();
+    u32 c0 = ci - c;
+    u64 w0 = wi - w;
+#pragma unroll
+    for (int v = 0; v < (int)(kTotalsThreads / kWave); ++v)
+        if (v < wid) {
+            c0 += s_c[v];
+            w0 += s_w[v];
+        }
+    if (b < e || (threadIdx.x == kTotalsThreads - 1)) {
+        // Level starts inside this thread's run (the end of the last level counts as one).
+        u32 cc = c0;
+        u64 ww = w0;
+        int k = 0;
+        while (k <= a.nlev && a.tile0[k] < b) ++k;
+        for (u32 i = b; i < e; ++i) {
+            for (; k <= a.nlev && a.tile0[k] == i; ++k) {
+                lev_c[k] = cc;
+                lev_w[k] = ww;
+            }
+            const u32 v = tile_sums[i];
+            cc += v >> 16;
+            ww += v & 0xFFFFu;
+        }
+        if (e == nt)
+            for (; k <= a.nlev; ++k) {  // (several threads may hold the end: the same values)
+                lev_c[k] = cc;
+                lev_w[k] = ww;
+            }
+    }
+    __syncthreads();
+    {
+        int k = 0;
+        while (k + 1 < a.nlev && a.tile0[k + 1] <= b) ++k;
+        for (u32 i = b; i < e; ++i) {
+            while (k + 1 < a.nlev && a.tile0[k + 1] <= i) ++k;
+            tile_pre[i] = ((u64)(c0 - lev_c[k]) << 32) | saturate32(w0 - lev_w[k]);
+            const u32 v = tile_sums[i];
+            c0 += v >> 16;
+            w0 += v & 0xFFFFu;
+        }
+    }
+    if (threadIdx.x < (u32)a.nlev) {
+        const u32 k = threadIdx.x;
+        meta[kMetaU + a.lv[k].L] = lev_c[k + 1] - lev_c[k];
+        meta[kMetaS + a.lv[k].L] = saturate32(lev_w[k + 1] - lev_w[k]);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && R >= 0) {
+        meta[kMetaRoot] = a.lv[a.nlev - 1].mask[0];
+        level_bases(meta, R);
+    }
+    if (host_meta) {  // the build's readback: one word per thread
+        __syncthreads();
+        for (u32 i = threadIdx.x; i < kMetaWords; i += blockDim.x) host_meta[i] = meta[i];
+        __threadfence_system();
+    }
+}
+
+__global__ __launch_bounds__(kTileThreads) void k_offsets(MArgs a, const u64* __restrict__ tile_pre) {
+    const int k = level_of_tile(a, blockIdx.x);
+    const MLevel& l = a.lv[k];
+    const u32 base = (blockIdx.x - a.tile0[k]) * kTileNodes + threadIdx.x;
+    const u64 pre = tile_pre[blockIdx.x];
+    u32 v[kTileRounds], ex[kTileRounds], id[kTileRounds];
+#pragma unroll
+    for (int j = 0; j < kTileRounds; ++j) {
+        const u32 i = base + j * kTileThreads;
+        const bool first = i < l.n && ((l.first[i / 64] >> (i & 63)) & 1ull);
+        v[j] = first ? 1u : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < kTileRounds; ++j) {
+        const u32 i = base + j * kTileThreads;
+        id[j] = (v[j] && !l.lone) ? l.id[i] : 0u;
+        if (v[j]) v[j] = (1u << 16) | node_words(l.mask[i], l.leaf);
+    }
+    block_exclusive_scan_rounds<kTileRounds>(v, ex, OpSum{});
+#pragma unroll
+    for (int j = 0; j < kTileRounds; ++j) {
+        if (!v[j]) continue;
+        const u32 rank = (u32)(pre >> 32) + (ex[j] >> 16);
+        const u32 off = saturate32((u64)(u32)pre + (ex[j] & 0xFFFFu));
+        l.uniq[rank] = base + j * kTileThreads;
+        l.off[rank] = off;
+        if (!l.lone) l.tab[min(id[j], l.slots - 1)] = ((u64)rank << 32) | off;
+    }
+}
+
+// --- the words -------------------------------------------------------------------------------
+
+// Every level's words in one launch, a grid-stride loop over the levels' blocks (their number is
+// known on the device only, so no readback comes between): unique node r of an inner level as
+// [mask, absolute offsets of its partial children], of the leaf level as [mask, (lo, hi) of each
+// partial slice's leafmask] (src/CompressedShadow.cpp:326-392).
+__global__ __launch_bounds__(kNodeThreads) void k_write_words(MArgs a, const u32* __restrict__ meta, u32* __restrict__ out,
+                                                              u64 cap) {
+    __shared__ u32 s_first[kMaxLevels + 1], s_U[kMaxLevels], s_base[kMaxLevels];
+    if (threadIdx.x < (u32)a.nlev) {
+        s_U[threadIdx.x] = meta[kMetaU + a.lv[threadIdx.x].L];
+        s_base[threadIdx.x] = meta[kMetaB + a.lv[threadIdx.x].L];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        u32 acc = 0;
+        for (int k = 0; k < a.nlev; ++k) {
+            s_first[k] = acc;
+            acc += (s_U[k] + kNodeThreads - 1) / kNodeThreads;
+        }
+        s_first[a.nlev] = acc;
+    }
+    __syncthreads();
+    const u32 total = meta[kMetaW];
+    if (total >= 0xFFFFFFFEu || total > cap) return;  // the host reports it
+    const u32 nb = s_first[a.nlev];
+    for (u32 vb = blockIdx.x; vb < nb; vb += gridDim.x) {
+        int k = 0;
+        while (k + 1 < a.nlev && vb >= s_first[k + 1]) ++k;
+        const MLevel& l = a.lv[k];
+        const u32 r = (vb - s_first[k]) * blockDim.x + threadIdx.x;
+        if (r >= s_U[k]) continue;
+        const u32 i = l.uniq[r];
+        const u32 o = s_base[k] + l.off[r];
+        const u32 m = l.mask[i];
+        out[o] = m;
+        const u32 kc = num_children(m);
+        if (!kc) continue;
+        if (l.leaf) {
+            const u64* p = a.leafm + (size_t)i * 8;  // a first occurrence heads its run: its own row
+            u64 v[8];
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j) v[j] = (j < kc) ? p[j] : 0ull;
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j)
+                if (j < kc) {
+                    out[o + 1 + 2 * j] = (u32)v[j];
+                    out[o + 2 + 2 * j] = (u32)(v[j] >> 32);
+                }
+            continue;
+        }
+        const int c = a.child(k);
+        if (c < 0) continue;
+        const MLevel& lc = a.lv[c];
+        const u32 s = l.cstart[i];
+        u32 id[8], co[8];
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? lc.id[min(s + j, lc.n - 1)] : 0u;
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j) co[j] = (j < kc) ? (u32)lc.tab[min(id[j], lc.slots - 1)] : 0u;
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j)
+            if (j < kc) out[o + 1 + j] = s_base[c] + co[j];
+    }
+}
+
+// --- launches --------------------------------------------------------------------------------
+
+static dim3 grid_of(u32 n, u32 block) { return dim3(ceil_div<u32>(n ? n : 1, block)); }
+
+// The children's identities of level k: those of the leaf level reach its non-heads here.
+static ChildIds children_of(const MArgs& a, int k, bool sorted) {
+    const int c = a.child(k);
+    if (c < 0) return ChildIds{nullptr, nullptr, 1u};
+    return ChildIds{a.lv[c].id, (a.lv[c].leaf && !sorted) ? a.heads : nullptr, a.lv[c].n};
+}
+
+void merge_insert(const MArgs& a, int k, const u64* hash, u32* meta, u32 hbits, hipStream_t s) {
+    const MLevel& l = a.lv[k];
+    if (l.leaf)
+        CPVS_LAUNCH("insert_leaf", k_insert_leaf, grid_of(l.n, kLeafWindow), dim3(kLeafInsertThreads), 0, s, l.mask, a.leafm,
+                    a.heads, hash, l.n, l.tab, l.slots, l.id, meta + kMetaFull, hbits);
+    else
+        CPVS_LAUNCH("insert_inner", k_insert_inner, grid_of(l.n, kInsertBlock), dim3(kInsertBlock), 0, s, l.mask, l.cstart,
+                    children_of(a, k, false), l.n, l.tab, l.slots, l.id, meta + kMetaFull, hbits);
+}
+
+void merge_sort_level(const MArgs& a, int k, const SortScratch& t, u32* meta, hipStream_t s) {
+    const MLevel& l = a.lv[k];
+    const ChildIds ch = children_of(a, k, true);
+    if (l.leaf)
+        CPVS_LAUNCH("sortkeys", k_sortkeys_leaf, grid_of(l.n, 256), dim3(256), 0, s, l.mask, a.leafm, a.heads, l.n, t.skey,
+                    t.sval);
+    else
+        CPVS_LAUNCH("sortkeys", k_sortkeys_inner, grid_of(l.n, 256), dim3(256), 0, s, l.mask, l.cstart, ch, l.n, t.skey,
+                    t.sval);
+    radix_sort_pairs(t.skey, t.sval, t.ktmp, t.vtmp, l.n, 32, t.sort_scratch, s);
+    device_scan(SegHeadIn{t.skey}, SegStartOut{t.seg}, l.n, OpMax{}, nullptr, t.scan_scratch, s);
+    if (l.leaf)
+        CPVS_LAUNCH("representative", k_representative<LeafEq>, grid_of(l.n, 256), dim3(256), 0, s, t.sval, t.seg, l.n,
+                    LeafEq{l.mask, a.leafm, a.heads, l.n}, l.id, meta + kMetaSortColl);
+    else
+        CPVS_LAUNCH("representative", k_representative<InnerEq>, grid_of(l.n, 256), dim3(256), 0, s, t.sval, t.seg, l.n,
+                    InnerEq{l.mask, l.cstart, ch.id, ch.n}, l.id, meta + kMetaSortColl);
+}
+
+void merge_finish(const MArgs& a, bool sorted, u32* tile_sums, u64* tile_pre, u32* meta, int R, u32* host_meta,
+                  hipStream_t s) {
+    const u32 nt = a.tile0[a.nlev];
+    if (sorted)
+        CPVS_LAUNCH("resolve", k_resolve<true>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums, meta + kMetaColl);
+    else
+        CPVS_LAUNCH("resolve", k_resolve<false>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums, meta + kMetaColl);
+    CPVS_LAUNCH("totals", k_totals, dim3(1), dim3(kTotalsThreads), 0, s, a, tile_sums, tile_pre, meta, R, host_meta);
+    CPVS_LAUNCH("offsets", k_offsets, dim3(nt), dim3(kTileThreads), 0, s, a, tile_pre);
+}
+
+void merge_write(const MArgs& a, const u32* meta, u32* out, u64 cap, hipStream_t s) {
+    u32 most = 0;  // blocks of the largest possible write (every node unique)
+    for (int k = 0; k < a.nlev; ++k) most += ceil_div<u32>(a.lv[k].n, kNodeThreads);
+    CPVS_LAUNCH("write_words", k_write_words, dim3(most < 2048 ? most : 2048), dim3(kNodeThreads), 0, s, a, meta, out, cap);
+}
+
+}  // namespace cpvs
