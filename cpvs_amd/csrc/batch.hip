@@ -33,15 +33,14 @@ int Worker::create() {
     return CPVS_OK;
 }
 
-int Worker::forest_staging(size_t bytes) {
-    if (bytes <= fpin_bytes) return CPVS_OK;
+int Worker::staging(Staging& st, size_t bytes) {
+    if (bytes <= st.bytes) return CPVS_OK;
     CPVS_HIP_CHECK(hipStreamSynchronize(stream));  // no copy still reads the old staging
-    if (fpin) (void)hipHostFree(fpin);
-    fpin = nullptr;
-    fpin_bytes = 0;
+    if (st.p) (void)hipHostFree(st.p);
+    st = Staging{};
     const size_t want = bytes + (bytes >> 2);
-    CPVS_HIP_CHECK(hipHostMalloc(&fpin, want, kPinnedFlags));
-    fpin_bytes = want;
+    CPVS_HIP_CHECK(hipHostMalloc(&st.p, want, kPinnedFlags));
+    st.bytes = want;
     return CPVS_OK;
 }
 
@@ -49,9 +48,10 @@ void Worker::destroy() {
     if (stream) (void)hipStreamSynchronize(stream);
     arena.release();
     levels.release();
-    if (fpin) (void)hipHostFree(fpin);
-    fpin = nullptr;
-    fpin_bytes = 0;
+    for (Staging* st : {&forest, &pyramids}) {
+        if (st->p) (void)hipHostFree(st->p);
+        *st = Staging{};
+    }
     if (pinned) (void)hipHostFree(pinned);
     if (stream) (void)hipStreamDestroy(stream);
     pinned = nullptr;
@@ -263,8 +263,6 @@ int run_forests(cpvs_ctx* ctx, const cpvs_batch_item* items, uint32_t count, con
     }
     ForestOpts fo;
     fo.merge_mode = ctx->merge_mode;
-    fo.leaf_cols = cfg.leaf_cols;
-    fo.leaf_waves = cfg.leaf_waves;
     fo.graph = cfg.graph != 0;
 
     std::atomic<uint32_t> next{0};
@@ -321,10 +319,12 @@ int run_forests(cpvs_ctx* ctx, const cpvs_batch_item* items, uint32_t count, con
                 const uint32_t f = next.fetch_add(1, std::memory_order_relaxed);
                 if (f >= forests.size()) break;
                 const uint32_t g0 = forests[f].first, g1 = forests[f].second;
-                size_t lv_bytes = 0;
+                size_t lv_bytes = pyramids_rec_bytes(g1 - g0);
                 for (uint32_t g = g0; g < g1; ++g) lv_bytes += pyramid_levels_bytes(items[order[groups[g].begin]].N, false);
                 int lrc = w->levels.reserve(lv_bytes, w->stream);
+                if (lrc == CPVS_OK) lrc = w->staging(w->pyramids, pyramids_rec_bytes(g1 - g0));
                 std::vector<cpvs_pyramid> pyr(g1 - g0);
+                std::vector<cpvs_pyramid*> pyrs;
                 std::vector<ForestIn> fin;
                 std::vector<uint32_t> idx;
                 for (uint32_t g = g0; g < g1 && lrc == CPVS_OK; ++g) {
@@ -335,12 +335,13 @@ int run_forests(cpvs_ctx* ctx, const cpvs_batch_item* items, uint32_t count, con
                     p.n = levels_of(it.N);
                     p.depth = const_cast<float*>(it.depth);
                     p.borrowed = true;
-                    lrc = pyramid_build_levels(&p, false, w->stream, &w->levels, true);
+                    pyrs.push_back(&p);
                     for (uint32_t j = groups[g].begin; j < groups[g].end; ++j) {
                         fin.push_back(ForestIn{&p, items[order[j]].zTileIndex, items[order[j]].zTileNum});
                         idx.push_back(order[j]);
                     }
                 }
+                if (lrc == CPVS_OK) lrc = pyramids_build(pyrs.data(), g1 - g0, w->pyramids.p, w->levels, w->stream);
                 if (lrc == CPVS_OK) lrc = build_range(w, fin, idx, 0, (uint32_t)fin.size());
                 if (lrc != CPVS_OK) {
                     char msg[600];

@@ -55,223 +55,63 @@ __global__ __launch_bounds__(256) void k_classify(const u64* __restrict__ coord,
 // ---------------------------------------------------------------------------------------
 
 // ---------------------------------------------------------------------------------------
-// The leaf kernel: kLeafCols level-3 columns per wave, one texel per lane.
-// * All loads of a wave's columns are issued together (column info, then the depth blocks and
-//   the first 64 breadth-first indices of each column); the columns are then walked one after the
-//   other with no memory wait.  A column of more than 64 nodes (box walls) loads the indices of
-//   its later 64-node chunks in the loop.
+// The leaf kernels.  k_leaf_lanes walks one column per lane (leaf_lane), for launches with enough
+// columns to fill the chip that way, and leaves walls and steep columns to k_leaf_waves, one column
+// per wave and one texel per lane (leaf_column).  In the latter:
 // * Which nodes differ from their predecessor follows from the texels alone.  With
 //   h_t = f_t + 8 - 8*zs, node q changes iff some h_t - 8q lies in [0, 14]: q = floor(h_t/8), or
 //   q = floor(h_t/8) - 1 when h_t mod 8 != 7.  Each texel flags at most two nodes in LDS and a
 //   ballot over the flags read back gives a chunk's changed nodes at once; only those (the run
-//   heads, 1.3 M of 6.7 M leaves at 8192^2) get compares.
-// * The kernel is bound by instruction issue: the per-run-head work is wave-uniform, and the
-//   scalar unit is one per CU, shared by its four SIMDs.  What cut it: the changed nodes from LDS
-//   flags and one ballot instead of two wave OR-reductions (0.262 -> 0.244 ms), lane inserts by
-//   v_writelane and run heads propagated head by head (0.239 ms), the wave's columns walked by a
-//   bitmask of those with nodes (0.224 ms), slice counts from per-chunk offsets (0.217 ms), and
-//   simpler flag addressing (0.209 ms).  The vector units are now the busier (73%, scalar 57%).
+//   heads) get compares.
 // * Only a run's first node stores its mask and leafmasks: the merge and the final write read
 //   those of first occurrences only, and a key's first occurrence is always the first node of a
 //   run (breadth-first order grows with z inside a column).  Every node stores the breadth-first
 //   index of its run's first node.
 // * A run head's leafmasks go to the row at its own breadth-first index (8 slots per node), so the
 //   leaf insert, the key compares and the write find them at the node's index, with no slot map.
-// * Measured on MI355X (earlier forms of the kernel): 8 columns per wave 0.31 ms, 4 columns 0.32
-//   ms, 16 columns 0.42 ms; one
-//   column per one-wave workgroup (loads issued per column, run heads found by a ballot per node)
-//   0.55 ms; one lane per node over LDS-staged columns 0.51 ms (64 texels of work per node).
-//   Workgroups of 1, 2, 4 and 8 waves: 0.308, 0.315, 0.320 and 0.335 ms.
+// Measured at 8192^2 (1 M columns, 6.7 M nodes): 8 columns per wave for all, bound by instruction issue
+// (vector units 73% busy, scalar 57%), 210 us; lanes 96 us and waves 49 us for the rest, whose
+// columns hold most of the nodes (2, 4 and 8 of them in turn per wave took 51, 63 and 77 us: a wave
+// waits for each column's chunks).  Small maps are all latency: 256^2 13 -> 4 us and 1024^2
+// 17 -> 9 us with one column per wave instead of 8.
 // Workgroups are dealt to the XCDs in turn (block b to XCD b mod kXcds), each XCD with its own L2.
-// XCD x takes the contiguous units [x*unit_chunk, (x+1)*unit_chunk): neighbouring columns, whose
-// 8-texel depth rows share 128-byte lines, are then read through one L2.
+// XCD x takes the contiguous units [x*chunk, (x+1)*chunk): neighbouring columns, whose 8-texel depth
+// rows share 128-byte lines, are then read through one L2.  A list fills only its first units, so
+// there consecutive units go to different XCDs.
 // ---------------------------------------------------------------------------------------
-
-// kList: the wave's columns are col_list[c0 .. c0+7], *n_list of them in all (with several z-tiles,
-// the z-tile's columns with leaf nodes in column order; or those that k_leaf_lanes left), and the
-// workgroups stride over the list; ncol (at most the leaf node count) bounds it.
-// Otherwise the wave's columns are c0 .. c0+7 of all ncol.
-template <bool kList, u32 kCols>
-__global__ __launch_bounds__(64 * kLeafWaves) void k_leaf_waves(LeafColumns lc, u32 ncol, u32 nleaf,
-                                                                const float* __restrict__ depth, u32 N, u32 T,
-                                                                const float2* __restrict__ lv3,
-                                                                u32* __restrict__ mask_out, u64* __restrict__ leafm,
-                                                                u32* __restrict__ runhead, u64* __restrict__ hash_out,
-                                                                u32 unit_chunk,
-                                                                u64* __restrict__ tab, u32 tab_slots,
-                                                                const u32* __restrict__ col_list,
-                                                                const u32* __restrict__ n_list) {
-    // Per lane: f_t and the breadth-first index of node `lane` of each of the wave's columns (a lane
-    // only ever reads back its own entries, so the arrays need no barrier).
-    __shared__ int s_f[kLeafWaves][kCols][64];
-    __shared__ u32 s_b[kLeafWaves][kCols][64];
-    // A chunk's changed-node flags (leaf_column): byte j + 1 for node q0 + j, byte 65 a sink.
-    __shared__ uint8_t s_chg[kLeafWaves][128];
-    // The wave index is uniform across the wave; saying so keeps the column bases in scalar registers.
-    const u32 lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // Workgroups are dealt to the XCDs in turn; XCD x takes the contiguous units [x*unit_chunk, ...).
-    // A column list fills only its first units, so there consecutive units go to different XCDs.
-    u32 unit = kList ? blockIdx.x : (blockIdx.x % kXcds) * unit_chunk + blockIdx.x / kXcds;
-    const u32 nvalid = kList ? min(*n_list, ncol) : ncol;  // columns of this launch
-    do {
-    const u32 c0 = (unit * kLeafWaves + wave) * kCols;
-    if (kList && c0 >= nvalid) break;
-    // Every load below is unconditional (addresses clamped into range, values masked afterwards), so
-    // the compiler counts them exactly and waits only for what each step uses.
-    const u32 clast = kList ? (nvalid ? nvalid - 1 : 0u) : ncol - 1;
-    // lane k < kCols: column c0 + k of the launch (list entries past nvalid are never read)
-    const u32 my_slot = min(c0 + (lane & (kCols - 1)), clast);
-    const u32 my_col = kList ? (nvalid ? col_list[my_slot] : 0u) : my_slot;
-    uint4 ci = lc.info[my_col];
-    if (lane >= kCols || c0 + lane >= nvalid) ci = make_uint4(0u, 0u, 0u, 0u);
-    // Addresses are a wave-uniform base (the column's block, its run of indices) plus a per-lane
-    // offset computed once, so every load takes its address from scalar registers and one vector
-    // offset, with no per-column vector arithmetic.
-    // Byte offset of texel (lane & 7, lane >> 3) of a column's block: below 2^32 (N <= 2^21), so a
-    // load takes it as its 32-bit vector offset from the block's scalar base.
-    const u32 loff = 4u * ((lane >> 3) * N + (lane & 7));
-    float d[kCols];
-    // Without a list, a wave's columns are c0 .. c0+7 of one row of level-3 texels when the row
-    // holds a multiple of 8 columns: their blocks are 32 bytes apart, one base and immediate offsets.
-    const bool row_run = !kList && lc.w3 >= kCols && c0 + kCols <= ncol;
-    if (row_run) {
-        const u32 x3 = c0 & (lc.w3 - 1), y3 = c0 >> lc.w3_shift;
-        const char* blk = reinterpret_cast<const char*>(depth + ((size_t)(8 * y3) * N + 8 * x3)) + loff;
-#pragma unroll
-        for (u32 k = 0; k < kCols; ++k) {
-            const float* p = reinterpret_cast<const float*>(blk + 32 * k);
-            if (T > 1) {
-                d[k] = 0.0f;
-                if (__builtin_amdgcn_readlane(ci.x, k) != 0u) d[k] = *p;
-            } else {
-                d[k] = __builtin_nontemporal_load(p);
-            }
-        }
-    } else if (T > 1) {
-        // A column with no leaf node in this z-tile (most columns of a tile) is not read: its f
-        // values are never used.  With one z-tile every column has nodes, and the check would only
-        // cost issue slots.
-#pragma unroll
-        for (u32 k = 0; k < kCols; ++k) {
-            const u32 c = kList ? __builtin_amdgcn_readlane(my_col, k) : min(c0 + k, clast);
-            const u32 x3 = c & (lc.w3 - 1), y3 = c >> lc.w3_shift;
-            const float* blk = depth + ((size_t)(8 * y3) * N + 8 * x3);
-            d[k] = 0.0f;
-            if (__builtin_amdgcn_readlane(ci.x, k) != 0u) d[k] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(blk) + loff);
-        }
-    } else {
-#pragma unroll
-        for (u32 k = 0; k < kCols; ++k) {
-            const u32 c = kList ? __builtin_amdgcn_readlane(my_col, k) : min(c0 + k, clast);
-            const u32 x3 = c & (lc.w3 - 1), y3 = c >> lc.w3_shift;
-            const float* blk = depth + ((size_t)(8 * y3) * N + 8 * x3);
-            // Nontemporal: the map's last read (the merge kernels that follow keep more of the L2).
-            d[k] = __builtin_nontemporal_load(reinterpret_cast<const float*>(reinterpret_cast<const char*>(blk) + loff));
-        }
-    }
-    u32 b[kCols];
-#pragma unroll
-    for (u32 k = 0; k < kCols; ++k) {
-        const u32 cnt = __builtin_amdgcn_readlane(ci.x, k), st = __builtin_amdgcn_readlane(ci.y, k);
-        const u32* run = lc.bfs + (cnt ? st : 0u);  // st + lane < nleaf for lane < cnt: the counts sum to it
-        b[k] = run[(lane < cnt) ? lane : 0u];
-    }
-    const float HT = (float)(N * T);
-    // The columns' minimum and maximum f from their level-3 pyramid texels (the 8x8 blocks' depth
-    // minimum and maximum): lane k < kCols holds column k's, lane k + kCols its maximum.
-    // A block holding a NaN takes them from its texels instead (the pyramid keeps a NaN only as a
-    // first operand, so its extremes do not tell).
-    const float2 ext = lv3[my_col];
-    const int fext = leaf_f(((lane & kCols) ? ext.y : ext.x) * HT);
-    u32 nan_cols = 0;
-#pragma unroll
-    for (u32 k = 0; k < kCols; ++k) {
-        const float D = d[k] * HT;
-        if (__ballot(!(D == D))) nan_cols |= 1u << k;
-        s_f[wave][k][lane] = leaf_f(D);
-        s_b[wave][k][lane] = b[k];
-    }
-
-    // The wave's columns with leaf nodes (ci is zero for lanes past the launch's columns).
-    for (u32 todo = (u32)__ballot(ci.x != 0u); todo; todo &= todo - 1u) {
-        const u32 k = (u32)__builtin_ctz(todo);
-        const u32 cnt = __builtin_amdgcn_readlane(ci.x, k);
-        const u32 base = __builtin_amdgcn_readlane(ci.y, k);
-        const int zs = (int)__builtin_amdgcn_readlane(ci.z, k);
-        const int f = s_f[wave][k][lane];
-        int fmin = __builtin_amdgcn_readlane(fext, k), fmax = __builtin_amdgcn_readlane(fext, k + kCols);
-        if ((nan_cols >> k) & 1u) {
-            fmin = __ockl_wfred_min_i32(f);
-            fmax = __ockl_wfred_max_i32(f);
-        }
-        // (with one wave per workgroup its flags sit at a constant LDS address)
-        leaf_column(f, fmin, fmax, zs, cnt, s_b[wave][k][lane], lc.bfs + base, 0u, nleaf,
-                    kLeafWaves == 1 ? s_chg[0] : s_chg[wave], lane, mask_out, leafm, runhead, hash_out);
-    }
-    unit += gridDim.x;
-    } while (kList);
-    // The leaf level's merge table is cleared here, after all the work (stores issued earlier
-    // would be waited for with the loads): this kernel leaves HBM bandwidth to spare.
-    clear_table(tab, tab_slots);
+__device__ inline LeafCol map_column(const LeafColumns& lc, const float* depth, u32 N, float HT, u32 col) {
+    const uint4 ci = lc.info[col];
+    const u32 x = even_bits(col), y = even_bits(col >> 1);
+    return LeafCol{col, depth + ((size_t)(8 * y) * N + 8 * x), N, HT, ci.x, ci.y, (int)ci.z, 0u};
 }
 
-// The same with one column per lane (leaf_lane), for launches with enough columns to fill the chip
-// that way: a workgroup takes 16 x 16 columns, each of its waves 8 x 8 (whose nodes lie close together
-// in breadth-first order), or 256 columns of the list.
+// kList: the columns col_list[0 .. *n_list), at most ncol (the z-tile's columns with leaf nodes, or
+// those that k_leaf_lanes left), over which the waves stride; otherwise all ncol of them.
 template <bool kList>
-struct MapCols {
-    LeafColumns lc;
-    const float* depth;
-    u32 N;
-    float HT;
-    const u32* list;
-    u32 nlist, first, tx, ty;
-    __device__ void operator()(u32 slot, LeafCol& c) const {
-        u32 x, y;
-        uint4 ci = make_uint4(0u, 0u, 0u, 0u);
-        if (kList) {
-            const bool in = first + slot < nlist;
-            const u32 col = in ? list[first + slot] : 0u;
-            x = col & (lc.w3 - 1);
-            y = col >> lc.w3_shift;
-            if (in) ci = lc.info[col];
-        } else {
-            x = 16 * tx + 8 * ((slot >> 6) & 1u) + (slot & 7u);
-            y = 16 * ty + 8 * (slot >> 7) + ((slot >> 3) & 7u);
-            ci = lc.info[(y << lc.w3_shift) + x];
-        }
-        c.col = (y << lc.w3_shift) + x;
-        c.blk = depth + ((size_t)(8 * y) * N + 8 * x);
-        c.pitch = N;
-        c.HT = HT;
-        c.cnt = ci.x;
-        c.start = ci.y;
-        c.zs = (int)ci.z;
-        c.gtag = 0;
+__global__ __launch_bounds__(64) void k_leaf_waves(LeafColumns lc, u32 ncol, const float* __restrict__ depth, u32 N, u32 T,
+                                                   const float2* __restrict__ lv3, LeafOut o, u32 chunk,
+                                                   u64* __restrict__ tab, u32 tab_slots,
+                                                   const u32* __restrict__ col_list, const u32* __restrict__ n_list) {
+    __shared__ uint8_t s_chg[128];
+    const u32 n = kList ? min(*n_list, ncol) : ncol;
+    for (u32 u = kList ? blockIdx.x : (blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds; u < n; u += gridDim.x) {
+        const LeafCol c = map_column(lc, depth, N, (float)(N * T), kList ? col_list[u] : u);
+        if (c.cnt) leaf_wave(c, lv3 + (size_t)even_bits(c.col >> 1) * lc.w3 + even_bits(c.col), o, s_chg, threadIdx.x);
+        if (!kList) break;
     }
-};
-
-// Even bits of v, packed.
-__device__ inline u32 even_bits(u32 v) {
-    v &= 0x55555555u;
-    v = (v | (v >> 1)) & 0x33333333u;
-    v = (v | (v >> 2)) & 0x0F0F0F0Fu;
-    v = (v | (v >> 4)) & 0x00FF00FFu;
-    return (v | (v >> 8)) & 0xFFFFu;
+    clear_table(tab, tab_slots);  // after all the work: stores issued earlier would be waited for with the loads
 }
 
 template <bool kList>
 __global__ __launch_bounds__(kLaneThreads) void k_leaf_lanes(LeafColumns lc, u32 ncol, const float* __restrict__ depth, u32 N,
-                                                             u32 T, LeafOut o, u32 unit_chunk, u64* __restrict__ tab,
+                                                             u32 T, LeafOut o, u32 chunk, u64* __restrict__ tab,
                                                              u32 tab_slots, const u32* __restrict__ col_list,
                                                              const u32* __restrict__ n_list) {
-    // Tiles of a map in Morton order, a contiguous range of them per XCD; a list's in turn.
-    const u32 unit = kList ? blockIdx.x : (blockIdx.x % kXcds) * unit_chunk + blockIdx.x / kXcds;
-    MapCols<kList> cols{lc, depth, N, (float)(N * T), col_list, 0u, unit * kLaneThreads, even_bits(unit), even_bits(unit >> 1)};
-    if (kList) cols.nlist = min(*n_list, ncol);
-    if (unit * kLaneThreads < (kList ? cols.nlist : ncol)) {
-        LeafCol c;
-        cols(threadIdx.x, c);
+    const u32 unit = kList ? blockIdx.x : (blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds;
+    const u32 n = kList ? min(*n_list, ncol) : ncol, u = unit * kLaneThreads + threadIdx.x;
+    if (unit * kLaneThreads < n) {
+        LeafCol c{};
+        if (u < n) c = map_column(lc, depth, N, (float)(N * T), kList ? col_list[u] : u);
         leaf_lanes(c, o);
     }
     clear_table(tab, tab_slots);
@@ -675,7 +515,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         }
     }
     u32* tile_sums = A.take<u32>(ntiles);
-    u64* tile_pre = A.take<u64>(ntiles);
+    ulonglong2* tile_pre = A.take<ulonglong2>(tile_pre_count(ntiles));
     u64* leafm = leaf ? A.take<u64>(c2 * 8) : nullptr;
     // The run heads' key hashes, from the leaf kernel to the leaf insert, in the place of the leaf
     // level's unique list and offsets (two arrays side by side), which k_offsets writes later.
@@ -707,7 +547,6 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         lc.info = colinfo;
         lc.bfs = colbfs;
         lc.w3 = w3;
-        lc.w3_shift = (u32)__builtin_ctz(w3);
         if (col_list)
             device_scan(ColPairIn{colinfo}, ColListOut{colinfo, clist, nclist, ncol}, ncol, OpSum64{}, nullptr, scan_scratch, s);
         else
@@ -744,33 +583,28 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         if (leaf && L == 2) {
             // With a column list, at most min(columns, leaf nodes) columns have nodes.
             const u32 bound = col_list ? std::min(ncol, c) : ncol;
-            const u32 units = ceil_div<u32>(bound, kLeafWaves * kLeafCols);
-            const u32 unit_chunk = ceil_div<u32>(units, kXcds);
             const u32 slots = use_table ? (u32)clear_slots : 0u;  // the merge's tables are cleared here
+            // (the list of slow columns lies where the identities are written later)
+            const LeafOut lo{colbfs, lv[2].mask, leafm, runhead, leaf_hash, lv[2].id, meta + kMetaSlow, c};
             if (lane_leaf) {
-                // (the list of slow columns lies where the identities are written later)
-                const LeafOut lo{colbfs, lv[2].mask, leafm, runhead, leaf_hash, lv[2].id, meta + kMetaSlow, c};
-                const u32 tiles = ceil_div<u32>(bound, kLaneThreads);
-                const u32 chunk = ceil_div<u32>(tiles, kXcds);
+                const u32 units = ceil_div<u32>(bound, kLaneThreads), chunk = ceil_div<u32>(units, kXcds);
                 if (col_list)
-                    CPVS_LAUNCH("leaf_lanes", k_leaf_lanes<true>, dim3(tiles), dim3(kLaneThreads), 0, s, lc, bound, p->depth,
+                    CPVS_LAUNCH("leaf_lanes", k_leaf_lanes<true>, dim3(units), dim3(kLaneThreads), 0, s, lc, bound, p->depth,
                                 N, T, lo, chunk, tab, slots, clist, nclist);
                 else
                     CPVS_LAUNCH("leaf_lanes", k_leaf_lanes<false>, dim3(chunk * kXcds), dim3(kLaneThreads), 0, s, lc, bound,
                                 p->depth, N, T, lo, chunk, tab, slots, nullptr, nullptr);
-                const u32 sbound = std::min(bound, c);
-                CPVS_LAUNCH("leaf_waves", (k_leaf_waves<true, kSlowCols>),
-                            dim3(std::min(ceil_div<u32>(sbound, kLeafWaves * kSlowCols), kSlowWaves / kLeafWaves)),
-                            dim3(64 * kLeafWaves), 0, s, lc, sbound, c, p->depth, N, T, p->lv[3], lv[2].mask, leafm, runhead,
-                            leaf_hash, 0u, tab, 0u, lv[2].id, meta + kMetaSlow);
-            } else if (col_list)
-                CPVS_LAUNCH("leaf_waves", (k_leaf_waves<true, kLeafCols>), dim3(unit_chunk * kXcds), dim3(64 * kLeafWaves), 0, s, lc,
-                            bound, c, p->depth, N, T, p->lv[3], lv[2].mask, leafm, runhead, nullptr, unit_chunk, tab,
-                            slots, clist, nclist);
-            else
-                CPVS_LAUNCH("leaf_waves", (k_leaf_waves<false, kLeafCols>), dim3(unit_chunk * kXcds), dim3(64 * kLeafWaves), 0, s, lc,
-                            bound, c, p->depth, N, T, p->lv[3], lv[2].mask, leafm, runhead, nullptr, unit_chunk, tab,
-                            slots, nullptr, nullptr);
+                const u32 most = std::min(bound, c);
+                CPVS_LAUNCH("leaf_waves", k_leaf_waves<true>, dim3(std::min(most, kSlowWaves)), dim3(64), 0, s, lc, most,
+                            p->depth, N, T, p->lv[3], lo, 0u, tab, 0u, lv[2].id, meta + kMetaSlow);
+            } else if (col_list) {
+                CPVS_LAUNCH("leaf_waves", k_leaf_waves<true>, dim3(std::min(bound, kSlowWaves)), dim3(64), 0, s, lc, bound,
+                            p->depth, N, T, p->lv[3], lo, 0u, tab, slots, clist, nclist);
+            } else {
+                const u32 chunk = ceil_div<u32>(bound, kXcds);
+                CPVS_LAUNCH("leaf_waves", k_leaf_waves<false>, dim3(chunk * kXcds), dim3(64), 0, s, lc, bound, p->depth, N, T,
+                            p->lv[3], lo, chunk, tab, slots, nullptr, nullptr);
+            }
             break;
         }
         // A level is classified inside its emit scan when that scan loads its outputs' prefetch
@@ -910,7 +744,7 @@ size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_
         slots += level_slots(cnt, L, R, Ls, use_table, leaf, small_leaf);
         ntiles += ceil_div<u32>((u32)cnt[L], kTileNodes);
     }
-    need += arena_bytes(slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(ntiles, 8);
+    need += arena_bytes(slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(tile_pre_count(ntiles), 16);
     const size_t c2 = leaf ? (cnt[2] ? cnt[2] : 1) : 1;
     if (leaf) need += arena_bytes(c2 * 8, 8) + 2 * arena_bytes(c2, 4);  // leafmask rows, run heads, column map
     if (col_list) need += arena_bytes(ncol, 4) + arena_bytes(1, 4);

@@ -62,14 +62,14 @@ __device__ inline u32 classify_node(u64 c, const float2* __restrict__ lv, const 
 }
 
 
-// Leaf columns: per level-3 texel one record {partial cells, first leaf's index in column order,
-// first partial z cell, 0}, so a column's scalars come in one load.  The counts (x, z) come from
+// Leaf columns: per level-3 texel, in Morton order, one record {partial cells, first leaf's index in
+// column order, first partial z cell, 0}, so a column's scalars come in one load and a node's four
+// columns in one line.  The counts (x, z) come from
 // the node-count pass, the starts (y) from a scan of the counts.
 struct LeafColumns {
     uint4* info;
     u32* bfs;       // (column start + z - zs) -> breadth-first index of the leaf node
     u32 w3;         // N >> 3
-    u32 w3_shift;   // log2(w3)
 };
 
 struct ColCountIn {
@@ -151,14 +151,14 @@ struct EmitChildrenOut {
         if (cols.bfs) {
             // (the column records read lie inside the level even for a node past its level's
             // emitted children)
-            const u32 xc = min(x, cols.w3 - 2) & ~1u, yc = min(y, cols.w3 - 2);
+            const u32 at = morton2(min(x, cols.w3 - 2) & ~1u, min(y, cols.w3 - 2) & ~1u);
             // Leaf children: children ch and ch + 4 lie in one column, so the node's (at most
             // four) column records are loaded first, all together, and the stores follow.
             uint4 ci[4];
 #pragma unroll
             for (u32 q = 0; q < 4; ++q) {
                 ci[q] = make_uint4(0u, 0u, 0u, 0u);
-                if (m & ((2u << (2 * q)) | (2u << (2 * (q + 4))))) ci[q] = cols.info[(yc + (q >> 1)) * cols.w3 + xc + (q & 1)];
+                if (m & ((2u << (2 * q)) | (2u << (2 * (q + 4))))) ci[q] = cols.info[at + q];
             }
 #pragma unroll
             for (u32 ch = 0; ch < 8; ++ch) {
@@ -339,8 +339,6 @@ __device__ inline void leaf_column(int f, int fmin, int fmax, int zs, u32 cnt, u
 }
 
 constexpr u32 kXcds = 8;
-constexpr u32 kLeafCols = 1;
-constexpr u32 kLeafWaves = 1;
 
 // ---------------------------------------------------------------------------------------
 // Leaf columns, one column per lane.  A smooth surface crosses an 8x8 block in a few slices, all
@@ -372,7 +370,7 @@ struct LeafOut {
     u32* mask;
     u64* leafm;
     u32* runhead;
-    u64* hash;  // key hash of every run head whose column a lane walked, 0 for the others'
+    u64* hash;  // key hash of every run head whose column a lane walked, 0 for the others' (null: no lanes)
     u32* slow;  // the columns left to the wave-per-column kernel, *n_slow of them
     u32* n_slow;
     u32 nleaf;
@@ -467,6 +465,25 @@ __device__ inline bool leaf_lane(const LeafCol& c, const LeafOut& o) {
         }
     }
     return true;
+}
+
+// One column by a wave, lane = texel (all arguments but the lane's texel are wave-uniform); ext: its
+// level-3 pyramid texel, the block's depth minimum and maximum (a block holding a NaN takes its
+// extremes from its texels instead: the pyramid keeps a NaN only as a first operand).
+__device__ inline void leaf_wave(const LeafCol& c, const float2* ext, const LeafOut& o, uint8_t* fl, u32 lane) {
+    const float d = c.blk[(size_t)(lane >> 3) * c.pitch + (lane & 7)];
+    const u32 b = o.bfs[c.start + min(lane, c.cnt - 1)];
+    const float2 e = *ext;
+    const float D = d * c.HT;
+    const int f = leaf_f(D);
+    int fmin = leaf_f(e.x * c.HT), fmax = leaf_f(e.y * c.HT);
+    if (__ballot(!(D == D))) {
+        fmin = __ockl_wfred_min_i32(f);
+        fmax = __ockl_wfred_max_i32(f);
+    }
+    fmin = __builtin_amdgcn_readfirstlane(fmin);
+    fmax = __builtin_amdgcn_readfirstlane(fmax);
+    leaf_column(f, fmin, fmax, c.zs, c.cnt, b, o.bfs + c.start, c.gtag, o.nleaf, fl, lane, o.mask, o.leafm, o.runhead, o.hash);
 }
 
 // The lanes' columns, those set aside appended to the list (one atomic per wave).
@@ -730,8 +747,7 @@ enum : int {
 
 // Launches over this many columns walk them one per lane (a map's are then at least 16 x 16).
 constexpr u64 kLaneLeafMin = 1u << 15;
-constexpr u32 kSlowCols = 1;
-constexpr u32 kSlowWaves = 8192;  // waves that stride over the columns left to them: the chip's 32 per CU
+constexpr u32 kSlowWaves = 8192;  // waves that stride over a list of columns: the chip's 32 per CU
 
 inline u32 table_slots(u32 n) {
     u32 S = 1024;

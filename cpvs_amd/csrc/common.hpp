@@ -24,6 +24,25 @@ __host__ __device__ inline u32 unpack_x(u64 c) { return (u32)(c & 0x1FFFFF); }
 __host__ __device__ inline u32 unpack_y(u64 c) { return (u32)((c >> 21) & 0x1FFFFF); }
 __host__ __device__ inline u32 unpack_z(u64 c) { return (u32)((c >> 42) & 0x1FFFFF); }
 
+// Morton order of 2-D cells: x in the even bits, y in the odd ones (16 bits each).  Leaf columns are
+// numbered so: a node's 2 x 2 columns follow one another, and neighbouring columns' nodes lie close
+// together in breadth-first order, which is Morton order in three dimensions.
+__host__ __device__ inline u32 spread_bits(u32 v) {
+    v &= 0xFFFFu;
+    v = (v | (v << 8)) & 0x00FF00FFu;
+    v = (v | (v << 4)) & 0x0F0F0F0Fu;
+    v = (v | (v << 2)) & 0x33333333u;
+    return (v | (v << 1)) & 0x55555555u;
+}
+__host__ __device__ inline u32 even_bits(u32 v) {
+    v &= 0x55555555u;
+    v = (v | (v >> 1)) & 0x33333333u;
+    v = (v | (v >> 2)) & 0x0F0F0F0Fu;
+    v = (v | (v >> 4)) & 0x00FF00FFu;
+    return (v | (v >> 8)) & 0xFFFFu;
+}
+__host__ __device__ inline u32 morton2(u32 x, u32 y) { return spread_bits(x) | (spread_bits(y) << 1); }
+
 // getNumChildren (CompressedShadowUtil.h:80-85): number of partial children.
 __host__ __device__ inline u32 num_children(u32 mask) { return (u32)__builtin_popcount(mask & 0xAAAAu); }
 

@@ -35,8 +35,7 @@ struct FItem {
     const float* depth;            // the map (level 0)
     const float2* lv[kMaxLevels];  // pyramid levels >= 3
     u32 N, T, t, R;                // side, zTileNum, zTileIndex, root level (numLevels - 2)
-    u32 w3, w3_shift, col_base;    // leaf columns: N/8 per side, first column record
-    u32 pad;
+    u32 w3, col_base;              // leaf columns: N/8 per side, first column record (a map's in Morton order)
 };
 
 // Node coordinates at levels >= 3 with the DAG's index: x, y < 2^13 (N <= 65536), z < 2^18
@@ -90,8 +89,9 @@ __global__ __launch_bounds__(256) void k_forest_counts(const FCountRec* __restri
         const u32 j = base + k * 256 + threadIdx.x;
         if (j < w * w) {
             int s;
-            const u32 c = exact ? reachable_cells(it.lv, j % w, j / w, L, (int)it.R, it.N, it.T, zlo, zhi, &s)
-                                : partial_cells(lv[j], h, zlo, zhi, &s);
+            const u32 x = colc ? even_bits(j) : j & (w - 1), y = colc ? even_bits(j >> 1) : j / w;
+            const u32 c = exact ? reachable_cells(it.lv, x, y, L, (int)it.R, it.N, it.T, zlo, zhi, &s)
+                                : partial_cells(lv[(size_t)y * w + x], h, zlo, zhi, &s);
             if (colc) colc[j] = make_uint4(c, 0u, (u32)max(s, 0), r.item);
             acc += c;
         }
@@ -200,12 +200,12 @@ struct FEmitOut {
         if (colbfs) {
             const FItem& it = items[g];
             const uint4* info = colinfo + it.col_base;
-            const u32 xc = min(x, it.w3 - 2) & ~1u, yc = min(y, it.w3 - 2);  // inside the DAG's columns
+            const u32 at = morton2(min(x, it.w3 - 2) & ~1u, min(y, it.w3 - 2) & ~1u);  // inside the DAG's columns
             uint4 ci[4];
 #pragma unroll
             for (u32 q = 0; q < 4; ++q) {
                 ci[q] = make_uint4(0u, 0u, 0u, 0u);
-                if (m & ((2u << (2 * q)) | (2u << (2 * (q + 4))))) ci[q] = info[(yc + (q >> 1)) * it.w3 + xc + (q & 1)];
+                if (m & ((2u << (2 * q)) | (2u << (2 * (q + 4))))) ci[q] = info[at + q];
             }
 #pragma unroll
             for (u32 ch = 0; ch < 8; ++ch) {
@@ -227,109 +227,40 @@ struct FEmitOut {
 };
 
 // ---------------------------------------------------------------------------------------
-// 3. Leaves: the single build's column waves (build.hip, k_leaf_waves) over the forest's list of
-//    columns with leaf nodes.  A column's record names its DAG (.w), whose map, size and z-tile
-//    give the column's depth block and scale.  kCols columns per wave, kWaves waves per group.
+// 3. Leaves: the single build's kernels (build.hip) over the forest's list of columns with leaf nodes.
+//    A column's record names its DAG (.w), whose map, size and z-tile give the column's depth block
+//    and scale.
 // ---------------------------------------------------------------------------------------
-template <u32 kCols, u32 kWaves>
-__global__ __launch_bounds__(64 * kWaves) void k_forest_leaf(const uint4* __restrict__ colinfo, const u32* __restrict__ colbfs,
-                                                             const FItem* __restrict__ items, u32 nleaf,
-                                                             u32* __restrict__ mask_out, u64* __restrict__ leafm,
-                                                             u32* __restrict__ runhead, u64* __restrict__ hash_out,
-                                                             u64* __restrict__ tab, u32 tab_slots,
-                                                             const u32* __restrict__ col_list, const u32* __restrict__ n_list,
-                                                             u32 list_cap) {
-    __shared__ int s_f[kWaves][kCols][64];
-    __shared__ u32 s_b[kWaves][kCols][64];
-    __shared__ uint8_t s_chg[kWaves][128];  // each wave's changed-node flags (leaf_column)
-    const u32 lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const u32 nvalid = min(*n_list, list_cap);
-    for (u32 c0 = (blockIdx.x * kWaves + wave) * kCols; c0 < nvalid; c0 += gridDim.x * kWaves * kCols) {
-    const u32 clast = nvalid ? nvalid - 1 : 0u;
-    const u32 my_col = nvalid ? col_list[min(c0 + (lane & (kCols - 1)), clast)] : 0u;
-    uint4 ci = colinfo[my_col];
-    if (lane >= kCols || c0 + lane >= nvalid) ci = make_uint4(0u, 0u, 0u, 0u);
-    float d[kCols];
-    float HT[kCols];
-#pragma unroll
-    for (u32 k = 0; k < kCols; ++k) {
-        const u32 c = __builtin_amdgcn_readlane(my_col, k);
-        const FItem& it = items[__builtin_amdgcn_readlane(ci.w, k)];
-        const u32 local = c - it.col_base;
-        const u32 x3 = local & (it.w3 - 1), y3 = local >> it.w3_shift;
-        HT[k] = (float)(it.N * it.T);
-        const float* blk = it.depth + ((size_t)(8 * y3) * it.N + 8 * x3);  // uniform base, per-lane offset
-        d[k] = 0.0f;
-        const u32 loff = 4u * ((lane >> 3) * it.N + (lane & 7));  // bytes, below 2^32 (N <= 65536)
-        if (__builtin_amdgcn_readlane(ci.x, k) != 0u)
-            d[k] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(blk) + loff);
-    }
-    u32 b[kCols];
-#pragma unroll
-    for (u32 k = 0; k < kCols; ++k) {
-        const u32 cnt = __builtin_amdgcn_readlane(ci.x, k), st = __builtin_amdgcn_readlane(ci.y, k);
-        const u32* run = colbfs + (cnt ? st : 0u);
-        b[k] = run[(lane < cnt) ? lane : 0u];
-    }
-    // The columns' minimum and maximum f from their DAGs' level-3 pyramid texels (lane k < kCols:
-    // column k's minimum, lane k + kCols its maximum), or from the texels for a block with a NaN.
-    int fext;
-    {
-        const uint4 cj = colinfo[my_col];  // lanes k and k + kCols read column k's record
-        const FItem& it = items[cj.w];
-        const float2 ext = it.lv[3][my_col - it.col_base];
-        fext = leaf_f(((lane & kCols) ? ext.y : ext.x) * (float)(it.N * it.T));
-    }
-    u32 nan_cols = 0;
-#pragma unroll
-    for (u32 k = 0; k < kCols; ++k) {
-        const float D = d[k] * HT[k];
-        if (__ballot(!(D == D))) nan_cols |= 1u << k;
-        s_f[wave][k][lane] = leaf_f(D);
-        s_b[wave][k][lane] = b[k];
-    }
+__device__ inline LeafCol forest_column(const uint4* colinfo, const FItem* items, u32 col, const float2** ext) {
+    const uint4 ci = colinfo[col];
+    const FItem& it = items[ci.w];
+    const u32 x = even_bits(col - it.col_base), y = even_bits((col - it.col_base) >> 1);
+    if (ext) *ext = it.lv[3] + (size_t)y * it.w3 + x;
+    return LeafCol{col, it.depth + ((size_t)(8 * y) * it.N + 8 * x), it.N, (float)(it.N * it.T), ci.x, ci.y, (int)ci.z, ci.w << 16};
+}
 
-    // The wave's columns with leaf nodes (ci is zero for lanes past the list).
-    for (u32 todo = (u32)__ballot(ci.x != 0u); todo; todo &= todo - 1u) {
-        const u32 k = (u32)__builtin_ctz(todo);
-        const u32 cnt = __builtin_amdgcn_readlane(ci.x, k);
-        const u32 base = __builtin_amdgcn_readlane(ci.y, k);
-        const int zs = (int)__builtin_amdgcn_readlane(ci.z, k);
-        const u32 gtag = __builtin_amdgcn_readlane(ci.w, k) << 16;
-        const int f = s_f[wave][k][lane];
-        int fmin = __builtin_amdgcn_readlane(fext, k), fmax = __builtin_amdgcn_readlane(fext, k + kCols);
-        if ((nan_cols >> k) & 1u) {
-            fmin = __ockl_wfred_min_i32(f);
-            fmax = __ockl_wfred_max_i32(f);
-        }
-        leaf_column(f, fmin, fmax, zs, cnt, s_b[wave][k][lane], colbfs + base, gtag, nleaf,
-                    kWaves == 1 ? s_chg[0] : s_chg[wave], lane, mask_out, leafm, runhead, hash_out);
-    }
+__global__ __launch_bounds__(64) void k_forest_waves(const uint4* __restrict__ colinfo, const FItem* __restrict__ items,
+                                                     LeafOut o, u64* __restrict__ tab, u32 tab_slots,
+                                                     const u32* __restrict__ col_list, const u32* __restrict__ n_list,
+                                                     u32 list_cap) {
+    __shared__ uint8_t s_chg[128];
+    const u32 n = min(*n_list, list_cap);
+    for (u32 u = blockIdx.x; u < n; u += gridDim.x) {
+        const float2* ext;
+        const LeafCol c = forest_column(colinfo, items, col_list[u], &ext);
+        if (c.cnt) leaf_wave(c, ext, o, s_chg, threadIdx.x);
     }
     clear_table(tab, tab_slots);
 }
 
-// The same with one column per lane (leaf_lane) over the list.
 __global__ __launch_bounds__(kLaneThreads) void k_forest_lanes(const uint4* __restrict__ colinfo, const FItem* __restrict__ items,
                                                                LeafOut o, u64* __restrict__ tab, u32 tab_slots,
                                                                const u32* __restrict__ col_list,
                                                                const u32* __restrict__ n_list, u32 list_cap) {
-    const u32 n = min(*n_list, list_cap), k = blockIdx.x * kLaneThreads + threadIdx.x;
+    const u32 n = min(*n_list, list_cap), u = blockIdx.x * kLaneThreads + threadIdx.x;
     if (blockIdx.x * kLaneThreads < n) {
         LeafCol c{};
-        if (k < n) {
-            c.col = col_list[k];
-            const uint4 ci = colinfo[c.col];
-            const FItem& it = items[ci.w];
-            const u32 local = c.col - it.col_base, x3 = local & (it.w3 - 1), y3 = local >> it.w3_shift;
-            c.blk = it.depth + ((size_t)(8 * y3) * it.N + 8 * x3);
-            c.pitch = it.N;
-            c.HT = (float)(it.N * it.T);
-            c.cnt = ci.x;
-            c.start = ci.y;
-            c.zs = (int)ci.z;
-            c.gtag = ci.w << 16;
-        }
+        if (u < n) c = forest_column(colinfo, items, col_list[u], nullptr);
         leaf_lanes(c, o);
     }
     clear_table(tab, tab_slots);
@@ -450,36 +381,6 @@ constexpr int kRetrySort = -1010;
 constexpr int kRetryFull = -1011;
 constexpr int kRetryExact = -1012;  // the counts exceed the emitted nodes (a map with NaN depths)
 
-// Launches the leaf kernels: one column per lane and a wave for each column left over, or, below
-// kLaneLeafMin columns, waves only, in the shape the options name.  n_slow and slow: the columns
-// left over (room for lo.nleaf).
-void launch_leaf(const ForestOpts& o, u32 units_cols, hipStream_t s, const uint4* colinfo, const u32* colbfs,
-                 const FItem* items, u32 nleaf, u32* mask, u64* leafm, u32* runhead, u64* hash, u32* slow, u32* n_slow,
-                 u64* tab, u32 slots, const u32* clist, const u32* nclist, u32 cap) {
-    if (hash) {
-        const LeafOut lo{colbfs, mask, leafm, runhead, hash, slow, n_slow, nleaf};
-        CPVS_LAUNCH("forest_lanes", k_forest_lanes, dim3(ceil_div<u32>(units_cols, kLaneThreads)), dim3(kLaneThreads), 0, s,
-                    colinfo, items, lo, tab, slots, clist, nclist, cap);
-        CPVS_LAUNCH("forest_leaf", (k_forest_leaf<kSlowCols, 1>), dim3(std::min(ceil_div<u32>(units_cols, kSlowCols), kSlowWaves)),
-                    dim3(64), 0, s, colinfo, colbfs, items, nleaf, mask, leafm, runhead, hash, tab, 0u, slow, n_slow, cap);
-        return;
-    }
-    const u32 per = o.leaf_cols * o.leaf_waves;
-    const dim3 grid((units_cols + per - 1) / per);
-    if (o.leaf_cols == 4 && o.leaf_waves == 1)
-        CPVS_LAUNCH("forest_leaf", (k_forest_leaf<4, 1>), grid, dim3(64), 0, s, colinfo, colbfs, items, nleaf, mask, leafm,
-                    runhead, nullptr, tab, slots, clist, nclist, cap);
-    else if (o.leaf_cols == 4)
-        CPVS_LAUNCH("forest_leaf", (k_forest_leaf<4, 2>), grid, dim3(128), 0, s, colinfo, colbfs, items, nleaf, mask, leafm,
-                    runhead, nullptr, tab, slots, clist, nclist, cap);
-    else if (o.leaf_waves == 1)
-        CPVS_LAUNCH("forest_leaf", (k_forest_leaf<8, 1>), grid, dim3(64), 0, s, colinfo, colbfs, items, nleaf, mask, leafm,
-                    runhead, nullptr, tab, slots, clist, nclist, cap);
-    else
-        CPVS_LAUNCH("forest_leaf", (k_forest_leaf<8, 2>), grid, dim3(128), 0, s, colinfo, colbfs, items, nleaf, mask, leafm,
-                    runhead, nullptr, tab, slots, clist, nclist, cap);
-}
-
 // Pinned staging of one forest build.
 struct Stage {
     u32* partials;  // nblocks + M (root masks)
@@ -522,7 +423,6 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         it.t = x.t;
         it.R = (u32)(x.p->n - 2);
         it.w3 = x.p->N >> 3;
-        it.w3_shift = (u32)__builtin_ctz(it.w3);
         it.col_base = (u32)ncol;
         ncol += (u64)it.w3 * it.w3;
         Rmax = std::max(Rmax, (int)it.R);
@@ -544,11 +444,11 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
                2 * arena_bytes((size_t)M * kKL, 4) + arena_bytes(M, sizeof(u32*)) +
                arena_bytes(kMetaWords + 2 * (size_t)M + (size_t)M * kKL, 4);
     };
-    int rc = w.forest_staging(stage_bytes(nblocks));
+    int rc = w.staging(w.forest, stage_bytes(nblocks));
     if (rc) return rc;
     Stage st;
     {
-        char* p = static_cast<char*>(w.fpin);
+        char* p = static_cast<char*>(w.forest.p);
         st.partials = carve<u32>(p, nblocks + M);
         st.items = carve<FItem>(p, M);
         st.recs = carve<FCountRec>(p, recs.size());
@@ -662,7 +562,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         need += (L > 2 ? arena_bytes(c, 8) + arena_bytes(c, 4) : 0) + 4 * arena_bytes(c, 4) +  // no coords, starts at leaves
                 arena_bytes(first_words((u32)c), 8);
     }
-    need += arena_bytes(tab_slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(ntiles, 8);
+    need += arena_bytes(tab_slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(tile_pre_count(ntiles), 16);
     need += arena_bytes(c2 * 8, 8) + 2 * arena_bytes(c2, 4);  // leafmask rows, run heads, column map
     need += arena_bytes(ncol, 4) + arena_bytes(1, 4);
     if (!use_table) need += 5 * arena_bytes(cmax, 4) + arena_bytes(sort_scratch_words(cmax), 4);
@@ -699,7 +599,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         }
     }
     u32* tile_sums = A.take<u32>(ntiles);
-    u64* tile_pre = A.take<u64>(ntiles);
+    ulonglong2* tile_pre = A.take<ulonglong2>(tile_pre_count(ntiles));
     // The run heads' key hashes, from the leaf kernel to the leaf insert, in the place of the leaf
     // level's unique list and offsets (two arrays side by side), which k_offsets writes later.
     u64* leaf_hash = (C[2] && std::min<u64>(ncol, C[2]) >= kLaneLeafMin) ? reinterpret_cast<u64*>(lv.uniq[2]) : nullptr;
@@ -754,10 +654,20 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
                 device_scan(ChildCountIn{lv.mask[L]}, emit, c, OpSum{}, meta + kMetaC + L, scan_scratch, s);
             }
         }
-        if (C[2]) {  // (its kernel clears every level's table)
-            const u32 bound = (u32)std::min<u64>(ncol, C[2]);
-            launch_leaf(o, bound, s, colinfo, colbfs, items, (u32)C[2], lv.mask[2], leafm, runhead, leaf_hash, lv.id[2],
-                        meta + kMetaSlow, tab, use_table ? (u32)tab_slots : 0u, clist, nclist, bound);
+        if (C[2]) {
+            // At most min(columns, leaf nodes) columns are listed.  The first kernel clears the tables.
+            const u32 bound = (u32)std::min<u64>(ncol, C[2]), clear = use_table ? (u32)tab_slots : 0u;
+            const LeafOut lo{colbfs, lv.mask[2], leafm, runhead, leaf_hash, lv.id[2], meta + kMetaSlow, (u32)C[2]};
+            const dim3 waves(std::min(bound, kSlowWaves));
+            if (leaf_hash) {
+                CPVS_LAUNCH("forest_lanes", k_forest_lanes, grid_of(bound, kLaneThreads), dim3(kLaneThreads), 0, s, colinfo,
+                            items, lo, tab, clear, clist, nclist, bound);
+                CPVS_LAUNCH("forest_waves", k_forest_waves, waves, dim3(64), 0, s, colinfo, items, lo, tab, 0u, lv.id[2],
+                            meta + kMetaSlow, bound);
+            } else {
+                CPVS_LAUNCH("forest_waves", k_forest_waves, waves, dim3(64), 0, s, colinfo, items, lo, tab, clear, clist,
+                            nclist, bound);
+            }
         } else if (use_table) {
             CPVS_LAUNCH("table_clear", k_table_clear, grid_of(tab_slots, 256), dim3(256), 0, s, tab, (u32)tab_slots);
         }

@@ -65,11 +65,15 @@ struct Worker {
     Arena arena;   // build scratch
     Arena levels;  // pyramid levels of the item being built (of all maps of a forest)
     u64* pinned = nullptr;
-    void* fpin = nullptr;  // a forest's pinned staging (count partials, tables, readback), grown as needed
-    size_t fpin_bytes = 0;
+    struct Staging {  // pinned host memory, grown as needed
+        void* p = nullptr;
+        size_t bytes = 0;
+    };
+    Staging forest;    // a forest's count partials, tables and readback
+    Staging pyramids;  // its pyramids' records
     int create();  // on the current device
     void destroy();
-    int forest_staging(size_t bytes);  // ensures fpin holds bytes (waits for the stream first)
+    int staging(Staging& st, size_t bytes);  // ensures st holds bytes (waits for the stream before it replaces it)
 };
 
 // forest.hip: many DAGs built as one forest with one launch chain (see there).
@@ -79,8 +83,6 @@ struct ForestIn {
 };
 struct ForestOpts {
     int merge_mode = CPVS_MERGE_TABLE;
-    u32 leaf_cols = 8;    // leaf kernel: level-3 columns per wave (4 or 8)
-    u32 leaf_waves = 1;   // leaf kernel: waves per workgroup (1 or 2)
     bool graph = false;   // capture the level chain between the two readbacks in a hipGraph
 };
 constexpr int kForestTooLarge = -1002;  // a level's words or nodes exceed 32 bits: split the forest
@@ -197,9 +199,13 @@ struct cpvs_container {
 namespace cpvs {
 
 // pyramid.hip.  Levels go to a new allocation owned by p, or, when `into` is given, to that
-// arena (p then does not own them; the arena is reset, or with append the levels follow what it
-// holds, within a reservation the caller made).
-int pyramid_build_levels(cpvs_pyramid* p, bool store_all, hipStream_t s, Arena* into = nullptr, bool append = false);
+// arena, which is reset (p then does not own them).
+int pyramid_build_levels(cpvs_pyramid* p, bool store_all, hipStream_t s, Arena* into = nullptr);
+// The levels >= 3 of n maps' pyramids (ps[i]->depth, N and n set), in three launches for all of them, into
+// the arena (within a reservation of their pyramid_levels_bytes and pyramids_rec_bytes(n)).  pinned:
+// pyramids_rec_bytes(n) bytes of pinned host memory, in use until the stream has passed the copy.
+size_t pyramids_rec_bytes(u32 n);
+int pyramids_build(cpvs_pyramid* const* ps, u32 n, void* pinned, Arena& into, hipStream_t s);
 // Exact node counts per level for z-tile t of T.  Each count workgroup writes its partial count
 // to partials[block] (pinned host memory, kPinnedPartials entries; may be null), and
 // sum_node_counts adds them up per level once the stream has reached that point: cnt[L] = nodes

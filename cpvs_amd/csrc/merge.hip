@@ -231,78 +231,83 @@ __device__ inline void level_bases(u32* meta, int R) {
 
 __device__ inline u32 saturate32(u64 v) { return v > 0xFFFFFFFFull ? 0xFFFFFFFFu : (u32)v; }
 
-// One workgroup: a scan over all tiles, each thread a contiguous run of them.  A tile's prefix is
-// relative to its level's first tile; word sums run in 64 bits, and a prefix or a level total at
-// or above 2^32 is stored saturated, so that the host rejects the DAG.
+// One workgroup: a scan over all tiles of all levels, four to a thread at a time.  tile_pre gets
+// (first occurrences, words) before each tile, then, after the tiles, before each level and at the
+// end; k_offsets subtracts its level's.  A level's total at or above 2^32 words is stored
+// saturated, so that the host rejects the DAG.  (Levels' starts are kept in LDS: looked up in the
+// kernel's arguments by a varying index they took twice the scan's time.)
 constexpr u32 kTotalsThreads = 1024;
 __global__ __launch_bounds__(kTotalsThreads) void k_totals(MArgs a, const u32* __restrict__ tile_sums,
-                                                           u64* __restrict__ tile_pre, u32* __restrict__ meta, int R,
+                                                           ulonglong2* __restrict__ tile_pre, u32* __restrict__ meta, int R,
                                                            u32* __restrict__ host_meta) {
-    __shared__ u32 s_c[kTotalsThreads / kWave];
-    __shared__ u64 s_w[kTotalsThreads / kWave];
-    __shared__ u32 lev_c[kMaxLevels + 1];  // first occurrences and words before each level
+    constexpr u32 kWaves = kTotalsThreads / kWave, kPer = 4;
+    __shared__ u32 s_c[2][kWaves], s_w[2][kWaves], s_tile0[kMaxLevels + 1];
+    __shared__ u32 lev_c[kMaxLevels + 1];
     __shared__ u64 lev_w[kMaxLevels + 1];
-    const u32 nt = a.tile0[a.nlev];
-    const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
-    const u32 E = ceil_div<u32>(nt, kTotalsThreads);
-    const u32 b = min(threadIdx.x * E, nt), e = min(b + E, nt);
-    u32 c = 0;
-    u64 w = 0;
-#pragma unroll 4
-    for (u32 i = b; i < e; ++i) {
-        const u32 v = tile_sums[i];
-        c += v >> 16;
-        w += v & 0xFFFFu;
-    }
-    const u32 ci = wave_inclusive_scan(c, OpSum{});
-    const u64 wi = wave_inclusive_scan(w, OpSum64{});
-    if (lane == kWave - 1) {
-        s_c[wid] = ci;
-        s_w[wid] = wi;
-    }
-    __syncthreads();
-    u32 c0 = ci - c;
-    u64 w0 = wi - w;
+    const u32 nt = a.tile0[a.nlev], nlev = (u32)a.nlev;
+    const u32 lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+    if (threadIdx.x <= nlev) s_tile0[threadIdx.x] = a.tile0[threadIdx.x];
+    u32 run_c = 0;  // of the chunks before
+    u64 run_w = 0;
+    u32 v[kPer];
+    auto load = [&](u32 t0) {
 #pragma unroll
-    for (int v = 0; v < (int)(kTotalsThreads / kWave); ++v)
-        if (v < wid) {
-            c0 += s_c[v];
-            w0 += s_w[v];
+        for (u32 j = 0; j < kPer; ++j) v[j] = (t0 + j < nt) ? tile_sums[t0 + j] : 0u;
+    };
+    load(threadIdx.x * kPer);
+    u32 buf = 0;
+    for (u32 base = 0; base < nt; base += kTotalsThreads * kPer, buf ^= 1u) {
+        const u32 t0 = base + threadIdx.x * kPer;
+        u32 x[kPer], c = 0, w = 0;  // (a chunk of 4096 tiles of at most 17408 words fits 32 bits)
+#pragma unroll
+        for (u32 j = 0; j < kPer; ++j) {
+            x[j] = v[j];
+            c += v[j] >> 16;
+            w += v[j] & 0xFFFFu;
         }
-    if (b < e || (threadIdx.x == kTotalsThreads - 1)) {
-        // Level starts inside this thread's run (the end of the last level counts as one).
-        u32 cc = c0;
-        u64 ww = w0;
-        int k = 0;
-        while (k <= a.nlev && a.tile0[k] < b) ++k;
-        for (u32 i = b; i < e; ++i) {
-            for (; k <= a.nlev && a.tile0[k] == i; ++k) {
+        load(t0 + kTotalsThreads * kPer);  // the next chunk's, while this one is scanned
+        const u32 ci = wave_inclusive_scan(c, OpSum{}), wi = wave_inclusive_scan(w, OpSum{});
+        if (lane == kWave - 1) {
+            s_c[buf][wid] = ci;
+            s_w[buf][wid] = wi;
+        }
+        __syncthreads();  // (also: the levels' first tiles are in; the other buffer's readers are done)
+        u32 pc = 0, pw = 0, tc = 0, tw = 0;
+#pragma unroll
+        for (u32 u = 0; u < kWaves; ++u) {
+            if (u == wid) {
+                pc = tc;
+                pw = tw;
+            }
+            tc += s_c[buf][u];
+            tw += s_w[buf][u];
+        }
+        u32 cc = run_c + pc + ci - c;
+        u64 ww = run_w + pw + wi - w;
+        run_c += tc;
+        run_w += tw;
+        u32 k = 0;
+        while (k < nlev && s_tile0[k] < t0) ++k;
+#pragma unroll
+        for (u32 j = 0; j < kPer; ++j) {
+            if (t0 + j >= nt) break;
+            if (k < nlev && s_tile0[k] == t0 + j) {  // a level's first tile (every level has one)
                 lev_c[k] = cc;
                 lev_w[k] = ww;
+                ++k;
             }
-            const u32 v = tile_sums[i];
-            cc += v >> 16;
-            ww += v & 0xFFFFu;
+            tile_pre[t0 + j] = make_ulonglong2(cc, ww);
+            cc += x[j] >> 16;
+            ww += x[j] & 0xFFFFu;
         }
-        if (e == nt)
-            for (; k <= a.nlev; ++k) {  // (several threads may hold the end: the same values)
-                lev_c[k] = cc;
-                lev_w[k] = ww;
-            }
+    }
+    if (threadIdx.x == 0) {
+        lev_c[nlev] = run_c;
+        lev_w[nlev] = run_w;
     }
     __syncthreads();
-    {
-        int k = 0;
-        while (k + 1 < a.nlev && a.tile0[k + 1] <= b) ++k;
-        for (u32 i = b; i < e; ++i) {
-            while (k + 1 < a.nlev && a.tile0[k + 1] <= i) ++k;
-            tile_pre[i] = ((u64)(c0 - lev_c[k]) << 32) | saturate32(w0 - lev_w[k]);
-            const u32 v = tile_sums[i];
-            c0 += v >> 16;
-            w0 += v & 0xFFFFu;
-        }
-    }
-    if (threadIdx.x < (u32)a.nlev) {
+    if (threadIdx.x <= nlev) tile_pre[nt + threadIdx.x] = make_ulonglong2(lev_c[threadIdx.x], lev_w[threadIdx.x]);
+    if (threadIdx.x < nlev) {
         const u32 k = threadIdx.x;
         meta[kMetaU + a.lv[k].L] = lev_c[k + 1] - lev_c[k];
         meta[kMetaS + a.lv[k].L] = saturate32(lev_w[k + 1] - lev_w[k]);
@@ -319,11 +324,13 @@ __global__ __launch_bounds__(kTotalsThreads) void k_totals(MArgs a, const u32* _
     }
 }
 
-__global__ __launch_bounds__(kTileThreads) void k_offsets(MArgs a, const u64* __restrict__ tile_pre) {
+__global__ __launch_bounds__(kTileThreads) void k_offsets(MArgs a, const ulonglong2* __restrict__ tile_pre) {
     const int k = level_of_tile(a, blockIdx.x);
     const MLevel& l = a.lv[k];
     const u32 base = (blockIdx.x - a.tile0[k]) * kTileNodes + threadIdx.x;
-    const u64 pre = tile_pre[blockIdx.x];
+    const ulonglong2 pre = tile_pre[blockIdx.x], lev = tile_pre[a.tile0[a.nlev] + k];
+    const u32 rank0 = (u32)(pre.x - lev.x);
+    const u64 off0 = pre.y - lev.y;
     u32 v[kTileRounds], ex[kTileRounds], id[kTileRounds];
 #pragma unroll
     for (int j = 0; j < kTileRounds; ++j) {
@@ -341,8 +348,8 @@ __global__ __launch_bounds__(kTileThreads) void k_offsets(MArgs a, const u64* __
 #pragma unroll
     for (int j = 0; j < kTileRounds; ++j) {
         if (!v[j]) continue;
-        const u32 rank = (u32)(pre >> 32) + (ex[j] >> 16);
-        const u32 off = saturate32((u64)(u32)pre + (ex[j] & 0xFFFFu));
+        const u32 rank = rank0 + (ex[j] >> 16);
+        const u32 off = saturate32(off0 + (ex[j] & 0xFFFFu));
         l.uniq[rank] = base + j * kTileThreads;
         l.off[rank] = off;
         if (!l.lone) l.tab[min(id[j], l.slots - 1)] = ((u64)rank << 32) | off;
@@ -455,7 +462,7 @@ void merge_sort_level(const MArgs& a, int k, const SortScratch& t, u32* meta, hi
                     InnerEq{l.mask, l.cstart, ch.id, ch.n}, l.id, meta + kMetaSortColl);
 }
 
-void merge_finish(const MArgs& a, bool sorted, u32* tile_sums, u64* tile_pre, u32* meta, int R, u32* host_meta,
+void merge_finish(const MArgs& a, bool sorted, u32* tile_sums, ulonglong2* tile_pre, u32* meta, int R, u32* host_meta,
                   hipStream_t s) {
     const u32 nt = a.tile0[a.nlev];
     if (sorted)

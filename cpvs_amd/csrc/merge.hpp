@@ -38,6 +38,7 @@ constexpr u32 kTileThreads = 256;
 constexpr int kTileRounds = 4;
 constexpr u32 kTileNodes = kTileThreads * kTileRounds;
 
+inline size_t tile_pre_count(u32 tiles) { return (size_t)tiles + kMaxLevels + 1; }
 inline size_t first_words(u32 n) { return (n + 63) / 64; }  // 64-bit words of MLevel::first
 
 // Launches.  insert_level: identities of level k of `a` by its table (a.lv[k].tab, cleared before);
@@ -49,10 +50,10 @@ struct SortScratch {
 };
 void merge_sort_level(const MArgs& a, int k, const SortScratch& t, u32* meta, hipStream_t s);
 // After every level has its identities: first occurrences (with the key compares of the table
-// merge), their ranks and word offsets, level totals in meta.  tile_sums and tile_pre: one entry
-// per tile.  R >= 0: a single build, whose level bases and root mask go to meta too.  host_meta
+// merge), their ranks and word offsets, level totals in meta.  tile_sums: one entry per tile;
+// tile_pre: tile_pre_count(tiles).  R >= 0: a single build, whose level bases and root mask go to meta too.  host_meta
 // (pinned, may be null) receives meta.
-void merge_finish(const MArgs& a, bool sorted, u32* tile_sums, u64* tile_pre, u32* meta, int R, u32* host_meta,
+void merge_finish(const MArgs& a, bool sorted, u32* tile_sums, ulonglong2* tile_pre, u32* meta, int R, u32* host_meta,
                   hipStream_t s);
 // A single build's words, level bases from meta, into out; nothing when they exceed cap words.
 void merge_write(const MArgs& a, const u32* meta, u32* out, u64 cap, hipStream_t s);

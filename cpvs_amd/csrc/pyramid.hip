@@ -9,6 +9,8 @@
 // build reads depth directly and pyramid levels >= 3 (src/CompressedShadow.cpp:104-106,162-166).
 // Every (min, max) is combined as min(min(a,b), min(c,d)) over the 2x2 block [a b; c d]
 // exactly as constructRange/setRow/find do (src/MinMaxHierarchy.cpp:29-49).
+#include <vector>
+
 #include "internal.hpp"
 
 namespace cpvs {
@@ -21,12 +23,12 @@ __device__ inline float2 combine4(float2 a, float2 b, float2 c, float2 d) {
     return make_float2(smin(smin(a.x, b.x), smin(c.x, d.x)), smax(smax(a.y, b.y), smax(c.y, d.y)));
 }
 
+// Tile (bx, by) / 64 of one level.
 template <bool ROOT>
-__global__ __launch_bounds__(256) void k_pyr_tile(const float* __restrict__ in, u32 W, PyrOut out) {
+__device__ inline void pyr_tile(const float* __restrict__ in, u32 W, const PyrOut& out, u32 bx, u32 by) {
     __shared__ float2 s_a[16 * 16];
     __shared__ float2 s_b[8 * 8];
     const u32 t = threadIdx.x, tx = t & 15, ty = t >> 4;
-    const u32 bx = blockIdx.x * 64, by = blockIdx.y * 64;
     const u32 x0 = bx + 4 * tx, y0 = by + 4 * ty;
 
     float2 p[4][4];  // p[row][col] of the 4x4 input patch as (min, max)
@@ -99,9 +101,14 @@ __global__ __launch_bounds__(256) void k_pyr_tile(const float* __restrict__ in, 
     }
 }
 
+template <bool ROOT>
+__global__ __launch_bounds__(256) void k_pyr_tile(const float* __restrict__ in, u32 W, PyrOut out) {
+    pyr_tile<ROOT>(in, W, out, blockIdx.x * 64, blockIdx.y * 64);
+}
+
 // One block reduces an input level of width W <= 32 (all of it in LDS) down to 1x1.
 template <bool ROOT>
-__global__ __launch_bounds__(256) void k_pyr_small(const float* __restrict__ in, u32 W, PyrOut out, int nout) {
+__device__ inline void pyr_small(const float* __restrict__ in, u32 W, const PyrOut& out, int nout) {
     __shared__ float2 s_a[32 * 32];
     __shared__ float2 s_b[16 * 16];
     for (u32 i = threadIdx.x; i < W * W; i += blockDim.x) {
@@ -133,6 +140,38 @@ __global__ __launch_bounds__(256) void k_pyr_small(const float* __restrict__ in,
     }
 }
 
+template <bool ROOT>
+__global__ __launch_bounds__(256) void k_pyr_small(const float* __restrict__ in, u32 W, PyrOut out, int nout) {
+    pyr_small<ROOT>(in, W, out, nout);
+}
+
+// The same for many maps in one launch: record r's tiles are the blocks [recs[r].block0,
+// recs[r + 1].block0); of the small form, block r is record r.  A batch of 32 maps spent a quarter of
+// its time on 64 launches of a few microseconds each.
+struct PyrRec {
+    const float* in;
+    PyrOut out;
+    u32 W, block0;
+    int nout, root;
+};
+template <bool ROOT>
+__global__ __launch_bounds__(256) void k_pyr_tiles(const PyrRec* __restrict__ recs, u32 n) {
+    u32 lo = 0, hi = n;  // recs[lo].block0 <= blockIdx.x < recs[hi].block0
+    while (hi - lo > 1) {
+        const u32 mid = (lo + hi) >> 1;
+        if (recs[mid].block0 <= blockIdx.x) lo = mid;
+        else hi = mid;
+    }
+    const PyrRec& r = recs[lo];
+    const u32 b = blockIdx.x - r.block0, per = r.W / 64;
+    pyr_tile<ROOT>(r.in, r.W, r.out, (b % per) * 64, (b / per) * 64);
+}
+__global__ __launch_bounds__(256) void k_pyr_smalls(const PyrRec* __restrict__ recs) {
+    const PyrRec& r = recs[blockIdx.x];
+    if (r.root) pyr_small<true>(r.in, r.W, r.out, r.nout);
+    else pyr_small<false>(r.in, r.W, r.out, r.nout);
+}
+
 size_t pyramid_levels_bytes(u32 N, bool store_all) {
     int n = 1;
     while ((1u << (n - 1)) < N) ++n;
@@ -143,7 +182,7 @@ size_t pyramid_levels_bytes(u32 N, bool store_all) {
     return arena_bytes(total ? total : 1, sizeof(float2));
 }
 
-int pyramid_build_levels(cpvs_pyramid* p, bool store_all, hipStream_t s, Arena* into, bool append) {
+int pyramid_build_levels(cpvs_pyramid* p, bool store_all, hipStream_t s, Arena* into) {
     const u32 N = p->N;
     const int n = p->n;
     // Store levels 1-2 only when asked, or when the octree uses them (no leafmasks, N < 16).
@@ -157,10 +196,8 @@ int pyramid_build_levels(cpvs_pyramid* p, bool store_all, hipStream_t s, Arena* 
         total += w * w;
     }
     if (into) {
-        if (!append) {
-            const int rc = into->reserve(arena_bytes(total ? total : 1, sizeof(float2)), s);
-            if (rc) return rc;
-        }
+        const int rc = into->reserve(arena_bytes(total ? total : 1, sizeof(float2)), s);
+        if (rc) return rc;
         p->levels = into->take<float2>(total ? total : 1);
         p->levels_owned = false;
         if (into->used > into->cap) {
@@ -205,6 +242,67 @@ int pyramid_build_levels(cpvs_pyramid* p, bool store_all, hipStream_t s, Arena* 
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "pyramid launch", __FILE__, __LINE__);
+    return CPVS_OK;
+}
+
+size_t pyramids_rec_bytes(u32 n) { return arena_bytes(3 * (size_t)n, sizeof(PyrRec)); }
+
+int pyramids_build(cpvs_pyramid* const* ps, u32 n, void* pinned, Arena& into, hipStream_t s) {
+    // A map's steps: its first six levels (tiles of the map, or for N < 64 all of it at once), then
+    // tiles again while the level is at least 64 wide (N >= 4096), then the rest at once.
+    std::vector<PyrRec> step[3];  // root tiles, further tiles, small
+    u32 blocks[2] = {0, 0};
+    for (u32 i = 0; i < n; ++i) {
+        cpvs_pyramid* p = ps[i];
+        size_t off[kMaxLevels] = {}, total = 0;
+        for (int L = 3; L < p->n; ++L) {
+            off[L] = total;
+            total += (size_t)(p->N >> L) * (p->N >> L);
+        }
+        p->levels = into.take<float2>(total ? total : 1);
+        p->levels_owned = false;
+        for (int L = 3; L < p->n; ++L) p->lv[L] = p->levels + off[L];
+        int at = 0;
+        for (u32 W = p->N; W > 1;) {
+            PyrRec r = {};
+            r.in = at == 0 ? p->depth : reinterpret_cast<const float*>(p->lv[at]);
+            r.W = W;
+            r.root = at == 0;
+            const bool tiles = W >= 64;
+            int nout = 6;
+            if (!tiles)
+                for (nout = 0; (W >> nout) > 1;) ++nout;
+            r.nout = nout;
+            for (int k = 0; k < 6 && k < nout; ++k) r.out.lv[k] = (at + 1 + k < p->n) ? p->lv[at + 1 + k] : nullptr;
+            const int kind = tiles ? (at == 0 ? 0 : 1) : 2;
+            if (tiles) {
+                r.block0 = blocks[kind];
+                blocks[kind] += (W / 64) * (W / 64);
+            }
+            step[kind].push_back(r);
+            at += nout;
+            W = tiles ? W / 64 : 1;
+        }
+    }
+    PyrRec* d = into.take<PyrRec>(3 * (size_t)n);
+    if (into.used > into.cap) {
+        set_error("pyramids: the level arena holds %zu bytes, %zu needed", into.cap, into.used);
+        return CPVS_EINTERNAL;
+    }
+    PyrRec* h = static_cast<PyrRec*>(pinned);
+    u32 first[3], m = 0;
+    for (int k = 0; k < 3; ++k) {
+        first[k] = m;
+        for (const PyrRec& r : step[k]) h[m++] = r;
+    }
+    CPVS_HIP_CHECK(hipMemcpyAsync(d, h, sizeof(PyrRec) * m, hipMemcpyHostToDevice, s));
+    if (blocks[0])
+        CPVS_LAUNCH("pyr_tile_root", k_pyr_tiles<true>, dim3(blocks[0]), dim3(256), 0, s, d + first[0], (u32)step[0].size());
+    if (blocks[1])
+        CPVS_LAUNCH("pyr_tile", k_pyr_tiles<false>, dim3(blocks[1]), dim3(256), 0, s, d + first[1], (u32)step[1].size());
+    if (!step[2].empty())
+        CPVS_LAUNCH("pyr_small", k_pyr_smalls, dim3((u32)step[2].size()), dim3(256), 0, s, d + first[2]);
+    CPVS_HIP_CHECK(hipGetLastError());
     return CPVS_OK;
 }
 
@@ -253,8 +351,10 @@ __global__ __launch_bounds__(256) void k_node_counts(CountArgs a) {
         const u32 j = base + r * 256 + threadIdx.x;
         if (j < w * w) {
             int s;
-            const u32 c = a.exact ? reachable_cells(a.by_level, j % w, j / w, L, a.R, a.N, a.T, zlo, zhi, &s)
-                                  : partial_cells(a.lv[k][j], h, zlo, zhi, &s);
+            // Leaf columns are numbered in Morton order; the other levels are only counted.
+            const u32 x = colc ? even_bits(j) : j & (w - 1), y = colc ? even_bits(j >> 1) : j / w;
+            const u32 c = a.exact ? reachable_cells(a.by_level, x, y, L, a.R, a.N, a.T, zlo, zhi, &s)
+                                  : partial_cells(a.lv[k][(size_t)y * w + x], h, zlo, zhi, &s);
             if (colc) colc[j] = make_uint4(c, 0u, (u32)max(s, 0), 0u);
             acc += c;
         }

@@ -257,9 +257,10 @@ int cpvs_tune_batch(cpvs_ctx *ctx, const cpvs_batch_item *items, uint32_t count,
  * launch chain, every octree level one array over all of them, all counts from one launch and one
  * readback -- each forest holding maps of at most forest_mtexels x 2^20 texels of work (N^2 /
  * zTileNum per item; the z-tiles of one map stay in one forest and share its pyramid), `lanes`
- * forests at once.  leaf_cols (4 or 8) and leaf_waves (1 or 2) shape the forest's leaf kernel
- * (level-3 columns per wave, waves per workgroup); graph = 1 captures each forest's level chain in
- * a hipGraph and launches it as one.  Words are identical to cpvs_build's in every configuration.
+ * forests at once.  leaf_cols (4 or 8) and leaf_waves (1 or 2) are accepted and checked but change
+ * nothing any more: the leaf kernels take their shape from the number of columns.  graph = 1 captures
+ * each forest's level chain in a hipGraph and launches it as one.  Words are identical to
+ * cpvs_build's in every configuration.
  * Maps with N < 16 (no leafmask levels) are built one by one. */
 typedef struct cpvs_batch_config {
     uint32_t lanes;           /* 1..16 */
