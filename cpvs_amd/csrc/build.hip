@@ -26,6 +26,8 @@
 //      level bases root first, then one pass writes [mask, absolute child offsets] or
 //      [mask, lo, hi, ...] (src/CompressedShadow.cpp:326-392).
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 
@@ -357,7 +359,6 @@ u64 bound_words_of(const u64* cnt, int bottom, int R, bool leaf) {
 constexpr int kRetryWithSort = -1000;
 constexpr int kRetryFullTable = -1001;
 constexpr int kRetryExactCounts = -1002;  // the counts exceed the emitted nodes (a map with NaN depths)
-static_assert(sizeof(u32) * kMetaWords <= sizeof(u64) * kPinnedWords, "meta readback fits the pinned staging");
 
 
 // small_leaf: a leaf level of at least kSmallLeafTableMin nodes gets a merge table sized for a
@@ -367,17 +368,52 @@ static_assert(sizeof(u32) * kMetaWords <= sizeof(u64) * kPinnedWords, "meta read
 // the build runs again.
 __global__ void k_store_word(u32* dst, u32 v) { *dst = v; }
 
-// The staged words into the DAG's own buffer (16-byte vectors where both are aligned).
-__global__ __launch_bounds__(256) void k_copy_words(const u32* __restrict__ src, u32* __restrict__ dst, u64 n) {
-    const u64 stride = (u64)gridDim.x * blockDim.x;
-    const u64 i0 = (u64)blockIdx.x * blockDim.x + threadIdx.x;
-    if ((((uintptr_t)src | (uintptr_t)dst) & 15) == 0) {
-        const u64 n4 = n / 4;
-        for (u64 i = i0; i < n4; i += stride) reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
-        for (u64 i = 4 * n4 + i0; i < n; i += stride) dst[i] = src[i];
-    } else {
-        for (u64 i = i0; i < n; i += stride) dst[i] = src[i];
+constexpr u32 kHostReady = kMetaWords, kHostDone = kMetaWords + 1;  // flags behind the meta readback
+static_assert(sizeof(u32) * (kMetaWords + 2) <= sizeof(u64) * kPinnedWords, "the readback fits the pinned staging");
+
+// Waits until none of n words of pinned memory, which queued kernels of stream s store to, reads
+// `unset` any more.  Reading them is about 6 us quicker than a stream synchronisation (6 against 12 us
+// for an empty kernel), which takes over after kPollUs: longer waits should not keep a core busy, and
+// a kernel that fails never stores.
+constexpr double kPollUs = 500.0;
+int wait_words(const volatile u32* w, size_t n, u32 unset, hipStream_t s) {
+    size_t k = 0;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (u32 spins = 1;; ++spins) {
+        while (k < n && w[k] != unset) ++k;
+        if (k == n) {
+            std::atomic_thread_fence(std::memory_order_acquire);
+            return CPVS_OK;
+        }
+        __builtin_ia32_pause();
+        if ((spins & 63u) == 0 &&
+            std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count() > kPollUs)
+            break;
     }
+    CPVS_HIP_CHECK(hipStreamSynchronize(s));
+    for (; k < n; ++k)
+        if (w[k] == unset) {
+            set_error("build: a readback word was not stored");
+            return CPVS_EINTERNAL;
+        }
+    return CPVS_OK;
+}
+
+}  // namespace
+
+int wait_stream(u64* pinned, hipStream_t s) {
+    u32* done = reinterpret_cast<u32*>(pinned) + kHostDone;
+    *static_cast<volatile u32*>(done) = 0;
+    CPVS_LAUNCH("done", k_store_word, dim3(1), dim3(1), 0, s, done, 1u);
+    CPVS_HIP_CHECK(hipGetLastError());
+    return wait_words(done, 1, 0u, s);
+}
+
+namespace {
+
+int store_and_wait(u32* dst, u32 v, u64* pinned, hipStream_t s) {
+    CPVS_LAUNCH("store_word", k_store_word, dim3(1), dim3(1), 0, s, dst, v);
+    return wait_stream(pinned, s);
 }
 
 int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 t, u32 T, hipStream_t s, int merge_mode,
@@ -400,7 +436,8 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     CountLayout lay;
     rc = pyramid_node_counts(p, t, T, leaf, pinned_partials(pinned), colinfo, s, &lay, exact);
     if (rc) return rc;
-    CPVS_HIP_CHECK(hipStreamSynchronize(s));
+    rc = wait_words(pinned_partials(pinned), lay.block_start[lay.nlev] + 1, kUnsetCount, s);
+    if (rc) return rc;
     u64 cnt[kMaxLevels] = {};
     sum_node_counts(lay, pinned_partials(pinned), cnt);
     cnt[R] = 1;
@@ -408,31 +445,28 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         // No partial child of the root (a z-tile above or below every surface, a flat map): the
         // DAG is the root's childmask alone, written without any further kernel.
         const u32 word = pinned_partials(pinned)[lay.block_start[lay.nlev]];
-        if (into) {  // a caller's buffer: the word is stored by a kernel, nothing is allocated
-            if (into->cap < 1) {
-                set_error("build: the DAG has 1 word, the output holds %llu", (unsigned long long)into->cap);
-                return CPVS_EINVAL;
-            }
-            CPVS_LAUNCH("store_word", k_store_word, dim3(1), dim3(1), 0, s, into->words, word);
-            CPVS_HIP_CHECK(hipGetLastError());
-            CPVS_HIP_CHECK(hipStreamSynchronize(s));
-            into->nwords = 1;
-            into->root_mask = word;
-            return CPVS_OK;
+        if (into && into->cap < 1) {
+            set_error("build: the DAG has 1 word, the output holds %llu", (unsigned long long)into->cap);
+            return CPVS_EINVAL;
         }
         if (admit) {
             rc = admit->fn(admit->user, A, 0, sizeof(u32));
             if (rc) return rc;
         }
-        u32* d_words = static_cast<u32*>(alloc_words(ctx, admit, 1));
+        u32* d_words = into ? into->words : static_cast<u32*>(alloc_words(ctx, admit, 1));
         if (!d_words) {
             set_error("build: hipMalloc of one DAG word failed");
             return CPVS_ENOMEM;
         }
-        const hipError_t e = hipMemcpy(d_words, &word, sizeof(u32), hipMemcpyHostToDevice);  // an idle buffer
-        if (e != hipSuccess) {
-            ctx->buffers.give(d_words);
-            return hip_fail(e, "build root word", __FILE__, __LINE__);
+        rc = store_and_wait(d_words, word, pinned, s);
+        if (rc) {
+            if (!into) ctx->buffers.give(d_words);
+            return rc;
+        }
+        if (into) {
+            into->nwords = 1;
+            into->root_mask = word;
+            return CPVS_OK;
         }
         cpvs_dag* d = new cpvs_dag();
         d->ctx = ctx;
@@ -465,15 +499,9 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     const bool col_list = leaf && T > 1;  // compact the z-tile's columns with leaf nodes
     const int deepest = deepest_level(cnt, bottom, R);
     const int Ls = small_levels(cnt, deepest, R, use_table, leaf);
-    // Pre-merge words bound the DAG: mask and child pointers per node, two words per partial slice
-    // at the leaves.  The words are written into a staging area of that size right behind the
-    // merge (no host readback before the write), then copied to an exact allocation; a caller's
-    // output buffer (into) is written directly.
-    const u64 bound_words = bound_words_of(cnt, bottom, R, leaf);
-    const bool staged = !into;
-    const size_t need = build_scratch_bytes(cnt, R, leaf, ncol, col_list, use_table, small_leaf, staged);
+    const size_t need = build_scratch_bytes(cnt, R, leaf, ncol, col_list, use_table, small_leaf);
     if (admit) {
-        rc = admit->fn(admit->user, A, need, 4 * bound_words);
+        rc = admit->fn(admit->user, A, need, 4 * bound_words_of(cnt, bottom, R, leaf));
         if (rc) return rc;
     }
     bool moved = false;
@@ -536,7 +564,6 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     }
     u32* scan_scratch = A.take<u32>(scan_scratch_words(scan_n));
     srt.scan_scratch = scan_scratch;
-    u32* staging = staged ? A.take<u32>(bound_words + 17) : nullptr;
     if (A.used > A.cap) {
         set_error("build: scratch layout exceeds its reservation (%zu > %zu)", A.used, A.cap);
         return CPVS_EINTERNAL;
@@ -653,11 +680,15 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
             merge_sort_level(ma, L - deepest, srt, meta, s);
     }
     if (Ls < R) CPVS_LAUNCH("small_insert", k_small_insert, dim3(1), dim3(kSmallThreads), 0, s, sa);
-    // --- 4. first occurrences, offsets, bases, words; one readback -------------------------
+    // --- 4. first occurrences, offsets, bases, one readback, words -------------------------
+    // The host reads the totals that k_totals stores in pinned memory while k_offsets runs, so the
+    // words go straight to a buffer of their exact size and the GPU does not wait for the host.
+    volatile u32* host_meta = reinterpret_cast<volatile u32*>(pinned);
+    host_meta[kHostReady] = 0;
     merge_finish(ma, !use_table, tile_sums, tile_pre, meta, R, reinterpret_cast<u32*>(pinned), s);
-    merge_write(ma, meta, staged ? staging : into->words, staged ? bound_words : into->cap, s);
     CPVS_HIP_CHECK(hipGetLastError());
-    CPVS_HIP_CHECK(hipStreamSynchronize(s));  // k_totals copied meta into pinned
+    rc = wait_words(host_meta + kHostReady, 1, 0u, s);
+    if (rc) return rc;
     u32 hm[kMetaWords];
     std::memcpy(hm, pinned, sizeof(hm));
 
@@ -687,24 +718,23 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
                   (unsigned long long)into->cap);
         return CPVS_EINVAL;
     }
+    u32* d_words = into ? into->words : static_cast<u32*>(alloc_words(ctx, admit, total ? total : 1));
+    if (!d_words) {
+        set_error("build: hipMalloc of %llu DAG words failed", (unsigned long long)total);
+        return CPVS_ENOMEM;
+    }
+    merge_write(ma, meta, d_words, total, s);
+    rc = wait_stream(pinned, s);
+    if (rc) {
+        if (!into) ctx->buffers.give(d_words);
+        return rc;
+    }
     if (into) {
         into->nwords = total;
         into->root_mask = hm[kMetaRoot];
         return CPVS_OK;
     }
-    u32* d_words = static_cast<u32*>(alloc_words(ctx, admit, total ? total : 1));
-    if (!d_words) {
-        set_error("build: hipMalloc of %llu DAG words failed", (unsigned long long)total);
-        return CPVS_ENOMEM;
-    }
-    if (total) CPVS_LAUNCH("copy_words", k_copy_words, dim3(std::min<u64>(ceil_div<u64>(total, 1024), 4096)), dim3(256), 0, s,
-                           staging, d_words, total);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) {
-        ctx->buffers.give(d_words);
-        return hip_fail(e, "build write", __FILE__, __LINE__);
-    }
+
     cpvs_dag* d = new cpvs_dag();
     d->ctx = ctx;
     d->n = n;
@@ -728,8 +758,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
 }  // namespace
 
 // What build_once lays out: cnt the nodes per level (bottom .. R), ncol the leaf columns.
-size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_list, bool use_table, bool small_leaf,
-                           bool staged) {
+size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_list, bool use_table, bool small_leaf) {
     const int bottom = leaf ? 2 : 0;
     const int Ls = small_levels(cnt, deepest_level(cnt, bottom, R), R, use_table, leaf);
     size_t need = arena_bytes(kMetaWords, sizeof(u32)) + (leaf ? arena_bytes(ncol, sizeof(uint4)) : 0);
@@ -750,7 +779,6 @@ size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_
     if (col_list) need += arena_bytes(ncol, 4) + arena_bytes(1, 4);
     if (!use_table) need += 5 * arena_bytes(cmax, 4) + arena_bytes(sort_scratch_words(cmax), 4);
     need += arena_bytes(scan_scratch_words((leaf && ncol > cmax) ? ncol : cmax), 4);
-    if (staged) need += arena_bytes(bound_words_of(cnt, bottom, R, leaf) + 17, 4);
     return need + (1 << 20);
 }
 

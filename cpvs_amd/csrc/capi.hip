@@ -160,11 +160,12 @@ void* BufferCache::take_cached(size_t bytes, size_t limit) {
     void* p = fit_from(free_, bytes, most, &got);
     if (!p && !pending_.empty()) {
         auto it = pending_.lower_bound(bytes);
-        if (it != pending_.end() && it->first <= most) {
+        if (it != pending_.end() && it->first <= most && (pending_bytes >= kPendingBytes || pending_.size() >= kPendingCount)) {
             // Every buffer freed so far becomes idle with one device synchronisation (those freed
             // while it runs stay pending: their readers may have been queued after it began).
             std::multimap<size_t, void*> parked;
             parked.swap(pending_);
+            pending_bytes = 0;
             lk.unlock();
             (void)hipSetDevice(device);
             (void)hipDeviceSynchronize();
@@ -207,6 +208,7 @@ void BufferCache::park(void* p, bool idle) {
         if (it != live_.end()) live_.erase(it);
         if (bytes && cached + bytes <= kMaxBytes) {
             (idle ? free_ : pending_).emplace(bytes, p);
+            if (!idle) pending_bytes += bytes;
             cached += bytes;
         } else {
             drop = true;
@@ -242,6 +244,7 @@ size_t BufferCache::trim(size_t keep) {
                 auto it = std::prev(m->end());  // largest first
                 drop.push_back(it->second);
                 cached -= it->first;
+                if (m == &pending_) pending_bytes -= it->first;
                 freed += it->first;
                 m->erase(it);
             }
@@ -260,7 +263,7 @@ void BufferCache::release() {
         for (auto& kv : *m) (void)hipFree(kv.second);
         m->clear();
     }
-    cached = 0;
+    cached = pending_bytes = 0;
 }
 
 }  // namespace cpvs
@@ -386,8 +389,7 @@ int cpvs_pyramid_build(cpvs_ctx* ctx, const float* depth, int depth_on_device, u
         p->depth = const_cast<float*>(depth);
         p->borrowed = true;
     } else {
-        if (hipMalloc(&p->depth, bytes) != hipSuccess) {
-            (void)hipGetLastError();
+        if (!(p->depth = static_cast<float*>(ctx->buffers.take(bytes)))) {
             delete p;
             set_error("pyramid_build: hipMalloc of %zu bytes failed", bytes);
             return CPVS_ENOMEM;
@@ -395,7 +397,7 @@ int cpvs_pyramid_build(cpvs_ctx* ctx, const float* depth, int depth_on_device, u
         const hipError_t e = hipMemcpyAsync(p->depth, depth, bytes,
                                             depth_on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s);
         if (e != hipSuccess) {
-            hipFree(p->depth);
+            ctx->buffers.give(p->depth);
             delete p;
             return hip_fail(e, "pyramid depth copy", __FILE__, __LINE__);
         }
@@ -407,12 +409,9 @@ int cpvs_pyramid_build(cpvs_ctx* ctx, const float* depth, int depth_on_device, u
     // input is waited for, so the caller may reuse its buffer, and so is a caller's stream, which
     // the caller may destroy.
     p->pending = p->borrowed && s == ctx->stream;
-    if (rc == CPVS_OK && !p->pending) {
-        const hipError_t e = hipStreamSynchronize(s);
-        if (e != hipSuccess) rc = hip_fail(e, "pyramid sync", __FILE__, __LINE__);
-    }
+    if (rc == CPVS_OK && !p->pending) rc = wait_stream(ctx->pinned, s);
     if (rc != CPVS_OK) {
-        if (!p->borrowed && p->depth) hipFree(p->depth);
+        if (!p->borrowed && p->depth) ctx->buffers.give(p->depth);
         if (p->levels && p->levels_owned) ctx->buffers.give(p->levels);
         delete p;
         return rc;
@@ -475,7 +474,7 @@ int cpvs_pyramid_copy_level(const cpvs_pyramid* p, uint32_t level, float* host, 
 int cpvs_pyramid_destroy(cpvs_pyramid* p) {
     if (!p) return CPVS_OK;
     hipSetDevice(p->ctx->device);
-    if (!p->borrowed && p->depth) hipFree(p->depth);
+    if (!p->borrowed && p->depth) p->ctx->buffers.give(p->depth);
     if (p->levels && p->levels_owned) p->ctx->buffers.give(p->levels);
     delete p;
     return CPVS_OK;
@@ -522,8 +521,7 @@ int cpvs_estimate_build(cpvs_ctx* ctx, const cpvs_pyramid* p, uint32_t t, uint32
         for (int L = 0; L < n; ++L) nodes[L] = cnt[L];
     // (with a full-size leaf table, which a build may fall back to)
     if (scratch_bytes)
-        *scratch_bytes = build_scratch_bytes(cnt, R, leafm, ncol, leafm && T > 1, ctx->merge_mode == CPVS_MERGE_TABLE, false,
-                                             true);
+        *scratch_bytes = build_scratch_bytes(cnt, R, leafm, ncol, leafm && T > 1, ctx->merge_mode == CPVS_MERGE_TABLE, false);
     if (max_dag_bytes) *max_dag_bytes = 4 * words;
     return CPVS_OK;
     GUARD_END
@@ -744,6 +742,17 @@ int cpvs_container_top_levels(const cpvs_container* c, int* levels) {
     return CPVS_OK;
 }
 
+// The container's device buffers back to the cache (queued lookups may still read them).
+static void free_on_gpu(cpvs_container* c) {
+    c->ctx->buffers.give(c->d_dag);
+    c->ctx->buffers.give(c->d_grid);
+    c->ctx->buffers.give(c->d_top);
+    c->d_dag = nullptr;
+    c->d_grid = nullptr;
+    c->d_top = nullptr;
+    c->top_levels = 0;
+}
+
 int cpvs_container_copy_to_gpu(cpvs_container* c) {
     CHECK_ARG(c, "container_copy_to_gpu: NULL container");
     if (c->freed_cpu) {
@@ -781,16 +790,13 @@ int cpvs_container_copy_to_gpu(cpvs_container* c) {
     std::lock_guard<std::mutex> lk(ctx->mu);
     CPVS_HIP_CHECK(hipSetDevice(ctx->device));
     hipStream_t s = ctx->stream;
-    if (c->d_dag) hipFree(c->d_dag);
-    if (c->d_grid) hipFree(c->d_grid);
-    if (c->d_top) hipFree(c->d_top);
-    c->d_dag = nullptr;
-    c->d_grid = nullptr;
-    c->d_top = nullptr;
-    c->top_levels = 0;
-    if (hipMalloc(&c->d_dag, sizeof(u32) * (total ? total : 1)) != hipSuccess ||
-        hipMalloc(&c->d_grid, sizeof(u32) * cells) != hipSuccess) {
-        (void)hipGetLastError();
+    free_on_gpu(c);
+    c->on_gpu = false;
+    // From the buffer cache: a program that makes a container for every frame paid six hipMalloc and
+    // hipFree calls, each a wait for the device, for half of a 1024^2 frame's time.
+    c->d_dag = static_cast<u32*>(ctx->buffers.take(sizeof(u32) * (total ? total : 1)));
+    c->d_grid = static_cast<u32*>(ctx->buffers.take(sizeof(u32) * cells));
+    if (!c->d_dag || !c->d_grid) {
         set_error("container_copy_to_gpu: hipMalloc failed");
         return CPVS_ENOMEM;
     }
@@ -813,8 +819,7 @@ int cpvs_container_copy_to_gpu(cpvs_container* c) {
     }
     if (K > 0 && total < 0xFFFFFFFDull) {
         const u64 entries = (u64)cells << (3 * K);
-        if (hipMalloc(&c->d_top, sizeof(u64) * entries) != hipSuccess) {
-            (void)hipGetLastError();
+        if (!(c->d_top = static_cast<u64*>(ctx->buffers.take(sizeof(u64) * entries)))) {
             set_error("container_copy_to_gpu: hipMalloc of the %llu-entry top table failed",
                       (unsigned long long)entries);
             return CPVS_ENOMEM;
@@ -824,7 +829,8 @@ int cpvs_container_copy_to_gpu(cpvs_container* c) {
         if (rc) return rc;
         c->top_levels = (u32)K;
     }
-    CPVS_HIP_CHECK(hipStreamSynchronize(s));
+    const int rc = wait_stream(ctx->pinned, s);
+    if (rc) return rc;
     c->dag_words = total;
     c->dag_levels = dl;
     c->leafmasks = c->dags[0]->leafmasks;
@@ -998,9 +1004,7 @@ int cpvs_container_destroy(cpvs_container* c) {
     if (!c) return CPVS_OK;
     hipSetDevice(c->ctx->device);
     for (auto* d : c->dags) cpvs_dag_destroy(d);
-    if (c->d_dag) hipFree(c->d_dag);
-    if (c->d_grid) hipFree(c->d_grid);
-    if (c->d_top) hipFree(c->d_top);
+    free_on_gpu(c);
     delete c;
     return CPVS_OK;
 }

@@ -99,17 +99,23 @@ namespace cpvs {
 // for the device).
 // A freed buffer may still be read by work queued on any stream, so give() parks it as pending
 // and the free itself waits for nothing.  A pending buffer is handed out again only after a
-// device synchronisation that follows its free: take() performs one when no ready buffer fits and
-// a pending one would, which readies every pending buffer at once.  give_idle() is for buffers
+// device synchronisation that follows its free: take() performs one when no ready buffer fits, a
+// pending one would and kPendingBytes are pending, which readies every pending buffer at once.
+// Below that it allocates: a synchronisation costs about 9 us and the overlap of everything queued, a
+// hipMalloc 0.4 us (1 MB) to 14 us (16 MB), and a program that frees and rebuilds then pays one
+// synchronisation for several builds.  give_idle() is for buffers
 // the caller knows no queued work reads (a server's evicted DAG: no lookup pins it, its build has
 // completed); they are ready at once.
 struct BufferCache {
     static constexpr size_t kMaxBytes = size_t(2) << 30;
+    static constexpr size_t kPendingBytes = size_t(64) << 20;
+    static constexpr size_t kPendingCount = 32;
     std::mutex mu;
     std::multimap<size_t, void*> free_;     // size -> ready buffer
     std::multimap<size_t, void*> pending_;  // size -> freed buffer not yet known idle
     std::unordered_map<void*, size_t> live_;  // handed-out buffer -> its size
     size_t cached = 0;   // bytes in free_ and pending_
+    size_t pending_bytes = 0;
     uint64_t device_syncs = 0, trims = 0;
     int device = 0;
     void* take(size_t bytes);            // nullptr when hipMalloc fails (even after emptying the cache)
@@ -226,6 +232,9 @@ struct CountLayout {
 // (counts from level 1 up, which needs pyramid levels 1 and 2).
 // exact: count only the cells under a partial cell at every level above (slower; needed only
 // for maps with NaN depths, whose plain counts can exceed the octree's nodes).
+// Every word of partials that will be stored, the last one included, reads kUnsetCount until it is
+// (a workgroup counts at most 2^29 cells).
+constexpr u32 kUnsetCount = 0xFFFFFFFFu;
 int pyramid_node_counts(const cpvs_pyramid* p, u32 t, u32 T, bool leaf, u32* partials, uint4* col_info, hipStream_t s,
                         CountLayout* layout = nullptr, bool exact = false);
 void sum_node_counts(const CountLayout& lay, const u32* partials, u64* cnt);
@@ -261,10 +270,12 @@ struct DagOut {
 int build_dag(cpvs_ctx* ctx, Arena& A, u64* pinned, int merge_mode, const cpvs_pyramid* p, u32 t, u32 T, hipStream_t s,
               cpvs_dag** out, const Admit* admit = nullptr, DagOut* into = nullptr);
 
+// Waits for the work queued on s, as a stream synchronisation does but about 6 us sooner: a last kernel
+// stores a flag in pinned (a lane's or the context's, whose lock the caller holds) and the host reads it.
+int wait_stream(u64* pinned, hipStream_t s);
 // The scratch bytes that build_dag needs for a map with cnt[L] nodes at level L (root level R) and
 // ncol leaf columns (see build.hip).
-size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_list, bool use_table, bool small_leaf,
-                           bool staged);
+size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_list, bool use_table, bool small_leaf);
 
 // noalloc.hip: finds this device's fixed scratch (once per device); called by cpvs_ctx_create.
 int noalloc_setup(int device);

@@ -321,6 +321,11 @@ __global__ __launch_bounds__(kTotalsThreads) void k_totals(MArgs a, const u32* _
         __syncthreads();
         for (u32 i = threadIdx.x; i < kMetaWords; i += blockDim.x) host_meta[i] = meta[i];
         __threadfence_system();
+        __syncthreads();
+        if (threadIdx.x == 0) {  // ready: the host polls for it
+            reinterpret_cast<volatile u32*>(host_meta)[kMetaWords] = 1u;
+            __threadfence_system();
+        }
     }
 }
 

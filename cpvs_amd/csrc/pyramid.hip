@@ -9,6 +9,7 @@
 // build reads depth directly and pyramid levels >= 3 (src/CompressedShadow.cpp:104-106,162-166).
 // Every (min, max) is combined as min(min(a,b), min(c,d)) over the 2x2 block [a b; c d]
 // exactly as constructRange/setRow/find do (src/MinMaxHierarchy.cpp:29-49).
+#include <algorithm>
 #include <vector>
 
 #include "internal.hpp"
@@ -381,6 +382,7 @@ __global__ __launch_bounds__(256) void k_node_counts(CountArgs a) {
             }
             a.partials[a.block_start[a.nlev]] = m;
         }
+        __threadfence_system();  // (the host may poll for the words)
     }
 }
 
@@ -432,6 +434,7 @@ int pyramid_node_counts(const cpvs_pyramid* p, u32 t, u32 T, bool leaf, u32* par
         for (int k = 0; k < a.nlev; ++k) layout->level[k] = a.level[k];
         for (int k = 0; k <= a.nlev; ++k) layout->block_start[k] = a.block_start[k];
     }
+    if (partials) std::fill_n(partials, blocks + 1, kUnsetCount);
     if (blocks) CPVS_LAUNCH("node_counts", k_node_counts, dim3(blocks), dim3(256), 0, s, a);
     CPVS_HIP_CHECK(hipGetLastError());
     return CPVS_OK;
