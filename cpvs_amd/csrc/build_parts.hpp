@@ -680,15 +680,14 @@ __device__ inline u32 table_insert_group(u64* tab, u32 S, u64 h, u32 i, bool act
 }
 
 // The leaf level: only a run's first node is inserted (1.3 M of 6.7 M nodes at 8192^2), so each
-// thread takes kLeafPer nodes and a workgroup merges a window of kLeafWindow nodes in LDS.  The
-// window's distinct hashes are listed as they are found, and the list is spread over the threads
-// for the global inserts: a workgroup waits for about one global insert per thread, not per node.
+// thread takes kLeafPer nodes and a workgroup merges a window of kLeafPer * kLeafInsertThreads nodes
+// in LDS.  The window's distinct hashes are listed as they are found, and the list is spread over
+// the threads for the global inserts: a workgroup waits for about one global insert per thread, not
+// per node.  A small level would leave most of the chip idle and wait for four inserts in turn, so
+// up to kLeafOneMax nodes a thread takes one (2215 nodes of a 256^2 map: 17 -> 9 us).
 constexpr u32 kLeafInsertThreads = 256;
 constexpr u32 kLeafPer = 4;
-constexpr u32 kLeafWindow = kLeafInsertThreads * kLeafPer;
-constexpr u32 kLeafSlots = 2 * kLeafWindow;  // LDS table at most half full, so every probe ends
-static_assert(kLeafSlots <= 65536, "LDS slot numbers are listed as 16-bit values");
-
+constexpr u32 kLeafOneMax = 1u << 18;
 
 // Threads per workgroup of the write kernels (at 8192^2, 128 and 256 tie; 512 and 1024 are slower).
 constexpr u32 kNodeThreads = 256;
@@ -741,7 +740,8 @@ enum : int {
     kMetaSortColl = 4 * kMaxLevels + 3,  // 32-bit key collisions resolved by a scan (sort merge)
     kMetaFull = 4 * kMaxLevels + 4,      // table inserts that found no free slot (table merge)
     kMetaSlow = 4 * kMaxLevels + 5,      // leaf columns left to the wave-per-column kernel
-    kMetaWords = 4 * kMaxLevels + 6,
+    kMetaTicket = 4 * kMaxLevels + 6,    // workgroups of k_resolve that are done
+    kMetaWords = 4 * kMaxLevels + 7,
 };
 
 

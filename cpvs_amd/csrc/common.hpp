@@ -109,6 +109,12 @@ __device__ inline u32 reachable_cells(const float2* const* lvl, u32 x, u32 y, in
     return clip_cells(lo, hi, zlo, zhi, first);
 }
 
+// Waits until this wave's stores have been acknowledged.  Enough to order stores that bypass the
+// caches (pinned coherent host memory, agent-scope atomics) before a later flag or ticket; a fence of
+// device or system scope would first write the XCD's dirty L2 lines back (measured: 9 -> 25 us for the
+// node counts with one per workgroup).
+__device__ inline void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // 64-bit mixers for subtree keys (Stafford variant 13 finaliser of splitmix64).
 __host__ __device__ inline u64 mix64(u64 z) {
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;

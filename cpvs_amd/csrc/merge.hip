@@ -32,43 +32,45 @@ __global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 
     if (i < S) tab[i] = kEmptySlot;
 }
 
+template <u32 kPer>
 __global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
                                                                     const u32* __restrict__ runhead,
                                                                     const u64* __restrict__ hash, u32 n,
                                                                     u64* __restrict__ tab, u32 S, u32* __restrict__ tslot,
                                                                     u32* __restrict__ full, u32 hbits) {
-    __shared__ u64 gh[kLeafSlots];
-    __shared__ u32 gi[kLeafSlots];  // smallest node index of the slot's hash, then its global slot
-    __shared__ unsigned short glist[kLeafWindow];  // LDS slots in use
+    constexpr u32 kWindow = kPer * kLeafInsertThreads, kSlots = 2 * kWindow;  // at most half full: every probe ends
+    __shared__ u64 gh[kSlots];
+    __shared__ u32 gi[kSlots];  // smallest node index of the slot's hash, then its global slot
+    __shared__ unsigned short glist[kWindow];  // LDS slots in use
     __shared__ u32 gcount;
-    for (u32 j = threadIdx.x; j < kLeafSlots; j += blockDim.x) {
+    for (u32 j = threadIdx.x; j < kSlots; j += blockDim.x) {
         gh[j] = 0ull;  // 0 marks an empty LDS slot
         gi[j] = kNoRep;
     }
     if (threadIdx.x == 0) gcount = 0;
-    const u32 i0 = blockIdx.x * kLeafWindow + threadIdx.x;
-    u32 rh[kLeafPer];
+    const u32 i0 = blockIdx.x * kWindow + threadIdx.x;
+    u32 rh[kPer];
 #pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
+    for (u32 k = 0; k < kPer; ++k) {
         const u32 i = i0 + k * kLeafInsertThreads;
         rh[k] = (i < n) ? runhead[i] : kNoRep;
     }
     // The key hash of each run's first node (the run's smallest index): from the leaf kernel where
     // a lane walked its column, else from its mask and leafmasks (its row at its own index).
-    u64 h[kLeafPer];
+    u64 h[kPer];
 #pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
+    for (u32 k = 0; k < kPer; ++k) {
         const u32 i = i0 + k * kLeafInsertThreads;
         h[k] = (hash && rh[k] == i) ? hash[i] : 0ull;
     }
-    u32 hm[kLeafPer];
+    u32 hm[kPer];
 #pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
+    for (u32 k = 0; k < kPer; ++k) {
         const u32 i = i0 + k * kLeafInsertThreads;
         hm[k] = (rh[k] == i && h[k] == 0ull) ? mask[i] : 0u;
     }
 #pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
+    for (u32 k = 0; k < kPer; ++k) {
         const u32 i = i0 + k * kLeafInsertThreads;
         if (rh[k] != i) continue;
         if (h[k] == 0ull) h[k] = leaf_key_hash(hm[k], leafm + (size_t)i * 8);
@@ -76,13 +78,13 @@ __global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* _
         if (h[k] == 0ull) h[k] = 1ull;
     }
     __syncthreads();
-    u32 ls[kLeafPer];
+    u32 ls[kPer];
 #pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
+    for (u32 k = 0; k < kPer; ++k) {
         const u32 i = i0 + k * kLeafInsertThreads;
         ls[k] = 0;
         if (rh[k] != i) continue;
-        u32 sl = (u32)(h[k] ^ (h[k] >> 29)) & (kLeafSlots - 1);
+        u32 sl = (u32)(h[k] ^ (h[k] >> 29)) & (kSlots - 1);
         for (;;) {
             const u64 cur = atomicCAS(reinterpret_cast<unsigned long long*>(gh + sl), 0ull, (unsigned long long)h[k]);
             if (cur == 0ull) {
@@ -90,20 +92,20 @@ __global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* _
                 break;
             }
             if (cur == h[k]) break;
-            sl = (sl + 1) & (kLeafSlots - 1);
+            sl = (sl + 1) & (kSlots - 1);
         }
         atomicMin(gi + sl, i);
         ls[k] = sl;
     }
     __syncthreads();
-    const u32 m = gcount;  // at most kLeafWindow
+    const u32 m = gcount;  // at most kWindow
     for (u32 j = threadIdx.x; j < m; j += blockDim.x) {
         const u32 sl = glist[j];
         gi[sl] = table_insert(tab, S, gh[sl], gi[sl], full);
     }
     __syncthreads();
 #pragma unroll
-    for (u32 k = 0; k < kLeafPer; ++k) {
+    for (u32 k = 0; k < kPer; ++k) {
         const u32 i = i0 + k * kLeafInsertThreads;
         if (rh[k] == i) tslot[i] = gi[ls[k]];
     }
@@ -161,102 +163,41 @@ __device__ inline int level_of_tile(const MArgs& a, u32 tile) {
 
 __device__ inline u32 node_words(u32 m, u32 leaf) { return 1u + (num_children(m) << leaf); }
 
-template <bool kSorted>
-__global__ __launch_bounds__(kTileThreads) void k_resolve(MArgs a, u32* __restrict__ tile_sums, u32* __restrict__ collisions) {
-    __shared__ u32 s_wave[kTileThreads / kWave];
-    const int k = level_of_tile(a, blockIdx.x);
-    const MLevel& l = a.lv[k];
-    const u32 n = l.n, base = (blockIdx.x - a.tile0[k]) * kTileNodes + threadIdx.x;
-    // The loads of the tile's rounds are issued together, stage by stage.
-    u32 r[kTileRounds];
-    bool act[kTileRounds];
-#pragma unroll
-    for (int j = 0; j < kTileRounds; ++j) {
-        const u32 i = base + j * kTileThreads;
-        act[j] = i < n;
-        if (l.leaf && act[j]) act[j] = a.heads[i] == i;  // a first occurrence heads its run
-    }
-#pragma unroll
-    for (int j = 0; j < kTileRounds; ++j) r[j] = (act[j] && !l.lone) ? l.id[base + j * kTileThreads] : 0u;
-    if (!kSorted) {
-#pragma unroll
-        for (int j = 0; j < kTileRounds; ++j) r[j] = (act[j] && !l.lone) ? (u32)l.tab[min(r[j], l.slots - 1)] : 0u;
-    }
-    u32 acc = 0;  // first occurrences << 16 | their words (at most 1024 and 17408)
-#pragma unroll
-    for (int j = 0; j < kTileRounds; ++j) {
-        const u32 i = base + j * kTileThreads;
-        bool first = false;
-        if (act[j]) {
-            if (l.lone || r[j] >= n) r[j] = i;
-            first = r[j] == i;
-            const int kc = a.child(k);
-            if (!kSorted && l.lone && kc >= 0 && a.lv[kc].leaf) {
-                // A root over leaves (a 16 x 16 map) had no insert to store its children's identities.
-                u32 unused[8];
-                load_child_ids(ChildIds{a.lv[kc].id, a.heads, a.lv[kc].n}, l.cstart[i], num_children(l.mask[i]), unused);
-            }
-            if (!kSorted && !first) {
-                const bool same = l.leaf ? LeafEq{l.mask, a.leafm, nullptr, n}(i, r[j])
-                                         : InnerEq{l.mask, l.cstart, kc >= 0 ? a.lv[kc].id : nullptr, kc >= 0 ? a.lv[kc].n : 1u}(i, r[j]);
-                if (!same) {
-                    atomicAdd(collisions, 1u);  // two keys share a slot: the build is redone by sorting
-                    first = true;
-                }
-            }
-            if (first) acc += (1u << 16) | node_words(l.mask[i], l.leaf);
-        }
-        const u64 bits = __ballot(first);
-        if ((threadIdx.x & (kWave - 1)) == 0 && i < n) l.first[i / 64] = bits;
-    }
-    acc = block_reduce(acc, s_wave, OpSum{});
-    if (threadIdx.x == 0) tile_sums[blockIdx.x] = acc;
-}
-
-// B[R] = 0, B[L-1] = B[L] + S[L]; total = B[bottom] + S[bottom] (levels absent have S = 0).
-__device__ inline void level_bases(u32* meta, int R) {
-    u32 S[kMaxLevels];
-#pragma unroll
-    for (int L = 0; L < kMaxLevels; ++L) S[L] = meta[kMetaS + L];
-    unsigned long long acc = 0;
-#pragma unroll
-    for (int L = kMaxLevels - 1; L >= 0; --L) {
-        if (L <= R) {
-            meta[kMetaB + L] = (u32)acc;
-            acc += S[L];
-        }
-    }
-    meta[kMetaW] = (acc > 0xFFFFFFFFull) ? 0xFFFFFFFFu : (u32)acc;
-}
-
 __device__ inline u32 saturate32(u64 v) { return v > 0xFFFFFFFFull ? 0xFFFFFFFFu : (u32)v; }
 
 // One workgroup: a scan over all tiles of all levels, four to a thread at a time.  tile_pre gets
 // (first occurrences, words) before each tile, then, after the tiles, before each level and at the
 // end; k_offsets subtracts its level's.  A level's total at or above 2^32 words is stored
-// saturated, so that the host rejects the DAG.  (Levels' starts are kept in LDS: looked up in the
-// kernel's arguments by a varying index they took twice the scan's time.)
+// saturated, so that the host rejects the DAG.  Then the levels' bases (R >= 0): B[R] = 0, B[L-1] =
+// B[L] + S[L], and the readback.  Levels' first tiles and the metadata are kept in LDS: looked up in
+// the kernel's arguments by a varying index, and read back from memory, they took longer than the
+// scan.  tile_sums and meta are read at agent scope: in k_resolve's last workgroup they were stored
+// by other workgroups of the same launch.
 constexpr u32 kTotalsThreads = 1024;
-__global__ __launch_bounds__(kTotalsThreads) void k_totals(MArgs a, const u32* __restrict__ tile_sums,
-                                                           ulonglong2* __restrict__ tile_pre, u32* __restrict__ meta, int R,
-                                                           u32* __restrict__ host_meta) {
-    constexpr u32 kWaves = kTotalsThreads / kWave, kPer = 4;
-    __shared__ u32 s_c[2][kWaves], s_w[2][kWaves], s_tile0[kMaxLevels + 1];
+constexpr u32 kInlineTiles = 256;  // up to this many tiles k_resolve's last workgroup does this
+template <u32 kThreads>
+__device__ inline void merge_totals(const MArgs& a, const u32* tile_sums, ulonglong2* __restrict__ tile_pre,
+                                    u32* __restrict__ meta, int R, u32* __restrict__ host_meta) {
+    constexpr u32 kWaves = kThreads / kWave, kPer = 4;
+    __shared__ u32 s_c[2][kWaves], s_w[2][kWaves], s_tile0[kMaxLevels + 1], s_meta[kMetaWords];
     __shared__ u32 lev_c[kMaxLevels + 1];
     __shared__ u64 lev_w[kMaxLevels + 1];
     const u32 nt = a.tile0[a.nlev], nlev = (u32)a.nlev;
     const u32 lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     if (threadIdx.x <= nlev) s_tile0[threadIdx.x] = a.tile0[threadIdx.x];
+    for (u32 i = threadIdx.x; i < kMetaWords; i += kThreads)
+        s_meta[i] = __hip_atomic_load(meta + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     u32 run_c = 0;  // of the chunks before
     u64 run_w = 0;
     u32 v[kPer];
     auto load = [&](u32 t0) {
 #pragma unroll
-        for (u32 j = 0; j < kPer; ++j) v[j] = (t0 + j < nt) ? tile_sums[t0 + j] : 0u;
+        for (u32 j = 0; j < kPer; ++j)
+            v[j] = (t0 + j < nt) ? __hip_atomic_load(tile_sums + t0 + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
     };
     load(threadIdx.x * kPer);
     u32 buf = 0;
-    for (u32 base = 0; base < nt; base += kTotalsThreads * kPer, buf ^= 1u) {
+    for (u32 base = 0; base < nt; base += kThreads * kPer, buf ^= 1u) {
         const u32 t0 = base + threadIdx.x * kPer;
         u32 x[kPer], c = 0, w = 0;  // (a chunk of 4096 tiles of at most 17408 words fits 32 bits)
 #pragma unroll
@@ -265,7 +206,7 @@ __global__ __launch_bounds__(kTotalsThreads) void k_totals(MArgs a, const u32* _
             c += v[j] >> 16;
             w += v[j] & 0xFFFFu;
         }
-        load(t0 + kTotalsThreads * kPer);  // the next chunk's, while this one is scanned
+        load(t0 + kThreads * kPer);  // the next chunk's, while this one is scanned
         const u32 ci = wave_inclusive_scan(c, OpSum{}), wi = wave_inclusive_scan(w, OpSum{});
         if (lane == kWave - 1) {
             s_c[buf][wid] = ci;
@@ -309,24 +250,103 @@ __global__ __launch_bounds__(kTotalsThreads) void k_totals(MArgs a, const u32* _
     if (threadIdx.x <= nlev) tile_pre[nt + threadIdx.x] = make_ulonglong2(lev_c[threadIdx.x], lev_w[threadIdx.x]);
     if (threadIdx.x < nlev) {
         const u32 k = threadIdx.x;
-        meta[kMetaU + a.lv[k].L] = lev_c[k + 1] - lev_c[k];
-        meta[kMetaS + a.lv[k].L] = saturate32(lev_w[k + 1] - lev_w[k]);
+        s_meta[kMetaU + a.lv[k].L] = lev_c[k + 1] - lev_c[k];
+        s_meta[kMetaS + a.lv[k].L] = saturate32(lev_w[k + 1] - lev_w[k]);
     }
     __syncthreads();
     if (threadIdx.x == 0 && R >= 0) {
-        meta[kMetaRoot] = a.lv[a.nlev - 1].mask[0];
-        level_bases(meta, R);
-    }
-    if (host_meta) {  // the build's readback: one word per thread
-        __syncthreads();
-        for (u32 i = threadIdx.x; i < kMetaWords; i += blockDim.x) host_meta[i] = meta[i];
-        __threadfence_system();
-        __syncthreads();
-        if (threadIdx.x == 0) {  // ready: the host polls for it
-            reinterpret_cast<volatile u32*>(host_meta)[kMetaWords] = 1u;
-            __threadfence_system();
+        s_meta[kMetaRoot] = a.lv[a.nlev - 1].mask[0];
+        u64 acc = 0;
+        for (int L = R; L >= 0; --L) {  // (levels absent have no words)
+            s_meta[kMetaB + L] = saturate32(acc);
+            acc += s_meta[kMetaS + L];
         }
+        s_meta[kMetaW] = saturate32(acc);
     }
+    __syncthreads();
+    for (u32 i = threadIdx.x; i < kMetaWords; i += kThreads) {
+        if (host_meta) reinterpret_cast<volatile u32*>(host_meta)[i] = s_meta[i];
+        meta[i] = s_meta[i];
+    }
+    if (host_meta) {
+        wait_stores();
+        __syncthreads();
+        if (threadIdx.x == 0) reinterpret_cast<volatile u32*>(host_meta)[kMetaWords] = 1u;  // ready: the host polls for it
+    }
+}
+
+__global__ __launch_bounds__(kTotalsThreads) void k_totals(MArgs a, const u32* __restrict__ tile_sums,
+                                                           ulonglong2* __restrict__ tile_pre, u32* __restrict__ meta, int R,
+                                                           u32* __restrict__ host_meta) {
+    merge_totals<kTotalsThreads>(a, tile_sums, tile_pre, meta, R, host_meta);
+}
+
+template <bool kSorted>
+__global__ __launch_bounds__(kTileThreads) void k_resolve(MArgs a, u32* tile_sums, ulonglong2* __restrict__ tile_pre,
+                                                          u32* meta, int R, u32* __restrict__ host_meta) {
+    u32* collisions = meta + kMetaColl;
+    __shared__ u32 s_wave[kTileThreads / kWave];
+    const int k = level_of_tile(a, blockIdx.x);
+    const MLevel& l = a.lv[k];
+    const u32 n = l.n, base = (blockIdx.x - a.tile0[k]) * kTileNodes + threadIdx.x;
+    // The loads of the tile's rounds are issued together, stage by stage.
+    u32 r[kTileRounds];
+    bool act[kTileRounds];
+#pragma unroll
+    for (int j = 0; j < kTileRounds; ++j) {
+        const u32 i = base + j * kTileThreads;
+        act[j] = i < n;
+        if (l.leaf && act[j]) act[j] = a.heads[i] == i;  // a first occurrence heads its run
+    }
+#pragma unroll
+    for (int j = 0; j < kTileRounds; ++j) r[j] = (act[j] && !l.lone) ? l.id[base + j * kTileThreads] : 0u;
+    if (!kSorted) {
+#pragma unroll
+        for (int j = 0; j < kTileRounds; ++j) r[j] = (act[j] && !l.lone) ? (u32)l.tab[min(r[j], l.slots - 1)] : 0u;
+    }
+    u32 acc = 0;  // first occurrences << 16 | their words (at most 1024 and 17408)
+#pragma unroll
+    for (int j = 0; j < kTileRounds; ++j) {
+        const u32 i = base + j * kTileThreads;
+        bool first = false;
+        if (act[j]) {
+            if (l.lone || r[j] >= n) r[j] = i;
+            first = r[j] == i;
+            const int kc = a.child(k);
+            if (!kSorted && l.lone && kc >= 0 && a.lv[kc].leaf) {
+                // A root over leaves (a 16 x 16 map) had no insert to store its children's identities.
+                u32 unused[8];
+                load_child_ids(ChildIds{a.lv[kc].id, a.heads, a.lv[kc].n}, l.cstart[i], num_children(l.mask[i]), unused);
+            }
+            if (!kSorted && !first) {
+                const bool same = l.leaf ? LeafEq{l.mask, a.leafm, nullptr, n}(i, r[j])
+                                         : InnerEq{l.mask, l.cstart, kc >= 0 ? a.lv[kc].id : nullptr, kc >= 0 ? a.lv[kc].n : 1u}(i, r[j]);
+                if (!same) {
+                    atomicAdd(collisions, 1u);  // two keys share a slot: the build is redone by sorting
+                    __threadfence();  // counted before the workgroup's ticket
+                    first = true;
+                }
+            }
+            if (first) acc += (1u << 16) | node_words(l.mask[i], l.leaf);
+        }
+        const u64 bits = __ballot(first);
+        if ((threadIdx.x & (kWave - 1)) == 0 && i < n) l.first[i / 64] = bits;
+    }
+    acc = block_reduce(acc, s_wave, OpSum{});
+    if (gridDim.x > kInlineTiles) {  // k_totals follows
+        if (threadIdx.x == 0) tile_sums[blockIdx.x] = acc;
+        return;
+    }
+    // The last workgroup to finish does the totals: one launch less for small builds.
+    __shared__ u32 s_last;
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(tile_sums + blockIdx.x, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        wait_stores();
+        s_last = atomicAdd(meta + kMetaTicket, 1u) == gridDim.x - 1 ? 1u : 0u;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    merge_totals<kTileThreads>(a, tile_sums, tile_pre, meta, R, host_meta);
 }
 
 __global__ __launch_bounds__(kTileThreads) void k_offsets(MArgs a, const ulonglong2* __restrict__ tile_pre) {
@@ -440,9 +460,13 @@ static ChildIds children_of(const MArgs& a, int k, bool sorted) {
 
 void merge_insert(const MArgs& a, int k, const u64* hash, u32* meta, u32 hbits, hipStream_t s) {
     const MLevel& l = a.lv[k];
-    if (l.leaf)
-        CPVS_LAUNCH("insert_leaf", k_insert_leaf, grid_of(l.n, kLeafWindow), dim3(kLeafInsertThreads), 0, s, l.mask, a.leafm,
-                    a.heads, hash, l.n, l.tab, l.slots, l.id, meta + kMetaFull, hbits);
+    if (l.leaf && l.n <= kLeafOneMax)
+        CPVS_LAUNCH("insert_leaf", k_insert_leaf<1>, grid_of(l.n, kLeafInsertThreads), dim3(kLeafInsertThreads), 0, s, l.mask,
+                    a.leafm, a.heads, hash, l.n, l.tab, l.slots, l.id, meta + kMetaFull, hbits);
+    else if (l.leaf)
+        CPVS_LAUNCH("insert_leaf", k_insert_leaf<kLeafPer>, grid_of(l.n, kLeafPer * kLeafInsertThreads),
+                    dim3(kLeafInsertThreads), 0, s, l.mask, a.leafm, a.heads, hash, l.n, l.tab, l.slots, l.id,
+                    meta + kMetaFull, hbits);
     else
         CPVS_LAUNCH("insert_inner", k_insert_inner, grid_of(l.n, kInsertBlock), dim3(kInsertBlock), 0, s, l.mask, l.cstart,
                     children_of(a, k, false), l.n, l.tab, l.slots, l.id, meta + kMetaFull, hbits);
@@ -471,10 +495,13 @@ void merge_finish(const MArgs& a, bool sorted, u32* tile_sums, ulonglong2* tile_
                   hipStream_t s) {
     const u32 nt = a.tile0[a.nlev];
     if (sorted)
-        CPVS_LAUNCH("resolve", k_resolve<true>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums, meta + kMetaColl);
+        CPVS_LAUNCH("resolve", k_resolve<true>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums, tile_pre, meta, R,
+                    host_meta);
     else
-        CPVS_LAUNCH("resolve", k_resolve<false>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums, meta + kMetaColl);
-    CPVS_LAUNCH("totals", k_totals, dim3(1), dim3(kTotalsThreads), 0, s, a, tile_sums, tile_pre, meta, R, host_meta);
+        CPVS_LAUNCH("resolve", k_resolve<false>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums, tile_pre, meta, R,
+                    host_meta);
+    if (nt > kInlineTiles)
+        CPVS_LAUNCH("totals", k_totals, dim3(1), dim3(kTotalsThreads), 0, s, a, tile_sums, tile_pre, meta, R, host_meta);
     CPVS_LAUNCH("offsets", k_offsets, dim3(nt), dim3(kTileThreads), 0, s, a, tile_pre);
 }
 

@@ -382,7 +382,6 @@ __global__ __launch_bounds__(256) void k_node_counts(CountArgs a) {
             }
             a.partials[a.block_start[a.nlev]] = m;
         }
-        __threadfence_system();  // (the host may poll for the words)
     }
 }
 
