@@ -344,11 +344,11 @@ int deepest_level(const u64* cnt, int bottom, int R) {
 }
 // Slots of level L's table (0: the root and absent levels have none).  With the sort merge one entry
 // per node.
-u32 level_slots(const u64* cnt, int L, int R, int Ls, bool use_table, bool leaf, bool small_leaf) {
+u32 level_slots(const u64* cnt, int L, int R, int Ls, bool use_table, bool leaf, bool small_tables) {
     if (L >= R || !cnt[L]) return 0;
     if (!use_table) return (u32)cnt[L];
     if (L >= Ls) return small_slots((u32)cnt[L]);
-    return (leaf && L == 2) ? leaf_table_slots((u32)cnt[L], small_leaf) : table_slots((u32)cnt[L]);
+    return (leaf && L == 2) ? leaf_table_slots((u32)cnt[L], small_tables) : inner_table_slots((u32)cnt[L], small_tables);
 }
 u64 bound_words_of(const u64* cnt, int bottom, int R, bool leaf) {
     u64 w = 0;
@@ -361,11 +361,6 @@ constexpr int kRetryFullTable = -1001;
 constexpr int kRetryExactCounts = -1002;  // the counts exceed the emitted nodes (a map with NaN depths)
 
 
-// small_leaf: a leaf level of at least kSmallLeafTableMin nodes gets a merge table sized for a
-// quarter of them (only a run's first node is inserted: a fifth of them at 8192^2, with 4% of the
-// nodes distinct), which keeps the table's clear and its random accesses small; a table found too
-// small (maps of mostly distinct leaves, such as white noise) is reported as kRetryFullTable and
-// the build runs again.
 __global__ void k_store_word(u32* dst, u32 v) { *dst = v; }
 
 constexpr u32 kHostReady = kMetaWords, kHostDone = kMetaWords + 1;  // flags behind the meta readback
@@ -417,7 +412,7 @@ int store_and_wait(u32* dst, u32 v, u64* pinned, hipStream_t s) {
 }
 
 int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 t, u32 T, hipStream_t s, int merge_mode,
-               cpvs_dag** out, const Admit* admit, bool small_leaf, bool exact, DagOut* into) {
+               cpvs_dag** out, const Admit* admit, bool small_tables, bool exact, DagOut* into) {
     const int n = p->n;
     const int R = n - 2;
     const bool leaf = n >= 5 && ctx->leafmasks != 0;  // useLeafmasks (src/CompressedShadow.cpp:20-27)
@@ -499,7 +494,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     const bool col_list = leaf && T > 1;  // compact the z-tile's columns with leaf nodes
     const int deepest = deepest_level(cnt, bottom, R);
     const int Ls = small_levels(cnt, deepest, R, use_table, leaf);
-    const size_t need = build_scratch_bytes(cnt, R, leaf, ncol, col_list, use_table, small_leaf);
+    const size_t need = build_scratch_bytes(cnt, R, leaf, ncol, col_list, use_table, small_tables);
     if (admit) {
         rc = admit->fn(admit->user, A, need, 4 * bound_words_of(cnt, bottom, R, leaf));
         if (rc) return rc;
@@ -529,7 +524,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         lv[L].uniq = A.take<u32>(c);
         lv[L].off = A.take<u32>(c);
         lv[L].first = A.take<u64>(first_words((u32)c));
-        lv[L].slots = level_slots(cnt, L, R, Ls, use_table, leaf, small_leaf);
+        lv[L].slots = level_slots(cnt, L, R, Ls, use_table, leaf, small_tables);
         tab_slots += lv[L].slots;
         if (L < Ls) clear_slots += lv[L].slots;
         ntiles += ceil_div<u32>((u32)cnt[L], kTileNodes);
@@ -700,7 +695,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
             return CPVS_EINTERNAL;
         }
     }
-    if (use_table && hm[kMetaFull] != 0) return small_leaf ? kRetryFullTable : kRetryWithSort;
+    if (use_table && hm[kMetaFull] != 0) return small_tables ? kRetryFullTable : kRetryWithSort;
     if (use_table && hm[kMetaColl] != 0) return kRetryWithSort;
     if (deepest > bottom && hm[kMetaC + deepest] != 0) {
         set_error("build: level %d emitted children below the deepest level", deepest);
@@ -758,7 +753,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
 }  // namespace
 
 // What build_once lays out: cnt the nodes per level (bottom .. R), ncol the leaf columns.
-size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_list, bool use_table, bool small_leaf) {
+size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_list, bool use_table, bool small_tables) {
     const int bottom = leaf ? 2 : 0;
     const int Ls = small_levels(cnt, deepest_level(cnt, bottom, R), R, use_table, leaf);
     size_t need = arena_bytes(kMetaWords, sizeof(u32)) + (leaf ? arena_bytes(ncol, sizeof(uint4)) : 0);
@@ -770,7 +765,7 @@ size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_
         const bool is_leaf = leaf && L == 2;
         need += (is_leaf ? 0 : arena_bytes(c, 8) + arena_bytes(c, 4)) + 4 * arena_bytes(c, 4) +
                 arena_bytes(first_words((u32)c), 8);
-        slots += level_slots(cnt, L, R, Ls, use_table, leaf, small_leaf);
+        slots += level_slots(cnt, L, R, Ls, use_table, leaf, small_tables);
         ntiles += ceil_div<u32>((u32)cnt[L], kTileNodes);
     }
     need += arena_bytes(slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(tile_pre_count(ntiles), 16);
@@ -787,12 +782,12 @@ size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_
 // exact counts; each switch is made at most once.
 int build_dag(cpvs_ctx* ctx, Arena& A, u64* pinned, int merge_mode, const cpvs_pyramid* p, u32 t, u32 T, hipStream_t s,
               cpvs_dag** out, const Admit* admit, DagOut* into) {
-    bool small_leaf = true, exact = false;
+    bool small_tables = true, exact = false;
     int rc = CPVS_OK;
     for (int attempt = 0; attempt < 4; ++attempt) {
-        rc = build_once(ctx, A, pinned, p, t, T, s, merge_mode, out, admit, small_leaf, exact, into);
-        if (rc == kRetryFullTable && small_leaf) small_leaf = false;
-        else if (rc == kRetryWithSort && merge_mode != CPVS_MERGE_SORT) merge_mode = CPVS_MERGE_SORT, small_leaf = false;
+        rc = build_once(ctx, A, pinned, p, t, T, s, merge_mode, out, admit, small_tables, exact, into);
+        if (rc == kRetryFullTable && small_tables) small_tables = false;
+        else if (rc == kRetryWithSort && merge_mode != CPVS_MERGE_SORT) merge_mode = CPVS_MERGE_SORT, small_tables = false;
         else if (rc == kRetryExactCounts && !exact) exact = true;
         else break;
     }

@@ -624,7 +624,7 @@ constexpr u32 kMaxProbes = 256;
 __device__ inline u32 table_insert(u64* tab, u32 S, u64 h, u32 i, u32* full) {
     const u32 tag = (u32)(h >> 32);
     const u64 mine = ((u64)tag << 32) | i;
-    u32 slot = (u32)(h ^ (h >> 31)) & (S - 1);
+    u32 slot = __umulhi((u32)(h ^ (h >> 31)) * 0x9E3779B1u, S);
     for (u32 probe = 0; probe < kMaxProbes; ++probe) {
         u64 cur = __hip_atomic_load(tab + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (cur == kEmptySlot) {
@@ -636,7 +636,7 @@ __device__ inline u32 table_insert(u64* tab, u32 S, u64 h, u32 i, u32* full) {
             if ((u32)cur > i) atomicMin(reinterpret_cast<unsigned long long*>(tab + slot), (unsigned long long)mine);
             return slot;
         }
-        slot = (slot + 1) & (S - 1);
+        if (++slot == S) slot = 0;
     }
     atomicAdd(full, 1u);
     return slot;
@@ -749,14 +749,18 @@ enum : int {
 constexpr u64 kLaneLeafMin = 1u << 15;
 constexpr u32 kSlowWaves = 8192;  // waves that stride over a list of columns: the chip's 32 per CU
 
+// Slots for n keys, at most two thirds full.
 inline u32 table_slots(u32 n) {
-    u32 S = 1024;
-    while (S < n + n / 2 + 1) S <<= 1;
-    return S;
+    const u64 S = (u64)n + n / 2 + 1;
+    return S < 1024 ? 1024u : (u32)(S < 0xFFFFFFFFull ? S : 0xFFFFFFFFull);
 }
-// Below 2^20 leaf nodes the table is small anyway, and small maps have more distinct leaves per
-// node (measured: 256^2 and 512^2 maps fill 85-96% of a quarter-size table, 1024^2 40%, 8192^2 4%).
-constexpr u32 kSmallLeafTableMin = 1u << 20;
-inline u32 leaf_table_slots(u32 c, bool small) { return table_slots((small && c >= kSmallLeafTableMin) ? c / 4 : c); }
+// Large levels repeat their nodes (8192^2: 5% of the leaves and 15% of the nodes above them are
+// distinct, 1024^2 25-40%), and a table that is not needed costs its clear and, spread wide, a cache
+// miss for every probe and look-up: from 2^20 nodes on a leaf level gets slots for a quarter of its
+// nodes and an inner level for half.  A table found too small (maps of mostly distinct leaves, such
+// as white noise) is reported, and the build runs again with small = false.
+constexpr u32 kSmallTableMin = 1u << 20;
+inline u32 leaf_table_slots(u32 c, bool small) { return table_slots((small && c >= kSmallTableMin) ? c / 4 : c); }
+inline u32 inner_table_slots(u32 c, bool small) { return table_slots((small && c >= kSmallTableMin) ? c / 2 : c); }
 
 }  // namespace cpvs

@@ -399,7 +399,7 @@ T* carve(char*& p, size_t n) {
     return r;
 }
 
-int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const ForestOpts& o, int merge_mode, bool small_leaf,
+int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const ForestOpts& o, int merge_mode, bool small_tables,
                 bool exact, cpvs_dag** out) {
     const hipStream_t s = w.stream;
     const bool use_table = merge_mode == CPVS_MERGE_TABLE;
@@ -549,7 +549,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         const u32 c = (u32)C[L];
         cmax = std::max<u32>(cmax, c);
         if (!c) continue;
-        slots[L] = !use_table ? c : (L == 2) ? leaf_table_slots(c, small_leaf) : table_slots(c);
+        slots[L] = !use_table ? c : (L == 2) ? leaf_table_slots(c, small_tables) : inner_table_slots(c, small_tables);
         tab_slots += slots[L];
         ntiles += ceil_div<u32>(c, kTileNodes);
     }
@@ -728,7 +728,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
             return CPVS_EINTERNAL;
         }
     }
-    if (use_table && hm[kMetaFull] != 0) return small_leaf ? kRetryFull : kRetrySort;
+    if (use_table && hm[kMetaFull] != 0) return small_tables ? kRetryFull : kRetrySort;
     if (use_table && hm[kMetaColl] != 0) return kRetrySort;
     const u32* totals = st.back + kMetaWords;
     const u32* roots = totals + M;
@@ -825,11 +825,11 @@ int build_forest(cpvs_ctx* ctx, Worker& w, const ForestIn* items, u32 M, const F
     // As build_dag: a full table, a key collision and counts above the emitted nodes each switch to
     // their fallback once.
     int mode = o.merge_mode, rc = CPVS_OK;
-    bool small_leaf = true, exact = false;
+    bool small_tables = true, exact = false;
     for (int attempt = 0; attempt < 4; ++attempt) {
-        rc = forest_once(ctx, w, items, M, o, mode, small_leaf, exact, out);
-        if (rc == kRetryFull && small_leaf) small_leaf = false;
-        else if (rc == kRetrySort && mode != CPVS_MERGE_SORT) mode = CPVS_MERGE_SORT, small_leaf = false;
+        rc = forest_once(ctx, w, items, M, o, mode, small_tables, exact, out);
+        if (rc == kRetryFull && small_tables) small_tables = false;
+        else if (rc == kRetrySort && mode != CPVS_MERGE_SORT) mode = CPVS_MERGE_SORT, small_tables = false;
         else if (rc == kRetryExact && !exact) exact = true;
         else break;
     }

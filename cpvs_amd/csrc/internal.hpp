@@ -275,7 +275,7 @@ int build_dag(cpvs_ctx* ctx, Arena& A, u64* pinned, int merge_mode, const cpvs_p
 int wait_stream(u64* pinned, hipStream_t s);
 // The scratch bytes that build_dag needs for a map with cnt[L] nodes at level L (root level R) and
 // ncol leaf columns (see build.hip).
-size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_list, bool use_table, bool small_leaf);
+size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_list, bool use_table, bool small_tables);
 
 // noalloc.hip: finds this device's fixed scratch (once per device); called by cpvs_ctx_create.
 int noalloc_setup(int device);
