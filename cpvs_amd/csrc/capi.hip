@@ -641,7 +641,7 @@ int cpvs_dag_set_top_levels(cpvs_dag* d, int levels) {
     GUARD_BEGIN
     std::lock_guard<std::mutex> lk(ctx->mu);
     CPVS_HIP_CHECK(hipSetDevice(ctx->device));
-    u64* nt = nullptr;
+    u64 *nt = nullptr, *nl = nullptr;
     if (K > 0) {
         nt = static_cast<u64*>(ctx->buffers.take(sizeof(u64) << (3 * K)));
         if (!nt) {
@@ -650,15 +650,21 @@ int cpvs_dag_set_top_levels(cpvs_dag* d, int levels) {
         }
         ProfInstall prof(ctx->prof_on ? &ctx->prof : nullptr);
         int rc = launch_build_top(d->d_words, (u32)d->words, nullptr, 1u, d->n, (u32)K, nt, ctx->stream);
+        // (without memory for the links the lookups walk the words)
+        if (rc == CPVS_OK && !d->d_links && (nl = static_cast<u64*>(ctx->buffers.take(sizeof(u64) * d->words))))
+            rc = launch_links(nullptr, 1, LinkSeg{d->d_words, 0u, (u32)d->words, 0u, 0u}, link_blocks(d->words),
+                              (u32)d->words - 1, nullptr, nl, nullptr, ctx->stream);
         if (rc == CPVS_OK && hipStreamSynchronize(ctx->stream) != hipSuccess) rc = CPVS_EHIP;
         if (rc) {
             ctx->buffers.give(nt);
+            ctx->buffers.give(nl);
             if (rc == CPVS_EHIP) set_error("dag_set_top_levels: building the table failed");
             return rc;
         }
     }
     if (d->d_top) d->retired_tops.push_back(d->d_top);
     d->d_top = nt;
+    if (nl) d->d_links = nl;
     d->top_levels = (u32)K;
     return CPVS_OK;
     GUARD_END
@@ -675,6 +681,7 @@ int cpvs_dag_destroy(cpvs_dag* d) {
     hipSetDevice(d->ctx->device);
     if (d->d_words) d->ctx->buffers.give(d->d_words);
     if (d->d_top) d->ctx->buffers.give(d->d_top);
+    if (d->d_links) d->ctx->buffers.give(d->d_links);
     for (u64* t : d->retired_tops) d->ctx->buffers.give(t);
     delete d;
     return CPVS_OK;
@@ -747,6 +754,8 @@ static void free_on_gpu(cpvs_container* c) {
     c->ctx->buffers.give(c->d_dag);
     c->ctx->buffers.give(c->d_grid);
     c->ctx->buffers.give(c->d_top);
+    c->ctx->buffers.give(c->d_links);
+    c->d_links = nullptr;
     c->d_dag = nullptr;
     c->d_grid = nullptr;
     c->d_top = nullptr;
@@ -800,14 +809,36 @@ int cpvs_container_copy_to_gpu(cpvs_container* c) {
         set_error("container_copy_to_gpu: hipMalloc failed");
         return CPVS_ENOMEM;
     }
-    // combineDAGs (src/CompressedShadowContainer.cpp:52-69): concatenation in slot order.
+    // Without memory for the links the lookups walk the words.
+    c->d_links = static_cast<u64*>(ctx->buffers.take(sizeof(u64) * (total ? total : 1)));
+    // combineDAGs (src/CompressedShadowContainer.cpp:52-69): concatenation in slot order, in one launch
+    // with the links and the grid.
+    std::vector<LinkSeg> segs(cells);
     u64 off = 0;
+    u32 blocks = 0;
     for (size_t i = 0; i < cells; ++i) {
         const cpvs_dag* d = c->dags[i];
-        CPVS_HIP_CHECK(hipMemcpyAsync(c->d_dag + off, d->d_words, sizeof(u32) * d->words, hipMemcpyDeviceToDevice, s));
+        segs[i] = LinkSeg{d->d_words, (u32)off, (u32)d->words, grid[i], blocks};
         off += d->words;
+        blocks += link_blocks(d->words);
     }
-    CPVS_HIP_CHECK(hipMemcpyAsync(c->d_grid, grid.data(), sizeof(u32) * cells, hipMemcpyHostToDevice, s));
+    LinkSeg* d_segs = nullptr;
+    if (cells > 1) {
+        if (!(d_segs = static_cast<LinkSeg*>(ctx->buffers.take(sizeof(LinkSeg) * cells)))) {
+            set_error("container_copy_to_gpu: hipMalloc failed");
+            return CPVS_ENOMEM;
+        }
+        const hipError_t e = hipMemcpyAsync(d_segs, segs.data(), sizeof(LinkSeg) * cells, hipMemcpyHostToDevice, s);
+        if (e != hipSuccess) {
+            ctx->buffers.give(d_segs);
+            return hip_fail(e, "container table copy", __FILE__, __LINE__);
+        }
+    }
+    ProfInstall prof(ctx->prof_on ? &ctx->prof : nullptr);
+    const int lrc = launch_links(d_segs, (u32)cells, segs[0], blocks, total ? (u32)total - 1 : 0u, c->d_dag, c->d_links,
+                                 c->d_grid, s);
+    ctx->buffers.give(d_segs);  // (queued work may still read a given buffer)
+    if (lrc) return lrc;
     // The lookups' top table (launch_build_top): K levels below the grid cell, no more than the
     // DAGs' inner levels above the last (level 3 with leafmasks, 1 without) nor kMaxTopLevels, and
     // within kTopTableBytes; skipped below 3 levels, where it saves little.
@@ -824,7 +855,6 @@ int cpvs_container_copy_to_gpu(cpvs_container* c) {
                       (unsigned long long)entries);
             return CPVS_ENOMEM;
         }
-        ProfInstall prof(ctx->prof_on ? &ctx->prof : nullptr);
         int rc = launch_build_top(c->d_dag, (u32)total, c->d_grid, (u32)cells, dl, (u32)K, c->d_top, s);
         if (rc) return rc;
         c->top_levels = (u32)K;
@@ -901,7 +931,7 @@ int cpvs_container_evaluate(cpvs_container* c, const float* pos, uint32_t stride
     }
     CPVS_HIP_CHECK(hipSetDevice(c->ctx->device));
     ProfInstall prof(c->ctx->prof_on ? &c->ctx->prof : nullptr);
-    return launch_evaluate(c->d_dag, (u32)c->dag_words, c->d_grid, c->dag_levels, c->grid_levels, c->leafmasks, c->d_top,
+    return launch_evaluate(c->d_dag, c->d_links, (u32)c->dag_words, c->d_grid, c->dag_levels, c->grid_levels, c->leafmasks, c->d_top,
                            c->top_levels, pos, stride, count,
                            to_mat(m), vis, pick_stream(c->ctx, stream));
 }
@@ -918,7 +948,7 @@ int cpvs_container_evaluate_pcf(cpvs_container* c, const float* pos, uint32_t st
     }
     CPVS_HIP_CHECK(hipSetDevice(c->ctx->device));
     ProfInstall prof(c->ctx->prof_on ? &c->ctx->prof : nullptr);
-    return launch_evaluate_pcf(c->d_dag, (u32)c->dag_words, c->d_grid, c->dag_levels, c->grid_levels, c->leafmasks, c->d_top,
+    return launch_evaluate_pcf(c->d_dag, c->d_links, (u32)c->dag_words, c->d_grid, c->dag_levels, c->grid_levels, c->leafmasks, c->d_top,
                                c->top_levels, pos, stride, count,
                                to_mat(m), c->filter_size, vis, pick_stream(c->ctx, stream));
 }
@@ -932,7 +962,7 @@ int cpvs_container_evaluate_image(cpvs_container* c, const float* pos, uint32_t 
     }
     CPVS_HIP_CHECK(hipSetDevice(c->ctx->device));
     ProfInstall prof(c->ctx->prof_on ? &c->ctx->prof : nullptr);
-    return launch_evaluate_image(c->d_dag, (u32)c->dag_words, c->d_grid, c->dag_levels, c->grid_levels, c->leafmasks,
+    return launch_evaluate_image(c->d_dag, c->d_links, (u32)c->dag_words, c->d_grid, c->dag_levels, c->grid_levels, c->leafmasks,
                                  c->d_top, c->top_levels, pos, width, height,
                                  to_mat(m), vis, pick_stream(c->ctx, stream));
 }

@@ -182,6 +182,7 @@ struct cpvs_dag {
     bool leafmasks = false;                   // level 2 holds leafmask nodes (lookups stop there)
     uint64_t* d_top = nullptr;                // lookup top table (cpvs_dag_set_top_levels), or null
     uint32_t top_levels = 0;
+    uint64_t* d_links = nullptr;              // links (launch_links), made with the first table and kept, or null
     std::vector<uint64_t*> retired_tops;      // replaced tables, which DAG sets made earlier still name
 };
 
@@ -191,6 +192,7 @@ struct cpvs_container {
     std::vector<cpvs_dag*> dags;  // length^3 slots, index z*L^2 + y*L + x
     uint32_t filter_size = 1;
     uint32_t* d_dag = nullptr;   // combined words
+    uint64_t* d_links = nullptr;  // links over them (launch_links), or null
     uint64_t dag_words = 0;
     uint32_t* d_grid = nullptr;  // length^3 entries
     int dag_levels = 0, grid_levels = 0;
@@ -285,16 +287,27 @@ struct Mat4 {
     float m[16];
 };
 // leaf: the DAGs end in leafmask nodes at level 2; 0: they go down to level 0.  top (may be null):
-// the container's top table of topk levels (launch_build_top).
-int launch_evaluate(const u32* dag, u32 words, const u32* grid, int dl, int gl, int leaf, const u64* top, u32 topk,
+// the container's top table of topk levels (launch_build_top).  links (may be null): launch_links' array.
+int launch_evaluate(const u32* dag, const u64* links, u32 words, const u32* grid, int dl, int gl, int leaf, const u64* top, u32 topk,
                     const float* pos, u32 stride, u64 count, const Mat4& m, uint8_t* vis, hipStream_t s);
-int launch_evaluate_pcf(const u32* dag, u32 words, const u32* grid, int dl, int gl, int leaf, const u64* top, u32 topk,
+int launch_evaluate_pcf(const u32* dag, const u64* links, u32 words, const u32* grid, int dl, int gl, int leaf, const u64* top, u32 topk,
                         const float* pos, u32 stride, u64 count, const Mat4& m, u32 f, float* vis, hipStream_t s);
-int launch_evaluate_image(const u32* dag, u32 words, const u32* grid, int dl, int gl, int leaf, const u64* top, u32 topk,
+int launch_evaluate_image(const u32* dag, const u64* links, u32 words, const u32* grid, int dl, int gl, int leaf, const u64* top, u32 topk,
                           const float* pos, u32 width, u32 height, const Mat4& m, uint8_t* vis, hipStream_t s);
 // The top table of a container: cells x 8^K entries (the walk's state after K levels per cell);
 // grid null: one DAG of its own (cells 1, base 0).
 int launch_build_top(const u32* dag, u32 words, const u32* grid, u32 cells, int dl, u32 K, u64* top, hipStream_t s);
+// The links of DAGs (see k_links): one entry for each word.  segs (device memory): DAG k's words lie
+// in src and go to dag[off ..] (dag null: in place) and links[off ..] (links null: copied only), its
+// blocks are [block0, block0 + link_blocks(words)), grid[k] gets its grid entry (grid null: none).
+// segs null: the one DAG `one`.  last: the last word's index.
+struct LinkSeg {
+    const u32* src;
+    u32 off, words, grid, block0;
+};
+u32 link_blocks(u64 words);
+int launch_links(const LinkSeg* segs, u32 nseg, const LinkSeg& one, u32 blocks, u32 last, u32* dag, u64* links, u32* grid,
+                 hipStream_t s);
 // One DAG of a set, walked as a one-cell container.  base is 0, or the grid sentinel
 // 0xFFFFFFFF / 0xFFFFFFFE when the root is all shadow / all lit.
 struct DagDesc {
@@ -303,8 +316,9 @@ struct DagDesc {
     u32 base;
     u32 dl;    // numLevels
     u32 leaf;  // 1: leafmask nodes at level 2; 0: the DAG goes down to level 0
-    const u64* top;  // the DAG's lookup top table (launch_build_top, one cell), or null
-    u32 topk;        // its levels
+    const u64* top;    // the DAG's lookup top table (launch_build_top, one cell), or null
+    const u64* links;  // its links (launch_links; read with a top table), or null
+    u32 topk;          // the table's levels
 };
 // The descriptor of a built DAG (createTopLevelGrid sentinels for a one-cell grid,
 // src/CompressedShadowContainer.cpp:71-91).
@@ -316,6 +330,7 @@ inline DagDesc dag_desc(const cpvs_dag* d) {
     r.dl = (u32)d->n;
     r.leaf = d->leafmasks ? 1u : 0u;
     r.top = d->d_top;
+    r.links = d->d_links;
     r.topk = d->d_top ? d->top_levels : 0u;
     return r;
 }

@@ -108,3 +108,44 @@ def test_round_robin_tiles(ctx, dags, count):
     assert np.array_equal(got, want)
     for s in sh:
         s.close()
+
+
+@pytest.mark.parametrize("leafmasks", [1, 0])
+@pytest.mark.parametrize("N,length", [(8, 1), (16, 2), (64, 1), (64, 2), (128, 4), (256, 1)])
+@pytest.mark.parametrize("top", [0, 1, -1])
+def test_links_of_container_dags(ctx, N, length, top, leafmasks):
+    """Lookups through the container's links, over the words copied with them: cells of one word (empty
+    and full z-tiles) beside cells of many, below, at and above one tile of words."""
+    _say("links", N, length, top, leafmasks)
+    ctx.set_leafmasks(bool(leafmasks))
+    try:
+        c = cp.CompressedShadowContainer(length)
+        words, order = [], {}
+        for y in range(length):
+            for x in range(length):
+                D = O.gen_depth(N, SEED0 + 30 + y * length + x, 3, True)
+                for z in range(length):
+                    sh = cp.CompressedShadow.create(cp.MinMaxHierarchy(D), z, length)
+                    order[(z, y, x)] = sh.getDAG()
+                    n = sh.getNumLevels()
+                    c.set(sh, x, y, z)
+        words = [order[k] for k in sorted(order)]
+        c.setTopLevels(top)
+        c.moveToGPU()
+        w, grid = c.words_and_grid()
+        assert np.array_equal(w, np.concatenate(words))
+        assert np.array_equal(grid, O.top_level_grid(words))
+        q = np.random.default_rng(N + length).uniform(-1, 1, (20011, 4)).astype(np.float32)
+        got = c.evaluate(cp.DeviceArray.from_numpy(q)).numpy()
+        gl = length.bit_length() - 1
+        px = _np_paths(q, np.eye(4, dtype=np.float32), N * length)
+        want = np.zeros(len(q), np.uint8)
+        for y in range(length):
+            for x in range(length):
+                D = O.gen_depth(N, SEED0 + 30 + y * length + x, 3, True)
+                here = (px[0] // N == x) & (px[1] // N == y)
+                want[here] = O.brute_visible(D, length, px[0][here] % N, px[1][here] % N, px[2][here])
+        assert (n, gl) == c.info()[:2] and np.array_equal(got, want)
+        c.close()
+    finally:
+        ctx.set_leafmasks(True)
