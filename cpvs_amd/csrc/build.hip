@@ -139,7 +139,7 @@ struct Level {
     u32* id = nullptr;
     u32* uniq = nullptr;
     u32* off = nullptr;
-    u64* first = nullptr;
+    uint8_t* flag = nullptr;
     u64* tab = nullptr;
     u32 slots = 0;
 };
@@ -361,7 +361,8 @@ constexpr int kRetryFullTable = -1001;
 constexpr int kRetryExactCounts = -1002;  // the counts exceed the emitted nodes (a map with NaN depths)
 
 
-__global__ void k_store_word(u32* dst, u32 v) { *dst = v; }
+// *dst = v, plus 1 when *src (may be null) is not 0.
+__global__ void k_store_word(u32* dst, u32 v, const u32* src) { *dst = v + ((src && *src) ? 1u : 0u); }
 
 constexpr u32 kHostReady = kMetaWords, kHostDone = kMetaWords + 1;  // flags behind the meta readback
 static_assert(sizeof(u32) * (kMetaWords + 2) <= sizeof(u64) * kPinnedWords, "the readback fits the pinned staging");
@@ -396,18 +397,22 @@ int wait_words(const volatile u32* w, size_t n, u32 unset, hipStream_t s) {
 
 }  // namespace
 
-int wait_stream(u64* pinned, hipStream_t s) {
+// As wait_stream; *set (may be null) = whether the device word *src was not 0 then.
+static int wait_stream_word(u64* pinned, const u32* src, bool* set, hipStream_t s) {
     u32* done = reinterpret_cast<u32*>(pinned) + kHostDone;
     *static_cast<volatile u32*>(done) = 0;
-    CPVS_LAUNCH("done", k_store_word, dim3(1), dim3(1), 0, s, done, 1u);
+    CPVS_LAUNCH("done", k_store_word, dim3(1), dim3(1), 0, s, done, 1u, src);
     CPVS_HIP_CHECK(hipGetLastError());
-    return wait_words(done, 1, 0u, s);
+    const int rc = wait_words(done, 1, 0u, s);
+    if (set) *set = *static_cast<volatile u32*>(done) > 1;
+    return rc;
 }
+int wait_stream(u64* pinned, hipStream_t s) { return wait_stream_word(pinned, nullptr, nullptr, s); }
 
 namespace {
 
 int store_and_wait(u32* dst, u32 v, u64* pinned, hipStream_t s) {
-    CPVS_LAUNCH("store_word", k_store_word, dim3(1), dim3(1), 0, s, dst, v);
+    CPVS_LAUNCH("store_word", k_store_word, dim3(1), dim3(1), 0, s, dst, v, nullptr);
     return wait_stream(pinned, s);
 }
 
@@ -523,7 +528,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         lv[L].id = A.take<u32>(c);
         lv[L].uniq = A.take<u32>(c);
         lv[L].off = A.take<u32>(c);
-        lv[L].first = A.take<u64>(first_words((u32)c));
+        lv[L].flag = reinterpret_cast<uint8_t*>(A.take<u64>(flag_words((u32)c)));
         lv[L].slots = level_slots(cnt, L, R, Ls, use_table, leaf, small_tables);
         tab_slots += lv[L].slots;
         if (L < Ls) clear_slots += lv[L].slots;
@@ -654,14 +659,15 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     MArgs ma{};
     ma.leafm = leafm;
     ma.heads = runhead;
-    ma.nleaf = (u32)c2;
+    ma.sorted = !use_table;
     u32 tile = 0;
     for (int L = deepest; L <= R; ++L) {
         const Level& v = lv[L];
         ma.tile0[ma.nlev] = tile;
         tile += ceil_div<u32>(v.count, kTileNodes);
-        ma.lv[ma.nlev++] = MLevel{v.mask, v.cstart, v.id, v.tab, v.first, v.uniq, v.off, v.count, v.slots, L,
-                                  (leaf && L == 2) ? 1u : 0u, L == R ? 1u : 0u};
+        ma.lv[ma.nlev++] = MLevel{v.mask, v.cstart, v.id, v.tab, v.flag, v.uniq, v.off, v.count, v.slots, L,
+                                  (leaf && L == 2) ? 1u : 0u, L == R ? 1u : 0u,
+                                  (use_table && L < R && (L >= Ls || v.count <= kLateMax)) ? 1u : 0u};
     }
     ma.tile0[ma.nlev] = tile;
     // Without a leaf level its kernel did not clear the tables.
@@ -680,7 +686,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     // words go straight to a buffer of their exact size and the GPU does not wait for the host.
     volatile u32* host_meta = reinterpret_cast<volatile u32*>(pinned);
     host_meta[kHostReady] = 0;
-    merge_finish(ma, !use_table, tile_sums, tile_pre, meta, R, reinterpret_cast<u32*>(pinned), s);
+    merge_finish(ma, tile_sums, tile_pre, meta, R, reinterpret_cast<u32*>(pinned), s);
     CPVS_HIP_CHECK(hipGetLastError());
     rc = wait_words(host_meta + kHostReady, 1, 0u, s);
     if (rc) return rc;
@@ -719,7 +725,9 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         return CPVS_ENOMEM;
     }
     merge_write(ma, meta, d_words, total, s);
-    rc = wait_stream(pinned, s);
+    bool collided = false;  // the late levels' compares run beside the write
+    rc = wait_stream_word(pinned, use_table ? meta + kMetaColl : nullptr, &collided, s);
+    if (rc == CPVS_OK && collided) rc = kRetryWithSort;
     if (rc) {
         if (!into) ctx->buffers.give(d_words);
         return rc;
@@ -764,7 +772,7 @@ size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_
         if (L < R) cmax = cnt[L] > cmax ? (u32)cnt[L] : cmax;
         const bool is_leaf = leaf && L == 2;
         need += (is_leaf ? 0 : arena_bytes(c, 8) + arena_bytes(c, 4)) + 4 * arena_bytes(c, 4) +
-                arena_bytes(first_words((u32)c), 8);
+                arena_bytes(flag_words((u32)c), 8);
         slots += level_slots(cnt, L, R, Ls, use_table, leaf, small_tables);
         ntiles += ceil_div<u32>((u32)cnt[L], kTileNodes);
     }

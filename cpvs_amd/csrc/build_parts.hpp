@@ -226,9 +226,13 @@ __device__ inline int leaf_f(float D) {
 // leafmask row, partial slices in ascending order).  All loads are issued before the hash.
 __device__ inline u64 leaf_key_hash(u32 m, const u64* __restrict__ slot8) {
     const u32 k = num_children(m);
-    u64 v[8];
+    u64 v[8];  // (16 bytes a load: a row takes half the line look-ups)
 #pragma unroll
-    for (u32 j = 0; j < 8; ++j) v[j] = (j < k) ? slot8[j] : 0ull;
+    for (u32 j = 0; j < 8; j += 2) {
+        ulonglong2 x = make_ulonglong2(0ull, 0ull);
+        if (j < k) x = *reinterpret_cast<const ulonglong2*>(slot8 + j);
+        v[j] = x.x, v[j + 1] = x.y;
+    }
     LeafHash hs(m);
 #pragma unroll
     for (u32 j = 0; j < 8; ++j)
@@ -501,12 +505,11 @@ __device__ inline void leaf_lanes(const LeafCol& c, const LeafOut& o) {
 }
 
 // The identity of each node of a level for its parents' keys: equal for equal subtrees, different
-// otherwise (up to hash collisions, which k_resolve finds): the node's merge-table slot, or its first
-// occurrence's index with the sort merge.  With heads set the level is the leaf level and only runs'
-// first nodes (heads[c] == c) have theirs yet: a child takes its run's, and it is stored for the
-// child as well (each node has one parent).
+// otherwise (up to hash collisions, which the key compares find): the node's merge-table slot, or its
+// first occurrence's index with the sort merge.  With heads set the level is the leaf level and only
+// runs' first nodes (heads[c] == c) have one: a child's is its run's.
 struct ChildIds {
-    u32* id;
+    const u32* id;
     const u32* heads;
     u32 n;  // nodes of the level: bounds every index (first children past a level's emitted nodes)
 };
@@ -527,9 +530,6 @@ __device__ inline void load_child_ids(const ChildIds& c, u32 s, u32 k, u32 r[8])
     for (u32 j = 0; j < 8; ++j) h[j] = (j < k) ? c.heads[at[j]] : 0u;
 #pragma unroll
     for (u32 j = 0; j < 8; ++j) r[j] = (j < k) ? c.id[min(h[j], c.n - 1)] : 0u;
-#pragma unroll
-    for (u32 j = 0; j < 8; ++j)
-        if (j < k && h[j] != at[j]) c.id[at[j]] = r[j];
 }
 
 // Key hash of an inner node with mask m, k children and their identities r: a sum of (mask,
@@ -617,11 +617,14 @@ struct InnerEq {
 // 104 µs against a plain load.
 // A probe gives up after kMaxProbes occupied slots (a table too small for its keys: the leaf
 // level's table is sized for a quarter of its nodes), counts that in *full and returns a slot in
-// range; the host then builds again with a larger table (k_resolve reads whatever the returned slot
-// holds, bounds it and checks the keys, so every index that the rest of the build derives stays in
-// range).
+// range; the host then builds again with a larger table (whatever a slot holds is bounded where it is
+// used as an index).
+// occ: a node that the slot held (equal keys, unless hashes collide: the caller compares), or kNoRep
+// when this one took it first.  Every node of a slot is compared with one that came before it, so
+// compares that all hold make all the slot's keys equal.
 constexpr u32 kMaxProbes = 256;
-__device__ inline u32 table_insert(u64* tab, u32 S, u64 h, u32 i, u32* full) {
+__device__ inline u32 table_insert(u64* tab, u32 S, u64 h, u32 i, u32* full, u32& occ) {
+    occ = kNoRep;
     const u32 tag = (u32)(h >> 32);
     const u64 mine = ((u64)tag << 32) | i;
     u32 slot = __umulhi((u32)(h ^ (h >> 31)) * 0x9E3779B1u, S);
@@ -633,6 +636,7 @@ __device__ inline u32 table_insert(u64* tab, u32 S, u64 h, u32 i, u32* full) {
             if (cur == kEmptySlot) return slot;
         }
         if ((u32)(cur >> 32) == tag) {
+            occ = (u32)cur;
             if ((u32)cur > i) atomicMin(reinterpret_cast<unsigned long long*>(tab + slot), (unsigned long long)mine);
             return slot;
         }
@@ -640,43 +644,6 @@ __device__ inline u32 table_insert(u64* tab, u32 S, u64 h, u32 i, u32* full) {
     }
     atomicAdd(full, 1u);
     return slot;
-}
-
-// A table slot hit by many threads at once serialises their atomics, and equal keys are common
-// (flat regions repeat the same subtrees all over a level; a level of a few hundred thousand nodes
-// runs almost all at once, before any first occurrence has landed).  So each 256-thread workgroup
-// first merges its own equal hashes in an LDS table: only the smallest index of each distinct
-// hash in the group touches the global table, and the others take its slot.  Every thread of the
-// workgroup calls this (it has barriers).
-// Threads per insert workgroup (the LDS merge window).  Measured at 8192^2: 512 takes the inner
-// inserts 0.142 -> 0.136 ms against 256; 1024 gains nothing more.
-constexpr u32 kInsertBlock = 512;
-constexpr u32 kGroupSlots = 2 * kInsertBlock;
-
-__device__ inline u32 table_insert_group(u64* tab, u32 S, u64 h, u32 i, bool active, u32* full) {
-    __shared__ u64 gh[kGroupSlots];
-    __shared__ u32 gi[kGroupSlots];
-    __shared__ u32 gs[kGroupSlots];
-    for (u32 j = threadIdx.x; j < kGroupSlots; j += blockDim.x) {
-        gh[j] = 0ull;
-        gi[j] = kNoRep;
-    }
-    __syncthreads();
-    if (h == 0ull) h = 1ull;  // 0 marks an empty LDS slot
-    u32 ls = 0;
-    if (active) {
-        ls = (u32)(h ^ (h >> 29)) & (kGroupSlots - 1);
-        for (;;) {
-            const u64 cur = atomicCAS(reinterpret_cast<unsigned long long*>(gh + ls), 0ull, (unsigned long long)h);
-            if (cur == 0ull || cur == h) break;
-            ls = (ls + 1) & (kGroupSlots - 1);
-        }
-        atomicMin(gi + ls, i);
-    }
-    __syncthreads();
-    if (active && gi[ls] == i) gs[ls] = table_insert(tab, S, h, i, full);
-    __syncthreads();
-    return active ? gs[ls] : 0u;
 }
 
 // The leaf level: only a run's first node is inserted (1.3 M of 6.7 M nodes at 8192^2), so each
@@ -688,6 +655,8 @@ __device__ inline u32 table_insert_group(u64* tab, u32 S, u64 h, u32 i, bool act
 constexpr u32 kLeafInsertThreads = 256;
 constexpr u32 kLeafPer = 4;
 constexpr u32 kLeafOneMax = 1u << 18;
+// Inner levels of this many nodes take two a thread.
+constexpr u32 kInnerTwoMin = 1u << 20;
 
 // Threads per workgroup of the write kernels (at 8192^2, 128 and 256 tie; 512 and 1024 are slower).
 constexpr u32 kNodeThreads = 256;
@@ -740,8 +709,7 @@ enum : int {
     kMetaSortColl = 4 * kMaxLevels + 3,  // 32-bit key collisions resolved by a scan (sort merge)
     kMetaFull = 4 * kMaxLevels + 4,      // table inserts that found no free slot (table merge)
     kMetaSlow = 4 * kMaxLevels + 5,      // leaf columns left to the wave-per-column kernel
-    kMetaTicket = 4 * kMaxLevels + 6,    // workgroups of k_resolve that are done
-    kMetaWords = 4 * kMaxLevels + 7,
+    kMetaWords = 4 * kMaxLevels + 6,
 };
 
 

@@ -330,6 +330,7 @@ struct FWriteArgs {
 // Unique node r of level L (global rank order) into its DAG's buffer: [mask, absolute offsets of
 // the partial children] or [mask, lo, hi, ...] at the leaf level (src/CompressedShadow.cpp:326-392).
 __global__ __launch_bounds__(kNodeThreads) void k_forest_write(FWriteArgs a, FLevels lv, const u64* __restrict__ leafm,
+                                                                const u32* __restrict__ heads,
                                                                 const u32* __restrict__ base_off, const u32* __restrict__ B,
                                                                 u32* const* __restrict__ outp) {
     int k = 0;
@@ -362,7 +363,13 @@ __global__ __launch_bounds__(kNodeThreads) void k_forest_write(FWriteArgs a, FLe
     const u32 cb = B[gk - 1], co0 = base_off[gk - 1], s = lv.cstart[L][i];
     u32 id[8], co[8];
 #pragma unroll
-    for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? lv.id[L - 1][min(s + j, lv.count[L - 1] - 1)] : 0u;
+    for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(s + j, lv.count[L - 1] - 1) : 0u;
+    if (L == 3 && heads) {  // a leaf's identity is its run's first node's (table merge)
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(heads[id[j]], lv.count[2] - 1) : 0u;
+    }
+#pragma unroll
+    for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? lv.id[L - 1][id[j]] : 0u;
 #pragma unroll
     for (u32 j = 0; j < 8; ++j) co[j] = (j < kc) ? (u32)lv.tab[L - 1][min(id[j], lv.slots[L - 1] - 1)] : 0u;
 #pragma unroll
@@ -560,7 +567,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
     for (int L = Lmin; L <= Rmax; ++L) {
         const size_t c = C[L] ? C[L] : 1;
         need += (L > 2 ? arena_bytes(c, 8) + arena_bytes(c, 4) : 0) + 4 * arena_bytes(c, 4) +  // no coords, starts at leaves
-                arena_bytes(first_words((u32)c), 8);
+                arena_bytes(flag_words((u32)c), 8);
     }
     need += arena_bytes(tab_slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(tile_pre_count(ntiles), 16);
     need += arena_bytes(c2 * 8, 8) + 2 * arena_bytes(c2, 4);  // leafmask rows, run heads, column map
@@ -577,7 +584,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         if (rc) return rc;
     }
     FLevels lv{};
-    u64* first[kMaxLevels] = {};
+    uint8_t* flag[kMaxLevels] = {};
     for (int L = Lmin; L <= Rmax; ++L) {
         const size_t c = C[L] ? C[L] : 1;
         lv.coord[L] = (L > 2) ? A.take<u64>(c) : nullptr;
@@ -586,7 +593,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         lv.id[L] = A.take<u32>(c);
         lv.uniq[L] = A.take<u32>(c);
         lv.off[L] = A.take<u32>(c);
-        first[L] = A.take<u64>(first_words((u32)c));
+        flag[L] = reinterpret_cast<uint8_t*>(A.take<u64>(flag_words((u32)c)));
         lv.slots[L] = slots[L];
         lv.count[L] = (u32)c;
     }
@@ -675,15 +682,15 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         MArgs ma{};
         ma.leafm = leafm;
         ma.heads = runhead;
-        ma.nleaf = (u32)c2;
+        ma.sorted = !use_table;
         u32 tile = 0;
         for (int L = Lmin; L <= Rmax; ++L) {
             const u32 c = (u32)C[L];
             if (!c) continue;
             ma.tile0[ma.nlev] = tile;
             tile += ceil_div<u32>(c, kTileNodes);
-            ma.lv[ma.nlev++] = MLevel{lv.mask[L], lv.cstart[L], lv.id[L], lv.tab[L], first[L], lv.uniq[L], lv.off[L],
-                                      c, lv.slots[L], L, L == 2 ? 1u : 0u, 0u};
+            ma.lv[ma.nlev++] = MLevel{lv.mask[L], lv.cstart[L], lv.id[L], lv.tab[L], flag[L], lv.uniq[L], lv.off[L],
+                                      c, lv.slots[L], L, L == 2 ? 1u : 0u, 0u, 0u};
         }
         ma.tile0[ma.nlev] = tile;
         for (int k = 0; k < ma.nlev; ++k) {
@@ -693,7 +700,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
             else
                 merge_sort_level(ma, k, srt, meta, s);
         }
-        merge_finish(ma, !use_table, tile_sums, tile_pre, meta, -1, nullptr, s);
+        merge_finish(ma, tile_sums, tile_pre, meta, -1, nullptr, s);
         FBasesOut ho;
         ho.meta_host = st.back;
         ho.total = st.back + kMetaWords;
@@ -766,8 +773,8 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
     }
     wa.first[wa.nlev] = wblocks;
     if (e == hipSuccess && wblocks) {
-        CPVS_LAUNCH("forest_write", k_forest_write, dim3(wblocks), dim3(kNodeThreads), 0, s, wa, lv, leafm, boff, B,
-                    dptrs);
+        CPVS_LAUNCH("forest_write", k_forest_write, dim3(wblocks), dim3(kNodeThreads), 0, s, wa, lv, leafm,
+                    use_table ? runhead : nullptr, boff, B, dptrs);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);

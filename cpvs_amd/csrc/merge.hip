@@ -3,15 +3,17 @@
 // Bottom-up, each level takes one launch: the key of every node -- its mask and the partial
 // leafmasks, or its mask and its children's identities -- goes into the level's hash table, and the
 // slot it ends in is the node's own identity for its parents' keys.  Slots never move, so equal keys
-// have equal identities before anything is known of their order; what needs a finished table is
-// left to three launches over all levels at once:
-//   k_resolve   per node the smallest index in its slot, the full-key compare against it, and a bit
-//               for each first occurrence; the first occurrences and words of each 1024-node tile;
-//   k_totals    a scan of the tiles, the levels' totals and bases;
+// have equal identities before anything is known of their order.  A node's key is compared in the
+// same launch, in full, with that of a node that the slot already held.  What needs finished tables is
+// left to launches over all levels at once:
+//   k_firsts    per node the smallest index in its slot; a byte for each node, its words if it is that
+//               one; the first occurrences and words of each tile of nodes;
+//   k_totals    a scan of the tiles, the levels' totals and bases (k_offsets does it for few tiles);
 //   k_offsets   rank and word offset of every first occurrence, in index order, which is the order
 //               that mergeLevel's linear search gives (src/CompressedShadowUtil.h:154-182).
-// Ranks as identities took four launches a level (insert, resolve, scan, rank copies), and the copies
-// alone read and wrote every node of the leaf level.
+// Before, a launch over all nodes looked up each node's slot and compared its key with the first
+// occurrence's: 77 us and 209 MB of scattered reads of 690 us at 8192^2, 16 of 144 us at 1024^2.  Keys
+// are compared here while they are in registers: 8 z-tiles 2118 -> 1992 us, 32 maps 2182 -> 2086.
 //
 // Keys that a table cannot tell apart are found by the compares, and the build is done again with
 // the sort merge, whose identities are first occurrences' indices.
@@ -24,7 +26,7 @@ namespace cpvs {
 // One 64-bit word per slot: the key hash's high 32 bits (its tag) above the smallest node index
 // with that hash, so a probe touches one cache line and a new key costs one atomic.  ~0 marks an
 // empty slot (node indices stay below 2^32 - 1).  Two keys whose tags are equal and whose probe
-// chains meet share a slot; the full-key compare in k_resolve then sends the build down the
+// chains meet share a slot; the full-key compare of a later one then sends the build down the
 // sorting path, as for equal 64-bit hashes.
 
 __global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 S) {
@@ -32,100 +34,197 @@ __global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 
     if (i < S) tab[i] = kEmptySlot;
 }
 
+// The run heads of a window of kPer * kT nodes are listed in LDS; equal hashes meet in an LDS table,
+// the distinct ones are spread over the threads for the global inserts, and every head's key is then
+// compared with its window's first of that hash, that one's with the global slot's earlier node.  The
+// compares take four lanes to a pair of leafmask rows (16 bytes a lane): one lane to a row would touch
+// 64 lines with each load.  The rows are what the compares cost (83 MB at 8192^2: 57 -> 98 us).
+// What bounds it besides: the tables' atomics and coherent reads, performed at memory, about 7 G atomics/s.
+// (Windows of 4096 nodes, for fewer of them: 148 us, the dense windows' batches one after another.)
 template <u32 kPer>
 __global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
                                                                     const u32* __restrict__ runhead,
                                                                     const u64* __restrict__ hash, u32 n,
                                                                     u64* __restrict__ tab, u32 S, u32* __restrict__ tslot,
-                                                                    u32* __restrict__ full, u32 hbits) {
-    constexpr u32 kWindow = kPer * kLeafInsertThreads, kSlots = 2 * kWindow;  // at most half full: every probe ends
-    __shared__ u64 gh[kSlots];
-    __shared__ u32 gi[kSlots];  // smallest node index of the slot's hash, then its global slot
+                                                                    u32* __restrict__ meta, u32 hbits, u32 late) {
+    constexpr u32 kT = kLeafInsertThreads, kWindow = kPer * kT, kSlots = 2 * kWindow;  // at most half full: every probe ends
+    __shared__ u64 gh[kSlots];  // a hash, then its global slot << 32 | the node that the slot held before
+    __shared__ u32 gi[kSlots];  // smallest node index of the slot's hash
     __shared__ unsigned short glist[kWindow];  // LDS slots in use
-    __shared__ u32 gcount;
-    for (u32 j = threadIdx.x; j < kSlots; j += blockDim.x) {
-        gh[j] = 0ull;  // 0 marks an empty LDS slot
-        gi[j] = kNoRep;
-    }
-    if (threadIdx.x == 0) gcount = 0;
-    const u32 i0 = blockIdx.x * kWindow + threadIdx.x;
+    __shared__ unsigned short heads[kWindow], hslot[kWindow];  // the window's run heads and their LDS slots
+    __shared__ u32 gcount, nheads;
+    const u32 t = threadIdx.x, lane = t & (kWave - 1), i0 = blockIdx.x * kWindow;
+    if (t == 0) gcount = nheads = 0;
     u32 rh[kPer];
 #pragma unroll
     for (u32 k = 0; k < kPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
+        const u32 i = i0 + k * kT + t;
         rh[k] = (i < n) ? runhead[i] : kNoRep;
     }
-    // The key hash of each run's first node (the run's smallest index): from the leaf kernel where
-    // a lane walked its column, else from its mask and leafmasks (its row at its own index).
-    u64 h[kPer];
-#pragma unroll
-    for (u32 k = 0; k < kPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        h[k] = (hash && rh[k] == i) ? hash[i] : 0ull;
-    }
-    u32 hm[kPer];
-#pragma unroll
-    for (u32 k = 0; k < kPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        hm[k] = (rh[k] == i && h[k] == 0ull) ? mask[i] : 0u;
-    }
-#pragma unroll
-    for (u32 k = 0; k < kPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        if (rh[k] != i) continue;
-        if (h[k] == 0ull) h[k] = leaf_key_hash(hm[k], leafm + (size_t)i * 8);
-        h[k] = weaken_hash(h[k], hbits);
-        if (h[k] == 0ull) h[k] = 1ull;
+    for (u32 j = t; j < kSlots; j += kT) {
+        gh[j] = 0ull;  // 0 marks an empty LDS slot
+        gi[j] = kNoRep;
     }
     __syncthreads();
-    u32 ls[kPer];
+    {
+        u64 bits[kPer];
+        u32 total = 0, at = 0;
 #pragma unroll
-    for (u32 k = 0; k < kPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        ls[k] = 0;
-        if (rh[k] != i) continue;
-        u32 sl = (u32)(h[k] ^ (h[k] >> 29)) & (kSlots - 1);
+        for (u32 k = 0; k < kPer; ++k) {
+            bits[k] = __ballot(rh[k] == i0 + k * kT + t);  // (never past n)
+            total += (u32)__popcll(bits[k]);
+        }
+        if (lane == 0 && total) at = atomicAdd(&nheads, total);
+        at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+        for (u32 k = 0; k < kPer; ++k) {
+            if ((bits[k] >> lane) & 1ull) heads[at + (u32)__popcll(bits[k] & ((1ull << lane) - 1ull))] = (unsigned short)(k * kT + t);
+            at += (u32)__popcll(bits[k]);
+        }
+    }
+    __syncthreads();
+    const u32 nh = nheads;
+    for (u32 j = t; j < nh; j += kT) {
+        // The key hash of a run's first node (the run's smallest index): from the leaf kernel where a
+        // lane walked its column, else from its mask and leafmasks (its row at its own index).
+        const u32 i = i0 + heads[j];
+        u64 h = hash ? hash[i] : 0ull;
+        if (h == 0ull) h = leaf_key_hash(mask[i], leafm + (size_t)i * 8);
+        h = weaken_hash(h, hbits);
+        if (h == 0ull) h = 1ull;
+        u32 sl = (u32)(h ^ (h >> 29)) & (kSlots - 1);
         for (;;) {
-            const u64 cur = atomicCAS(reinterpret_cast<unsigned long long*>(gh + sl), 0ull, (unsigned long long)h[k]);
+            const u64 cur = atomicCAS(reinterpret_cast<unsigned long long*>(gh + sl), 0ull, (unsigned long long)h);
             if (cur == 0ull) {
                 glist[atomicAdd(&gcount, 1u)] = (unsigned short)sl;
                 break;
             }
-            if (cur == h[k]) break;
+            if (cur == h) break;
             sl = (sl + 1) & (kSlots - 1);
         }
         atomicMin(gi + sl, i);
-        ls[k] = sl;
+        hslot[j] = (unsigned short)sl;
     }
     __syncthreads();
     const u32 m = gcount;  // at most kWindow
-    for (u32 j = threadIdx.x; j < m; j += blockDim.x) {
+    for (u32 j = t; j < m; j += kT) {
         const u32 sl = glist[j];
-        gi[sl] = table_insert(tab, S, gh[sl], gi[sl], full);
+        u32 occ;
+        const u32 slot = table_insert(tab, S, gh[sl], gi[sl], meta + kMetaFull, occ);
+        gh[sl] = ((u64)slot << 32) | occ;
+    }
+    __syncthreads();
+    bool eq = true;
+    for (u32 j = t; j < nh; j += kT) tslot[i0 + heads[j]] = (u32)(gh[hslot[j]] >> 32);
+    for (u32 j = t / 4; j < nh && !late; j += kT / 4) {
+        const u32 i = i0 + heads[j], sl = hslot[j], rep = gi[sl];
+        const u32 with = (rep != i) ? rep : (u32)gh[sl];
+        if (with >= n) continue;
+        const u32 q = t & 3, ma = mask[i], mb = mask[with];
+        const u32 k = num_children(ma);
+        eq = eq && ma == mb;
+        if (2 * q < k) {
+            const ulonglong2 x = *reinterpret_cast<const ulonglong2*>(leafm + (size_t)i * 8 + 2 * q);
+            const ulonglong2 y = *reinterpret_cast<const ulonglong2*>(leafm + (size_t)with * 8 + 2 * q);
+            eq = eq && x.x == y.x && (2 * q + 1 >= k || x.y == y.y);
+        }
+    }
+    if (!eq) atomicAdd(meta + kMetaColl, 1u);  // two keys share a slot: the build is redone by sorting
+}
+
+// A table slot hit by many threads at once serialises their atomics, and equal keys are common
+// (flat regions repeat the same subtrees all over a level; a level of a few hundred thousand nodes
+// runs almost all at once, before any first occurrence has landed).  So each workgroup first merges
+// its own equal hashes in an LDS table, with the keys beside it for the compares: only the smallest
+// index of each distinct hash in the group touches the global table, and the others take its slot.
+// Threads per workgroup (the window): at 8192^2, 512 took the inner inserts 0.142 -> 0.136 ms against
+// 256; 1024 gained nothing more.
+constexpr u32 kInsertBlock = 512;
+
+template <u32 kPer>
+__global__ __launch_bounds__(kInsertBlock) void k_insert_inner(const u32* __restrict__ mask, const u32* __restrict__ cstart,
+                                                               ChildIds ch, u32 n, u64* __restrict__ tab, u32 S,
+                                                               u32* __restrict__ id, u32* __restrict__ meta, u32 hbits, u32 late) {
+    constexpr u32 kT = kInsertBlock, kSlots = 2 * kPer * kT;
+    __shared__ u64 gh[kSlots];
+    __shared__ u32 gi[kSlots];  // smallest node index of the slot's hash, then its global slot
+    const u32 t = threadIdx.x, i0 = blockIdx.x * (kPer * kT) + t;
+    u32 m[kPer], c[kPer], k[kPer], r[kPer][8], ls[kPer], rep[kPer], slot[kPer];
+    u64 h[kPer];
+#pragma unroll
+    for (u32 e = 0; e < kPer; ++e) {
+        const u32 i = i0 + e * kT;
+        m[e] = (i < n) ? mask[i] : 0u;
+        c[e] = (i < n) ? cstart[i] : 0u;
+    }
+    for (u32 j = t; j < kSlots; j += kT) {
+        gh[j] = 0ull;
+        gi[j] = kNoRep;
+    }
+#pragma unroll
+    for (u32 e = 0; e < kPer; ++e) {
+        k[e] = ch.id ? num_children(m[e]) : 0u;
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j) r[e][j] = 0u;
+        if (k[e]) load_child_ids(ch, c[e], k[e], r[e]);
+    }
+#pragma unroll
+    for (u32 e = 0; e < kPer; ++e) {
+        h[e] = weaken_hash(inner_key_hash(m[e], r[e]), hbits);
+        if (h[e] == 0ull) h[e] = 1ull;  // 0 marks an empty LDS slot
     }
     __syncthreads();
 #pragma unroll
-    for (u32 k = 0; k < kPer; ++k) {
-        const u32 i = i0 + k * kLeafInsertThreads;
-        if (rh[k] == i) tslot[i] = gi[ls[k]];
+    for (u32 e = 0; e < kPer; ++e) {
+        ls[e] = 0;
+        if (i0 + e * kT >= n) continue;
+        u32 sl = (u32)(h[e] ^ (h[e] >> 29)) & (kSlots - 1);
+        for (;;) {
+            const u64 cur = atomicCAS(reinterpret_cast<unsigned long long*>(gh + sl), 0ull, (unsigned long long)h[e]);
+            if (cur == 0ull || cur == h[e]) break;
+            sl = (sl + 1) & (kSlots - 1);
+        }
+        atomicMin(gi + sl, i0 + e * kT);
+        ls[e] = sl;
     }
-}
-
-__global__ __launch_bounds__(kInsertBlock) void k_insert_inner(const u32* __restrict__ mask, const u32* __restrict__ cstart,
-                                                               ChildIds ch, u32 n, u64* __restrict__ tab, u32 S,
-                                                               u32* __restrict__ id, u32* __restrict__ full, u32 hbits) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool act = i < n;
-    u64 h = 0;
-    if (act) {
-        const u32 m = mask[i], s = cstart[i];
-        const u32 k = ch.id ? num_children(m) : 0u;
-        u32 r[8] = {};
-        if (k) load_child_ids(ch, s, k, r);
-        h = weaken_hash(inner_key_hash(m, r), hbits);
+    __syncthreads();
+    // A node's key is compared with the group's smallest index of its hash, that one's with the table's.
+    u32 with[kPer];
+#pragma unroll
+    for (u32 e = 0; e < kPer; ++e) {
+        const u32 i = i0 + e * kT;
+        rep[e] = (i < n) ? gi[ls[e]] : kNoRep;
+        with[e] = (i < n) ? rep[e] : kNoRep;
+        slot[e] = kNoRep;
+        if (i < n && rep[e] == i) slot[e] = table_insert(tab, S, h[e], i, meta + kMetaFull, with[e]);
+        if (late) with[e] = kNoRep;
     }
-    const u32 slot = table_insert_group(tab, S, h, i, act, full);
-    if (act) id[i] = slot;
+    __syncthreads();
+#pragma unroll
+    for (u32 e = 0; e < kPer; ++e)
+        if (slot[e] != kNoRep) gi[ls[e]] = slot[e];
+    u32 mo[kPer], co[kPer];
+#pragma unroll
+    for (u32 e = 0; e < kPer; ++e) {
+        mo[e] = (with[e] < n) ? mask[with[e]] : m[e];
+        co[e] = (with[e] < n) ? cstart[with[e]] : 0u;
+    }
+    bool eq = true;
+#pragma unroll
+    for (u32 e = 0; e < kPer; ++e) {
+        eq = eq && mo[e] == m[e];
+        if (with[e] < n && mo[e] == m[e] && k[e]) {
+            u32 ro[8];
+            load_child_ids(ch, co[e], k[e], ro);
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j) eq = eq && ro[j] == r[e][j];
+        }
+    }
+    if (!eq) atomicAdd(meta + kMetaColl, 1u);  // two keys share a slot: the build is redone by sorting
+    __syncthreads();
+#pragma unroll
+    for (u32 e = 0; e < kPer; ++e)
+        if (i0 + e * kT < n) id[i0 + e * kT] = gi[ls[e]];
 }
 
 // --- the sort merge --------------------------------------------------------------------------
@@ -171,12 +270,11 @@ __device__ inline u32 saturate32(u64 v) { return v > 0xFFFFFFFFull ? 0xFFFFFFFFu
 // saturated, so that the host rejects the DAG.  Then the levels' bases (R >= 0): B[R] = 0, B[L-1] =
 // B[L] + S[L], and the readback.  Levels' first tiles and the metadata are kept in LDS: looked up in
 // the kernel's arguments by a varying index, and read back from memory, they took longer than the
-// scan.  tile_sums and meta are read at agent scope: in k_resolve's last workgroup they were stored
-// by other workgroups of the same launch.
+// scan.
 constexpr u32 kTotalsThreads = 1024;
-constexpr u32 kInlineTiles = 256;  // up to this many tiles k_resolve's last workgroup does this
+constexpr u32 kInlineTiles = 1024;  // up to this many tiles k_offsets' workgroups scan them themselves
 template <u32 kThreads>
-__device__ inline void merge_totals(const MArgs& a, const u32* tile_sums, ulonglong2* __restrict__ tile_pre,
+__device__ inline void merge_totals(const MArgs& a, const u32* __restrict__ tile_sums, ulonglong2* __restrict__ tile_pre,
                                     u32* __restrict__ meta, int R, u32* __restrict__ host_meta) {
     constexpr u32 kWaves = kThreads / kWave, kPer = 4;
     __shared__ u32 s_c[2][kWaves], s_w[2][kWaves], s_tile0[kMaxLevels + 1], s_meta[kMetaWords];
@@ -186,20 +284,20 @@ __device__ inline void merge_totals(const MArgs& a, const u32* tile_sums, ulongl
     const u32 lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
     if (threadIdx.x <= nlev) s_tile0[threadIdx.x] = a.tile0[threadIdx.x];
     for (u32 i = threadIdx.x; i < kMetaWords; i += kThreads)
-        s_meta[i] = __hip_atomic_load(meta + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_meta[i] = meta[i];
     u32 run_c = 0;  // of the chunks before
     u64 run_w = 0;
     u32 v[kPer];
     auto load = [&](u32 t0) {
 #pragma unroll
         for (u32 j = 0; j < kPer; ++j)
-            v[j] = (t0 + j < nt) ? __hip_atomic_load(tile_sums + t0 + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+            v[j] = (t0 + j < nt) ? tile_sums[t0 + j] : 0u;
     };
     load(threadIdx.x * kPer);
     u32 buf = 0;
     for (u32 base = 0; base < nt; base += kThreads * kPer, buf ^= 1u) {
         const u32 t0 = base + threadIdx.x * kPer;
-        u32 x[kPer], c = 0, w = 0;  // (a chunk of 4096 tiles of at most 17408 words fits 32 bits)
+        u32 x[kPer], c = 0, w = 0;  // (a chunk of 4096 tiles of at most 34816 words fits 32 bits)
 #pragma unroll
         for (u32 j = 0; j < kPer; ++j) {
             x[j] = v[j];
@@ -237,7 +335,7 @@ __device__ inline void merge_totals(const MArgs& a, const u32* tile_sums, ulongl
                 lev_w[k] = ww;
                 ++k;
             }
-            tile_pre[t0 + j] = make_ulonglong2(cc, ww);
+            if (tile_pre) tile_pre[t0 + j] = make_ulonglong2(cc, ww);
             cc += x[j] >> 16;
             ww += x[j] & 0xFFFFu;
         }
@@ -247,7 +345,7 @@ __device__ inline void merge_totals(const MArgs& a, const u32* tile_sums, ulongl
         lev_w[nlev] = run_w;
     }
     __syncthreads();
-    if (threadIdx.x <= nlev) tile_pre[nt + threadIdx.x] = make_ulonglong2(lev_c[threadIdx.x], lev_w[threadIdx.x]);
+    if (tile_pre && threadIdx.x <= nlev) tile_pre[nt + threadIdx.x] = make_ulonglong2(lev_c[threadIdx.x], lev_w[threadIdx.x]);
     if (threadIdx.x < nlev) {
         const u32 k = threadIdx.x;
         s_meta[kMetaU + a.lv[k].L] = lev_c[k + 1] - lev_c[k];
@@ -281,103 +379,109 @@ __global__ __launch_bounds__(kTotalsThreads) void k_totals(MArgs a, const u32* _
     merge_totals<kTotalsThreads>(a, tile_sums, tile_pre, meta, R, host_meta);
 }
 
+// First occurrences as bytes: flag[node] = the node's words if it is its key's first, else 0; and each
+// tile's first occurrences << 16 | their words (at most 2048 and 34816).  The loads of the tile's
+// rounds are issued together, stage by stage.
 template <bool kSorted>
-__global__ __launch_bounds__(kTileThreads) void k_resolve(MArgs a, u32* tile_sums, ulonglong2* __restrict__ tile_pre,
-                                                          u32* meta, int R, u32* __restrict__ host_meta) {
-    u32* collisions = meta + kMetaColl;
+__global__ __launch_bounds__(kTileThreads) void k_firsts(MArgs a, u32* __restrict__ tile_sums) {
     __shared__ u32 s_wave[kTileThreads / kWave];
     const int k = level_of_tile(a, blockIdx.x);
     const MLevel& l = a.lv[k];
     const u32 n = l.n, base = (blockIdx.x - a.tile0[k]) * kTileNodes + threadIdx.x;
-    // The loads of the tile's rounds are issued together, stage by stage.
-    u32 r[kTileRounds];
-    bool act[kTileRounds];
+    u32 r[kTilePer], m[kTilePer];
+    bool act[kTilePer];
 #pragma unroll
-    for (int j = 0; j < kTileRounds; ++j) {
+    for (u32 j = 0; j < kTilePer; ++j) {
         const u32 i = base + j * kTileThreads;
         act[j] = i < n;
         if (l.leaf && act[j]) act[j] = a.heads[i] == i;  // a first occurrence heads its run
     }
 #pragma unroll
-    for (int j = 0; j < kTileRounds; ++j) r[j] = (act[j] && !l.lone) ? l.id[base + j * kTileThreads] : 0u;
-    if (!kSorted) {
-#pragma unroll
-        for (int j = 0; j < kTileRounds; ++j) r[j] = (act[j] && !l.lone) ? (u32)l.tab[min(r[j], l.slots - 1)] : 0u;
-    }
-    u32 acc = 0;  // first occurrences << 16 | their words (at most 1024 and 17408)
-#pragma unroll
-    for (int j = 0; j < kTileRounds; ++j) {
+    for (u32 j = 0; j < kTilePer; ++j) {
         const u32 i = base + j * kTileThreads;
-        bool first = false;
-        if (act[j]) {
-            if (l.lone || r[j] >= n) r[j] = i;
-            first = r[j] == i;
-            const int kc = a.child(k);
-            if (!kSorted && l.lone && kc >= 0 && a.lv[kc].leaf) {
-                // A root over leaves (a 16 x 16 map) had no insert to store its children's identities.
-                u32 unused[8];
-                load_child_ids(ChildIds{a.lv[kc].id, a.heads, a.lv[kc].n}, l.cstart[i], num_children(l.mask[i]), unused);
-            }
-            if (!kSorted && !first) {
-                const bool same = l.leaf ? LeafEq{l.mask, a.leafm, nullptr, n}(i, r[j])
-                                         : InnerEq{l.mask, l.cstart, kc >= 0 ? a.lv[kc].id : nullptr, kc >= 0 ? a.lv[kc].n : 1u}(i, r[j]);
-                if (!same) {
-                    atomicAdd(collisions, 1u);  // two keys share a slot: the build is redone by sorting
-                    __threadfence();  // counted before the workgroup's ticket
-                    first = true;
-                }
-            }
-            if (first) acc += (1u << 16) | node_words(l.mask[i], l.leaf);
-        }
-        const u64 bits = __ballot(first);
-        if ((threadIdx.x & (kWave - 1)) == 0 && i < n) l.first[i / 64] = bits;
+        r[j] = (act[j] && !l.lone) ? l.id[i] : i;
+        m[j] = act[j] ? l.mask[i] : 0u;
+    }
+    if (!kSorted && !l.lone) {
+#pragma unroll
+        for (u32 j = 0; j < kTilePer; ++j) r[j] = act[j] ? (u32)l.tab[min(r[j], l.slots - 1)] : 0u;
+    }
+    u32 acc = 0;
+#pragma unroll
+    for (u32 j = 0; j < kTilePer; ++j) {
+        const u32 i = base + j * kTileThreads;
+        const u32 w = (act[j] && r[j] == i) ? node_words(m[j], l.leaf) : 0u;
+        if (i < n) l.flag[i] = (uint8_t)w;
+        acc += w ? (1u << 16) | w : 0u;
     }
     acc = block_reduce(acc, s_wave, OpSum{});
-    if (gridDim.x > kInlineTiles) {  // k_totals follows
-        if (threadIdx.x == 0) tile_sums[blockIdx.x] = acc;
-        return;
-    }
-    // The last workgroup to finish does the totals: one launch less for small builds.
-    __shared__ u32 s_last;
-    if (threadIdx.x == 0) {
-        __hip_atomic_store(tile_sums + blockIdx.x, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        wait_stores();
-        s_last = atomicAdd(meta + kMetaTicket, 1u) == gridDim.x - 1 ? 1u : 0u;
-    }
-    __syncthreads();
-    if (!s_last) return;
-    merge_totals<kTileThreads>(a, tile_sums, tile_pre, meta, R, host_meta);
+    if (threadIdx.x == 0) tile_sums[blockIdx.x] = acc;
 }
 
-__global__ __launch_bounds__(kTileThreads) void k_offsets(MArgs a, const ulonglong2* __restrict__ tile_pre) {
-    const int k = level_of_tile(a, blockIdx.x);
+// The flags of a thread's kTilePer consecutive nodes of a tile.
+__device__ inline u64 tile_flags(const MLevel& l, u32 tile, u32& i) {
+    i = tile * kTileNodes + threadIdx.x * kTilePer;
+    if (i >= l.n) return 0ull;
+    const u64 v = *reinterpret_cast<const u64*>(l.flag + i);
+    const u32 have = l.n - i;
+    return have < kTilePer ? v & ((1ull << (8 * have)) - 1ull) : v;
+}
+
+// kInline: at most kInlineTiles tiles; each workgroup adds up those of its level before its own, and one
+// more workgroup (the first, which the host waits for) does the totals meanwhile.
+template <bool kInline>
+__global__ __launch_bounds__(kTileThreads) void k_offsets(MArgs a, const u32* __restrict__ tile_sums,
+                                                          const ulonglong2* __restrict__ tile_pre, u32* __restrict__ meta, int R,
+                                                          u32* __restrict__ host_meta) {
+    if (kInline && blockIdx.x == 0) {
+        merge_totals<kTileThreads>(a, tile_sums, nullptr, meta, R, host_meta);
+        return;
+    }
+    const u32 b = kInline ? blockIdx.x - 1 : blockIdx.x;
+    const int k = level_of_tile(a, b);
     const MLevel& l = a.lv[k];
-    const u32 base = (blockIdx.x - a.tile0[k]) * kTileNodes + threadIdx.x;
-    const ulonglong2 pre = tile_pre[blockIdx.x], lev = tile_pre[a.tile0[a.nlev] + k];
-    const u32 rank0 = (u32)(pre.x - lev.x);
-    const u64 off0 = pre.y - lev.y;
-    u32 v[kTileRounds], ex[kTileRounds], id[kTileRounds];
-#pragma unroll
-    for (int j = 0; j < kTileRounds; ++j) {
-        const u32 i = base + j * kTileThreads;
-        const bool first = i < l.n && ((l.first[i / 64] >> (i & 63)) & 1ull);
-        v[j] = first ? 1u : 0u;
+    u32 i0;
+    const u64 v = tile_flags(l, b - a.tile0[k], i0);
+    u32 rank;
+    u64 off;
+    if constexpr (kInline) {
+        __shared__ u32 s_c[kTileThreads / kWave], s_w[kTileThreads / kWave];
+        u32 c = 0, w = 0;  // (1024 tiles of at most 34816 words fit 32 bits)
+        for (u32 t = a.tile0[k] + threadIdx.x; t < b; t += kTileThreads) {
+            const u32 x = tile_sums[t];
+            c += x >> 16;
+            w += x & 0xFFFFu;
+        }
+        rank = block_reduce(c, s_c, OpSum{});
+        off = block_reduce(w, s_w, OpSum{});
+    } else {
+        const ulonglong2 pre = tile_pre[b], lev = tile_pre[a.tile0[a.nlev] + k];
+        rank = (u32)(pre.x - lev.x);
+        off = pre.y - lev.y;
     }
+    u32 sum[1] = {0}, ex[1];
 #pragma unroll
-    for (int j = 0; j < kTileRounds; ++j) {
-        const u32 i = base + j * kTileThreads;
-        id[j] = (v[j] && !l.lone) ? l.id[i] : 0u;
-        if (v[j]) v[j] = (1u << 16) | node_words(l.mask[i], l.leaf);
+    for (u32 q = 0; q < kTilePer; ++q) {
+        const u32 w = (u32)(v >> (8 * q)) & 0xFFu;
+        sum[0] += w ? (1u << 16) | w : 0u;
     }
-    block_exclusive_scan_rounds<kTileRounds>(v, ex, OpSum{});
+    block_exclusive_scan_rounds<1>(sum, ex, OpSum{});
+    if (!v) return;
+    rank += ex[0] >> 16;
+    off += ex[0] & 0xFFFFu;
+    u32 id[kTilePer];
 #pragma unroll
-    for (int j = 0; j < kTileRounds; ++j) {
-        if (!v[j]) continue;
-        const u32 rank = rank0 + (ex[j] >> 16);
-        const u32 off = saturate32(off0 + (ex[j] & 0xFFFFu));
-        l.uniq[rank] = base + j * kTileThreads;
-        l.off[rank] = off;
-        if (!l.lone) l.tab[min(id[j], l.slots - 1)] = ((u64)rank << 32) | off;
+    for (u32 q = 0; q < kTilePer; ++q) id[q] = (((v >> (8 * q)) & 0xFFu) && !l.lone) ? l.id[i0 + q] : 0u;
+#pragma unroll
+    for (u32 q = 0; q < kTilePer; ++q) {
+        const u32 w = (u32)(v >> (8 * q)) & 0xFFu;
+        if (!w) continue;
+        const u32 o = saturate32(off);
+        l.uniq[rank] = i0 + q;
+        l.off[rank] = o;
+        if (!l.lone) l.tab[min(id[q], l.slots - 1)] = ((u64)rank << 32) | o;
+        ++rank;
+        off += w;
     }
 }
 
@@ -387,8 +491,56 @@ __global__ __launch_bounds__(kTileThreads) void k_offsets(MArgs a, const ulonglo
 // known on the device only, so no readback comes between): unique node r of an inner level as
 // [mask, absolute offsets of its partial children], of the leaf level as [mask, (lo, hi) of each
 // partial slice's leafmask] (src/CompressedShadow.cpp:326-392).
-__global__ __launch_bounds__(kNodeThreads) void k_write_words(MArgs a, const u32* __restrict__ meta, u32* __restrict__ out,
-                                                              u64 cap) {
+// The blocks from `writers` on make the compares that the late levels' inserts left out, one node a
+// thread, each with its slot's first occurrence.  An insert of a small level is one chain of reads and
+// atomics whatever its size, and the compare would make it longer; here it runs beside the write, and
+// the host takes its collisions with the end of the write (256^2 100 -> 94.5 us, 1024^2 147 -> 141).
+__device__ inline void compare_late(const MArgs& a, u32 block, u32* meta) {
+    int k = 0;
+    for (; k < a.nlev; ++k) {
+        if (!a.lv[k].late) continue;
+        const u32 nb = (a.lv[k].n + kNodeThreads - 1) / kNodeThreads;
+        if (block < nb) break;
+        block -= nb;
+    }
+    if (k == a.nlev) return;
+    const MLevel& l = a.lv[k];
+    const u32 i = block * kNodeThreads + threadIdx.x;
+    if (i >= l.n || (l.leaf && a.heads[i] != i)) return;
+    const u32 rank = (u32)(l.tab[min(l.id[i], l.slots - 1)] >> 32);  // (k_offsets' entry)
+    const u32 r = (rank < l.n) ? l.uniq[rank] : i;
+    if (r == i || r >= l.n) return;
+    const u32 m = l.mask[i], mr = l.mask[r];
+    bool same = m == mr;
+    if (l.leaf) {
+        const ulonglong2 *x = reinterpret_cast<const ulonglong2*>(a.leafm + (size_t)i * 8),
+                         *y = reinterpret_cast<const ulonglong2*>(a.leafm + (size_t)r * 8);
+        const u32 kk = same ? num_children(m) : 0u;
+#pragma unroll
+        for (u32 q = 0; q < 4; ++q)
+            if (2 * q < kk) same = same && x[q].x == y[q].x && (2 * q + 1 >= kk || x[q].y == y[q].y);
+    } else {
+        const int kc = a.child(k);
+        const ChildIds ch =
+            kc >= 0 ? ChildIds{a.lv[kc].id, a.lv[kc].leaf ? a.heads : nullptr, a.lv[kc].n} : ChildIds{nullptr, nullptr, 1u};
+        const u32 c = l.cstart[i], cr = l.cstart[r];
+        const u32 kk = (same && ch.id) ? num_children(m) : 0u;
+        if (kk) {
+            u32 x[8], y[8];
+            load_child_ids(ch, c, kk, x);
+            load_child_ids(ch, cr, kk, y);
+#pragma unroll
+            for (u32 q = 0; q < 8; ++q) same = same && x[q] == y[q];
+        }
+    }
+    if (!same) atomicAdd(meta + kMetaColl, 1u);
+}
+
+__global__ __launch_bounds__(kNodeThreads) void k_write_words(MArgs a, u32* meta, u32* __restrict__ out, u64 cap, u32 writers) {
+    if (blockIdx.x >= writers) {
+        compare_late(a, blockIdx.x - writers, meta);
+        return;
+    }
     __shared__ u32 s_first[kMaxLevels + 1], s_U[kMaxLevels], s_base[kMaxLevels];
     if (threadIdx.x < (u32)a.nlev) {
         s_U[threadIdx.x] = meta[kMetaU + a.lv[threadIdx.x].L];
@@ -407,7 +559,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_write_words(MArgs a, const u32
     const u32 total = meta[kMetaW];
     if (total >= 0xFFFFFFFEu || total > cap) return;  // the host reports it
     const u32 nb = s_first[a.nlev];
-    for (u32 vb = blockIdx.x; vb < nb; vb += gridDim.x) {
+    for (u32 vb = blockIdx.x; vb < nb; vb += writers) {
         int k = 0;
         while (k + 1 < a.nlev && vb >= s_first[k + 1]) ++k;
         const MLevel& l = a.lv[k];
@@ -438,7 +590,13 @@ __global__ __launch_bounds__(kNodeThreads) void k_write_words(MArgs a, const u32
         const u32 s = l.cstart[i];
         u32 id[8], co[8];
 #pragma unroll
-        for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? lc.id[min(s + j, lc.n - 1)] : 0u;
+        for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(s + j, lc.n - 1) : 0u;
+        if (lc.leaf && !a.sorted) {  // (children_of)
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(a.heads[id[j]], lc.n - 1) : 0u;
+        }
+#pragma unroll
+        for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? lc.id[id[j]] : 0u;
 #pragma unroll
         for (u32 j = 0; j < 8; ++j) co[j] = (j < kc) ? (u32)lc.tab[min(id[j], lc.slots - 1)] : 0u;
 #pragma unroll
@@ -451,7 +609,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_write_words(MArgs a, const u32
 
 static dim3 grid_of(u32 n, u32 block) { return dim3(ceil_div<u32>(n ? n : 1, block)); }
 
-// The children's identities of level k: those of the leaf level reach its non-heads here.
+// The children's identities of level k.
 static ChildIds children_of(const MArgs& a, int k, bool sorted) {
     const int c = a.child(k);
     if (c < 0) return ChildIds{nullptr, nullptr, 1u};
@@ -462,14 +620,17 @@ void merge_insert(const MArgs& a, int k, const u64* hash, u32* meta, u32 hbits, 
     const MLevel& l = a.lv[k];
     if (l.leaf && l.n <= kLeafOneMax)
         CPVS_LAUNCH("insert_leaf", k_insert_leaf<1>, grid_of(l.n, kLeafInsertThreads), dim3(kLeafInsertThreads), 0, s, l.mask,
-                    a.leafm, a.heads, hash, l.n, l.tab, l.slots, l.id, meta + kMetaFull, hbits);
+                    a.leafm, a.heads, hash, l.n, l.tab, l.slots, l.id, meta, hbits, l.late);
     else if (l.leaf)
         CPVS_LAUNCH("insert_leaf", k_insert_leaf<kLeafPer>, grid_of(l.n, kLeafPer * kLeafInsertThreads),
-                    dim3(kLeafInsertThreads), 0, s, l.mask, a.leafm, a.heads, hash, l.n, l.tab, l.slots, l.id,
-                    meta + kMetaFull, hbits);
+                    dim3(kLeafInsertThreads), 0, s, l.mask, a.leafm, a.heads, hash, l.n, l.tab, l.slots, l.id, meta,
+                    hbits, l.late);
+    else if (l.n >= kInnerTwoMin)
+        CPVS_LAUNCH("insert_inner", k_insert_inner<2>, grid_of(l.n, 2 * kInsertBlock), dim3(kInsertBlock), 0, s, l.mask,
+                    l.cstart, children_of(a, k, false), l.n, l.tab, l.slots, l.id, meta, hbits, l.late);
     else
-        CPVS_LAUNCH("insert_inner", k_insert_inner, grid_of(l.n, kInsertBlock), dim3(kInsertBlock), 0, s, l.mask, l.cstart,
-                    children_of(a, k, false), l.n, l.tab, l.slots, l.id, meta + kMetaFull, hbits);
+        CPVS_LAUNCH("insert_inner", k_insert_inner<1>, grid_of(l.n, kInsertBlock), dim3(kInsertBlock), 0, s, l.mask, l.cstart,
+                    children_of(a, k, false), l.n, l.tab, l.slots, l.id, meta, hbits, l.late);
 }
 
 void merge_sort_level(const MArgs& a, int k, const SortScratch& t, u32* meta, hipStream_t s) {
@@ -491,24 +652,29 @@ void merge_sort_level(const MArgs& a, int k, const SortScratch& t, u32* meta, hi
                     InnerEq{l.mask, l.cstart, ch.id, ch.n}, l.id, meta + kMetaSortColl);
 }
 
-void merge_finish(const MArgs& a, bool sorted, u32* tile_sums, ulonglong2* tile_pre, u32* meta, int R, u32* host_meta,
-                  hipStream_t s) {
+void merge_finish(const MArgs& a, u32* tile_sums, ulonglong2* tile_pre, u32* meta, int R, u32* host_meta, hipStream_t s) {
     const u32 nt = a.tile0[a.nlev];
-    if (sorted)
-        CPVS_LAUNCH("resolve", k_resolve<true>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums, tile_pre, meta, R,
-                    host_meta);
+    if (a.sorted)
+        CPVS_LAUNCH("firsts", k_firsts<true>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums);
     else
-        CPVS_LAUNCH("resolve", k_resolve<false>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums, tile_pre, meta, R,
+        CPVS_LAUNCH("firsts", k_firsts<false>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums);
+    if (nt <= kInlineTiles) {
+        CPVS_LAUNCH("offsets", k_offsets<true>, dim3(nt + 1), dim3(kTileThreads), 0, s, a, tile_sums, nullptr, meta, R,
                     host_meta);
-    if (nt > kInlineTiles)
-        CPVS_LAUNCH("totals", k_totals, dim3(1), dim3(kTotalsThreads), 0, s, a, tile_sums, tile_pre, meta, R, host_meta);
-    CPVS_LAUNCH("offsets", k_offsets, dim3(nt), dim3(kTileThreads), 0, s, a, tile_pre);
+        return;
+    }
+    CPVS_LAUNCH("totals", k_totals, dim3(1), dim3(kTotalsThreads), 0, s, a, tile_sums, tile_pre, meta, R, host_meta);
+    CPVS_LAUNCH("offsets", k_offsets<false>, dim3(nt), dim3(kTileThreads), 0, s, a, tile_sums, tile_pre, nullptr, R, nullptr);
 }
 
-void merge_write(const MArgs& a, const u32* meta, u32* out, u64 cap, hipStream_t s) {
-    u32 most = 0;  // blocks of the largest possible write (every node unique)
-    for (int k = 0; k < a.nlev; ++k) most += ceil_div<u32>(a.lv[k].n, kNodeThreads);
-    CPVS_LAUNCH("write_words", k_write_words, dim3(most < 2048 ? most : 2048), dim3(kNodeThreads), 0, s, a, meta, out, cap);
+void merge_write(const MArgs& a, u32* meta, u32* out, u64 cap, hipStream_t s) {
+    u32 most = 0, compares = 0;  // blocks of the largest possible write (every node unique), and of compare_late
+    for (int k = 0; k < a.nlev; ++k) {
+        most += ceil_div<u32>(a.lv[k].n, kNodeThreads);
+        if (a.lv[k].late) compares += ceil_div<u32>(a.lv[k].n, kNodeThreads);
+    }
+    const u32 writers = most < 2048 ? most : 2048;
+    CPVS_LAUNCH("write_words", k_write_words, dim3(writers + compares), dim3(kNodeThreads), 0, s, a, meta, out, cap, writers);
 }
 
 }  // namespace cpvs
