@@ -78,8 +78,9 @@ __global__ __launch_bounds__(256) void k_classify(const u64* __restrict__ coord,
 // 17 -> 9 us with one column per wave instead of 8.
 // Workgroups are dealt to the XCDs in turn (block b to XCD b mod kXcds), each XCD with its own L2.
 // XCD x takes the contiguous units [x*chunk, (x+1)*chunk): neighbouring columns, whose 8-texel depth
-// rows share 128-byte lines, are then read through one L2.  A list fills only its first units, so
-// there consecutive units go to different XCDs.
+// rows share 128-byte lines, are then read through one L2.  Of a list each XCD takes a contiguous
+// eighth (list_share) where a wave takes one column; k_leaf_lanes' list (of a z-tile) fills only its
+// first workgroups, 256 columns each, so there consecutive ones go to different XCDs.
 // ---------------------------------------------------------------------------------------
 __device__ inline LeafCol map_column(const LeafColumns& lc, const float* depth, u32 N, float HT, u32 col) {
     const uint4 ci = lc.info[col];
@@ -95,11 +96,12 @@ __global__ __launch_bounds__(64) void k_leaf_waves(LeafColumns lc, u32 ncol, con
                                                    u64* __restrict__ tab, u32 tab_slots,
                                                    const u32* __restrict__ col_list, const u32* __restrict__ n_list) {
     __shared__ uint8_t s_chg[128];
-    const u32 n = kList ? min(*n_list, ncol) : ncol;
-    for (u32 u = kList ? blockIdx.x : (blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds; u < n; u += gridDim.x) {
+    const u32 b = blockIdx.x;
+    const ListShare share = kList ? list_share(min(*n_list, ncol), b, gridDim.x)
+                                  : ListShare{(b % kXcds) * chunk + b / kXcds, ncol, ncol};
+    for (u32 u = share.u0; u < share.end; u += share.step) {
         const LeafCol c = map_column(lc, depth, N, (float)(N * T), kList ? col_list[u] : u);
         if (c.cnt) leaf_wave(c, lv3 + (size_t)even_bits(c.col >> 1) * lc.w3 + even_bits(c.col), o, s_chg, threadIdx.x);
-        if (!kList) break;
     }
     clear_table(tab, tab_slots);  // after all the work: stores issued earlier would be waited for with the loads
 }
@@ -622,10 +624,10 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
                     CPVS_LAUNCH("leaf_lanes", k_leaf_lanes<false>, dim3(chunk * kXcds), dim3(kLaneThreads), 0, s, lc, bound,
                                 p->depth, N, T, lo, chunk, tab, slots, nullptr, nullptr);
                 const u32 most = std::min(bound, c);
-                CPVS_LAUNCH("leaf_waves", k_leaf_waves<true>, dim3(std::min(most, kSlowWaves)), dim3(64), 0, s, lc, most,
+                CPVS_LAUNCH("leaf_waves", k_leaf_waves<true>, dim3(list_waves(most)), dim3(64), 0, s, lc, most,
                             p->depth, N, T, p->lv[3], lo, 0u, tab, 0u, lv[2].id, meta + kMetaSlow);
             } else if (col_list) {
-                CPVS_LAUNCH("leaf_waves", k_leaf_waves<true>, dim3(std::min(bound, kSlowWaves)), dim3(64), 0, s, lc, bound,
+                CPVS_LAUNCH("leaf_waves", k_leaf_waves<true>, dim3(list_waves(bound)), dim3(64), 0, s, lc, bound,
                             p->depth, N, T, p->lv[3], lo, 0u, tab, slots, clist, nclist);
             } else {
                 const u32 chunk = ceil_div<u32>(bound, kXcds);

@@ -490,6 +490,18 @@ __device__ inline void leaf_wave(const LeafCol& c, const float2* ext, const Leaf
     leaf_column(f, fmin, fmax, c.zs, c.cnt, b, o.bfs + c.start, c.gtag, o.nleaf, fl, lane, o.mask, o.leafm, o.runhead, o.hash);
 }
 
+// The entries of a list of n columns that workgroup b of g takes: u0, u0 + step, ... below end.  XCD x
+// (workgroups x, x + kXcds, ...) takes a contiguous range: a 2 x 2 group's columns follow one another
+// in the list, and their nodes one another in breadth-first order, so their run heads share lines,
+// which one L2 then writes once (8192^2: 47 -> 35 us, 8 z-tiles 27 -> 19 us each; the walks wrote 110 MB).  g is a multiple of kXcds.
+struct ListShare {
+    u32 u0, end, step;
+};
+__device__ inline ListShare list_share(u32 n, u32 b, u32 g) {
+    const u32 chunk = (n + kXcds - 1) / kXcds, x = b % kXcds;
+    return ListShare{x * chunk + b / kXcds, min(n, (x + 1) * chunk), g / kXcds};
+}
+
 // The lanes' columns, those set aside appended to the list (one atomic per wave).
 __device__ inline void leaf_lanes(const LeafCol& c, const LeafOut& o) {
     const bool slow = !leaf_lane(c, o);
@@ -716,6 +728,7 @@ enum : int {
 // Launches over this many columns walk them one per lane (a map's are then at least 16 x 16).
 constexpr u64 kLaneLeafMin = 1u << 15;
 constexpr u32 kSlowWaves = 8192;  // waves that stride over a list of columns: the chip's 32 per CU
+inline u32 list_waves(u32 most) { return most < kSlowWaves ? (most + kXcds - 1) / kXcds * kXcds : kSlowWaves; }
 
 // Slots for n keys, at most two thirds full.
 inline u32 table_slots(u32 n) {

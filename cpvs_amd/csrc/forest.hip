@@ -244,8 +244,8 @@ __global__ __launch_bounds__(64) void k_forest_waves(const uint4* __restrict__ c
                                                      const u32* __restrict__ col_list, const u32* __restrict__ n_list,
                                                      u32 list_cap) {
     __shared__ uint8_t s_chg[128];
-    const u32 n = min(*n_list, list_cap);
-    for (u32 u = blockIdx.x; u < n; u += gridDim.x) {
+    const ListShare share = list_share(min(*n_list, list_cap), blockIdx.x, gridDim.x);
+    for (u32 u = share.u0; u < share.end; u += share.step) {
         const float2* ext;
         const LeafCol c = forest_column(colinfo, items, col_list[u], &ext);
         if (c.cnt) leaf_wave(c, ext, o, s_chg, threadIdx.x);
@@ -665,7 +665,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
             // At most min(columns, leaf nodes) columns are listed.  The first kernel clears the tables.
             const u32 bound = (u32)std::min<u64>(ncol, C[2]), clear = use_table ? (u32)tab_slots : 0u;
             const LeafOut lo{colbfs, lv.mask[2], leafm, runhead, leaf_hash, lv.id[2], meta + kMetaSlow, (u32)C[2]};
-            const dim3 waves(std::min(bound, kSlowWaves));
+            const dim3 waves(list_waves(bound));
             if (leaf_hash) {
                 CPVS_LAUNCH("forest_lanes", k_forest_lanes, grid_of(bound, kLaneThreads), dim3(kLaneThreads), 0, s, colinfo,
                             items, lo, tab, clear, clist, nclist, bound);
