@@ -30,6 +30,17 @@ __device__ inline u32 fmix32(u32 h) {
 // ---------------------------------------------------------------------------------------
 // 1. Inner classification: createChildmask (src/CompressedShadowUtil.cpp:20-54).
 // ---------------------------------------------------------------------------------------
+// The childmask of the node at level-L cell z from its 2 x 2 texels' rows a and b (L > 0).
+__device__ inline u32 classify_texels(u32 z, float h, float4 a, float4 b) {
+    const float mn[4] = {a.x, a.z, b.x, b.z}, mx[4] = {a.y, a.w, b.y, b.w};  // texel (x + (q&1), y + (q>>1))
+    u32 mask = 0;
+#pragma unroll
+    for (u32 ch = 0; ch < 8; ++ch) {
+        const u32 q = ch & 3;
+        mask |= classify_cell(z + (ch >> 2), mn[q] * h, mx[q] * h) << (2 * ch);
+    }
+    return mask;
+}
 // The cell is clamped into the level: a node past a level's emitted children (counts that
 // exceed them, which the host then reports) still reads inside the pyramid.
 __device__ inline u32 classify_node(u64 c, const float2* __restrict__ lv, const float* __restrict__ depth, u32 N, int L,
@@ -37,30 +48,17 @@ __device__ inline u32 classify_node(u64 c, const float2* __restrict__ lv, const 
     const u32 w = N >> L;
     const u32 x = min(unpack_x(c), w - 2) & ~1u, y = min(unpack_y(c), w - 2), z = unpack_z(c);
     const float h = (float)((N >> L) * T);
-    float mn[4], mx[4];  // texel (x + (q&1), y + (q>>1))
-    if (L > 0) {
-        const float4 a = *reinterpret_cast<const float4*>(lv + (size_t)y * w + x);
-        const float4 b = *reinterpret_cast<const float4*>(lv + (size_t)(y + 1) * w + x);
-        mn[0] = a.x; mx[0] = a.y; mn[1] = a.z; mx[1] = a.w;
-        mn[2] = b.x; mx[2] = b.y; mn[3] = b.z; mx[3] = b.w;
-    } else {
-        const float2 a = *reinterpret_cast<const float2*>(depth + (size_t)y * N + x);
-        const float2 b = *reinterpret_cast<const float2*>(depth + (size_t)(y + 1) * N + x);
-        mn[0] = mx[0] = a.x; mn[1] = mx[1] = a.y;
-        mn[2] = mx[2] = b.x; mn[3] = mx[3] = b.y;
-    }
+    if (L > 0)
+        return classify_texels(z, h, *reinterpret_cast<const float4*>(lv + (size_t)y * w + x),
+                               *reinterpret_cast<const float4*>(lv + (size_t)(y + 1) * w + x));
+    const float2 a = *reinterpret_cast<const float2*>(depth + (size_t)y * N + x);
+    const float2 b = *reinterpret_cast<const float2*>(depth + (size_t)(y + 1) * N + x);
+    const float d[4] = {a.x, a.y, b.x, b.y};
     u32 mask = 0;
 #pragma unroll
-    for (u32 ch = 0; ch < 8; ++ch) {
-        const u32 q = ch & 3, cz = z + (ch >> 2);
-        u32 bits;
-        if (L > 0) bits = classify_cell(cz, mn[q] * h, mx[q] * h);
-        else bits = classify_mid(cz, mn[q] * h);
-        mask |= bits << (2 * ch);
-    }
+    for (u32 ch = 0; ch < 8; ++ch) mask |= classify_mid(z + (ch >> 2), d[ch & 3] * h) << (2 * ch);
     return mask;
 }
-
 
 // Leaf columns: per level-3 texel, in Morton order, one record {partial cells, first leaf's index in
 // column order, first partial z cell, 0}, so a column's scalars come in one load and a node's four
@@ -173,8 +171,8 @@ struct EmitChildrenOut {
 #pragma unroll
         for (u32 ch = 0; ch < 8; ++ch) {
             if (!(m & (2u << (2 * ch)))) continue;
-            const u32 cx = x + (ch & 1), cy = y + ((ch >> 1) & 1), cz = z + (ch >> 2);
-            if (j < child_cap) child_coord[j] = pack_xyz(2 * cx, 2 * cy, 2 * cz);
+            // pack_xyz of the doubled child cell (no field of a node with children is near its width)
+            if (j < child_cap) child_coord[j] = 2 * c + pack_xyz(2 * (ch & 1), 2 * ((ch >> 1) & 1), 2 * (ch >> 2));
             ++j;
         }
     }
