@@ -67,9 +67,10 @@ __device__ inline u64 xcd_query(u32 chunk) {
     return (u64)((blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds) * blockDim.x + threadIdx.x;
 }
 
-// Threads per workgroup of the flat and PCF lookups (measured on 16.6 M G-buffer queries: 64, 128,
+// Threads per workgroup of the flat lookups (measured on 16.6 M G-buffer queries: 64, 128,
 // 256, 512 and 1024 threads took 0.301, 0.297, 0.289, 0.277 and 0.276 ms walking every level; with
-// the 7-level top table, 512 and 1024 threads take 0.159 and 0.150 ms).
+// the 7-level top table, 512 and 1024 threads take 0.159 and 0.150 ms; with links and 6 levels 256, 512
+// and 1024 take 0.135, 0.132 and 0.123 ms, 4.2 M random queries over 64 DAGs 43.0, 41.5 and 40.6 us).
 constexpr u32 kLookupThreads = 1024;
 
 // traverse.cs:43-48: path = int(((ndc + 1) * 0.5) * float(R - 1)), clamped to [0, R-1]
@@ -401,7 +402,11 @@ __device__ inline u32 walk_slice(const GridDag& g, u32 px, u32 py, u32 pz, u64& 
     return 1u;
 }
 
-__global__ __launch_bounds__(kLookupThreads) void k_evaluate_pcf(GridDag g, Mat4 M, const float* __restrict__ pos, u32 stride,
+// Lanes whose windows cross blocks take up to four walks where others take one, and a workgroup keeps
+// its place until its last wave ends: 1024, 512 and 256 threads take 37.7, 31.4 and 29.2 us (3 x 3 over
+// 1920 x 1080 points; 128 and 64 as 256).
+constexpr u32 kPcfThreads = 256;
+__global__ __launch_bounds__(kPcfThreads) void k_evaluate_pcf(GridDag g, Mat4 M, const float* __restrict__ pos, u32 stride,
                                                       u64 count, u32 f, float* __restrict__ vis, u32 chunk) {
     const u64 i = xcd_query(chunk);
     if (i >= count) return;
@@ -440,13 +445,13 @@ int launch_evaluate_pcf(const u32* dag, const u64* links, u32 words, const u32* 
                         const float* pos, u32 stride, u64 count, const Mat4& m, u32 f, float* vis, hipStream_t s) {
     if (count == 0) return CPVS_OK;
     const GridDag g = grid_dag(dag, links, words, grid, dl, gl, leaf, top, topk, m);
-    const u64 blocks = (count + kLookupThreads - 1) / kLookupThreads;
+    const u64 blocks = (count + kPcfThreads - 1) / kPcfThreads;
     if (blocks > 0x7FFFFFF0ull) {
         set_error("evaluate_pcf: %llu points exceed one launch", (unsigned long long)count);
         return CPVS_EINVAL;
     }
     const u32 chunk = (u32)((blocks + kXcds - 1) / kXcds);
-    CPVS_LAUNCH("evaluate_pcf", k_evaluate_pcf, dim3(chunk * kXcds), dim3(kLookupThreads), 0, s, g, m, pos, stride, count, f, vis, chunk);
+    CPVS_LAUNCH("evaluate_pcf", k_evaluate_pcf, dim3(chunk * kXcds), dim3(kPcfThreads), 0, s, g, m, pos, stride, count, f, vis, chunk);
     CPVS_HIP_CHECK(hipGetLastError());
     return CPVS_OK;
 }
