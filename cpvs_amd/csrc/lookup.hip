@@ -637,7 +637,9 @@ __global__ __launch_bounds__(256) void k_dagset_eval(const DagDesc* __restrict__
 // ranges of equal length, so each XCD's L2 holds the upper levels of its own DAGs only and every
 // XCD has the same work whatever the number of groups (6.3 M lookups over 48 DAGs, three groups:
 // 222 -> 78 us against whole groups per XCD, which left five XCDs idle).
-constexpr u32 kRRGroup = 16;
+// Groups of 16, 8 and 4 DAGs: 69.8, 65.5 and 72.1 us: a workgroup waits for its longest walks, but a
+// row of fewer points shares its lines with other workgroups.
+constexpr u32 kRRGroup = 8;
 
 __global__ __launch_bounds__(64 * kRRGroup) void k_dagset_eval_rr(const DagDesc* __restrict__ set, u32 nset, u32 tiles,
                                                                u32 chunk, u32 kblocks, const float* __restrict__ ndc,
