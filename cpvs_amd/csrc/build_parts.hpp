@@ -656,17 +656,8 @@ __device__ inline u32 table_insert(u64* tab, u32 S, u64 h, u32 i, u32* full, u32
     return slot;
 }
 
-// The leaf level: only a run's first node is inserted (1.3 M of 6.7 M nodes at 8192^2), so each
-// thread takes kLeafPer nodes and a workgroup merges a window of kLeafPer * kLeafInsertThreads nodes
-// in LDS.  The window's distinct hashes are listed as they are found, and the list is spread over
-// the threads for the global inserts: a workgroup waits for about one global insert per thread, not
-// per node.  A small level would leave most of the chip idle and wait for four inserts in turn, so
-// up to kLeafOneMax nodes a thread takes one (2215 nodes of a 256^2 map: 17 -> 9 us).
 constexpr u32 kLeafInsertThreads = 256;
-constexpr u32 kLeafPer = 4;
-constexpr u32 kLeafOneMax = 1u << 18;
-// Inner levels of this many nodes take two a thread.
-constexpr u32 kInnerTwoMin = 1u << 20;
+constexpr u32 kInnerTwoMin = 1u << 20, kInnerSmallMax = 1u << 18;
 
 // Threads per workgroup of the write kernels (at 8192^2, 128 and 256 tie; 512 and 1024 are slower).
 constexpr u32 kNodeThreads = 256;

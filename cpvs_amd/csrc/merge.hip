@@ -34,60 +34,47 @@ __global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 
     if (i < S) tab[i] = kEmptySlot;
 }
 
-// The run heads of a window of kPer * kT nodes are listed in LDS; equal hashes meet in an LDS table,
+// The run heads of a window of kT nodes are listed in LDS; equal hashes meet in an LDS table,
 // the distinct ones are spread over the threads for the global inserts, and every head's key is then
 // compared with its window's first of that hash, that one's with the global slot's earlier node.  The
 // compares take four lanes to a pair of leafmask rows (16 bytes a lane): one lane to a row would touch
 // 64 lines with each load.  The rows are what the compares cost (83 MB at 8192^2: 57 -> 98 us).
 // What bounds it besides: the tables' atomics and coherent reads, performed at memory, about 7 G atomics/s.
-// (Windows of 4096 nodes, for fewer of them: 148 us, the dense windows' batches one after another.)
-template <u32 kPer>
+// One node a thread: where heads lie dense, a thread with several walks their reads and atomics one
+// after another (4 a thread 99 us, 16 a thread 148 us at 8192^2, one 77; 30, 18 at 2048^2).  Windows of
+// 512 and 1024 meet fewer equal hashes than they lose to workgroups waiting: 32 maps 227, 248, 287 us.
 __global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* __restrict__ mask, const u64* __restrict__ leafm,
                                                                     const u32* __restrict__ runhead,
                                                                     const u64* __restrict__ hash, u32 n,
                                                                     u64* __restrict__ tab, u32 S, u32* __restrict__ tslot,
                                                                     u32* __restrict__ meta, u32 hbits, u32 late) {
-    constexpr u32 kT = kLeafInsertThreads, kWindow = kPer * kT, kSlots = 2 * kWindow;  // at most half full: every probe ends
+    constexpr u32 kT = kLeafInsertThreads, kSlots = 2 * kT;  // at most half full: every probe ends
     __shared__ u64 gh[kSlots];  // a hash, then its global slot << 32 | the node that the slot held before
     __shared__ u32 gi[kSlots];  // smallest node index of the slot's hash
-    __shared__ unsigned short glist[kWindow];  // LDS slots in use
-    __shared__ unsigned short heads[kWindow], hslot[kWindow];  // the window's run heads and their LDS slots
+    __shared__ unsigned short glist[kT];  // LDS slots in use
+    __shared__ unsigned short heads[kT], hslot[kT];  // the window's run heads and their LDS slots
     __shared__ u32 gcount, nheads;
-    const u32 t = threadIdx.x, lane = t & (kWave - 1), i0 = blockIdx.x * kWindow;
+    const u32 t = threadIdx.x, lane = t & (kWave - 1), i0 = blockIdx.x * kT;
     if (t == 0) gcount = nheads = 0;
-    u32 rh[kPer];
-#pragma unroll
-    for (u32 k = 0; k < kPer; ++k) {
-        const u32 i = i0 + k * kT + t;
-        rh[k] = (i < n) ? runhead[i] : kNoRep;
-    }
+    const bool head = i0 + t < n && runhead[i0 + t] == i0 + t;
     for (u32 j = t; j < kSlots; j += kT) {
         gh[j] = 0ull;  // 0 marks an empty LDS slot
         gi[j] = kNoRep;
     }
     __syncthreads();
     {
-        u64 bits[kPer];
-        u32 total = 0, at = 0;
-#pragma unroll
-        for (u32 k = 0; k < kPer; ++k) {
-            bits[k] = __ballot(rh[k] == i0 + k * kT + t);  // (never past n)
-            total += (u32)__popcll(bits[k]);
-        }
-        if (lane == 0 && total) at = atomicAdd(&nheads, total);
+        const u64 bits = __ballot(head);
+        u32 at = 0;
+        if (lane == 0 && bits) at = atomicAdd(&nheads, (u32)__popcll(bits));
         at = __builtin_amdgcn_readfirstlane(at);
-#pragma unroll
-        for (u32 k = 0; k < kPer; ++k) {
-            if ((bits[k] >> lane) & 1ull) heads[at + (u32)__popcll(bits[k] & ((1ull << lane) - 1ull))] = (unsigned short)(k * kT + t);
-            at += (u32)__popcll(bits[k]);
-        }
+        if (head) heads[at + (u32)__popcll(bits & ((1ull << lane) - 1ull))] = (unsigned short)t;
     }
     __syncthreads();
     const u32 nh = nheads;
-    for (u32 j = t; j < nh; j += kT) {
+    if (t < nh) {
         // The key hash of a run's first node (the run's smallest index): from the leaf kernel where a
         // lane walked its column, else from its mask and leafmasks (its row at its own index).
-        const u32 i = i0 + heads[j];
+        const u32 i = i0 + heads[t];
         u64 h = hash ? hash[i] : 0ull;
         if (h == 0ull) h = leaf_key_hash(mask[i], leafm + (size_t)i * 8);
         h = weaken_hash(h, hbits);
@@ -103,19 +90,18 @@ __global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* _
             sl = (sl + 1) & (kSlots - 1);
         }
         atomicMin(gi + sl, i);
-        hslot[j] = (unsigned short)sl;
+        hslot[t] = (unsigned short)sl;
     }
     __syncthreads();
-    const u32 m = gcount;  // at most kWindow
-    for (u32 j = t; j < m; j += kT) {
-        const u32 sl = glist[j];
+    if (t < gcount) {
+        const u32 sl = glist[t];
         u32 occ;
         const u32 slot = table_insert(tab, S, gh[sl], gi[sl], meta + kMetaFull, occ);
         gh[sl] = ((u64)slot << 32) | occ;
     }
     __syncthreads();
     bool eq = true;
-    for (u32 j = t; j < nh; j += kT) tslot[i0 + heads[j]] = (u32)(gh[hslot[j]] >> 32);
+    if (t < nh) tslot[i0 + heads[t]] = (u32)(gh[hslot[t]] >> 32);
     for (u32 j = t / 4; j < nh && !late; j += kT / 4) {
         const u32 i = i0 + heads[j], sl = hslot[j], rep = gi[sl];
         const u32 with = (rep != i) ? rep : (u32)gh[sl];
@@ -137,15 +123,14 @@ __global__ __launch_bounds__(kLeafInsertThreads) void k_insert_leaf(const u32* _
 // runs almost all at once, before any first occurrence has landed).  So each workgroup first merges
 // its own equal hashes in an LDS table, with the keys beside it for the compares: only the smallest
 // index of each distinct hash in the group touches the global table, and the others take its slot.
-// Threads per workgroup (the window): at 8192^2, 512 took the inner inserts 0.142 -> 0.136 ms against
-// 256; 1024 gained nothing more.
-constexpr u32 kInsertBlock = 512;
-
-template <u32 kPer>
-__global__ __launch_bounds__(kInsertBlock) void k_insert_inner(const u32* __restrict__ mask, const u32* __restrict__ cstart,
-                                                               ChildIds ch, u32 n, u64* __restrict__ tab, u32 S,
-                                                               u32* __restrict__ id, u32* __restrict__ meta, u32 hbits, u32 late) {
-    constexpr u32 kT = kInsertBlock, kSlots = 2 * kPer * kT;
+// The window: levels up to kInnerSmallMax nodes are one chain of reads and atomics for each workgroup,
+// shorter in small ones (256 threads against 512: 7.6-10 us against 8.4-10.5); above, larger windows meet
+// more equal keys (32 maps, 6.4 M nodes: 256 nodes 169 us, 512 165, two a thread 155).
+template <u32 kPer, u32 kT>
+__global__ __launch_bounds__(kT) void k_insert_inner(const u32* __restrict__ mask, const u32* __restrict__ cstart, ChildIds ch,
+                                                     u32 n, u64* __restrict__ tab, u32 S, u32* __restrict__ id,
+                                                     u32* __restrict__ meta, u32 hbits, u32 late) {
+    constexpr u32 kSlots = 2 * kPer * kT;
     __shared__ u64 gh[kSlots];
     __shared__ u32 gi[kSlots];  // smallest node index of the slot's hash, then its global slot
     const u32 t = threadIdx.x, i0 = blockIdx.x * (kPer * kT) + t;
@@ -618,18 +603,17 @@ static ChildIds children_of(const MArgs& a, int k, bool sorted) {
 
 void merge_insert(const MArgs& a, int k, const u64* hash, u32* meta, u32 hbits, hipStream_t s) {
     const MLevel& l = a.lv[k];
-    if (l.leaf && l.n <= kLeafOneMax)
-        CPVS_LAUNCH("insert_leaf", k_insert_leaf<1>, grid_of(l.n, kLeafInsertThreads), dim3(kLeafInsertThreads), 0, s, l.mask,
+    if (l.leaf)
+        CPVS_LAUNCH("insert_leaf", k_insert_leaf, grid_of(l.n, kLeafInsertThreads), dim3(kLeafInsertThreads), 0, s, l.mask,
                     a.leafm, a.heads, hash, l.n, l.tab, l.slots, l.id, meta, hbits, l.late);
-    else if (l.leaf)
-        CPVS_LAUNCH("insert_leaf", k_insert_leaf<kLeafPer>, grid_of(l.n, kLeafPer * kLeafInsertThreads),
-                    dim3(kLeafInsertThreads), 0, s, l.mask, a.leafm, a.heads, hash, l.n, l.tab, l.slots, l.id, meta,
-                    hbits, l.late);
     else if (l.n >= kInnerTwoMin)
-        CPVS_LAUNCH("insert_inner", k_insert_inner<2>, grid_of(l.n, 2 * kInsertBlock), dim3(kInsertBlock), 0, s, l.mask,
-                    l.cstart, children_of(a, k, false), l.n, l.tab, l.slots, l.id, meta, hbits, l.late);
+        CPVS_LAUNCH("insert_inner", (k_insert_inner<2, 512>), grid_of(l.n, 1024), dim3(512), 0, s, l.mask, l.cstart,
+                    children_of(a, k, false), l.n, l.tab, l.slots, l.id, meta, hbits, l.late);
+    else if (l.n > kInnerSmallMax)
+        CPVS_LAUNCH("insert_inner", (k_insert_inner<1, 512>), grid_of(l.n, 512), dim3(512), 0, s, l.mask, l.cstart,
+                    children_of(a, k, false), l.n, l.tab, l.slots, l.id, meta, hbits, l.late);
     else
-        CPVS_LAUNCH("insert_inner", k_insert_inner<1>, grid_of(l.n, kInsertBlock), dim3(kInsertBlock), 0, s, l.mask, l.cstart,
+        CPVS_LAUNCH("insert_inner", (k_insert_inner<1, 256>), grid_of(l.n, 256), dim3(256), 0, s, l.mask, l.cstart,
                     children_of(a, k, false), l.n, l.tab, l.slots, l.id, meta, hbits, l.late);
 }
 
