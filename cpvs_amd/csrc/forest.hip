@@ -333,48 +333,51 @@ __global__ __launch_bounds__(kNodeThreads) void k_forest_write(FWriteArgs a, FLe
                                                                 const u32* __restrict__ heads,
                                                                 const u32* __restrict__ base_off, const u32* __restrict__ B,
                                                                 u32* const* __restrict__ outp) {
+    __shared__ u32 s_out[kStageWords];
     int k = 0;
     while (k + 1 < a.nlev && blockIdx.x >= a.first[k + 1]) ++k;
     const int L = a.level[k];
-    const u32 r = (blockIdx.x - a.first[k]) * blockDim.x + threadIdx.x;
-    if (r >= a.U[k]) return;
-    const u32 i = lv.uniq[L][r];
-    const u32 m = lv.mask[L][i];
-    const u32 g = m >> 16;
-    const size_t gk = (size_t)g * kKL + L;
-    const u32 o = B[gk] + (lv.off[L][r] - base_off[gk]);
-    u32* out = outp[g];
-    out[o] = m & 0xFFFFu;
-    const u32 kc = num_children(m);
-    if (!kc) return;
-    if (L == 2) {
-        const u64* p = leafm + (size_t)i * 8;  // a first occurrence heads its run: its own row
-        u64 v[8];
+    const u32 r0 = (blockIdx.x - a.first[k]) * kNodeThreads, r1 = min(r0 + kNodeThreads, a.U[k]) - 1, r = r0 + threadIdx.x;
+    // Ranks are DAG-major: the nodes are one DAG's if the first and the last are.
+    const u32 g0 = lv.mask[L][lv.uniq[L][r0]] >> 16, g1 = lv.mask[L][lv.uniq[L][r1]] >> 16;
+    u32 o = 0, n = 0, g = g0, w[17];
+    if (r <= r1) {
+        const u32 i = lv.uniq[L][r];
+        const u32 m = lv.mask[L][i];
+        o = lv.off[L][r];
+        g = m >> 16;
+        w[0] = m & 0xFFFFu;
+        const u32 kc = num_children(m);
+        n = 1 + (kc << (L == 2 ? 1 : 0));
+        if (L == 2) {
+            leaf_row(leafm + (size_t)i * 8, kc, w + 1);  // a first occurrence heads its run: its own row
+        } else if (kc) {
+            const size_t gk = (size_t)g * kKL + L;
+            const u32 cb = B[gk - 1] - base_off[gk - 1], s = lv.cstart[L][i];
+            u32 id[8];
 #pragma unroll
-        for (u32 j = 0; j < 8; ++j) v[j] = (j < kc) ? p[j] : 0ull;
+            for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(s + j, lv.count[L - 1] - 1) : 0u;
+            if (L == 3 && heads) {  // a leaf's identity is its run's first node's (table merge)
 #pragma unroll
-        for (u32 j = 0; j < 8; ++j)
-            if (j < kc) {
-                out[o + 1 + 2 * j] = (u32)v[j];
-                out[o + 2 + 2 * j] = (u32)(v[j] >> 32);
+                for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(heads[id[j]], lv.count[2] - 1) : 0u;
             }
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? lv.id[L - 1][id[j]] : 0u;
+#pragma unroll
+            for (u32 j = 0; j < 8; ++j) w[1 + j] = (j < kc) ? cb + (u32)lv.tab[L - 1][min(id[j], lv.slots[L - 1] - 1)] : 0u;
+        }
+    }
+    const size_t gk = (size_t)g * kKL + L;
+    if (g0 == g1) {  // (workgroup-uniform)
+        // out: where the level's offset 0 would lie
+        stage_words(s_out, lv.off[L][r0], o, n, w, outp[g0] + (ptrdiff_t)B[gk] - (ptrdiff_t)base_off[gk], 0xFFFFFFFFu);
         return;
     }
-    const u32 cb = B[gk - 1], co0 = base_off[gk - 1], s = lv.cstart[L][i];
-    u32 id[8], co[8];
+    if (!n) return;
+    u32* out = outp[g] + B[gk] + (o - base_off[gk]);
 #pragma unroll
-    for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(s + j, lv.count[L - 1] - 1) : 0u;
-    if (L == 3 && heads) {  // a leaf's identity is its run's first node's (table merge)
-#pragma unroll
-        for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(heads[id[j]], lv.count[2] - 1) : 0u;
-    }
-#pragma unroll
-    for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? lv.id[L - 1][id[j]] : 0u;
-#pragma unroll
-    for (u32 j = 0; j < 8; ++j) co[j] = (j < kc) ? (u32)lv.tab[L - 1][min(id[j], lv.slots[L - 1] - 1)] : 0u;
-#pragma unroll
-    for (u32 j = 0; j < 8; ++j)
-        if (j < kc) out[o + 1 + j] = cb + (co[j] - co0);
+    for (u32 j = 0; j < 17; ++j)
+        if (j < n) out[j] = w[j];
 }
 
 // ---------------------------------------------------------------------------------------

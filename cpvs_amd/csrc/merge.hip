@@ -526,7 +526,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_write_words(MArgs a, u32* meta
         compare_late(a, blockIdx.x - writers, meta);
         return;
     }
-    __shared__ u32 s_first[kMaxLevels + 1], s_U[kMaxLevels], s_base[kMaxLevels];
+    __shared__ u32 s_first[kMaxLevels + 1], s_U[kMaxLevels], s_base[kMaxLevels], s_out[kStageWords];
     if (threadIdx.x < (u32)a.nlev) {
         s_U[threadIdx.x] = meta[kMetaU + a.lv[threadIdx.x].L];
         s_base[threadIdx.x] = meta[kMetaB + a.lv[threadIdx.x].L];
@@ -548,45 +548,35 @@ __global__ __launch_bounds__(kNodeThreads) void k_write_words(MArgs a, u32* meta
         int k = 0;
         while (k + 1 < a.nlev && vb >= s_first[k + 1]) ++k;
         const MLevel& l = a.lv[k];
-        const u32 r = (vb - s_first[k]) * blockDim.x + threadIdx.x;
-        if (r >= s_U[k]) continue;
-        const u32 i = l.uniq[r];
-        const u32 o = s_base[k] + l.off[r];
-        const u32 m = l.mask[i];
-        out[o] = m;
-        const u32 kc = num_children(m);
-        if (!kc) continue;
-        if (l.leaf) {
-            const u64* p = a.leafm + (size_t)i * 8;  // a first occurrence heads its run: its own row
-            u64 v[8];
+        const u32 r0 = (vb - s_first[k]) * kNodeThreads, r = r0 + threadIdx.x;
+        u32 o = 0, n = 0, w[17];
+        if (r < s_U[k]) {
+            const u32 i = l.uniq[r];
+            o = l.off[r];
+            w[0] = l.mask[i];
+            const u32 kc = num_children(w[0]);
+            n = node_words(w[0], l.leaf);
+            if (l.leaf) {
+                leaf_row(a.leafm + (size_t)i * 8, kc, w + 1);  // a first occurrence heads its run: its own row
+            } else if (const int c = a.child(k); c >= 0 && kc) {
+                const MLevel& lc = a.lv[c];
+                const u32 s = l.cstart[i];
+                u32 id[8];
 #pragma unroll
-            for (u32 j = 0; j < 8; ++j) v[j] = (j < kc) ? p[j] : 0ull;
+                for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(s + j, lc.n - 1) : 0u;
+                if (lc.leaf && !a.sorted) {  // (children_of)
 #pragma unroll
-            for (u32 j = 0; j < 8; ++j)
-                if (j < kc) {
-                    out[o + 1 + 2 * j] = (u32)v[j];
-                    out[o + 2 + 2 * j] = (u32)(v[j] >> 32);
+                    for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(a.heads[id[j]], lc.n - 1) : 0u;
                 }
-            continue;
+#pragma unroll
+                for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? lc.id[id[j]] : 0u;
+#pragma unroll
+                for (u32 j = 0; j < 8; ++j) w[1 + j] = (j < kc) ? s_base[c] + (u32)lc.tab[min(id[j], lc.slots - 1)] : 0u;
+            } else {
+                n = 1;
+            }
         }
-        const int c = a.child(k);
-        if (c < 0) continue;
-        const MLevel& lc = a.lv[c];
-        const u32 s = l.cstart[i];
-        u32 id[8], co[8];
-#pragma unroll
-        for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(s + j, lc.n - 1) : 0u;
-        if (lc.leaf && !a.sorted) {  // (children_of)
-#pragma unroll
-            for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? min(a.heads[id[j]], lc.n - 1) : 0u;
-        }
-#pragma unroll
-        for (u32 j = 0; j < 8; ++j) id[j] = (j < kc) ? lc.id[id[j]] : 0u;
-#pragma unroll
-        for (u32 j = 0; j < 8; ++j) co[j] = (j < kc) ? (u32)lc.tab[min(id[j], lc.slots - 1)] : 0u;
-#pragma unroll
-        for (u32 j = 0; j < 8; ++j)
-            if (j < kc) out[o + 1 + j] = s_base[c] + co[j];
+        stage_words(s_out, l.off[r0], o, n, w, out + s_base[k], total - s_base[k]);
     }
 }
 
