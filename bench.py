@@ -43,25 +43,22 @@ def pct(xs, p):
 
 
 def table_slots(n):
-    """Slots of a merge hash table for n keys: the power of two >= max(1024, n + n/2 + 1)."""
-    S = 1024
-    while S < n + n // 2 + 1:
-        S <<= 1
-    return S
+    """Slots of a merge table for n keys (build_parts.hpp's table_slots)."""
+    return max(1024, n + n // 2 + 1)
 
 
 def leaf_waves_bytes(N, nodes_leaf):
-    """Algorithmic bytes of k_leaf_waves: the 8x8 depth block of every level-3 column (256 B) and,
+    """Algorithmic bytes of the leaf kernels: the 8x8 depth block of every level-3 column (256 B) and,
     per leaf node, its breadth-first index read and its run head's index written (8 B).  The first
     node of each run also writes its mask and leafmasks; those bytes are left out, so the figure is
-    a lower bound.  The kernel also clears the leaf level's merge table (leaf_table_clear_bytes),
+    a lower bound.  The kernels also clear the merge tables (the leaf level's: leaf_table_clear_bytes),
     which is not part of the leaf computation."""
     return 256 * (N // 8) ** 2 + 8 * nodes_leaf
 
 
 def leaf_table_clear_bytes(nodes_leaf):
     """The leaf level's merge table (8 B per slot, sized for a quarter of the leaf nodes), cleared
-    at the end of k_leaf_waves."""
+    at the end of the first leaf kernel."""
     return 8 * table_slots(nodes_leaf // 4)
 
 
@@ -846,30 +843,37 @@ def main():
         log(f"    {k:18s} {ms / prof_steps:9.3f} ms/step  {cnt // prof_steps:5d} launches/step")
 
     nodes, uniq = levels
+    leaf_name = "leaf_lanes" if "leaf_lanes" in prof else "leaf_waves"
     algo = {  # algorithmic bytes per profiled step of the kernels with a closed form
-        "leaf_waves": leaf_waves_bytes(N, int(nodes[2])),
+        leaf_name: leaf_waves_bytes(N, int(nodes[2])),
         "pyr_tile_root": pyramid_root_bytes(N),
         "evaluate4": 17 * nq,
     }
 
     traffic = load_traffic(N)
 
+    # The leaf level takes two launches: smooth columns one per lane, then walls one per wave.
+    leaf_parts = [k for k in ("leaf_lanes", "leaf_waves") if k in prof]
+
     def roof(name):
         ms, cnt = prof[name]
+        if name == "leaf_lanes":
+            ms = sum(prof[k][0] for k in leaf_parts)
         per_launch_ms = ms / cnt
         bytes_per_launch = algo[name] / (cnt / prof_steps)
         ach = bytes_per_launch / (per_launch_ms * 1e-3) / 1e9
         return {"kernel": name, "bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": traffic.get(name),
+                "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": (sum(traffic[k] for k in leaf_parts if k in traffic) or None) if name == "leaf_lanes"
+                else traffic.get(name),
                 "avg_launch_us": round(per_launch_ms * 1e3, 2),
                 "bytes_per_launch": int(bytes_per_launch)}
 
-    rname = dominant[0] if dominant[0] in algo else "leaf_waves"
+    rname = dominant[0] if dominant[0] in algo else leaf_name
     roofline = roof(rname)
-    if rname == "leaf_waves":
-        # The HBM roofline is the ceiling; what holds the kernel below it is instruction issue.
-        roofline["limiter"] = ("instruction issue (SQ counters: vector units 73% and scalar units 57% busy; the "
-                               "per-column flags and wave-uniform per-run-head work), not HBM bandwidth")
+    if rname == leaf_name:
+        # The HBM roofline is the ceiling; what holds the kernels below it:
+        roofline["limiter"] = ("leaf_lanes: depth loads, then scattered stores of leafmask rows (a fifth of its time); "
+                               "leaf_waves: scattered stores of run heads; not HBM bandwidth")
         roofline["table_clear_bytes"] = leaf_table_clear_bytes(int(nodes[2]))
     pyramid_roofline = roof("pyr_tile_root")
     lookup_roofline = roof("evaluate4")
