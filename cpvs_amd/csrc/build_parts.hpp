@@ -1,8 +1,8 @@
 // build_parts.hpp -- device code shared by the single-map build (build.hip) and the forest build
-// of many maps (forest.hip): classification, leaf hashing, the merge tables and their kernels,
-// the rank and size scans' functors, the metadata layout and the word writers.
+// of many maps (forest.hip): classification, the leaf columns, leaf hashing, the merge tables, the
+// metadata layout and the staging of words.
 //
-// The subtree merge works on node indices, masks, child ranks and leafmasks only, so a forest of
+// The subtree merge works on node indices, masks, child identities and leafmasks only, so a forest of
 // many DAGs goes through the same merge kernels: its mask words carry the DAG's index in their
 // upper 16 bits (hash and key compares then never merge across DAGs, and num_children() reads
 // the low 16 bits only).
