@@ -809,8 +809,23 @@ int cpvs_container_copy_to_gpu(cpvs_container* c) {
         set_error("container_copy_to_gpu: hipMalloc failed");
         return CPVS_ENOMEM;
     }
-    // Without memory for the links the lookups walk the words.
-    c->d_links = static_cast<u64*>(ctx->buffers.take(sizeof(u64) * (total ? total : 1)));
+    // The lookups' top table (launch_build_top): K levels below the grid cell, no more than the
+    // DAGs' inner levels above the last (level 3 with leafmasks, 1 without) nor kMaxTopLevels, and
+    // within kTopTableBytes; skipped below 3 levels, where it saves little.
+    const int lead = dl - 1 - (c->dags[0]->leafmasks ? 3 : 1);
+    int K = (c->top_request < 0) ? std::min(lead, kMaxTopLevels) : std::min(c->top_request, lead);
+    if (c->top_request < 0) {
+        while (K > 0 && ((u64)cells << (3 * K)) * sizeof(u64) > kTopTableBytes) --K;
+        if (K < 3) K = 0;
+    }
+    if (K > 0 && total < 0xFFFFFFFDull) {
+        const u64 entries = (u64)cells << (3 * K);
+        if (!(c->d_top = static_cast<u64*>(ctx->buffers.take(sizeof(u64) * entries)))) {
+            set_error("container_copy_to_gpu: hipMalloc of the %llu-entry top table failed",
+                      (unsigned long long)entries);
+            return CPVS_ENOMEM;
+        }
+    }
     // combineDAGs (src/CompressedShadowContainer.cpp:52-69): concatenation in slot order, in one launch
     // with the links and the grid.
     std::vector<LinkSeg> segs(cells);
@@ -834,28 +849,15 @@ int cpvs_container_copy_to_gpu(cpvs_container* c) {
             return hip_fail(e, "container table copy", __FILE__, __LINE__);
         }
     }
+    // The links last: without memory for them the lookups walk the words.
+    c->d_links = static_cast<u64*>(ctx->buffers.take(sizeof(u64) * (total ? total : 1)));
     ProfInstall prof(ctx->prof_on ? &ctx->prof : nullptr);
     const int lrc = launch_links(d_segs, (u32)cells, segs[0], blocks, total ? (u32)total - 1 : 0u, c->d_dag, c->d_links,
                                  c->d_grid, s);
     ctx->buffers.give(d_segs);  // (queued work may still read a given buffer)
     if (lrc) return lrc;
-    // The lookups' top table (launch_build_top): K levels below the grid cell, no more than the
-    // DAGs' inner levels above the last (level 3 with leafmasks, 1 without) nor kMaxTopLevels, and
-    // within kTopTableBytes; skipped below 3 levels, where it saves little.
-    const int lead = dl - 1 - (c->dags[0]->leafmasks ? 3 : 1);
-    int K = (c->top_request < 0) ? std::min(lead, kMaxTopLevels) : std::min(c->top_request, lead);
-    if (c->top_request < 0) {
-        while (K > 0 && ((u64)cells << (3 * K)) * sizeof(u64) > kTopTableBytes) --K;
-        if (K < 3) K = 0;
-    }
-    if (K > 0 && total < 0xFFFFFFFDull) {
-        const u64 entries = (u64)cells << (3 * K);
-        if (!(c->d_top = static_cast<u64*>(ctx->buffers.take(sizeof(u64) * entries)))) {
-            set_error("container_copy_to_gpu: hipMalloc of the %llu-entry top table failed",
-                      (unsigned long long)entries);
-            return CPVS_ENOMEM;
-        }
-        int rc = launch_build_top(c->d_dag, (u32)total, c->d_grid, (u32)cells, dl, (u32)K, c->d_top, s);
+    if (c->d_top) {
+        const int rc = launch_build_top(c->d_dag, (u32)total, c->d_grid, (u32)cells, dl, (u32)K, c->d_top, s);
         if (rc) return rc;
         c->top_levels = (u32)K;
     }
