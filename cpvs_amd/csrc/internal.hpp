@@ -305,6 +305,7 @@ struct LinkSeg {
     const u32* src;
     u32 off, words, grid, block0;
 };
+constexpr size_t kLinksOneLevelBytes = size_t(2) << 20;  // (cpvs_container_copy_to_gpu)
 u32 link_blocks(u64 words);
 int launch_links(const LinkSeg* segs, u32 nseg, const LinkSeg& one, u32 blocks, u32 last, u32* dag, u64* links, u32* grid,
                  hipStream_t s);

@@ -21,6 +21,7 @@ struct GridDag {
     u32 last;  // the DAG's last word: every read is clamped to it
     u32 leaf;  // 1: leafmask nodes at level 2; 0: the DAG goes down to level 0
     u32 topk;
+    u32 nobase;  // 1: no walk needs its DAG's base, and the table's entries hold the grid's sentinels
     float lim, half;  // R - 1 and half of it, for R = 2^(dl + gl - 1) cells per axis
     int proj;         // kProjIdentity, kProjAffine or kProjFull
 };
@@ -52,6 +53,7 @@ static GridDag grid_dag(const u32* dag, const u64* links, u32 words, const u32* 
     g.last = words ? words - 1 : 0u;
     g.leaf = leaf ? 1u : 0u;
     g.topk = top ? topk : 0u;
+    g.nobase = (g.topk && (links || dl - 2 - (int)g.topk < (leaf ? 3 : 1))) ? 1u : 0u;  // (links, or no level left to walk)
     g.lim = (float)((1u << (dl + gl - 1)) - 1u);
     g.half = 0.5f * g.lim;
     g.proj = proj_kind(m);
@@ -308,7 +310,7 @@ __device__ inline u32 walk_start(const GridDag& g, u32 px, u32 py, u32 pz, Start
         cell = ((pz >> sh) * G + (py >> sh)) * G + (px >> sh);
     }
     st.base = 0;
-    if (!(g.topk && g.links)) {  // (the table's entries hold the sentinels, the links need no base)
+    if (!g.nobase) {
         st.base = g.grid[cell];
         if (st.base == 0xFFFFFFFFu) return 0u;
         if (st.base == 0xFFFFFFFEu) return 1u;
