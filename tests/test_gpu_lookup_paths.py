@@ -111,7 +111,7 @@ def test_round_robin_tiles(ctx, dags, count):
 
 
 @pytest.mark.parametrize("leafmasks", [1, 0])
-@pytest.mark.parametrize("N,length", [(8, 1), (16, 2), (64, 1), (64, 2), (128, 4), (256, 1)])
+@pytest.mark.parametrize("N,length", [(8, 1), (16, 2), (64, 1), (64, 2), (128, 4), (256, 1), (256, 4)])
 @pytest.mark.parametrize("top", [0, 1, -1])
 def test_links_of_container_dags(ctx, N, length, top, leafmasks):
     """Lookups through the container's links, over the words copied with them: cells of one word (empty
