@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 
 // the distinct ones are spread over the threads for the global inserts, and every head's key is then
 // compared with its window's first of that hash, that one's with the global slot's earlier node.  The
 // compares take four lanes to a pair of leafmask rows (16 bytes a lane): one lane to a row would touch
-// 64 lines with each load.  The rows are what the compares cost (83 MB at 8192^2: 57 -> 98 us).
+// 64 lines with each load.  The rows are what the compares cost (at 8192^2, with four nodes a thread: 57 -> 98 us).
 // What bounds it besides: the tables' atomics and coherent reads, performed at memory, about 7 G atomics/s.
 // One node a thread: where heads lie dense, a thread with several walks their reads and atomics one
 // after another (4 a thread 99 us, 16 a thread 148 us at 8192^2, one 77; 30, 18 at 2048^2).  Windows of
