@@ -849,6 +849,10 @@ int build_dag(cpvs_ctx* ctx, Arena& A, u64* pinned, int merge_mode, const cpvs_p
         else if (rc == kRetryExactCounts && !exact) exact = true;
         else break;
     }
+    // The host acts on readbacks that kernels store before the last launches end, so a build that fails
+    // here may still be writing its scratch and reading its map.  The scratch is the context's (or, for
+    // cpvs_build_noalloc, the device's) and the next call may come on another stream.
+    if (rc != CPVS_OK) (void)hipStreamSynchronize(s);
     if (rc == kRetryFullTable || rc == kRetryWithSort || rc == kRetryExactCounts) {
         set_error("build: no consistent build after every fallback (status %d)", rc);
         return CPVS_EINTERNAL;
