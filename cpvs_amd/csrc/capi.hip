@@ -614,10 +614,17 @@ int cpvs_dag_traverse(cpvs_dag* d, const float* ndc, uint64_t count, int try_lea
 }  // extern "C"
 
 namespace cpvs {
-void dag_destroy_idle(cpvs_dag* d) {
-    if (!d) return;
-    if (d->d_words) d->ctx->buffers.give_idle(d->d_words);
+// Destroys a DAG; its words, lookup tables and links go back to the cache by `give`.
+static void destroy_dag(cpvs_dag* d, void (BufferCache::*give)(void*)) {
+    BufferCache& bc = d->ctx->buffers;
+    (bc.*give)(d->d_words);
+    (bc.*give)(d->d_top);
+    (bc.*give)(d->d_links);
+    for (u64* t : d->retired_tops) (bc.*give)(t);
     delete d;
+}
+void dag_destroy_idle(cpvs_dag* d) {
+    if (d) destroy_dag(d, &BufferCache::give_idle);
 }
 }  // namespace cpvs
 
@@ -679,11 +686,7 @@ int cpvs_dag_top_levels(const cpvs_dag* d, int* levels) {
 int cpvs_dag_destroy(cpvs_dag* d) {
     if (!d) return CPVS_OK;
     hipSetDevice(d->ctx->device);
-    if (d->d_words) d->ctx->buffers.give(d->d_words);
-    if (d->d_top) d->ctx->buffers.give(d->d_top);
-    if (d->d_links) d->ctx->buffers.give(d->d_links);
-    for (u64* t : d->retired_tops) d->ctx->buffers.give(t);
-    delete d;
+    destroy_dag(d, &BufferCache::give);
     return CPVS_OK;
 }
 

@@ -253,7 +253,7 @@ struct Admit {
     void* (*alloc)(void* user, size_t bytes) = nullptr;
 };
 
-// Destroys a DAG whose words no queued work reads: its buffer is ready for reuse at once.
+// Destroys a DAG whose words and tables no queued work reads: their buffers are ready for reuse at once.
 void dag_destroy_idle(cpvs_dag* d);
 // Bytes of the stored pyramid levels of an N x N map (levels >= 3, or all with store_all).
 size_t pyramid_levels_bytes(u32 N, bool store_all);
