@@ -90,7 +90,7 @@ __device__ inline LeafCol map_column(const LeafColumns& lc, const float* depth, 
 template <bool kList>
 __global__ __launch_bounds__(64) void k_leaf_waves(LeafColumns lc, u32 ncol, const float* __restrict__ depth, u32 N, u32 T,
                                                    const float2* __restrict__ lv3, LeafOut o, u32 chunk,
-                                                   u64* __restrict__ tab, u32 tab_slots,
+                                                   u64* __restrict__ tab, u64 tab_slots,
                                                    const u32* __restrict__ col_list, const u32* __restrict__ n_list) {
     __shared__ uint8_t s_chg[128];
     const u32 b = blockIdx.x;
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(64) void k_leaf_waves(LeafColumns lc, u32 ncol, con
 template <bool kList>
 __global__ __launch_bounds__(kLaneThreads) void k_leaf_lanes(LeafColumns lc, u32 ncol, const float* __restrict__ depth, u32 N,
                                                              u32 T, LeafOut o, u32 chunk, u64* __restrict__ tab,
-                                                             u32 tab_slots, const u32* __restrict__ col_list,
+                                                             u64 tab_slots, const u32* __restrict__ col_list,
                                                              const u32* __restrict__ n_list) {
     const u32 unit = kList ? blockIdx.x : (blockIdx.x % kXcds) * chunk + blockIdx.x / kXcds;
     const u32 n = kList ? min(*n_list, ncol) : ncol, u = unit * kLaneThreads + threadIdx.x;
@@ -391,9 +391,9 @@ int deepest_level(const u64* cnt, int bottom, int R) {
 // per node.
 u32 level_slots(const u64* cnt, int L, int R, int Ls, bool use_table, bool leaf, bool small_tables) {
     if (L >= R || !cnt[L]) return 0;
-    if (!use_table) return (u32)cnt[L];
+    if (!use_table) return (u32)std::min<u64>(cnt[L], 0xFFFFFFFFull);
     if (L >= Ls) return small_slots((u32)cnt[L]);
-    return (leaf && L == 2) ? leaf_table_slots((u32)cnt[L], small_tables) : inner_table_slots((u32)cnt[L], small_tables);
+    return (leaf && L == 2) ? leaf_table_slots(cnt[L], small_tables) : inner_table_slots(cnt[L], small_tables);
 }
 u64 bound_words_of(const u64* cnt, int bottom, int R, bool leaf) {
     u64 w = 0;
@@ -573,7 +573,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         lv[L].id = A.take<u32>(c);
         lv[L].uniq = A.take<u32>(c);
         lv[L].off = A.take<u32>(c);
-        lv[L].flag = reinterpret_cast<uint8_t*>(A.take<u64>(flag_words((u32)c)));
+        lv[L].flag = reinterpret_cast<uint8_t*>(A.take<u64>(flag_words(c)));
         lv[L].slots = level_slots(cnt, L, R, Ls, use_table, leaf, small_tables);
         tab_slots += lv[L].slots;
         if (L < Ls) clear_slots += lv[L].slots;
@@ -660,7 +660,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         if (leaf && L == 2) {
             // With a column list, at most min(columns, leaf nodes) columns have nodes.
             const u32 bound = col_list ? std::min(ncol, c) : ncol;
-            const u32 slots = use_table ? (u32)clear_slots : 0u;  // the merge's tables are cleared here
+            const u64 slots = use_table ? clear_slots : 0u;  // the merge's tables are cleared here
             // (the list of slow columns lies where the identities are written later)
             const LeafOut lo{colbfs, lv[2].mask, leafm, runhead, leaf_hash, lv[2].id, meta + kMetaSlow, c};
             if (lane_leaf) {
@@ -721,8 +721,7 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     }
     ma.tile0[ma.nlev] = tile;
     // Without a leaf level its kernel did not clear the tables.
-    if (use_table && clear_slots && !(leaf && deepest == 2))
-        CPVS_LAUNCH("table_clear", k_table_clear, grid1d((u32)clear_slots), dim3(256), 0, s, tab, (u32)clear_slots);
+    if (use_table && clear_slots && !(leaf && deepest == 2)) table_clear(tab, clear_slots, s);
     for (int L = deepest; L < std::min(R, Ls); ++L) {
         if (use_table)
             merge_insert(ma, L - deepest, leaf_hash, meta,
@@ -815,23 +814,23 @@ size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_
     const int bottom = leaf ? 2 : 0;
     const int Ls = small_levels(cnt, deepest_level(cnt, bottom, R), R, use_table, leaf);
     size_t need = arena_bytes(kMetaWords, sizeof(u32)) + (leaf ? arena_bytes(ncol, sizeof(uint4)) : 0);
-    u32 cmax = 1, ntiles = 0;
-    size_t slots = 0;
+    // (64 bits throughout: estimates are asked for maps that no build takes)
+    size_t cmax = 1, ntiles = 0, slots = 0;
     for (int L = bottom; L <= R; ++L) {
         const size_t c = cnt[L] ? cnt[L] : 1;
-        if (L < R) cmax = cnt[L] > cmax ? (u32)cnt[L] : cmax;
+        if (L < R) cmax = std::max<size_t>(cmax, cnt[L]);
         const bool is_leaf = leaf && L == 2;
         need += (is_leaf ? 0 : arena_bytes(c, 8) + arena_bytes(c, 4)) + 4 * arena_bytes(c, 4) +
-                arena_bytes(flag_words((u32)c), 8);
+                arena_bytes(flag_words(c), 8);
         slots += level_slots(cnt, L, R, Ls, use_table, leaf, small_tables);
-        ntiles += ceil_div<u32>((u32)cnt[L], kTileNodes);
+        ntiles += ceil_div<size_t>(cnt[L], kTileNodes);
     }
     need += arena_bytes(slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(tile_pre_count(ntiles), 16);
     const size_t c2 = leaf ? (cnt[2] ? cnt[2] : 1) : 1;
     if (leaf) need += arena_bytes(c2 * 8, 8) + 2 * arena_bytes(c2, 4);  // leafmask rows, run heads, column map
     if (col_list) need += arena_bytes(ncol, 4) + arena_bytes(1, 4);
     if (!use_table) need += 5 * arena_bytes(cmax, 4) + arena_bytes(sort_scratch_words(cmax), 4);
-    need += arena_bytes(scan_scratch_words((leaf && ncol > cmax) ? ncol : cmax), 4);
+    need += arena_bytes(scan_scratch_words(leaf ? std::max<size_t>(ncol, cmax) : cmax), 4);
     return need + (1 << 20);
 }
 

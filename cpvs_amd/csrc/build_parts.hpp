@@ -182,10 +182,11 @@ struct EmitChildrenOut {
 // Empty slot of the merge hash tables (see table_insert).
 constexpr u64 kEmptySlot = ~0ull;
 
-// Grid-stride clear of a merge table, folded into a kernel that runs before the table is used.
-__device__ inline void clear_table(u64* tab, u32 slots) {
+// Grid-stride clear of the merge tables, folded into a kernel that runs before they are used.  A level's
+// slots fit 32 bits; those of all levels, which lie in one run, need not.
+__device__ inline void clear_table(u64* tab, u64 slots) {
     const u32 stride = gridDim.x * blockDim.x;
-    for (u32 j = blockIdx.x * blockDim.x + threadIdx.x; j < slots; j += stride) tab[j] = kEmptySlot;
+    for (u64 j = (u64)blockIdx.x * blockDim.x + threadIdx.x; j < slots; j += stride) tab[j] = kEmptySlot;
 }
 
 // Key hash of a leaf node (wave-uniform): two 32-bit multiply-xorshift streams over the low and
@@ -762,14 +763,14 @@ inline u32 table_slots(u64 n) {
 // nodes and an inner level for half.  A table found too small (maps of mostly distinct leaves, such
 // as white noise) is reported, and the build runs again with small = false.
 constexpr u32 kSmallTableMin = 1u << 20;
-inline u32 leaf_table_slots(u32 c, bool small) { return table_slots((small && c >= kSmallTableMin) ? c / 4 : c); }
+inline u32 leaf_table_slots(u64 c, bool small) { return table_slots((small && c >= kSmallTableMin) ? c / 4 : c); }
 // Small inner levels' tables are at most a quarter full: each probe is a read from memory, and where
 // every key is distinct (the upper levels of a forest, whose keys hold the DAG's index) the longest run
 // of occupied slots in a two-thirds table is tens of probes (32 maps: 3 K nodes 22.9 -> 9.9 us, 18 K
 // nodes 14.7 -> 9.5; the batch 2047 -> 2011, a server's burst 360 -> 351).
 constexpr u32 kSparseTableMax = 1u << 17;
-inline u32 inner_table_slots(u32 c, bool small) {
-    return c < kSparseTableMax ? table_slots((u64)c * 8 / 3) : table_slots((small && c >= kSmallTableMin) ? c / 2 : c);
+inline u32 inner_table_slots(u64 c, bool small) {
+    return c < kSparseTableMax ? table_slots(c * 8 / 3) : table_slots((small && c >= kSmallTableMin) ? c / 2 : c);
 }
 
 }  // namespace cpvs

@@ -240,7 +240,7 @@ __device__ inline LeafCol forest_column(const uint4* colinfo, const FItem* items
 }
 
 __global__ __launch_bounds__(64) void k_forest_waves(const uint4* __restrict__ colinfo, const FItem* __restrict__ items,
-                                                     LeafOut o, u64* __restrict__ tab, u32 tab_slots,
+                                                     LeafOut o, u64* __restrict__ tab, u64 tab_slots,
                                                      const u32* __restrict__ col_list, const u32* __restrict__ n_list,
                                                      u32 list_cap) {
     __shared__ uint8_t s_chg[128];
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(64) void k_forest_waves(const uint4* __restrict__ c
 }
 
 __global__ __launch_bounds__(kLaneThreads) void k_forest_lanes(const uint4* __restrict__ colinfo, const FItem* __restrict__ items,
-                                                               LeafOut o, u64* __restrict__ tab, u32 tab_slots,
+                                                               LeafOut o, u64* __restrict__ tab, u64 tab_slots,
                                                                const u32* __restrict__ col_list,
                                                                const u32* __restrict__ n_list, u32 list_cap) {
     const u32 n = min(*n_list, list_cap), u = blockIdx.x * kLaneThreads + threadIdx.x;
@@ -570,7 +570,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
     for (int L = Lmin; L <= Rmax; ++L) {
         const size_t c = C[L] ? C[L] : 1;
         need += (L > 2 ? arena_bytes(c, 8) + arena_bytes(c, 4) : 0) + 4 * arena_bytes(c, 4) +  // no coords, starts at leaves
-                arena_bytes(flag_words((u32)c), 8);
+                arena_bytes(flag_words(c), 8);
     }
     need += arena_bytes(tab_slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(tile_pre_count(ntiles), 16);
     need += arena_bytes(c2 * 8, 8) + 2 * arena_bytes(c2, 4);  // leafmask rows, run heads, column map
@@ -596,7 +596,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         lv.id[L] = A.take<u32>(c);
         lv.uniq[L] = A.take<u32>(c);
         lv.off[L] = A.take<u32>(c);
-        flag[L] = reinterpret_cast<uint8_t*>(A.take<u64>(flag_words((u32)c)));
+        flag[L] = reinterpret_cast<uint8_t*>(A.take<u64>(flag_words(c)));
         lv.slots[L] = slots[L];
         lv.count[L] = (u32)c;
     }
@@ -679,7 +679,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
                             nclist, bound);
             }
         } else if (use_table) {
-            CPVS_LAUNCH("table_clear", k_table_clear, grid_of(tab_slots, 256), dim3(256), 0, s, tab, (u32)tab_slots);
+            table_clear(tab, tab_slots, s);
         }
         // Bottom-up merge over every level with nodes (roots included: a root is alone in its DAG).
         MArgs ma{};

@@ -29,10 +29,7 @@ namespace cpvs {
 // chains meet share a slot; the full-key compare of a later one then sends the build down the
 // sorting path, as for equal 64-bit hashes.
 
-__global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 S) {
-    const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < S) tab[i] = kEmptySlot;
-}
+__global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u64 slots) { clear_table(tab, slots); }
 
 // The run heads of a window of kT nodes are listed in LDS; equal hashes meet in an LDS table,
 // the distinct ones are spread over the threads for the global inserts, and every head's key is then
@@ -589,6 +586,11 @@ static ChildIds children_of(const MArgs& a, int k, bool sorted) {
     const int c = a.child(k);
     if (c < 0) return ChildIds{nullptr, nullptr, 1u};
     return ChildIds{a.lv[c].id, (a.lv[c].leaf && !sorted) ? a.heads : nullptr, a.lv[c].n};
+}
+
+void table_clear(u64* tab, u64 slots, hipStream_t s) {
+    const u64 blocks = (slots + 255) / 256;
+    CPVS_LAUNCH("table_clear", k_table_clear, dim3((u32)(blocks < 65536 ? blocks : 65536)), dim3(256), 0, s, tab, slots);
 }
 
 void merge_insert(const MArgs& a, int k, const u64* hash, u32* meta, u32 hbits, hipStream_t s) {

@@ -41,8 +41,8 @@ constexpr u32 kTileNodes = kTileThreads * kTilePer;
 
 constexpr u32 kLateMax = 1u << 18;  // nodes of a level whose compares a single build leaves to merge_write
 
-inline size_t tile_pre_count(u32 tiles) { return (size_t)tiles + kMaxLevels + 1; }
-inline size_t flag_words(u32 n) { return ((size_t)n + 7) / 8; }  // 64-bit words of MLevel::flag
+inline size_t tile_pre_count(size_t tiles) { return tiles + kMaxLevels + 1; }
+inline size_t flag_words(size_t n) { return (n + 7) / 8; }  // 64-bit words of MLevel::flag
 
 // Launches.  insert_level: identities of level k of `a` by its table (a.lv[k].tab, cleared before);
 // hash: the leaf level's key hashes from the leaf kernel, or null.
@@ -60,6 +60,7 @@ void merge_finish(const MArgs& a, u32* tile_sums, ulonglong2* tile_pre, u32* met
 // the late levels' key collisions in meta (kMetaColl).
 void merge_write(const MArgs& a, u32* meta, u32* out, u64 cap, hipStream_t s);
 
-__global__ __launch_bounds__(256) void k_table_clear(u64* __restrict__ tab, u32 S);
+// Empties `slots` table slots (where no leaf kernel does).
+void table_clear(u64* tab, u64 slots, hipStream_t s);
 
 }  // namespace cpvs

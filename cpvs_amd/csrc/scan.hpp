@@ -319,7 +319,7 @@ struct ArrOutExclusive {
 // Scratch words (u32) needed by device_scan and device_scan_from_partials for n elements: one
 // 64-bit partial per one-round tile (the finest tiling any path uses) and one more.  Monotone in
 // n, so it covers every scan of at most n elements (callers size scratch for their largest scan).
-inline size_t scan_scratch_words(u32 n) { return 2 * ((size_t)ceil_div<u32>(n ? n : 1, kScanThreads) + 1); }
+inline size_t scan_scratch_words(size_t n) { return 2 * (ceil_div<size_t>(n ? n : 1, kScanThreads) + 1); }
 
 // Reduce and down-sweep with R-round tiles (at most kScanPartialsInline of them).
 template <class In, class Out, class Op, int R>
@@ -420,9 +420,9 @@ __global__ __launch_bounds__(kSortThreads) void k_radix_scatter(const u32* __res
 constexpr u32 kSmallSort = 4096;
 
 // Scratch words for radix_sort_pairs with n pairs.
-inline size_t sort_scratch_words(u32 n) {
-    const u32 nb = ceil_div<u32>(n ? n : 1, kSortTile);
-    return (size_t)256 * nb + scan_scratch_words(256 * nb);
+inline size_t sort_scratch_words(size_t n) {
+    const size_t nb = ceil_div<size_t>(n ? n : 1, kSortTile);
+    return 256 * nb + scan_scratch_words(256 * nb);
 }
 
 // Sorts keys[0..n) with values by the low `bits` bits of the key (a multiple of 8).
