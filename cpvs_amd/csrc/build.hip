@@ -308,7 +308,7 @@ __device__ inline u32 lds_insert(u64* tab, u32 S, u64 h, u32 i) {
 // then copied to the level's own.  The identities are also kept in LDS (two buffers: a level and its
 // children), where the next level's keys read them, and a level's masks and child starts are loaded
 // while the level below is inserted.
-__global__ __launch_bounds__(kSmallThreads) void k_small_insert(SmallArgs a) {
+__global__ __launch_bounds__(kSmallThreads) void k_small_insert(SmallArgs a, u32 hbits) {
     __shared__ u64 tab[kSmallSlots];
     __shared__ u32 s_id[2][kSmallMax];
     __shared__ SmallLevels lv;
@@ -348,7 +348,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_insert(SmallArgs a) {
                     for (u32 j = 0; j < 8; ++j) r[j] = (j < k) ? s_id[(L - 1) & 1][min(pc[e] + j, kSmallMax - 1)] : 0u;
                 }
             }
-            h[e] = inner_key_hash(pm[e], r);
+            h[e] = weaken_hash(inner_key_hash(pm[e], r), hbits);
         }
         if (L + 1 < a.R) load(L + 1);
         __syncthreads();  // the table is clear
@@ -729,7 +729,8 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
         else
             merge_sort_level(ma, L - deepest, srt, meta, s);
     }
-    if (Ls < R) CPVS_LAUNCH("small_insert", k_small_insert, dim3(1), dim3(kSmallThreads), 0, s, sa);
+    if (Ls < R) CPVS_LAUNCH("small_insert", k_small_insert, dim3(1), dim3(kSmallThreads), 0, s, sa,
+                             ctx->inner_hash_bits.load());
     // --- 4. first occurrences, offsets, bases, one readback, words -------------------------
     // The host reads the totals that k_totals stores in pinned memory while k_offsets runs, so the
     // words go straight to a buffer of their exact size and the GPU does not wait for the host.
