@@ -401,6 +401,14 @@ u64 bound_words_of(const u64* cnt, int bottom, int R, bool leaf) {
     return w;
 }
 
+// The nodes' cells are read for the last time by the level scans, a sort's arrays by its last level, and
+// the tables are emptied or written after that: one region holds all three.  Each with its own place, a
+// sort without leafmasks needed 20% more than the fixed scratch of cpvs_build_noalloc was sized by.
+size_t sort_bytes(size_t cmax) { return 5 * arena_bytes(cmax, 4) + arena_bytes(sort_scratch_words(cmax), 4); }
+size_t shared_bytes(size_t cell_bytes, size_t tab_slots, size_t cmax, bool use_table) {
+    return std::max({cell_bytes, arena_bytes(tab_slots, 8), use_table ? 0 : sort_bytes(cmax)});
+}
+
 constexpr int kRetryWithSort = -1000;
 constexpr int kRetryFullTable = -1001;
 constexpr int kRetryExactCounts = -1002;  // the counts exceed the emitted nodes (a map with NaN depths)
@@ -563,23 +571,32 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     Level lv[kMaxLevels];
     u32 ntiles = 0;
     size_t tab_slots = 0, clear_slots = 0;  // of all levels; of those whose tables a launch must clear
+    size_t cell_bytes = 0;
+    for (int L = bottom; L <= R; ++L) {
+        lv[L].slots = level_slots(cnt, L, R, Ls, use_table, leaf, small_tables);
+        tab_slots += lv[L].slots;
+        if (L < Ls) clear_slots += lv[L].slots;
+        if (!(leaf && L == 2)) cell_bytes += arena_bytes(cnt[L] ? cnt[L] : 1, sizeof(u64));
+    }
+    const size_t shared_cap = shared_bytes(cell_bytes, tab_slots, cmax, use_table);
+    char* const shared = A.take<char>(shared_cap);
+    Arena cells, sorting;
+    cells.base = sorting.base = shared;
+    cells.cap = sorting.cap = shared_cap;
+    u64* const tab = reinterpret_cast<u64*>(shared);
     for (int L = bottom; L <= R; ++L) {
         const size_t c = cnt[L] ? cnt[L] : 1;
         const bool is_leaf = leaf && L == 2;
         lv[L].count = (u32)cnt[L];
-        lv[L].coord = is_leaf ? nullptr : A.take<u64>(c);
+        lv[L].coord = is_leaf ? nullptr : cells.take<u64>(c);
         lv[L].mask = A.take<u32>(c);
         lv[L].cstart = is_leaf ? nullptr : A.take<u32>(c);
         lv[L].id = A.take<u32>(c);
         lv[L].uniq = A.take<u32>(c);
         lv[L].off = A.take<u32>(c);
         lv[L].flag = reinterpret_cast<uint8_t*>(A.take<u64>(flag_words(c)));
-        lv[L].slots = level_slots(cnt, L, R, Ls, use_table, leaf, small_tables);
-        tab_slots += lv[L].slots;
-        if (L < Ls) clear_slots += lv[L].slots;
         ntiles += ceil_div<u32>((u32)cnt[L], kTileNodes);
     }
-    u64* tab = A.take<u64>(tab_slots);
     {
         u64* t0 = tab;  // deepest level first: the tables to clear are one run
         for (int L = bottom; L <= R; ++L) {
@@ -600,16 +617,16 @@ int build_once(cpvs_ctx* ctx, Arena& A, u64* pinned, const cpvs_pyramid* p, u32 
     u32* nclist = col_list ? A.take<u32>(1) : nullptr;
     SortScratch srt{};
     if (!use_table) {
-        srt.skey = A.take<u32>(cmax);
-        srt.sval = A.take<u32>(cmax);
-        srt.ktmp = A.take<u32>(cmax);
-        srt.vtmp = A.take<u32>(cmax);
-        srt.seg = A.take<u32>(cmax);
-        srt.sort_scratch = A.take<u32>(sort_scratch_words(cmax));
+        srt.skey = sorting.take<u32>(cmax);
+        srt.sval = sorting.take<u32>(cmax);
+        srt.ktmp = sorting.take<u32>(cmax);
+        srt.vtmp = sorting.take<u32>(cmax);
+        srt.seg = sorting.take<u32>(cmax);
+        srt.sort_scratch = sorting.take<u32>(sort_scratch_words(cmax));
     }
     u32* scan_scratch = A.take<u32>(scan_scratch_words(scan_n));
     srt.scan_scratch = scan_scratch;
-    if (A.used > A.cap) {
+    if (A.used > A.cap || cells.used > shared_cap || sorting.used > shared_cap) {
         set_error("build: scratch layout exceeds its reservation (%zu > %zu)", A.used, A.cap);
         return CPVS_EINTERNAL;
     }
@@ -816,21 +833,21 @@ size_t build_scratch_bytes(const u64* cnt, int R, bool leaf, u32 ncol, bool col_
     const int Ls = small_levels(cnt, deepest_level(cnt, bottom, R), R, use_table, leaf);
     size_t need = arena_bytes(kMetaWords, sizeof(u32)) + (leaf ? arena_bytes(ncol, sizeof(uint4)) : 0);
     // (64 bits throughout: estimates are asked for maps that no build takes)
-    size_t cmax = 1, ntiles = 0, slots = 0;
+    size_t cmax = 1, ntiles = 0, slots = 0, cells = 0;
     for (int L = bottom; L <= R; ++L) {
         const size_t c = cnt[L] ? cnt[L] : 1;
         if (L < R) cmax = std::max<size_t>(cmax, cnt[L]);
         const bool is_leaf = leaf && L == 2;
-        need += (is_leaf ? 0 : arena_bytes(c, 8) + arena_bytes(c, 4)) + 4 * arena_bytes(c, 4) +
+        cells += is_leaf ? 0 : arena_bytes(c, 8);
+        need += (is_leaf ? 0 : arena_bytes(c, 4)) + 4 * arena_bytes(c, 4) +
                 arena_bytes(flag_words(c), 8);
         slots += level_slots(cnt, L, R, Ls, use_table, leaf, small_tables);
         ntiles += ceil_div<size_t>(cnt[L], kTileNodes);
     }
-    need += arena_bytes(slots, 8) + arena_bytes(ntiles, 4) + arena_bytes(tile_pre_count(ntiles), 16);
+    need += shared_bytes(cells, slots, cmax, use_table) + arena_bytes(ntiles, 4) + arena_bytes(tile_pre_count(ntiles), 16);
     const size_t c2 = leaf ? (cnt[2] ? cnt[2] : 1) : 1;
     if (leaf) need += arena_bytes(c2 * 8, 8) + 2 * arena_bytes(c2, 4);  // leafmask rows, run heads, column map
     if (col_list) need += arena_bytes(ncol, 4) + arena_bytes(1, 4);
-    if (!use_table) need += 5 * arena_bytes(cmax, 4) + arena_bytes(sort_scratch_words(cmax), 4);
     need += arena_bytes(scan_scratch_words(leaf ? std::max<size_t>(ncol, cmax) : cmax), 4);
     return need + (1 << 20);
 }

@@ -36,3 +36,22 @@ def test_counts_beyond_32_bits(table, per_node):
         c[2] = nodes
         need.append(scratch_bytes(c, 15, True, 8192 * 8192, table=table, small=False))
     assert need[1] - need[0] >= per_node * ((1 << 34) - (1 << 32))
+
+
+# Counts whose builds fitted the fixed scratch when one table, of the largest level's size, and one set of
+# sort arrays served all levels: without leafmasks, halving and quartering levels, next to its end.
+FITTING = [
+    ([794417, 411119, 212758, 110104, 56980, 29487, 15260, 1], False),
+    ([747276, 386278, 199672, 103213, 53352, 27578, 14255, 1], True),
+    ([962560, 329728, 93184, 25000, 6600, 1800, 450, 60, 1], False),
+    ([962560, 329728, 93184, 25000, 6600, 1800, 450, 60, 1], True),
+]
+
+
+@pytest.mark.parametrize("cnt,table", FITTING, ids=lambda v: str(v[0]) if isinstance(v, list) else ("table" if v else "sort"))
+def test_fixed_scratch_takes_what_it_took(cnt, table):
+    limit = C.CDLL(_lib.LIB_PATH).cpvs_build_noalloc_scratch_bytes
+    limit.restype = C.c_size_t
+    c = cnt + [0] * (LEVELS - len(cnt))
+    for small in (True, False):
+        assert scratch_bytes(c, len(cnt) - 1, False, table=table, small=small) <= limit()
