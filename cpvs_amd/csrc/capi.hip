@@ -658,7 +658,8 @@ int cpvs_dag_set_top_levels(cpvs_dag* d, int levels) {
         ProfInstall prof(ctx->prof_on ? &ctx->prof : nullptr);
         int rc = launch_build_top(d->d_words, (u32)d->words, nullptr, 1u, d->n, (u32)K, nt, ctx->stream);
         // (without memory for the links the lookups walk the words)
-        if (rc == CPVS_OK && !d->d_links && (nl = static_cast<u64*>(ctx->buffers.take(sizeof(u64) * d->words))))
+        if (rc == CPVS_OK && !d->d_links && links_pay(lead - K, d->words) &&
+            (nl = static_cast<u64*>(ctx->buffers.take(sizeof(u64) * d->words))))
             rc = launch_links(nullptr, 1, LinkSeg{d->d_words, 0u, (u32)d->words, 0u, 0u}, link_blocks(d->words),
                               (u32)d->words - 1, nullptr, nl, nullptr, ctx->stream);
         if (rc == CPVS_OK && hipStreamSynchronize(ctx->stream) != hipSuccess) rc = CPVS_EHIP;
@@ -852,12 +853,8 @@ int cpvs_container_copy_to_gpu(cpvs_container* c) {
             return hip_fail(e, "container table copy", __FILE__, __LINE__);
         }
     }
-    // Links pay where a walk takes two levels or more below the table; with one, only while they stay in
-    // an XCD's L2 beside the table and the words (64 DAGs of 256^2, one level, 2.8 MB of links: 3 M random
-    // lookups 22.4 us without, 23.7 with).  They are taken last: without memory for them the lookups walk
-    // the words.
-    const int left = lead - (c->d_top ? K : 0);
-    if (left >= 2 || (left == 1 && sizeof(u64) * total <= kLinksOneLevelBytes))
+    // The links are taken last: without memory for them the lookups walk the words.
+    if (links_pay(lead - (c->d_top ? K : 0), total))
         c->d_links = static_cast<u64*>(ctx->buffers.take(sizeof(u64) * (total ? total : 1)));
     ProfInstall prof(ctx->prof_on ? &ctx->prof : nullptr);
     const int lrc = launch_links(d_segs, (u32)cells, segs[0], blocks, total ? (u32)total - 1 : 0u, c->d_dag, c->d_links,

@@ -305,7 +305,13 @@ struct LinkSeg {
     const u32* src;
     u32 off, words, grid, block0;
 };
-constexpr size_t kLinksOneLevelBytes = size_t(2) << 20;  // (cpvs_container_copy_to_gpu)
+// Links pay where a walk takes two levels or more below the top table; with one, only while they stay in
+// an XCD's L2 beside the table and the words (64 DAGs of 256^2, one level, 2.8 MB of links: 3 M random
+// lookups 22.4 us without, 23.7 with); with none, nothing reads them.
+constexpr size_t kLinksOneLevelBytes = size_t(2) << 20;
+inline bool links_pay(int levels_left, u64 words) {
+    return levels_left >= 2 || (levels_left == 1 && sizeof(u64) * words <= kLinksOneLevelBytes);
+}
 u32 link_blocks(u64 words);
 int launch_links(const LinkSeg* segs, u32 nseg, const LinkSeg& one, u32 blocks, u32 last, u32* dag, u64* links, u32* grid,
                  hipStream_t s);

@@ -160,7 +160,12 @@ int cpvs_container_set_filter_size(cpvs_container *c, uint32_t size);
 /* copyToGPU (src/CompressedShadowContainer.cpp:31-46): combineDAGs (:52-69) and
  * createTopLevelGrid (:71-91) on the device.  Grid sentinels are 0xFFFFFFFF (shadow) and
  * 0xFFFFFFFE (visible), the values shader/traverse.cs:85-88 tests.  Every slot holds a DAG of the
- * same numLevels and leafmask mode (one traverse.cs walks them all). */
+ * same numLevels and leafmask mode (one traverse.cs walks them all).
+ * Device memory: 4 bytes for each word of the DAGs, the grid and the top table (below), and links,
+ * 8 bytes for each word, where lookups walk two levels or more below the table, or one and the links
+ * take at most 2 MiB.  The links are allocated last; without memory for them lookups walk the words
+ * instead (same results).  A replaced or destroyed container's buffers go to the context's cache of
+ * freed buffers (cpvs_ctx_release_scratch frees it). */
 int cpvs_container_copy_to_gpu(cpvs_container *c);
 /* No counterpart in the reference (its lookup walks every level, shader/traverse.cs:89-133).
  * copy_to_gpu also builds a top table: per grid cell, the walk's state after its first K levels,
@@ -302,7 +307,9 @@ int cpvs_dag_evaluate(const cpvs_dag *dag, const float *ndc, uint32_t stride, ui
  * cpvs_dag_evaluate, by DAG sets created after the call and by server lookups; results are the
  * same with any setting.  Built on the context stream, synchronously; call it while no lookup on
  * the DAG is queued.  A replaced table is kept until the DAG is destroyed (DAG sets created earlier
- * name it).  Its bytes are not counted in a server's budget.  top_levels reports the levels built. */
+ * name it).  The first table with levels left to walk below it also makes the DAG's links, 8 bytes for
+ * each word (as cpvs_container_copy_to_gpu), kept until the DAG is destroyed.  Neither is counted in a
+ * server's budget.  top_levels reports the levels built. */
 int cpvs_dag_set_top_levels(cpvs_dag *d, int levels);
 int cpvs_dag_top_levels(const cpvs_dag *d, int *levels);
 

@@ -61,3 +61,29 @@ def test_server_dags_give_their_tables_back(evict):
             srv.close()
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("levels,links", [(5, False), (4, True), (3, True)])
+def test_links_only_where_a_walk_reads_them(levels, links):
+    """A 256^2 DAG has 5 inner levels above the last: with all of them in the table no walk takes a link,
+    with one or two left (and links of less than 2 MiB) it does."""
+    _say("links rule", levels)
+    c = cp.Context(0)
+    try:
+        mm = cp.MinMaxHierarchy(O.gen_depth(256, SEED0 + 82, 8, True), ctx=c)
+        cs = cp.CompressedShadow.create(mm)
+        mm.close()
+        words = cs.num_words()
+        q = cp.DeviceArray.from_numpy(O.gen_queries_uniform(SEED0 + 83, 4096, 3), ctx=c)
+        want = cs.evaluate(q).numpy()
+        srv = cp.Server(serial=True, ctx=c)  # (its statistics report the cache)
+        c.release_scratch()
+        cs.setTopLevels(levels)
+        assert cs.top_levels() == levels
+        assert np.array_equal(cs.evaluate(q).numpy(), want)
+        before = srv.stats()["cached_bytes"]
+        cs.close()
+        assert srv.stats()["cached_bytes"] - before == 4 * words + 8 * 8 ** levels + (8 * words if links else 0)
+        srv.close()
+    finally:
+        c.close()
