@@ -21,7 +21,8 @@
 
 namespace cpvs {
 
-int Worker::create() {
+int Worker::create(BufferCache* cache) {
+    arena.cache = levels.cache = cache;
     CPVS_HIP_CHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&pinned), kPinnedBytes, kPinnedFlags);
     if (e != hipSuccess) {
@@ -93,7 +94,7 @@ int build_pyramid(cpvs_ctx* ctx, Worker& w, const cpvs_batch_item& it, cpvs_pyra
 int ensure_lanes(cpvs_ctx* ctx, uint32_t lanes) {
     while (ctx->lanes.size() < lanes) {
         Worker* w = new Worker();
-        const int rc = w->create();
+        const int rc = w->create(&ctx->buffers);
         if (rc) {
             delete w;
             return rc;

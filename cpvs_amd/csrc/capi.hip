@@ -75,8 +75,9 @@ int Arena::reserve(size_t bytes, hipStream_t s, bool* moved) {
         cap = 0;
     }
     size_t want = bytes + (bytes >> 3);
-    if (hipMalloc(&base, want) != hipSuccess) {
-        base = nullptr;
+    if (cache) base = static_cast<char*>(cache->new_memory(want));
+    else if (hipMalloc(&base, want) != hipSuccess) base = nullptr;
+    if (!base) {
         (void)hipGetLastError();
         set_error("scratch arena: hipMalloc of %zu bytes failed", want);
         return CPVS_ENOMEM;
@@ -111,6 +112,7 @@ int cpvs_ctx_create(int device, cpvs_ctx** out) {
     cpvs_ctx* c = new cpvs_ctx();
     c->device = device;
     c->buffers.device = device;
+    c->arena.cache = &c->buffers;
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0)
         c->num_cus = cus;
@@ -184,18 +186,21 @@ void* BufferCache::take_cached(size_t bytes, size_t limit) {
 void* BufferCache::take(size_t bytes) {
     bytes = bytes ? bytes : 1;
     if (void* p = take_cached(bytes)) return p;
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        release();  // the cached buffers may be what is missing
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-    }
+    void* p = new_memory(bytes);
+    if (!p) return nullptr;
     std::lock_guard<std::mutex> lk(mu);
     live_[p] = bytes;
     return p;
+}
+
+void* BufferCache::new_memory(size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    release();  // the cached buffers may be what is missing
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
 }
 
 void BufferCache::park(void* p, bool idle) {
@@ -1053,8 +1058,7 @@ int cpvs_container_destroy(cpvs_container* c) {
 int cpvs_device_alloc(cpvs_ctx* ctx, uint64_t bytes, void** dptr) {
     CHECK_ARG(ctx && dptr, "device_alloc: NULL argument");
     CPVS_HIP_CHECK(hipSetDevice(ctx->device));
-    if (hipMalloc(dptr, bytes ? bytes : 1) != hipSuccess) {
-        (void)hipGetLastError();
+    if (!(*dptr = ctx->buffers.new_memory(bytes ? bytes : 1))) {
         set_error("device_alloc: hipMalloc of %llu bytes failed", (unsigned long long)bytes);
         return CPVS_ENOMEM;
     }

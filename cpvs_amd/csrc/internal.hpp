@@ -25,6 +25,8 @@ constexpr uint64_t kTopTableMaxBytes = 1ull << 30;
 
 void set_error(const char* fmt, ...);
 
+struct BufferCache;
+
 // Bump allocator over one device buffer, reset per build.  Grows (after a stream sync) when a
 // build needs more than it holds.
 struct Arena {
@@ -32,6 +34,7 @@ struct Arena {
     size_t cap = 0;
     size_t used = 0;
     bool fixed = false;  // a caller's buffer of `cap` bytes: never grown (reserve fails beyond it)
+    BufferCache* cache = nullptr;  // the context's, emptied before a growth fails for want of memory
     // Ensure capacity and reset `used`; *moved (optional) tells whether the buffer was reallocated
     // (its contents are then lost).
     int reserve(size_t bytes, hipStream_t s, bool* moved = nullptr);
@@ -71,7 +74,7 @@ struct Worker {
     };
     Staging forest;    // a forest's count partials, tables and readback
     Staging pyramids;  // its pyramids' records
-    int create();  // on the current device
+    int create(BufferCache* cache);  // on the current device; cache: the context's
     void destroy();
     int staging(Staging& st, size_t bytes);  // ensures st holds bytes (waits for the stream before it replaces it)
 };
@@ -119,6 +122,8 @@ struct BufferCache {
     uint64_t device_syncs = 0, trims = 0;
     int device = 0;
     void* take(size_t bytes);            // nullptr when hipMalloc fails (even after emptying the cache)
+    // hipMalloc, tried again with the cache emptied when memory is short; nullptr on failure.
+    void* new_memory(size_t bytes);
     // A cached buffer of at most min(2 * bytes, limit) bytes, or nullptr; never allocates.
     void* take_cached(size_t bytes, size_t limit = ~size_t(0));
     void give(void* p);                  // p from take(); null is ignored

@@ -384,7 +384,7 @@ int cpvs_server_create(cpvs_ctx* ctx, uint32_t lanes, uint64_t hbm_budget_bytes,
     int rc = CPVS_OK;
     for (uint32_t i = 0; i < nl && rc == CPVS_OK; ++i) {
         Worker* w = new Worker();
-        rc = w->create();
+        rc = w->create(&ctx->buffers);
         if (rc) delete w;
         else s->lanes.push_back(w);
     }
@@ -394,7 +394,7 @@ int cpvs_server_create(cpvs_ctx* ctx, uint32_t lanes, uint64_t hbm_budget_bytes,
             s->lk = s->lanes[0];
         } else {
             s->lk = new Worker();
-            rc = s->lk->create();
+            rc = s->lk->create(&ctx->buffers);
             if (rc) {
                 delete s->lk;
                 s->lk = nullptr;
