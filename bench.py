@@ -51,15 +51,28 @@ def leaf_waves_bytes(N, nodes_leaf):
     """Algorithmic bytes of the leaf kernels: the 8x8 depth block of every level-3 column (256 B) and,
     per leaf node, its breadth-first index read and its run head's index written (8 B).  The first
     node of each run also writes its mask and leafmasks; those bytes are left out, so the figure is
-    a lower bound.  The kernels also clear the merge tables (the leaf level's: leaf_table_clear_bytes),
-    which is not part of the leaf computation."""
+    a lower bound.  The kernels also clear the merge tables (cleared_table_bytes), which is not part of
+    the leaf computation."""
     return 256 * (N // 8) ** 2 + 8 * nodes_leaf
 
 
-def leaf_table_clear_bytes(nodes_leaf):
-    """The leaf level's merge table (8 B per slot, sized for a quarter of the leaf nodes), cleared
-    at the end of the first leaf kernel."""
-    return 8 * table_slots(nodes_leaf // 4)
+def cleared_table_bytes(nodes):
+    """The merge tables cleared at the end of the first leaf kernel (8 B per slot): those of the levels
+    below the first with more than 4096 nodes from the root down, by build_parts.hpp's size rules (a
+    quarter of the leaves and half of the inner nodes from 2^20 on, inner tables below 2^17 nodes at most
+    a quarter full).  nodes: per octree level, leaves at level 2."""
+    levels = [int(c) for c in nodes]
+    top = max(L for L, c in enumerate(levels) if c)
+    while top >= 3 and levels[top] <= 4096:
+        top -= 1
+    slots = 0
+    for L in range(2, top + 1):
+        c = levels[L]
+        if L == 2:
+            slots += table_slots(c // 4 if c >= 1 << 20 else c)
+        else:
+            slots += table_slots(c * 8 // 3 if c < 1 << 17 else c // 2 if c >= 1 << 20 else c)
+    return 8 * slots
 
 
 def host_cpu():
@@ -178,8 +191,7 @@ def run_tiled(cp, np, ctx, full=65536, tile=8192, boxes=16384, nq=1 << 26, batch
     cands = [cp.batch_config(lanes=batch_lanes, forest_mtexels=0)] + \
         [cp.batch_config(lanes=ln, forest_mtexels=mt) for ln in (1, 2, 4) for mt in (64, 256, 512, 1024)] + \
         [cp.batch_config(lanes=ln, forest_mtexels=mt) for ln in (6, 8) for mt in (128, 256, 512)] + \
-        [cp.batch_config(lanes=2, forest_mtexels=64, leaf_cols=4), cp.batch_config(lanes=2, forest_mtexels=64, graph=True),
-         cp.batch_config(lanes=4, forest_mtexels=256, leaf_waves=2), cp.batch_config(lanes=3, forest_mtexels=256)]
+        [cp.batch_config(lanes=2, forest_mtexels=64, graph=True), cp.batch_config(lanes=3, forest_mtexels=256)]
     best, tune_ms = cp.tune_batch_config(bd, cands, bt)
     cfg = cands[best]
     log(f"[bench] tiled: tuner picked {cfg.as_dict()} ({[round(m, 1) for m in tune_ms]} ms)")
@@ -320,14 +332,13 @@ def run_batched(cp, np, ctx, maps=256, kmin=8, kmax=13, qper=1 << 20, reps=3):
         return out, list(done), time.perf_counter() - t0
 
     # warm-up of the plain path (arena sizing), then the autotuner picks the batch configuration:
-    # forests (many maps through one launch chain) of several sizes on 1-4 lanes, leaf kernel
-    # shapes, hipGraph capture, and one map per launch chain on 4 or 8 lanes.
+    # forests (many maps through one launch chain) of several sizes on 1-4 lanes, hipGraph capture,
+    # and one map per launch chain on 4 or 8 lanes.
     for sh in plain_once()[0]:
         sh.close()
     cands = [cp.batch_config(lanes=ln, forest_mtexels=0) for ln in (4, 8)] + \
         [cp.batch_config(lanes=ln, forest_mtexels=mt) for ln in (1, 2, 4) for mt in (64, 256, 1024)] + \
-        [cp.batch_config(lanes=2, forest_mtexels=256, leaf_cols=4), cp.batch_config(lanes=2, forest_mtexels=256, leaf_waves=2),
-         cp.batch_config(lanes=2, forest_mtexels=256, graph=True)]
+        [cp.batch_config(lanes=2, forest_mtexels=256, graph=True)]
     bi, tms = cp.tune_batch_config(depths, cands)
     best = cands[bi].as_dict()
     tune_ms = {json.dumps(c.as_dict(), sort_keys=True): m for c, m in zip(cands, tms)}
@@ -874,7 +885,7 @@ def main():
         # The HBM roofline is the ceiling; what holds the kernels below it:
         roofline["limiter"] = ("leaf_lanes: depth loads, then scattered stores of leafmask rows (a fifth of its time); "
                                "leaf_waves: scattered stores of run heads; not HBM bandwidth")
-        roofline["table_clear_bytes"] = leaf_table_clear_bytes(int(nodes[2]))
+        roofline["table_clear_bytes"] = cleared_table_bytes(nodes)
     pyramid_roofline = roof("pyr_tile_root")
     lookup_roofline = roof("evaluate4")
     # Dependent gathers from a cache-resident DAG: set by load throughput and L2 locality, not HBM.
