@@ -152,6 +152,15 @@ void* fit_from(std::multimap<size_t, void*>& m, size_t bytes, size_t most, size_
     m.erase(it);
     return p;
 }
+// Waits for everything queued on the current device; false if that failed.  hipFree synchronises the
+// device as hipDeviceSynchronize does (1 us more), but that call fails, and invalidates the capture, while
+// any stream of the process captures a graph: another lane of a batch with graph = 1, or a caller's.
+bool wait_for_device() {
+    void* p = nullptr;
+    if (hipMalloc(&p, 1) == hipSuccess && hipFree(p) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
 }  // namespace
 
 void* BufferCache::take_cached(size_t bytes, size_t limit) {
@@ -170,11 +179,13 @@ void* BufferCache::take_cached(size_t bytes, size_t limit) {
             pending_bytes = 0;
             lk.unlock();
             (void)hipSetDevice(device);
-            (void)hipDeviceSynchronize();
+            const bool idle = wait_for_device();
             lk.lock();
             ++device_syncs;
-            free_.insert(parked.begin(), parked.end());
-            p = fit_from(free_, bytes, most, &got);
+            (idle ? free_ : pending_).insert(parked.begin(), parked.end());
+            if (idle) p = fit_from(free_, bytes, most, &got);
+            else
+                for (auto& kv : parked) pending_bytes += kv.first;
         }
     }
     if (!p) return nullptr;

@@ -102,7 +102,7 @@ namespace cpvs {
 // for the device).
 // A freed buffer may still be read by work queued on any stream, so give() parks it as pending
 // and the free itself waits for nothing.  A pending buffer is handed out again only after a
-// device synchronisation that follows its free: take() performs one when no ready buffer fits, a
+// device synchronisation that follows its free (wait_for_device): take() performs one when no ready buffer fits, a
 // pending one would and kPendingBytes are pending, which readies every pending buffer at once.
 // Below that it allocates: a synchronisation costs about 9 us and the overlap of everything queued, a
 // hipMalloc 0.4 us (1 MB) to 14 us (16 MB), and a program that frees and rebuilds then pays one
