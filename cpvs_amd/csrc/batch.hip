@@ -2,8 +2,8 @@
 // (many DAGs queried in one launch).
 //
 // The reference builds maps one after another (src/DeferredRenderer.cpp:150-187, one
-// CompressedShadow::create per tile and z-tile).  One build is a chain of ~60 short launches
-// with three host readbacks; small maps leave the GPU idle between them.  A batch runs L lanes,
+// CompressedShadow::create per tile and z-tile).  One build is a chain of 12 to 33 short
+// launches with two host readbacks; small maps leave the GPU idle between them.  A batch runs L lanes,
 // each a host thread with its own stream, scratch arena, pyramid-level arena and pinned staging,
 // pulling maps from one queue in decreasing size (so a lane's arenas grow on its first map and
 // are reused after).  Every map goes through the same kernels as cpvs_build, so the DAG words

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void k_classify(const u64* __restrict__ coord,
 // * A run head's leafmasks go to the row at its own breadth-first index (8 slots per node), so the
 //   leaf insert, the key compares and the write find them at the node's index, with no slot map.
 // Measured at 8192^2 (1 M columns, 6.7 M nodes): 8 columns per wave for all, bound by instruction issue
-// (vector units 73% busy, scalar 57%), 210 us; lanes 96 us and waves 35 us (49 before list_share) for the rest, whose
+// (vector units 73% busy, scalar 57%), 210 us; lanes 103 us and waves 34 us (49 before list_share) for the rest, whose
 // columns hold most of the nodes (2, 4 and 8 of them in turn per wave took 51, 63 and 77 us: a wave
 // waits for each column's chunks).  Small maps are all latency: 256^2 13 -> 4 us and 1024^2
 // 17 -> 9 us with one column per wave instead of 8.

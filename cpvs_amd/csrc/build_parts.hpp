@@ -548,6 +548,8 @@ __device__ inline void load_child_ids(const ChildIds& c, u32 s, u32 k, u32 r[8])
 // differences' sum mod 2^64, then a mixer that is a bijection.  Two 32-bit multiplies per child
 // instead of a chain of two 64-bit ones: in the one-workgroup merge of the small levels, four waves
 // per SIMD hash four nodes per thread and level, and a chain's multiplies alone were much of its time.
+// The constants are published ones with well spread bits: splitmix64's increment (2^64 over the golden
+// ratio), two of xxHash64's primes, the rrmxmx mixer's multiplier and wyhash's default secrets.
 __device__ inline u64 inner_key_hash(u32 m, const u32 (&r)[8]) {
     constexpr u64 kMul[9] = {0x9E3779B97F4A7C15ull, 0xC2B2AE3D27D4EB4Full, 0x165667B19E3779F9ull, 0xD6E8FEB86659FD93ull,
                              0xA0761D6478BD642Full, 0xE7037ED1A0B428DBull, 0x8EBC6AF09C88C6E3ull, 0x589965CC75374CC3ull,

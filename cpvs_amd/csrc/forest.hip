@@ -2,8 +2,8 @@
 //
 // The reference builds one DAG after another (src/DeferredRenderer.cpp:150-187: every z-tile of
 // every tile, each create() a separate pass over its own vectors).  One build here is a chain of
-// about 60 launches and three host readbacks; a small map keeps the GPU busy for only a few of
-// them.  A forest builds M DAGs (maps of any sizes, and z-tiles of one map sharing its pyramid)
+// 12 (256^2) to 33 (8192^2) launches with two host readbacks; a small map keeps the GPU busy for only a
+// few of them.  A forest builds M DAGs (maps of any sizes, and z-tiles of one map sharing its pyramid)
 // with the launches of one build:
 //   * every octree level L is one array over all DAGs, DAG-major: DAG f's level-L nodes form one
 //     segment, in its own breadth-first order.  DAGs are ordered by root level, highest first; a

@@ -2,9 +2,10 @@
 // src/CompressedShadowContainer.cpp:93-124) and CompressedShadow::traverse
 // (src/CompressedShadow.cpp:404-463).
 //
-// One thread per query.  The walk is a chain of dependent 4-byte loads, one per level; the
-// upper levels are shared by every query and stay in L2, so throughput is set by how many
-// walks are in flight and by the locality of neighbouring queries.  The image entry point
+// One thread per query.  A walk reads an entry of the top table, where there is one, for its first levels
+// and then one 8-byte link a level (k_links), each depending on the last; without links, two dependent
+// 4-byte words a level.  The upper levels are shared by every query and stay in L2, so throughput is set by how
+// many walks are in flight and by the locality of neighbouring queries.  The image entry point
 // gives each wave an 8x8 pixel tile so neighbouring lanes follow the same DAG paths.
 // Compiled with -ffp-contract=off: the matrix product, the divide and the quantisation round
 // exactly as written, as the reference's float expressions do.
