@@ -153,8 +153,9 @@ void* fit_from(std::multimap<size_t, void*>& m, size_t bytes, size_t most, size_
     return p;
 }
 // Waits for everything queued on the current device; false if that failed.  hipFree synchronises the
-// device as hipDeviceSynchronize does (1 us more), but that call fails, and invalidates the capture, while
-// any stream of the process captures a graph: another lane of a batch with graph = 1, or a caller's.
+// device as hipDeviceSynchronize does, if more slowly (32-36 us against 18-24 beside a few launches), but that
+// call fails, and invalidates the capture, while any stream of the process captures a graph: another
+// lane of a batch with graph = 1, or a caller's.
 bool wait_for_device() {
     void* p = nullptr;
     if (hipMalloc(&p, 1) == hipSuccess && hipFree(p) == hipSuccess) return true;

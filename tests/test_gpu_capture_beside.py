@@ -19,12 +19,13 @@ def test_reused_buffers_leave_a_capture_alone():
     c = cp.Context(0)
     other = cp.Context(0)  # its stream is captured
     try:
-        N = 4096
+        N = 8192
         img = cp.gen_depth(N, 0x43505653 + 5, 512, True, ctx=c)
         small = cp.DeviceArray((64,), np.uint32, ctx=other)
-        mm = cp.MinMaxHierarchy(img, ctx=c)
-        want = mm.getLevel(5)
-        mm.close()  # 64 MiB of depth and its levels are pending
+        two = [cp.MinMaxHierarchy(img, ctx=c) for _ in range(2)]
+        want = two[0].getLevel(5)
+        for mm in two:
+            mm.close()  # 256 MiB of depth and its levels each: enough pending for the cache to wait
         begun, done, rc = threading.Event(), threading.Event(), {}
 
         def capture():
