@@ -55,6 +55,8 @@ void Worker::destroy() {
     }
     if (pinned) (void)hipHostFree(pinned);
     if (stream) (void)hipStreamDestroy(stream);
+    if (capture) (void)hipStreamDestroy(capture);
+    capture = nullptr;
     pinned = nullptr;
     stream = nullptr;
 }

@@ -637,10 +637,7 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
     CPVS_HIP_CHECK(hipMemcpyAsync(nxt, st.nxt, sizeof(u32) * M * kKL, hipMemcpyHostToDevice, s));
 
     // --- the level chain (optionally captured) ----------------------------------------------------
-    hipGraph_t graph = nullptr;
-    const bool capture = o.graph && !t_prof;  // per-kernel timing records events: launch directly then
-    if (capture) CPVS_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    {
+    auto chain = [&](hipStream_t s) {
         if (ncol)
             device_scan(ColPairIn{colinfo}, ColListOut{colinfo, clist, nclist, (u32)ncol}, (u32)ncol, OpSum64{}, nullptr,
                         scan_scratch, s);
@@ -711,20 +708,38 @@ int forest_once(cpvs_ctx* ctx, Worker& w, const ForestIn* in, u32 M, const Fores
         ho.uniq = ho.root + M;
         CPVS_LAUNCH("forest_bases", k_forest_bases, grid_of(M, 256), dim3(256), 0, s, items, M, lv, seg, nxt, boff, B, meta,
                     Lmin, ho);
+    };
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    if (o.graph && !t_prof) {  // (per-kernel timing records events: launch directly then)
+        // Any thread of the process that synchronises the device or copies on the null stream meanwhile
+        // invalidates the capture, and the stream stays unusable: so the capture has a stream of its own,
+        // which is replaced then, and the chain, of which nothing was launched, is launched directly.
+        hipError_t ec = w.capture ? hipSuccess : hipStreamCreateWithFlags(&w.capture, hipStreamNonBlocking);
+        if (ec == hipSuccess) ec = hipStreamBeginCapture(w.capture, hipStreamCaptureModeThreadLocal);
+        if (ec == hipSuccess) {
+            chain(w.capture);
+            ec = hipStreamEndCapture(w.capture, &graph);
+        }
+        if (ec == hipSuccess) ec = hipGetLastError();
+        if (ec == hipSuccess) ec = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        if (ec != hipSuccess) {
+            exec = nullptr;
+            if (w.capture) (void)hipStreamDestroy(w.capture);
+            w.capture = nullptr;
+            (void)hipGetLastError();
+        }
     }
-    hipError_t e = hipGetLastError();
-    if (capture) {
-        const hipError_t ec = hipStreamEndCapture(s, &graph);
-        if (e == hipSuccess) e = ec;
-        hipGraphExec_t exec = nullptr;
-        if (e == hipSuccess) e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        if (e == hipSuccess) e = hipGraphLaunch(exec, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (exec) (void)hipGraphExecDestroy(exec);
-        if (graph) (void)hipGraphDestroy(graph);
-    } else if (e == hipSuccess) {
-        e = hipStreamSynchronize(s);
+    hipError_t e = hipSuccess;
+    if (exec) {
+        e = hipGraphLaunch(exec, s);
+    } else {
+        chain(s);
+        e = hipGetLastError();
     }
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (exec) (void)hipGraphExecDestroy(exec);
+    if (graph) (void)hipGraphDestroy(graph);
     if (e != hipSuccess) return hip_fail(e, "forest level chain", __FILE__, __LINE__);
 
     const u32* hm = st.back;

@@ -65,6 +65,7 @@ constexpr unsigned kPinnedFlags = hipHostMallocCoherent | hipHostMallocMapped;
 // pinned readback staging.  Lanes run concurrently from their own host threads.
 struct Worker {
     hipStream_t stream = nullptr;
+    hipStream_t capture = nullptr;  // forests' graphs are captured on it (made when first needed)
     Arena arena;   // build scratch
     Arena levels;  // pyramid levels of the item being built (of all maps of a forest)
     u64* pinned = nullptr;
@@ -104,16 +105,16 @@ namespace cpvs {
 // and the free itself waits for nothing.  A pending buffer is handed out again only after a
 // wait for the device (wait_for_device) that follows its free: take() performs one when no ready buffer
 // fits, a pending one would, and kPendingBytes or kPendingCount buffers are pending; it readies every
-// pending buffer at once.  Below that it allocates, 0.4 us (1 MB) to 14 us (16 MB) until the program's
-// buffers go round.  A wait costs 30 us and, with hundreds of launches since the last one, up to 210, and
-// the overlap of everything queued: 8192^2 builds take 672, 658 and 647 us with 64, 256 and 512 MB, 256^2
-// ones 107 and 101 with 32 and 256 buffers.  give_idle() is for buffers
+// pending buffer at once.
+// Below that it allocates: a wait costs about 9 us and the overlap of everything queued, a
+// hipMalloc 0.4 us (1 MB) to 14 us (16 MB), and a program that frees and rebuilds then pays one
+// wait for several builds.  give_idle() is for buffers
 // the caller knows no queued work reads (a server's evicted DAG: no lookup pins it, its build has
 // completed); they are ready at once.
 struct BufferCache {
     static constexpr size_t kMaxBytes = size_t(2) << 30;
-    static constexpr size_t kPendingBytes = size_t(512) << 20;
-    static constexpr size_t kPendingCount = 256;
+    static constexpr size_t kPendingBytes = size_t(64) << 20;
+    static constexpr size_t kPendingCount = 32;
     std::mutex mu;
     std::multimap<size_t, void*> free_;     // size -> ready buffer
     std::multimap<size_t, void*> pending_;  // size -> freed buffer not yet known idle

@@ -264,7 +264,9 @@ int cpvs_tune_batch(cpvs_ctx *ctx, const cpvs_batch_item *items, uint32_t count,
  * zTileNum per item; the z-tiles of one map stay in one forest and share its pyramid), `lanes`
  * forests at once.  leaf_cols (4 or 8) and leaf_waves (1 or 2) are accepted and checked but change
  * nothing any more: the leaf kernels take their shape from the number of columns.  graph = 1 captures
- * each forest's level chain in a hipGraph and launches it as one.  Words are identical to
+ * each forest's level chain in a hipGraph and launches it as one; a capture that another thread's device
+ * synchronisation or copy on the null stream invalidates is launched directly (HIP refuses that thread's
+ * call too: copy results, with cpvs_dag_copy_words and the like, after the batch).  Words are identical to
  * cpvs_build's in every configuration.
  * Maps with N < 16 (no leafmask levels) are built one by one. */
 typedef struct cpvs_batch_config {

@@ -1,5 +1,6 @@
-"""Calls on one thread while another thread captures a graph on a stream of its own: the buffer cache's wait
-for the device must not invalidate the capture, as hipDeviceSynchronize does.  Needs a GPU."""
+"""Graph captures beside other work.  A device synchronisation on any thread invalidates every capture of the
+process, and fails itself without waiting: a batch's lanes must get by without their graph, and the
+buffer cache must not take the failed wait for done.  Needs a GPU."""
 import ctypes as C
 import threading
 
@@ -7,49 +8,99 @@ import numpy as np
 import pytest
 
 import cpvs_amd as cp
-import oracle as O
 
 pytestmark = pytest.mark.gpu
+SEED0 = 0x43505653
 THREAD_LOCAL = 1  # hipStreamCaptureModeThreadLocal, as a batch's lanes capture
 
 
-def test_reused_buffers_leave_a_capture_alone():
-    print("[case] buffers reused beside a capture", flush=True)
+@pytest.mark.parametrize("lanes", [1, 4])
+def test_graph_forests_beside_device_synchronisations(lanes):
+    print("[case] graph forests beside synchronisations", lanes, flush=True)
     hip = C.CDLL("libamdhip64.so")
     c = cp.Context(0)
-    other = cp.Context(0)  # its stream is captured
     try:
-        N = 8192
-        img = cp.gen_depth(N, 0x43505653 + 5, 512, True, ctx=c)
-        small = cp.DeviceArray((64,), np.uint32, ctx=other)
-        two = [cp.MinMaxHierarchy(img, ctx=c) for _ in range(2)]
-        want = two[0].getLevel(5)
-        for mm in two:
-            mm.close()  # 256 MiB of depth and its levels each: enough pending for the cache to wait
+        maps = [cp.gen_depth(N, SEED0 + 400 + i, max(1, 32 * N * N >> 20), True, ctx=c)
+                for i, N in enumerate([256, 512, 1024] * 4)]
+        plain = []
+        for d in maps:
+            cs = cp.CompressedShadow.create(cp.MinMaxHierarchy(d, ctx=c))
+            plain.append(cs.getDAG())
+            cs.close()
+        stop = threading.Event()
+
+        def sync():
+            while not stop.is_set():
+                hip.hipDeviceSynchronize()
+
+        t = threading.Thread(target=sync)
+        t.start()
+        built = []
+        try:
+            for _ in range(6):
+                built.append(cp.build_batch(maps, ctx=c,
+                                            config=cp.batch_config(lanes=lanes, forest_mtexels=1, graph=True))[0])
+        finally:
+            stop.set()
+            t.join(60)
+        for shadows in built:
+            for w, sh in zip(plain, shadows):
+                assert np.array_equal(sh.getDAG(), w)
+    finally:
+        c.close()
+
+
+def test_reused_buffers_wait_beside_a_capture():
+    """Lookups on a stream of their own read a container that is destroyed; the next pyramid's depth is
+    copied to a buffer of its size while a third stream, not the library's, is being captured."""
+    print("[case] buffers reused beside a capture", flush=True)
+    hip = C.CDLL("libamdhip64.so")
+    c, reader = cp.Context(0), cp.Context(0)  # (a stream each)
+    try:
+        big = cp.gen_depth(8192, SEED0 + 5, 512, True, ctx=c)
+        img = cp.gen_depth(2048, SEED0 + 6, 128, True, ctx=c)
+        q = cp.gen_queries_uniform(SEED0 + 7, 1 << 20, 4, ctx=c)
+        mm = cp.MinMaxHierarchy(big, borrow=True, ctx=c)
+        k = cp.CompressedShadowContainer(cp.CompressedShadow.create(mm))
+        k.setFilterSize(64)
+        k.copyToGPU()
+        vis = [cp.DeviceArray((1 << 20,), np.float32, ctx=c) for _ in range(2)]
+        k.evaluate_pcf(q, None, vis[0])
+        c.synchronize()
+        want = vis[0].numpy()
+        fill = cp.MinMaxHierarchy(cp.gen_depth(4096, SEED0 + 8, 512, True, ctx=c), ctx=c)
+        c.release_scratch()  # nothing ready: the next depth takes a pending buffer or new memory
+        fill.close()  # more than 64 MiB pending
         begun, done, rc = threading.Event(), threading.Event(), {}
 
         def capture():
-            rc["begin"] = hip.hipStreamBeginCapture(other.stream, THREAD_LOCAL)
+            s = C.c_void_p()
+            rc["create"] = hip.hipStreamCreateWithFlags(C.byref(s), 1)
+            rc["begin"] = hip.hipStreamBeginCapture(s, THREAD_LOCAL)
             begun.set()
             done.wait(60)
-            rc["copy"] = hip.hipMemcpyAsync(small.ptr, C.c_void_p(small.ptr.value + 128), C.c_size_t(128), 3, other.stream)
             g = C.c_void_p()
-            rc["end"] = hip.hipStreamEndCapture(other.stream, C.byref(g))
+            hip.hipStreamEndCapture(s, C.byref(g))  # (invalid by then, and the stream with it)
             if g:
                 hip.hipGraphDestroy(g)
+            hip.hipStreamDestroy(s)
             hip.hipGetLastError()
 
         t = threading.Thread(target=capture)
         t.start()
         try:
             assert begun.wait(60)
-            mm = cp.MinMaxHierarchy(img, ctx=c)  # takes the freed buffers, which needs the device idle
+            for _ in range(20):
+                k.evaluate_pcf(q, None, vis[1], stream=reader.stream)
+            k.close()
+            one = cp.MinMaxHierarchy(img, ctx=c)  # 16 MiB, the container's words' and links' sizes
         finally:
             done.set()
             t.join(60)
-        assert np.array_equal(mm.getLevel(5), want)
-        mm.close()
-        assert rc == {"begin": 0, "copy": 0, "end": 0}
+        reader.synchronize()
+        assert rc == {"create": 0, "begin": 0}
+        assert np.array_equal(vis[1].numpy(), want)
+        assert np.array_equal(one.getLevel(0), img.numpy())
     finally:
-        c.close()
-        other.close()
+        for x in (c, reader):
+            x.close()
